@@ -784,20 +784,23 @@ inline int compute_units() {
 // items of one row block x one span of tiles.  Two things are weighed: the rounds of 256 workgroups
 // the items make, and the L2 traffic of the 32 workgroups that run on one XCD at a time, which cover
 // 32 / s row blocks (one E block each) times s spans (one stream of C tiles each): s + 32 / s streams,
-// least for s = 4 .. 8.  The weight 0.165 is fitted to measurements at E [65536, 3584] x C [152064, 3584]
-// (1, 2, 4, 8, 16 spans: 70.8, 62.5, 53.9, 56.8, 59.4 ms).
+// least for s = 4 .. 8, and 32 + 1 for any s beyond 32.  The weight 0.165 is fitted to measurements at
+// E [65536, 3584] x C [152064, 3584] (1, 2, 4, 8, 16 spans: 70.8, 62.5, 53.9, 56.8, 59.4 ms).
+// Up to 64 spans are weighed, and as many as fill the chip where the row blocks are fewer than that takes: one row
+// block against 256000 classes of 2304 columns is 847 us in 64 spans (a quarter of the compute units) and 262 us in 250 (4.5 TB/s).
 inline int choose_span_count(int nrb, int nvt) {
   const int num_cu = compute_units();  // (the size query and the launch must see the same device)
   int best = 1;
   double best_cost = 1e300;
-  const int max_split = nvt < 64 ? nvt : 64;
+  const int most = num_cu / nrb > 64 ? num_cu / nrb : 64;
+  const int max_split = nvt < most ? nvt : most;
   for (int s = 1; s <= max_split; ++s) {
     const int64_t items = static_cast<int64_t>(nrb) * s;
     const int64_t rounds = (items + num_cu - 1) / num_cu;
     const int tiles_per_item = (nvt + s - 1) / s;
-    const double streams = (s <= 32) ? s + 32.0 / s : s + 1.0;
+    const double streams = (s <= 32) ? s + 32.0 / s : 33.0;
     const double traffic = 1.0 + 0.165 * (streams / 11.3137 - 1.0);
-    const double cost = static_cast<double>(rounds) * tiles_per_item * traffic + 0.02 * s;
+    const double cost = static_cast<double>(rounds) * tiles_per_item * traffic + 0.002 * s;
     if (cost < best_cost - 1e-9) {
       best_cost = cost;
       best = s;

@@ -602,18 +602,32 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   }
 }
 
-// lse[i] = ln(2) * (M + log2(sum_s sum_s * 2^(m_s - M))),  M = max_s m_s
-__global__ void lse_merge_kernel(const float2* partial, float* lse, int64_t b, int nsplit) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= b) return;
-  float m = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) m = fmaxf(m, partial[static_cast<int64_t>(s) * b + i].x);
-  float acc = 0.0f;
-  for (int s = 0; s < nsplit; ++s) {
-    const float2 ps = partial[static_cast<int64_t>(s) * b + i];
-    acc += ps.y * exp2f(ps.x - m);
+// lse[i] = ln(2) * (M + log2(sum_s sum_s * 2^(m_s - M))),  M = max_s m_s.  A workgroup merges 16 rows with 16 threads
+// each: the spans of a row are read in parallel (a row block with few neighbours has up to 256 of them, and one thread
+// per row took 25 us over 64), 16 neighbouring rows are one 128-byte line.
+constexpr int kMergeRows = 16, kMergeParts = 16;
+__global__ __launch_bounds__(kMergeRows * kMergeParts) void lse_merge_kernel(const float2* partial, float* lse, int64_t b,
+                                                                              int nsplit) {
+  __shared__ float2 s_part[kMergeParts][kMergeRows];
+  const int r = threadIdx.x % kMergeRows;
+  const int part = threadIdx.x / kMergeRows;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kMergeRows + r;
+  auto merge = [](float2 x, float2 y) {
+    const float m = fmaxf(x.x, y.x);
+    const float ms = (m == -INFINITY) ? 0.0f : m;
+    return make_float2(m, x.y * exp2f(x.x - ms) + y.y * exp2f(y.x - ms));
+  };
+  float2 acc = make_float2(-INFINITY, 0.0f);
+  if (i < b) {
+    for (int s = part; s < nsplit; s += kMergeParts) acc = merge(acc, partial[static_cast<int64_t>(s) * b + i]);
   }
-  lse[i] = (m + log2f(acc)) * kLn2;
+  s_part[part][r] = acc;
+  __syncthreads();
+  if (part == 0 && i < b) {
+#pragma unroll
+    for (int k = 1; k < kMergeParts; ++k) acc = merge(acc, s_part[k][r]);
+    lse[i] = (acc.x + log2f(acc.y)) * kLn2;
+  }
 }
 
 __global__ void fill_zero_kernel(float* p, int64_t n) {
@@ -736,8 +750,8 @@ static int lse_forward_impl(const void* e, const void* c, const void* bias, cons
   int st = (dtype == CCE_DTYPE_BF16) ? launch_lse_forward<BF16>(p, aligned, logit_avg != nullptr, stream)
                                      : launch_lse_forward<F16>(p, aligned, logit_avg != nullptr, stream);
   if (st != CCE_OK) return st;
-  hipLaunchKernelGGL(lse_merge_kernel, dim3(static_cast<unsigned>((b + 255) / 256)), dim3(256), 0, stream,
-                     p.partial, lse, b, p.nsplit);
+  hipLaunchKernelGGL(lse_merge_kernel, dim3(static_cast<unsigned>((b + kMergeRows - 1) / kMergeRows)),
+                     dim3(kMergeRows * kMergeParts), 0, stream, p.partial, lse, b, p.nsplit);
   return status_from_hip(hipGetLastError());
 }
 
