@@ -18,11 +18,14 @@
 // blocks of ROWS instead, each with the whole vocabulary: dE of a block is then complete after its one launch (written
 // once, no compensation buffer of [b, d]) and it is dC that is carried from block to block, as a pair of 16-bit
 // numbers with a [v, d] compensation buffer.  Same kernels, the roles of the two outputs exchanged.
+// Where the tiles of a product are few and their reduction long (dE of a thousand rows against 50000 classes: 16 tiles
+// of 800 stages on 256 compute units, and its mirror image, dC of a small vocabulary under many rows), the reduction
+// itself is cut: a tile becomes several items, each with a range of the reduction and an fp32 slot [rows, d] of its
+// own in the workspace, and split_sum_kernel adds the slots in a fixed order at the end (deterministic, no atomics).
 // Both products run on the tile loop of cce_tile4.h (direct-to-LDS loads, LDS transpose reads for the
 // operand whose reduction index is the row index).  Everything is enqueued on the caller's stream; nothing
 // is allocated, no host synchronisation.
-#include <queue>
-#include <vector>
+#include <algorithm>
 
 #include "cce_dense.h"
 #include "cce_tile4.h"
@@ -54,24 +57,35 @@ struct ProductParams {
   int d;
   int n_cls;            // classes in the chunk
   int tiles_n;          // column tiles of either output
-  int dc_tiles, dc_per_xcd;  // tiles of dC, slots per XCD
+  int dc_tiles, dc_per_xcd;  // items of dC (tiles x splits), places per XCD
   int de_tiles, de_per_xcd;
-  int de_first;              // the dE tiles have the longer reduction and take the first block ids
+  int de_first;              // the dE items have the longer reduction and take the first block ids
+  // A reduction cut into splits: split s of a tile runs over [s * len, min((s + 1) * len, total)) and leaves its
+  // result in slot s, `slot` floats behind the one before (one split: the whole reduction, slot unused).
+  int de_splits, dc_splits;
+  int de_len, dc_len;        // classes / rows per split, multiples of 64
+  int64_t de_slot, dc_slot;
+  int de_init;               // an fp32 d_e is written, not added to (the first launch on a set of slots)
 };
 
 constexpr int kProdThreads = 256;  // four waves, one per SIMD
 
-// Tile `block` of a group of `tiles` tiles (tiles_n column tiles wide).  Block ids that land on one XCD get
+// Item `block` of a group of `items` = tiles x splits items (tiles_n column tiles wide).  Block ids that land on one XCD get
 // consecutive places in an order that keeps the 32 tiles an XCD works on at a time on few operand panels: a tile
 // streams one A panel (its row of tiles) and one B panel (its column) through the XCD's L2, so 32 tiles of one or
 // two rows of a wide output need 2 + 16 panels where a block of 4 x 8 tiles needs 12.  The columns are therefore
 // cut into groups of at most 8 (as equal as possible), and the order walks a group row by row before it moves to
 // the next group (E [15356, 4096] x C [128256, 4096], 16 column tiles: backward 39.3 -> 38.1 ms).
-__device__ __forceinline__ bool product_tile_of(int block, int tiles, int per_xcd, int tiles_n, int& tm, int& tn) {
+// The splits of a reduction are walked one after the other: neighbours then share the same range of the operands.
+__device__ __forceinline__ bool product_tile_of(int block, int items, int splits, int per_xcd, int tiles_n, int& split,
+                                                int& tm, int& tn) {
   const int xcd = block & 7;
   const int slot = block >> 3;
   int lin = xcd * per_xcd + slot;
-  if (lin >= tiles) return false;
+  if (lin >= items) return false;
+  const int tiles = items / splits;
+  split = lin / tiles;
+  lin -= split * tiles;
   const int tiles_m = tiles / tiles_n;
   const int groups = (tiles_n + 7) / 8;
   const int narrow = tiles_n / groups;          // width of the narrow groups; the first `wide` groups have one more
@@ -97,27 +111,29 @@ __device__ __forceinline__ bool product_tile_of(int block, int tiles, int per_xc
 
 // dE[row][col] += sum_class dz[row][class] * C[class][col]
 template <typename T, bool SPLIT_DE>
-__device__ __forceinline__ void dense_de_tile(const ProductParams& p, int tm, int tn, unsigned char* smem) {
+__device__ __forceinline__ void dense_de_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
   using Tile = Tile4<T, false, true>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int64_t m0 = static_cast<int64_t>(tm) * Tile::TILE;
   const int n0 = tn * Tile::TILE;
+  const int k0 = split * p.de_len;
 
   typename Tile::Source s;
 #pragma unroll
   for (int q = 0; q < Tile::NQ1; ++q) {
     int64_t i = m0 + Tile::row_direct(q, g.wave, g.lane);
     i = (i < p.b) ? i : p.b - 1;  // rows past the end repeat the last one; their results are dropped
-    s.a_row[q] = p.dz + i * p.ldz + Tile::chunk_direct(g.wave, g.lane);
+    s.a_row[q] = p.dz + i * p.ldz + k0 + Tile::chunk_direct(g.wave, g.lane);
   }
   s.b_row[0] = nullptr;
   s.a_km = nullptr;
   s.a_stride = 0;
   // (columns past d: the last chunk inside the matrix once more; what they feed is dropped below)
-  s.b_km = p.c + min(n0 + Tile::chunk_kmajor(g.wave, g.lane), p.d - 8);
+  s.b_km = p.c + k0 * p.stride_cv + min(n0 + Tile::chunk_kmajor(g.wave, g.lane), p.d - 8);
   s.b_stride = p.stride_cv;
   s.b_rows = nullptr;
-  s.k_total = p.n_cls;
+  s.k_total = min(p.de_len, p.n_cls - k0);
+  float* const de_f32 = SPLIT_DE ? nullptr : p.de_f32 + split * p.de_slot;
 
   // What memory holds of a piece so far, fetched ahead of its use.
   struct Old {
@@ -134,7 +150,8 @@ __device__ __forceinline__ void dense_de_tile(const ProductParams& p, int tm, in
     if (ri >= p.b || cg >= p.d) return o;
     o.re = (p.valids != nullptr && !p.de_rows_by_number) ? static_cast<int64_t>(p.valids[ri]) : ri;
     if (!SPLIT_DE) {
-      const uint4* src = reinterpret_cast<const uint4*>(p.de_f32 + o.re * p.ld_de + cg);
+      if (p.de_init) return o;
+      const uint4* src = reinterpret_cast<const uint4*>(de_f32 + o.re * p.ld_de + cg);
       o.a = src[0];
       o.b = src[1];
     } else if (!p.first_chunk) {  // (never with de_lo == nullptr: a d_e written alone is a first chunk)
@@ -158,7 +175,7 @@ __device__ __forceinline__ void dense_de_tile(const ProductParams& p, int tm, in
     const int64_t ri = m0 + row;
     const int cg = n0 + col;
     if (!SPLIT_DE) {
-      float4* dst = reinterpret_cast<float4*>(p.de_f32 + o.re * p.ld_de + cg);
+      float4* dst = reinterpret_cast<float4*>(de_f32 + o.re * p.ld_de + cg);
       float4 a = __builtin_bit_cast(float4, o.a), b = __builtin_bit_cast(float4, o.b);
       a.x += v[0]; a.y += v[1]; a.z += v[2]; a.w += v[3];
       b.x += v[4]; b.y += v[5]; b.z += v[6]; b.w += v[7];
@@ -191,23 +208,24 @@ __device__ __forceinline__ void dense_de_tile(const ProductParams& p, int tm, in
 
 // dC[class][col] = sum_row dz[row][class] * E[row][col]; GATHER: the rows of E come through valids
 template <typename T, bool GATHER>
-__device__ __forceinline__ void dense_dc_tile(const ProductParams& p, int tm, int tn, unsigned char* smem) {
+__device__ __forceinline__ void dense_dc_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
   using Tile = Tile4<T, true, true, GATHER>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int m0 = tm * Tile::TILE;
   const int n0 = tn * Tile::TILE;
+  const int64_t k0 = static_cast<int64_t>(split) * p.dc_len;
 
   typename Tile::Source s;
   s.a_row[0] = nullptr;
   s.b_row[0] = nullptr;
   const int chunk = Tile::chunk_kmajor(g.wave, g.lane);
   // (columns past the matrix: the last chunk inside it once more; what they feed is dropped below)
-  s.a_km = p.dz + min(static_cast<int64_t>(m0 + chunk), p.ldz - 8);
+  s.a_km = p.dz + k0 * p.ldz + min(static_cast<int64_t>(m0 + chunk), p.ldz - 8);
   s.a_stride = p.ldz;
-  s.b_km = p.e + min(n0 + chunk, p.d - 8);
+  s.b_km = p.e + (GATHER ? 0 : k0 * p.stride_e) + min(n0 + chunk, p.d - 8);
   s.b_stride = p.stride_e;
-  s.b_rows = p.valids;
-  s.k_total = static_cast<int>(p.b);
+  s.b_rows = GATHER ? p.valids + k0 : nullptr;
+  s.k_total = static_cast<int>(min(static_cast<int64_t>(p.dc_len), p.b - k0));
 
   f32x16 acc[Tile::WM][Tile::WN];
   typename Tile::Loop loop = Tile::plan(s, g);
@@ -268,7 +286,7 @@ __device__ __forceinline__ void dense_dc_tile(const ProductParams& p, int tm, in
     const int cls = m0 + row;
     const int cg = n0 + col;
     if (cls >= p.n_cls || cg >= p.d) return;
-    const int64_t off = static_cast<int64_t>(cls) * p.ld_dc + cg;
+    const int64_t off = split * p.dc_slot + static_cast<int64_t>(cls) * p.ld_dc + cg;
     if (p.dc_fp32) {
       float4* dst = reinterpret_cast<float4*>(static_cast<float*>(p.d_c) + off);
       float4 a = make_float4(v[0], v[1], v[2], v[3]), b = make_float4(v[4], v[5], v[6], v[7]);
@@ -295,17 +313,51 @@ __global__ __launch_bounds__(kProdThreads, 1) void dense_products_kernel(Product
   const int first_blocks = (p.de_first ? p.de_per_xcd : p.dc_per_xcd) * 8;
   const bool first = static_cast<int>(blockIdx.x) < first_blocks;
   const int block = first ? blockIdx.x : blockIdx.x - first_blocks;
-  int tm, tn;
+  int split, tm, tn;
   if (first != (p.de_first != 0)) {
-    if (!product_tile_of(block, p.dc_tiles, p.dc_per_xcd, p.tiles_n, tm, tn)) return;
+    if (!product_tile_of(block, p.dc_tiles, p.dc_splits, p.dc_per_xcd, p.tiles_n, split, tm, tn)) return;
     if (p.valids != nullptr) {
-      dense_dc_tile<T, true>(p, tm, tn, smem);
+      dense_dc_tile<T, true>(p, split, tm, tn, smem);
     } else {
-      dense_dc_tile<T, false>(p, tm, tn, smem);
+      dense_dc_tile<T, false>(p, split, tm, tn, smem);
     }
   } else {
-    if (!product_tile_of(block, p.de_tiles, p.de_per_xcd, p.tiles_n, tm, tn)) return;
-    dense_de_tile<T, SPLIT_DE>(p, tm, tn, smem);
+    if (!product_tile_of(block, p.de_tiles, p.de_splits, p.de_per_xcd, p.tiles_n, split, tm, tn)) return;
+    dense_de_tile<T, SPLIT_DE>(p, split, tm, tn, smem);
+  }
+}
+
+// out[row(i)][:] (+)= sum over the slots of slot[s][i][:], in the order of the slots; eight columns per thread.  Bound
+// by reading the slots: 4 bytes per element and slot.
+template <typename T>
+__global__ __launch_bounds__(256) void split_sum_kernel(const float* slots, int splits, int64_t rows, int d, const int32_t* ids,
+                                                        void* out, int64_t ld_out, int out_fp32, int add) {
+  const int per_row = d / 8;
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (item >= rows * per_row) return;
+  const int64_t i = item / per_row;
+  const int col = static_cast<int>(item - i * per_row) * 8;
+  float v[8] = {};
+  for (int s = 0; s < splits; ++s) {
+    const float4* src = reinterpret_cast<const float4*>(slots + (s * rows + i) * d + col);
+    const float4 a = src[0], b = src[1];
+    v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
+    v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
+  }
+  const int64_t off = (ids != nullptr ? static_cast<int64_t>(ids[i]) : i) * ld_out + col;
+  if (out_fp32) {
+    float4* dst = reinterpret_cast<float4*>(static_cast<float*>(out) + off);
+    float4 a = make_float4(v[0], v[1], v[2], v[3]), b = make_float4(v[4], v[5], v[6], v[7]);
+    if (add) {
+      const float4 a0 = dst[0], b0 = dst[1];
+      a.x += a0.x; a.y += a0.y; a.z += a0.z; a.w += a0.w;
+      b.x += b0.x; b.y += b0.y; b.z += b0.z; b.w += b0.w;
+    }
+    dst[0] = a;
+    dst[1] = b;
+  } else {
+    *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + off) =
+        make_uint4(Elem<T>::pack2(v[0], v[1]), Elem<T>::pack2(v[2], v[3]), Elem<T>::pack2(v[4], v[5]), Elem<T>::pack2(v[6], v[7]));
   }
 }
 
@@ -330,98 +382,39 @@ __global__ __launch_bounds__(1024) void dz_colsum_kernel(const uint16_t* dz, int
   }
 }
 
-static int64_t dense_chunk_classes_uncached(int64_t b, int64_t v, int64_t d, int64_t max_dz_bytes, bool want_de,
-                                            bool want_dc);
-
-// Rounds the product launch of one chunk takes, in units of 256 reduction steps: n_long tiles of length
-// len_long and n_short tiles of len_short handed out in that order to 256 compute units as they fall free.
-static double product_makespan(int64_t n_long, int64_t len_long, int64_t n_short, int64_t len_short) {
-  const int cus = compute_units();
-  if (len_long < len_short) {
-    const int64_t n = n_long, l = len_long;
-    n_long = n_short; len_long = len_short; n_short = n; len_short = l;
-  }
-  // greedy list scheduling over a min-heap of the units' finishing times
-  std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> free_at;
-  for (int i = 0; i < cus; ++i) free_at.push(0);
-  int64_t worst = 0;
-  auto give = [&](int64_t n, int64_t len) {
-    for (int64_t t = 0; t < n; ++t) {
-      const int64_t end = free_at.top() + len;
-      free_at.pop();
-      free_at.push(end);
-      worst = end > worst ? end : worst;
-    }
-  };
-  give(n_long, len_long);
-  give(n_short, len_short);
-  return static_cast<double>(worst);
-}
-
-// Classes per chunk for a dz buffer of at most `max_dz_bytes`: a multiple of 256 up to 16384 that the buffer can
-// hold, chosen for the least estimated time of the whole vocabulary (whole chunks and the shorter last one): per
-// chunk the dz kernel and the product launch (dC tiles with a reduction over b rows, dE tiles with a reduction
-// over vc classes, the longer kind first, filling 256 compute units as they fall free).  0: the buffer cannot
-// hold 256 classes.
-static int64_t dense_chunk_classes(int64_t b, int64_t v, int64_t d, int64_t max_dz_bytes, bool want_de, bool want_dc) {
-  // The same questions come with every step of a training loop -- the size query with the caller's dz budget, then
-  // the call itself with the bytes that query answered -- so the last few answers of this thread are kept (the
-  // search simulates two schedules for each of up to 64 chunk sizes: 1-3 ms of host time per question).
-  struct Memo {
-    int64_t b, v, d, bytes, answer;
-    bool de, dc;
-  };
-  constexpr int kMemos = 8;
-  static thread_local Memo memo[kMemos] = {};
-  static thread_local int next_slot = 0;
-  for (int i = 0; i < kMemos; ++i) {
-    const Memo& m = memo[i];
-    if (m.b == b && m.v == v && m.d == d && m.bytes == max_dz_bytes && m.de == want_de && m.dc == want_dc && m.b != 0)
-      return m.answer;
-  }
-  const int64_t answer = dense_chunk_classes_uncached(b, v, d, max_dz_bytes, want_de, want_dc);
-  memo[next_slot] = {b, v, d, max_dz_bytes, answer, want_de, want_dc};
-  next_slot = (next_slot + 1) % kMemos;
-  return answer;
-}
-
-// Estimated time of one chunk of vc classes in units of 256 reduction steps of a tile: the dz kernel (row_tiles x
-// vc / 256 logit tiles of d / 256 units each, in rounds of 256) and the product launch.
-static double chunk_cost(int64_t b, int64_t d, int64_t vc, bool want_de, bool want_dc) {
-  const int64_t col_tiles = (d + 255) / 256;
-  const int64_t row_tiles = (b + 255) / 256;
-  const double products = product_makespan(want_dc ? vc / 256 * col_tiles : 0, row_tiles,
-                                           want_de ? row_tiles * col_tiles : 0, vc / 256);
-  const int64_t dz_tiles = row_tiles * (vc / 256);
-  const int64_t cus = compute_units();
-  const double dz = static_cast<double>((dz_tiles + cus - 1) / cus) * static_cast<double>(col_tiles);
-  return products + dz + 0.25;  // the constant only breaks ties towards fewer chunks: launches queue back to back
-}
-
-static int64_t dense_chunk_classes_uncached(int64_t b, int64_t v, int64_t d, int64_t max_dz_bytes, bool want_de,
-                                            bool want_dc) {
-  const int64_t v_pad = (v + 255) / 256 * 256;
-  int64_t top = max_dz_bytes / (b * 2) / 256 * 256;
-  if (top > 16384) top = 16384;
-  if (top < 256) return 0;
-  if (top >= v_pad) return v_pad;
-  int64_t best = top;
-  double best_cost = 1e300;
-  for (int64_t vc = top; vc >= 256; vc -= 256) {
-    // whole chunks, then the shorter last one
-    const int64_t full = v / vc;
-    const int64_t rest = (v - full * vc + 255) / 256 * 256;
-    double cost = static_cast<double>(full) * chunk_cost(b, d, vc, want_de, want_dc);
-    if (rest > 0) cost += chunk_cost(b, d, rest, want_de, want_dc);
-    if (cost < best_cost * (1.0 - 1e-9)) {
-      best = vc;
-      best_cost = cost;
-    }
-  }
-  return best;
-}
-
 static int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
+
+// Finishing time of a launch of n1 items of length l1 and n2 of length l2 handed out, longer kind first, to the compute
+// units as they fall free.  (With l1 >= l2 the units fall free at q l1 or (q + 1) l1, and the n2 short items end at the
+// n2 smallest of {free + k l2}.)
+static int64_t product_makespan(int64_t n1, int64_t l1, int64_t n2, int64_t l2) {
+  const int64_t cus = compute_units();
+  if (l1 < l2) {
+    std::swap(n1, n2);
+    std::swap(l1, l2);
+  }
+  const int64_t q = n1 / cus, r = n1 % cus;
+  const int64_t early = q * l1, late = (q + 1) * l1;
+  if (n2 == 0 || l2 == 0) return r > 0 ? late : early;
+  auto done_by = [&](int64_t t) {
+    return (cus - r) * ((t - early) / l2) + (t > late ? r * ((t - late) / l2) : 0);
+  };
+  auto first_end = [&](int64_t base) {  // the least base + k l2 by which all short items are done
+    int64_t lo = 0, hi = n2;
+    while (lo < hi) {
+      const int64_t k = (lo + hi) / 2;
+      if (done_by(base + k * l2) >= n2) hi = k; else lo = k + 1;
+    }
+    return base + lo * l2;
+  };
+  int64_t end = first_end(early);
+  if (r > 0) {
+    const int64_t other = first_end(late);
+    end = other < end ? other : end;
+    end = end < late ? late : end;
+  }
+  return end;
+}
 
 // How cce_backward_dense walks the [b, v] plane for a dz buffer of at most `max_dz_bytes`.
 //   by classes  chunks of `unit` classes, all b rows each: dC of a chunk is complete, dE is carried over the chunks
@@ -433,36 +426,157 @@ static int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 // rows outnumber the classes two to one (measured, E [65536, 3584] x C [19008, 3584]: 36.1 ms and 581 MB by classes
 // with 1024-class chunks, against the same 130 MB of dz by rows).  Only with 16-bit gradients: an fp32 dE is its own
 // accumulator.  unit == 0: not even the smallest plan (256 classes / rows) fits.
+//   splits      into how many ranges the reductions of dE and dC are cut.  The gradient that is carried may be cut in any
+//               walk (its slots are then what is carried, in place of the pair and its compensation term), the other one
+//               only where a single launch completes it.
 struct DensePlan {
   bool by_rows;
   int64_t unit;
-  int64_t fixed_bytes;
+  int de_splits, dc_splits;
+  int64_t fixed_bytes;  // what the size query promises to need beside the dz buffer
+  int64_t comp_bytes;   // the compensation term this plan keeps (0 where the carried gradient sits in slots)
   int64_t dz_bytes;
+  int64_t slot_bytes;   // of all slots
 };
 static bool dense_walks_by_rows(int64_t b, int64_t v, bool gradients_16bit) {
   return gradients_16bit && b >= 2 * ((v + 255) / 256 * 256);
 }
-static DensePlan dense_plan(int64_t b, int64_t v, int64_t d, bool gradients_16bit, int64_t max_dz_bytes) {
-  DensePlan pl;
-  pl.by_rows = dense_walks_by_rows(b, v, gradients_16bit);
+
+// A split of n steps of 64: multiples of whole stages, so that only the last one has a partial stage.
+static int64_t split_stages(int64_t stages, int splits) { return (stages + splits - 1) / splits; }
+
+// Estimated time of one launch pair (dz kernel, products) over `rows` rows and `cls` classes, in reduction stages of a
+// product tile (64 steps of 256 x 256; 1.65 us where all units are busy): the dz tiles in rounds of all units, d / 64
+// stages each, then the product items as they are handed out.  An item of a cut reduction leaves 256 KB of fp32 (and
+// takes them in first, where slots are carried): up to 6 stages of time where every unit does so at once.
+static double launch_cost(int64_t rows, int64_t cls, int64_t d, int de_splits, int dc_splits, bool carried) {
+  const int64_t cus = compute_units();
+  const int64_t tr = (rows + 255) / 256, tc = (cls + 255) / 256, tn = (d + 255) / 256;
+  const int64_t dz = (tr * tc + cus - 1) / cus * tn * 4;
+  auto item = [&](int64_t total, int splits, int64_t tiles) {
+    const int64_t len = split_stages((total + 63) / 64, splits);
+    if (splits == 1) return len;
+    const int64_t items = tiles * splits;
+    return len + (4 + 6 * (items < cus ? items : cus) / cus) * (carried ? 2 : 1);
+  };
+  return static_cast<double>(dz + product_makespan(tc * tn * dc_splits, item(rows, dc_splits, tc * tn),
+                                                   tr * tn * de_splits, item(cls, de_splits, tr * tn)));
+}
+
+// Adding the slots up at the end: a launch, and reading them at 4 TB/s (6.6 MB in the time of a stage).
+static double split_sum_cost(int64_t rows, int64_t d, int splits) {
+  return splits == 1 ? 0.0 : 4.0 + static_cast<double>(splits) * static_cast<double>(rows * d) * 4.0 / 6.6e6;
+}
+
+// At least this many stages per split: below, an item is mostly its own start and end.
+constexpr int64_t kMinSplitStages = 8;
+constexpr int64_t kMaxChunkClasses = 16384;
+
+static DensePlan dense_plan_uncached(int64_t b, int64_t v, int64_t d, bool g16, int64_t max_dz_bytes) {
+  DensePlan pl = {};
+  pl.by_rows = dense_walks_by_rows(b, v, g16);
+  pl.de_splits = pl.dc_splits = 1;
+  const int64_t v_pad = (v + 255) / 256 * 256, b_pad = (b + 255) / 256 * 256;
+  pl.fixed_bytes = pl.by_rows ? align256(v * d * 2) : (g16 ? align256(b * d * 2) : 0);
+  pl.comp_bytes = pl.fixed_bytes;
+  const int64_t budget = max_dz_bytes + pl.fixed_bytes;  // what a plan may take in all
+  double best = 1e300;
+
+  // Takes a plan in if it fits and is estimated to be faster.  A cut reduction has to win by 3 %.
+  auto consider = [&](int64_t unit, int de_splits, int dc_splits) {
+    const bool cut = de_splits > 1 || dc_splits > 1;
+    const bool carried_cut = pl.by_rows ? dc_splits > 1 : de_splits > 1;
+    const int64_t launches = pl.by_rows ? (b + unit - 1) / unit : (v + unit - 1) / unit;
+    if (launches > 1 && (pl.by_rows ? de_splits : dc_splits) > 1) return;
+    const int64_t comp = carried_cut ? 0 : pl.fixed_bytes;
+    const int64_t dz = align256((pl.by_rows ? unit * v_pad : b * unit) * 2);
+    const int64_t slots = align256((de_splits > 1 ? de_splits * b * d * 4 : 0)) + align256(dc_splits > 1 ? dc_splits * v * d * 4 : 0);
+    if (comp + dz + slots > budget) return;
+    const int64_t whole = pl.by_rows ? b / unit : v / unit;
+    const int64_t rest = pl.by_rows ? b - whole * unit : v - whole * unit;
+    const bool carried = launches > 1;
+    double cost = 0.0;
+    if (whole > 0)
+      cost += whole * (1.0 + (pl.by_rows ? launch_cost(unit, v, d, de_splits, dc_splits, carried)
+                                         : launch_cost(b, unit, d, de_splits, dc_splits, carried)));
+    if (rest > 0)
+      cost += 1.0 + (pl.by_rows ? launch_cost(rest, v, d, de_splits, dc_splits, carried)
+                                : launch_cost(b, rest, d, de_splits, dc_splits, carried));
+    cost += split_sum_cost(b, d, de_splits) + split_sum_cost(v, d, dc_splits);
+    if (cost * (cut ? 1.03 : 1.0) >= best * (1.0 - 1e-9)) return;
+    best = cost * (cut ? 1.03 : 1.0);
+    pl.unit = unit;
+    pl.de_splits = de_splits;
+    pl.dc_splits = dc_splits;
+    pl.comp_bytes = comp;
+    pl.dz_bytes = dz;
+    pl.slot_bytes = slots;
+  };
+
+  // ---- whole reductions
   if (pl.by_rows) {
-    const int64_t v_pad = (v + 255) / 256 * 256;
-    const int64_t b_pad = (b + 255) / 256 * 256;
-    pl.fixed_bytes = align256(v * d * 2);
     int64_t rb = max_dz_bytes / (v_pad * 2) / 256 * 256;
     if (rb > b_pad) rb = b_pad;
     if (rb >= 256) {  // blocks of equal size: the last one is not a sliver
       const int64_t blocks = (b + rb - 1) / rb;
       rb = ((b + blocks - 1) / blocks + 255) / 256 * 256;
+      consider(rb, 1, 1);
     }
-    pl.unit = rb >= 256 ? rb : 0;
-    pl.dz_bytes = align256(pl.unit * v_pad * 2);
   } else {
-    pl.fixed_bytes = gradients_16bit ? align256(b * d * 2) : 0;
-    pl.unit = dense_chunk_classes(b, v, d, max_dz_bytes, true, true);
-    pl.dz_bytes = align256(b * pl.unit * 2);
+    int64_t top = max_dz_bytes / (b * 2) / 256 * 256;
+    if (top > kMaxChunkClasses) top = kMaxChunkClasses;
+    if (top >= v_pad) consider(v_pad, 1, 1);
+    else
+      for (int64_t vc = top; vc >= 256; vc -= 256) consider(vc, 1, 1);
+  }
+
+  // ---- cut reductions, in as few launches as the budget allows (chunks past 16384 classes where the whole dz still
+  // stays in the last-level cache), and a launch or two more: the slots compete with dz for the budget
+  static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+  const int64_t dz_cap = budget < (int64_t(256) << 20) ? budget : (int64_t(256) << 20);
+  const int64_t along = pl.by_rows ? b_pad : v_pad;
+  int64_t most = dz_cap / ((pl.by_rows ? v_pad : b) * 2) / 256 * 256;
+  if (most > along) most = along;
+  if (most >= 256) {
+    const int64_t least = (along + most - 1) / most;
+    for (int64_t n = least; n <= least + 2; ++n) {
+      const int64_t unit = ((along + n - 1) / n + 255) / 256 * 256;
+      const int64_t rows = pl.by_rows ? unit : b, cls = pl.by_rows ? v : unit;
+      for (int se : kSplits) {
+        if (se > 1 && (cls + 63) / 64 < se * kMinSplitStages) break;
+        for (int sc : kSplits) {
+          if (sc > 1 && (rows + 63) / 64 < sc * kMinSplitStages) break;
+          consider(unit, se, sc);
+        }
+      }
+    }
   }
   return pl;
+}
+
+// The same questions come with every step of a training loop -- the size query with the caller's dz budget, then the
+// call itself with the bytes that query answered -- so the last few answers of this thread are kept (a search weighs
+// up to 64 chunk sizes and 400 ways to cut: 10 - 60 us of host time).
+static DensePlan dense_plan(int64_t b, int64_t v, int64_t d, bool g16, int64_t max_dz_bytes) {
+  struct Memo {
+    int64_t b, v, d, bytes;
+    bool g16;
+    int cus;
+    DensePlan answer;
+  };
+  constexpr int kMemos = 8;
+  static thread_local Memo memo[kMemos] = {};
+  static thread_local int next_slot = 0;
+  const int cus = compute_units();
+  for (int i = 0; i < kMemos; ++i) {
+    const Memo& m = memo[i];
+    if (m.b == b && m.v == v && m.d == d && m.bytes == max_dz_bytes && m.g16 == g16 && m.cus == cus && m.b != 0)
+      return m.answer;
+  }
+  memo[next_slot] = {b, v, d, max_dz_bytes, g16, cus, dense_plan_uncached(b, v, d, g16, max_dz_bytes)};
+  const DensePlan answer = memo[next_slot].answer;
+  next_slot = (next_slot + 1) % kMemos;
+  return answer;
 }
 
 }  // namespace cce
@@ -472,17 +586,18 @@ using namespace cce;
 extern "C" int64_t cce_backward_dense_workspace_bytes(int64_t b, int64_t v, int64_t d, int d_e_in_workspace,
                                                       int64_t max_dz_bytes) {
   if (b <= 0 || v <= 0 || d <= 0) return 0;
-  DensePlan pl = dense_plan(b, v, d, d_e_in_workspace != 0, max_dz_bytes);
+  const DensePlan pl = dense_plan(b, v, d, d_e_in_workspace != 0, max_dz_bytes);
   if (pl.unit == 0) {  // the smallest plan
     const int64_t v_pad = (v + 255) / 256 * 256;
-    pl.dz_bytes = align256(256 * (pl.by_rows ? v_pad : b) * 2);
+    return pl.fixed_bytes + align256(256 * (pl.by_rows ? v_pad : b) * 2);
   }
-  return pl.fixed_bytes + pl.dz_bytes;
+  return std::max(pl.comp_bytes + pl.dz_bytes + pl.slot_bytes, pl.fixed_bytes);
 }
 
 extern "C" int64_t cce_backward_dense_fixed_bytes(int64_t b, int64_t v, int64_t d, int d_e_in_workspace) {
   if (b <= 0 || v <= 0 || d <= 0) return 0;
-  return dense_plan(b, v, d, d_e_in_workspace != 0, 0).fixed_bytes;
+  if (dense_walks_by_rows(b, v, d_e_in_workspace != 0)) return align256(v * d * 2);
+  return d_e_in_workspace != 0 ? align256(b * d * 2) : 0;
 }
 
 extern "C" int64_t cce_backward_dense_dz_bytes(int64_t b, int64_t v, int64_t d, int d_e_in_workspace, int64_t units) {
@@ -521,18 +636,24 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
   if (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
     return workspace == nullptr ? CCE_ERR_WORKSPACE_TOO_SMALL : CCE_ERR_MISALIGNED;
 
-  // ---- plan: [16-bit compensation term of the gradient that is carried][dz buffer] ------------------------------
+  // ---- plan: [16-bit compensation term of the gradient that is carried][dz buffer][slots of dE][slots of dC] ------
   const bool split_de = (d_e != nullptr) && !d_e_is_fp32;
   // (the walk by rows needs the caller to have sized the workspace for it: a 16-bit d_e is what the size query's
   // flag says, and a d_c in fp32 beside it is added to in place)
   const bool by_rows = dense_walks_by_rows(b, v, split_de);
-  const int64_t comp_bytes = dense_plan(b, v, d, split_de, 0).fixed_bytes;
   // the plan the size query made (both gradients wanted), so that its answer always suffices
-  const DensePlan plan = dense_plan(b, v, d, split_de, workspace_bytes - comp_bytes);
+  const DensePlan plan = dense_plan(b, v, d, split_de, workspace_bytes - cce_backward_dense_fixed_bytes(b, v, d, split_de));
   if (plan.unit == 0) return CCE_ERR_WORKSPACE_TOO_SMALL;
-  uint16_t* dz = reinterpret_cast<uint16_t*>(static_cast<unsigned char*>(workspace) + comp_bytes);
+  unsigned char* const ws = static_cast<unsigned char*>(workspace);
+  uint16_t* dz = reinterpret_cast<uint16_t*>(ws + plan.comp_bytes);
+  float* const de_slots = reinterpret_cast<float*>(ws + plan.comp_bytes + plan.dz_bytes);
+  float* const dc_slots =
+      reinterpret_cast<float*>(ws + plan.comp_bytes + plan.dz_bytes + (plan.de_splits > 1 ? align256(plan.de_splits * b * d * 4) : 0));
   const int64_t vc = by_rows ? (v + 255) / 256 * 256 : plan.unit;
   const int64_t ldz = vc;
+  const bool de_cut = d_e != nullptr && plan.de_splits > 1;
+  const bool dc_cut = d_c != nullptr && plan.dc_splits > 1;
+  const bool pair_de = split_de && !de_cut;  // dE leaves the products as 16-bit numbers
 
   ProductParams p;
   p.dz = dz;
@@ -541,22 +662,43 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
   p.e = static_cast<const uint16_t*>(e);
   p.stride_e = stride_e;
   p.valids = valids;
-  p.de_f32 = split_de ? nullptr : static_cast<float*>(d_e);
-  p.de_hi = split_de ? static_cast<uint16_t*>(d_e) : nullptr;
-  p.de_lo = (split_de && !by_rows) ? static_cast<uint16_t*>(workspace) : nullptr;
-  p.ld_de = stride_e;
-  p.dc_fp32 = d_c_is_fp32;
-  p.ld_dc = stride_cv;
+  p.de_f32 = de_cut ? de_slots : (split_de ? nullptr : static_cast<float*>(d_e));
+  p.de_hi = pair_de ? static_cast<uint16_t*>(d_e) : nullptr;
+  p.de_lo = (pair_de && !by_rows) ? static_cast<uint16_t*>(workspace) : nullptr;
+  p.ld_de = de_cut ? d : stride_e;
+  p.dc_fp32 = dc_cut ? 1 : d_c_is_fp32;
+  p.ld_dc = dc_cut ? d : stride_cv;
   p.dc_accumulate = 0;
   p.dc_lo = nullptr;
   p.dc_first = 1;
-  p.de_rows_by_number = 0;
+  p.de_rows_by_number = de_cut ? 1 : 0;
+  p.de_init = 0;
   p.b = b;
   p.d = static_cast<int>(d);
+  p.de_slot = b * d;
+  p.dc_slot = v * d;
+  // Ranges of the reductions, fixed by the first launch, which is the largest: it fills every slot there is (seven stages
+  // cut in five make four ranges of two, the last of them short), a later one adds to as many of them as it has ranges.
+  const int64_t first_rows = by_rows ? std::min(plan.unit, b) : b, first_cls = by_rows ? v : std::min(vc, v);
+  p.de_len = static_cast<int>(split_stages((first_cls + 63) / 64, de_cut ? plan.de_splits : 1) * 64);
+  p.dc_len = static_cast<int>(split_stages((first_rows + 63) / 64, dc_cut ? plan.dc_splits : 1) * 64);
+  const int de_nslots = static_cast<int>((first_cls + p.de_len - 1) / p.de_len);
+  const int dc_nslots = static_cast<int>((first_rows + p.dc_len - 1) / p.dc_len);
+  p.tiles_n = static_cast<int>((d + 255) / 256);
+  auto set_items = [&](int64_t rows, int64_t cls) {  // the items of a launch over `rows` rows and `cls` classes
+    p.b = rows;
+    p.n_cls = static_cast<int>(cls);
+    p.de_splits = static_cast<int>((cls + p.de_len - 1) / p.de_len);
+    p.dc_splits = static_cast<int>((rows + p.dc_len - 1) / p.dc_len);
+    p.dc_tiles = (d_c != nullptr) ? static_cast<int>((cls + 255) / 256) * p.tiles_n * p.dc_splits : 0;
+    p.de_tiles = (d_e != nullptr) ? static_cast<int>((rows + 255) / 256) * p.tiles_n * p.de_splits : 0;
+    p.dc_per_xcd = (p.dc_tiles + 7) / 8;
+    p.de_per_xcd = (p.de_tiles + 7) / 8;
+    p.de_first = (std::min<int64_t>(p.de_len, cls) > std::min<int64_t>(p.dc_len, rows)) ? 1 : 0;
+  };
 
   using TileB = Tile4<BF16, true, true>;
   const int lds = TileB::LDS_BYTES;
-  const int tiles_n = static_cast<int>((d + 255) / 256);
   hipError_t err;
 #define CCE_LAUNCH_PRODUCT(KERN, BLOCKS)                                                            \
   do {                                                                                              \
@@ -566,19 +708,40 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
     if (err != hipSuccess) return status_from_hip(err);                                             \
     hipLaunchKernelGGL(kern, dim3(BLOCKS), dim3(kProdThreads), lds, stream, p);                     \
   } while (0)
+  // the products of the dz in the workspace (set_items() has been called), and dBias
+  auto products = [&](int64_t rows, int64_t cls, float* bias_out) -> int {
+    const int blocks = (p.dc_per_xcd + p.de_per_xcd) * 8;
+    if (blocks > 0) {
+      if (dtype == CCE_DTYPE_BF16) {
+        if (pair_de) CCE_LAUNCH_PRODUCT((dense_products_kernel<BF16, true>), blocks);
+        else CCE_LAUNCH_PRODUCT((dense_products_kernel<BF16, false>), blocks);
+      } else {
+        if (pair_de) CCE_LAUNCH_PRODUCT((dense_products_kernel<F16, true>), blocks);
+        else CCE_LAUNCH_PRODUCT((dense_products_kernel<F16, false>), blocks);
+      }
+    }
+    if (bias_out != nullptr) {
+      const unsigned cblocks = static_cast<unsigned>((cls + 63) / 64);
+      if (dtype == CCE_DTYPE_BF16)
+        hipLaunchKernelGGL(dz_colsum_kernel<BF16>, dim3(cblocks), dim3(1024), 0, stream, dz, ldz, rows, static_cast<int>(cls),
+                           bias_out);
+      else
+        hipLaunchKernelGGL(dz_colsum_kernel<F16>, dim3(cblocks), dim3(1024), 0, stream, dz, ldz, rows, static_cast<int>(cls),
+                           bias_out);
+    }
+    return status_from_hip(hipGetLastError());
+  };
+#undef CCE_LAUNCH_PRODUCT
 
   const size_t es = 2;
   if (by_rows) {
     // ---- blocks of rows, the whole vocabulary each ------------------------------------------------------------
     const int64_t rb = plan.unit;
     p.c = static_cast<const uint16_t*>(c);
-    p.n_cls = static_cast<int>(v);
     p.first_chunk = 1;  // d_e of a block is complete with its launch
-    p.tiles_n = tiles_n;
-    p.d_c = d_c;
-    p.dc_lo = (d_c != nullptr && !d_c_is_fp32) ? static_cast<uint16_t*>(workspace) : nullptr;
-    p.dc_tiles = (d_c != nullptr) ? static_cast<int>((v + 255) / 256) * tiles_n : 0;
-    p.dc_per_xcd = (p.dc_tiles + 7) / 8;
+    p.de_init = 1;      // ... also where it is cut
+    p.d_c = dc_cut ? static_cast<void*>(dc_slots) : d_c;
+    p.dc_lo = (d_c != nullptr && !dc_cut && !d_c_is_fp32) ? static_cast<uint16_t*>(workspace) : nullptr;
     for (int64_t r0 = 0; r0 < b; r0 += rb) {
       const int64_t n = (b - r0 < rb) ? (b - r0) : rb;
       // Rows are numbered through valids when there is one (absolute rows of e: only the list moves on); without
@@ -594,76 +757,45 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
       if (st != CCE_OK) return st;
       p.e = reinterpret_cast<const uint16_t*>(e_blk);
       p.valids = valids_blk;
-      p.de_hi = static_cast<uint16_t*>(d_e) + shift_rows * stride_e;
-      p.b = n;
+      if (pair_de) p.de_hi = static_cast<uint16_t*>(d_e) + shift_rows * stride_e;
       p.dc_first = (r0 == 0) ? 1 : 0;
-      p.dc_accumulate = (r0 == 0) ? 0 : 1;  // an fp32 d_c is written by the first block and added to by the others
-      p.de_tiles = static_cast<int>((n + 255) / 256) * tiles_n;
-      p.de_per_xcd = (p.de_tiles + 7) / 8;
-      p.de_first = (v > n) ? 1 : 0;
-      const int blocks = (p.dc_per_xcd + p.de_per_xcd) * 8;
-      if (dtype == CCE_DTYPE_BF16) CCE_LAUNCH_PRODUCT((dense_products_kernel<BF16, true>), blocks);
-      else CCE_LAUNCH_PRODUCT((dense_products_kernel<F16, true>), blocks);
-      if (d_bias != nullptr) {
-        const unsigned cblocks = static_cast<unsigned>((v + 63) / 64);
-        if (dtype == CCE_DTYPE_BF16)
-          hipLaunchKernelGGL(dz_colsum_kernel<BF16>, dim3(cblocks), dim3(1024), 0, stream, dz, ldz, n, static_cast<int>(v),
-                             d_bias);
-        else
-          hipLaunchKernelGGL(dz_colsum_kernel<F16>, dim3(cblocks), dim3(1024), 0, stream, dz, ldz, n, static_cast<int>(v),
-                             d_bias);
-      }
-      err = hipGetLastError();
-      if (err != hipSuccess) return status_from_hip(err);
+      p.dc_accumulate = (r0 == 0) ? 0 : 1;  // an fp32 d_c (or its slots) is written by the first block and added to by the others
+      set_items(n, v);
+      st = products(n, v, d_bias);
+      if (st != CCE_OK) return st;
     }
-    return status_from_hip(hipGetLastError());
+  } else {
+    for (int64_t v0 = 0; v0 < v; v0 += vc) {
+      const int64_t n = (v - v0 < vc) ? (v - v0) : vc;
+      const unsigned char* c_chunk = static_cast<const unsigned char*>(c) + v0 * stride_cv * es;
+      const void* bias_chunk = bias ? static_cast<const unsigned char*>(bias) + v0 * es : nullptr;
+      int st = dense_dz_launch(e, c_chunk, bias_chunk, lse, d_out, d_out_is_scalar, d_lse, valids, targets, dz, ldz, 0, 1,
+                               n_rows, b, n, d, stride_e, stride_cv, stride_cd, grad_scale, shift, target_offset + v0,
+                               softcap, dtype, stream);
+      if (st != CCE_OK) return st;
+      p.c = reinterpret_cast<const uint16_t*>(c_chunk);
+      p.first_chunk = (v0 == 0) ? 1 : 0;
+      p.de_init = (de_cut && v0 == 0) ? 1 : 0;  // (the caller's fp32 d_e is added to from the start)
+      p.d_c = nullptr;
+      if (d_c != nullptr)
+        p.d_c = dc_cut ? static_cast<void*>(dc_slots) : static_cast<unsigned char*>(d_c) + v0 * stride_cv * (d_c_is_fp32 ? 4 : 2);
+      set_items(b, n);
+      st = products(b, n, d_bias != nullptr ? d_bias + v0 : nullptr);
+      if (st != CCE_OK) return st;
+    }
   }
-  for (int64_t v0 = 0; v0 < v; v0 += vc) {
-    const int64_t n = (v - v0 < vc) ? (v - v0) : vc;
-    const unsigned char* c_chunk = static_cast<const unsigned char*>(c) + v0 * stride_cv * es;
-    const void* bias_chunk = bias ? static_cast<const unsigned char*>(bias) + v0 * es : nullptr;
-    int st = dense_dz_launch(e, c_chunk, bias_chunk, lse, d_out, d_out_is_scalar, d_lse, valids, targets, dz, ldz, 0, 1,
-                             n_rows, b, n, d, stride_e, stride_cv, stride_cd, grad_scale, shift, target_offset + v0,
-                             softcap, dtype, stream);
-    if (st != CCE_OK) return st;
-    p.c = reinterpret_cast<const uint16_t*>(c_chunk);
-    p.n_cls = static_cast<int>(n);
-    p.first_chunk = (v0 == 0) ? 1 : 0;
-    p.tiles_n = tiles_n;
-    p.d_c = nullptr;
-    p.dc_tiles = 0;
-    if (d_c != nullptr) {
-      p.d_c = static_cast<unsigned char*>(d_c) + v0 * stride_cv * (d_c_is_fp32 ? 4 : 2);
-      p.dc_tiles = static_cast<int>((n + 255) / 256) * tiles_n;
-    }
-    p.dc_per_xcd = (p.dc_tiles + 7) / 8;
-    p.de_tiles = (d_e != nullptr) ? static_cast<int>((b + 255) / 256) * tiles_n : 0;
-    p.de_per_xcd = (p.de_tiles + 7) / 8;
-    p.de_first = (n > b) ? 1 : 0;
-    const int blocks = (p.dc_per_xcd + p.de_per_xcd) * 8;
-    if (blocks > 0) {
-      if (dtype == CCE_DTYPE_BF16) {
-        if (split_de) CCE_LAUNCH_PRODUCT((dense_products_kernel<BF16, true>), blocks);
-        else CCE_LAUNCH_PRODUCT((dense_products_kernel<BF16, false>), blocks);
-      } else {
-        if (split_de) CCE_LAUNCH_PRODUCT((dense_products_kernel<F16, true>), blocks);
-        else CCE_LAUNCH_PRODUCT((dense_products_kernel<F16, false>), blocks);
-      }
-    }
-    if (d_bias != nullptr) {
-      const unsigned blocks = static_cast<unsigned>((n + 63) / 64);
-      if (dtype == CCE_DTYPE_BF16)
-        hipLaunchKernelGGL(dz_colsum_kernel<BF16>, dim3(blocks), dim3(1024), 0, stream, dz, ldz, b, static_cast<int>(n),
-                           d_bias + v0);
-      else
-        hipLaunchKernelGGL(dz_colsum_kernel<F16>, dim3(blocks), dim3(1024), 0, stream, dz, ldz, b, static_cast<int>(n),
-                           d_bias + v0);
-    }
-    err = hipGetLastError();
-    if (err != hipSuccess) return status_from_hip(err);
-  }
-#undef CCE_LAUNCH_PRODUCT
 
+  auto sum_slots = [&](const float* slots, int count, int64_t rows, const int32_t* ids, void* out, int64_t ld, int fp32, int add) {
+    const unsigned blocks = static_cast<unsigned>((rows * (d / 8) + 255) / 256);
+    if (dtype == CCE_DTYPE_BF16)
+      hipLaunchKernelGGL(split_sum_kernel<BF16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d), ids, out,
+                         ld, fp32, add);
+    else
+      hipLaunchKernelGGL(split_sum_kernel<F16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d), ids, out,
+                         ld, fp32, add);
+  };
+  if (de_cut) sum_slots(de_slots, de_nslots, b, valids, d_e, stride_e, d_e_is_fp32, 1);
+  if (dc_cut) sum_slots(dc_slots, dc_nslots, v, nullptr, d_c, stride_cv, d_c_is_fp32, 0);
   return status_from_hip(hipGetLastError());
 }
 
@@ -700,6 +832,11 @@ extern "C" int cce_backward_products(const void* dz, int64_t ldz, const void* c,
   p.de_lo = nullptr;
   p.ld_de = ld_de;
   p.de_rows_by_number = 1;
+  p.de_init = 0;
+  p.de_splits = p.dc_splits = 1;
+  p.de_len = static_cast<int>((n_cls + 63) / 64 * 64);
+  p.dc_len = static_cast<int>((b + 63) / 64 * 64);
+  p.de_slot = p.dc_slot = 0;
   p.first_chunk = 0;
   p.d_c = d_c;
   p.ld_dc = ld_dc;

@@ -35,3 +35,58 @@ def test_lse_forward_of_few_rows_fills_the_chip(shape):
     # fp32 sums of D <= 192 products of magnitude about 1, and of up to 66000 exponentials: the bound of
     # test_lse_forward_spans_of_many_tiles
     assert torch.allclose(lse.double(), want, atol=2e-4, rtol=2e-5)
+
+
+@pytest.mark.parametrize("shape,fp32_out", [((300, 9000, 128), False), ((300, 9000, 128), True), ((70, 20011, 192), False),
+                                            ((1100, 33000, 320), False), ((9001, 200, 128), False), ((5000, 520, 64), False),
+                                            ((2100, 2500, 64), False), ((2100, 2500, 64), True)])
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("budget", [1 << 28, 0])
+def test_backward_dense_cuts_long_reductions(shape, fp32_out, gathered, budget):
+    """Few tiles with a long reduction: the unfiltered backward cuts the reduction into slots and adds them up.  dE cut
+    (few rows, many classes; with less workspace over several chunks, or not at all), dC cut (a small vocabulary under many
+    rows), both cut; the caller's fp32 dE is added to.  Against the formulas in fp64."""
+    lib = _lib()
+    dev = torch.device("cuda:0")
+    N, V, D = shape
+    e, c, t, _ = make_inputs(N, V, D, torch.bfloat16, seed=7, planted=False, c_std=0.3)
+    ed, cd, td = e.to(dev), c.to(dev), t.to(dev)
+    rows = torch.arange(N, device=dev)
+    valids = None
+    if gathered:
+        rows = rows[torch.rand(N, generator=torch.Generator().manual_seed(3)).to(dev) < 0.8]
+        valids = rows.to(torch.int32)
+    B = rows.numel()
+    g = torch.rand((N,), generator=torch.Generator().manual_seed(4)).to(dev) + 0.5
+    logits = ed.double()[rows] @ cd.double().T
+    lse = torch.logsumexp(logits, dim=1)
+    dz = torch.exp(logits - lse[:, None])
+    dz[torch.arange(B, device=dev), td[rows]] -= 1.0
+    dz *= g[rows].double()[:, None]
+    want_dc = dz.T @ ed.double()[rows]
+    want_de = torch.zeros((N, D), dtype=torch.float64, device=dev)
+    want_de[rows] = dz @ cd.double()
+    gdt = torch.float32 if fp32_out else torch.bfloat16
+    de = torch.zeros((N, D), dtype=gdt, device=dev)
+    if fp32_out:
+        de += 1.0
+    dc = torch.full((V, D), float("nan"), dtype=gdt, device=dev)
+    smallest = lib.cce_backward_dense_workspace_bytes(B, V, D, 0 if fp32_out else 1, 0)
+    ws_bytes = lib.cce_backward_dense_workspace_bytes(B, V, D, 0 if fp32_out else 1, budget or 3 * smallest)
+    ws = torch.full((ws_bytes // 4 + 64,), float("nan"), device=dev)
+    p = lambda x: x.data_ptr() if x is not None else None
+    st = lib.cce_backward_dense(
+        p(ed), p(cd), None, p(lse.float()), p(g), 0, None, p(valids), p(td), p(de), p(dc), None,
+        (ws.data_ptr() + 255) // 256 * 256, ws_bytes, N, B, V, D, D, D, 1, 1.0, int(fp32_out), int(fp32_out), 0, 0, 0.0, 0,
+        torch.cuda.current_stream().cuda_stream)
+    assert st == 0, lib.cce_error_string(st)
+    torch.cuda.synchronize()
+    # dz and a 16-bit result are rounded to 8 bits once each (2^-9 relative, on sums of terms of either sign: a
+    # hundredth of the largest value of the row), fp32 results by dz alone
+    if fp32_out:
+        de -= 1.0
+    assert torch.isfinite(de).all() and torch.isfinite(dc).all()
+    for got, want in ((de, want_de), (dc, want_dc)):
+        scale = want.abs().amax(dim=1, keepdim=True)
+        assert ((got.double() - want).abs() <= 1e-2 * scale + 1e-2 * want.abs() + 1e-6).all()
+        assert (got.double() - want).norm() <= 6e-3 * want.norm()
