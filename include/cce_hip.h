@@ -285,6 +285,32 @@ int cce_backward_products(const void* dz, int64_t ldz, const void* c, int64_t st
                           float* d_e, int64_t ld_de, float* d_c, int64_t ld_dc, int d_c_accumulate,
                           int64_t b, int64_t n_cls, int64_t d, int dtype, void* stream);
 
+/*
+ * fp32 inputs.  The matrix cores multiply 16-bit numbers: every value is split into bf16 parts, x = hi + mid + lo, and a
+ * product is taken as its leading cross terms (`terms`: 6, what is left is below 2^-24 relative; or 3 of two parts,
+ * 16 bits), all in fp32 accumulators.  The reference gives this dtype to tl.dot (cut_cross_entropy/cce_lse_forward.py:81,
+ * cce_backward.py:170-302).
+ *
+ * cce_fp32_forward: lse[b] and neg_dot[b] as cce_lse_forward and cce_indexed_neg_dot define them; bias [v] float or NULL.
+ * cce_fp32_backward: the unfiltered gradients, arguments as for cce_backward_dense: d_e [n_rows, d] is added to (row
+ * stride ld_de), d_c [v, d] written (row stride ld_dc), d_bias [v] added to.
+ * Any alignment and width; stride_cd must be 1, else CCE_ERR_MISALIGNED.  `workspace` 256-byte aligned, of at least the
+ * bytes that the size query names (copies of e and of a chunk of c in parts; dz of a chunk).
+ */
+int64_t cce_fp32_forward_workspace_bytes(int64_t b, int64_t v, int64_t d, int terms);
+int cce_fp32_forward(const float* e, const float* c, const float* bias, const int32_t* valids, const int64_t* targets,
+                     float* lse, float* neg_dot, void* workspace, int64_t workspace_bytes,
+                     int64_t n_rows, int64_t b, int64_t v, int64_t d,
+                     int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
+                     int64_t shift, int64_t target_offset, float softcap, int terms, void* stream);
+int64_t cce_fp32_backward_workspace_bytes(int64_t b, int64_t v, int64_t d, int terms);
+int cce_fp32_backward(const float* e, const float* c, const float* bias, const float* lse, const float* d_out,
+                      int d_out_is_scalar, const float* d_lse, const int32_t* valids, const int64_t* targets,
+                      float* d_e, float* d_c, float* d_bias, void* workspace, int64_t workspace_bytes,
+                      int64_t n_rows, int64_t b, int64_t v, int64_t d,
+                      int64_t stride_e, int64_t stride_cv, int64_t stride_cd, int64_t ld_de, int64_t ld_dc,
+                      float grad_scale, int64_t shift, int64_t target_offset, float softcap, int terms, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -66,6 +66,12 @@ struct ProductParams {
   int de_len, dc_len;        // classes / rows per split, multiples of 64
   int64_t de_slot, dc_slot;
   int de_init;               // an fp32 d_e is written, not added to (the first launch on a set of slots)
+  // Operands and dz in 16-bit parts (TERMS): a row of c / e is [hi | mid | lo] of part_d columns each, a row of dz
+  // [hi | mid | lo] of dz_part classes each; e is compact and b, n_cls are multiples of 64 (rows and classes that pad
+  // them are zeros).  rows_out, cls_out: what of them exists; d may be anything (out_vec: 16-byte pieces may be stored).
+  int terms, part_d, dz_part, out_vec;
+  int64_t rows_out;
+  int cls_out;
 };
 
 constexpr int kProdThreads = 256;  // four waves, one per SIMD
@@ -107,6 +113,124 @@ __device__ __forceinline__ bool product_tile_of(int block, int items, int splits
   tm = lin / width;
   tn = first_col + (lin - tm * width);
   return true;
+}
+
+// Eight consecutive floats of a row from column `col` on, of `d` columns in all; `vec`: rows are 16-byte aligned and d a
+// multiple of 8.
+__device__ __forceinline__ void load_piece(const float* row, int col, int d, bool vec, float (&v)[8]) {
+  if (vec) {
+    const float4 a = *reinterpret_cast<const float4*>(row + col), b = *reinterpret_cast<const float4*>(row + col + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = (col + k < d) ? row[col + k] : 0.0f;
+  }
+}
+__device__ __forceinline__ void store_piece(float* row, int col, int d, bool vec, const float (&v)[8]) {
+  if (vec) {
+    *reinterpret_cast<float4*>(row + col) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(row + col + 4) = make_float4(v[4], v[5], v[6], v[7]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (col + k < d) row[col + k] = v[k];
+  }
+}
+
+// The two products of operands in parts, fp32 results: the tiles below without what 16-bit gradients need.
+__device__ __forceinline__ void terms_de_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
+  using Tile = Tile4<BF16, false, true, false, true>;
+  typename Tile::Geometry g = Tile::geometry(smem);
+  const int64_t m0 = static_cast<int64_t>(tm) * Tile::TILE;
+  const int n0 = tn * Tile::TILE;
+  const int k0 = split * p.de_len;
+  typename Tile::Source s;
+#pragma unroll
+  for (int q = 0; q < Tile::NQ1; ++q) {
+    int64_t i = m0 + Tile::row_direct(q, g.wave, g.lane);
+    i = (i < p.b) ? i : p.b - 1;  // rows past the end repeat the last one; their results are dropped
+    s.a_row[q] = p.dz + i * p.ldz + k0 + Tile::chunk_direct(g.wave, g.lane);
+  }
+  s.b_row[0] = nullptr;
+  s.a_km = nullptr;
+  s.a_stride = 0;
+  s.b_km = p.c + k0 * p.stride_cv + min(n0 + Tile::chunk_kmajor(g.wave, g.lane), p.part_d - 8);
+  s.b_stride = p.stride_cv;
+  s.b_rows = nullptr;
+  s.k_total = min(p.de_len, p.n_cls - k0);
+  s.a_part = p.dz_part;
+  s.b_part = p.part_d;
+  s.terms = p.terms;
+  float* const de = p.de_f32 + split * p.de_slot;
+
+  f32x16 acc[Tile::WM][Tile::WN];
+  typename Tile::Loop loop = Tile::plan(s, g);
+  typename Tile::Ids ids;
+  typename Tile::Ptrs ptrs;
+  Tile::prefetch(s, loop, ptrs, ids, g);
+  Tile::run(acc, s, loop, ptrs, ids, smem, g);
+  Tile::for_each_row_piece(acc, smem, g, [&](int row, int col, const float (&v)[8]) {
+    const int64_t ri = m0 + row;
+    const int cg = n0 + col;
+    if (ri >= p.rows_out || cg >= p.d) return;
+    const int64_t re = (p.valids != nullptr && !p.de_rows_by_number) ? static_cast<int64_t>(p.valids[ri]) : ri;
+    float out[8];
+    if (p.de_init) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) out[k] = v[k];
+    } else {
+      load_piece(de + re * p.ld_de, cg, p.d, p.out_vec != 0, out);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) out[k] += v[k];
+    }
+    store_piece(de + re * p.ld_de, cg, p.d, p.out_vec != 0, out);
+  });
+}
+
+__device__ __forceinline__ void terms_dc_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
+  using Tile = Tile4<BF16, true, true, false, true>;
+  typename Tile::Geometry g = Tile::geometry(smem);
+  const int m0 = tm * Tile::TILE;
+  const int n0 = tn * Tile::TILE;
+  const int64_t k0 = static_cast<int64_t>(split) * p.dc_len;
+  const int chunk = Tile::chunk_kmajor(g.wave, g.lane);
+  typename Tile::Source s;
+  s.a_row[0] = nullptr;
+  s.b_row[0] = nullptr;
+  s.a_km = p.dz + k0 * p.ldz + min(m0 + chunk, p.dz_part - 8);
+  s.a_stride = p.ldz;
+  s.b_km = p.e + k0 * p.stride_e + min(n0 + chunk, p.part_d - 8);
+  s.b_stride = p.stride_e;
+  s.b_rows = nullptr;
+  s.k_total = static_cast<int>(min(static_cast<int64_t>(p.dc_len), p.b - k0));
+  s.a_part = p.dz_part;
+  s.b_part = p.part_d;
+  s.terms = p.terms;
+  float* const dc = static_cast<float*>(p.d_c) + split * p.dc_slot;
+
+  f32x16 acc[Tile::WM][Tile::WN];
+  typename Tile::Loop loop = Tile::plan(s, g);
+  typename Tile::Ids ids;
+  typename Tile::Ptrs ptrs;
+  Tile::prefetch(s, loop, ptrs, ids, g);
+  Tile::run(acc, s, loop, ptrs, ids, smem, g);
+  Tile::for_each_row_piece(acc, smem, g, [&](int row, int col, const float (&v)[8]) {
+    const int cls = m0 + row;
+    const int cg = n0 + col;
+    if (cls >= p.cls_out || cg >= p.d) return;
+    float* dst = dc + static_cast<int64_t>(cls) * p.ld_dc;
+    float out[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) out[k] = v[k];
+    if (p.dc_accumulate) {
+      float old[8];
+      load_piece(dst, cg, p.d, p.out_vec != 0, old);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) out[k] += old[k];
+    }
+    store_piece(dst, cg, p.d, p.out_vec != 0, out);
+  });
 }
 
 // dE[row][col] += sum_class dz[row][class] * C[class][col]
@@ -327,36 +451,52 @@ __global__ __launch_bounds__(kProdThreads, 1) void dense_products_kernel(Product
   }
 }
 
+// The same for operands in parts.
+__global__ __launch_bounds__(kProdThreads, 1) void terms_products_kernel(ProductParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int first_blocks = (p.de_first ? p.de_per_xcd : p.dc_per_xcd) * 8;
+  const bool first = static_cast<int>(blockIdx.x) < first_blocks;
+  const int block = first ? blockIdx.x : blockIdx.x - first_blocks;
+  int split, tm, tn;
+  if (first != (p.de_first != 0)) {
+    if (!product_tile_of(block, p.dc_tiles, p.dc_splits, p.dc_per_xcd, p.tiles_n, split, tm, tn)) return;
+    terms_dc_tile(p, split, tm, tn, smem);
+  } else {
+    if (!product_tile_of(block, p.de_tiles, p.de_splits, p.de_per_xcd, p.tiles_n, split, tm, tn)) return;
+    terms_de_tile(p, split, tm, tn, smem);
+  }
+}
+
 // out[row(i)][:] (+)= sum over the slots of slot[s][i][:], in the order of the slots; eight columns per thread.  Bound
 // by reading the slots: 4 bytes per element and slot.
 template <typename T>
-__global__ __launch_bounds__(256) void split_sum_kernel(const float* slots, int splits, int64_t rows, int d, const int32_t* ids,
-                                                        void* out, int64_t ld_out, int out_fp32, int add) {
-  const int per_row = d / 8;
+__global__ __launch_bounds__(256) void split_sum_kernel(const float* slots, int splits, int64_t rows, int d, int ld_slot,
+                                                        const int32_t* ids, void* out, int64_t ld_out, int out_fp32, int add,
+                                                        int out_vec) {
+  const int per_row = (d + 7) / 8;
   const int64_t item = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (item >= rows * per_row) return;
   const int64_t i = item / per_row;
   const int col = static_cast<int>(item - i * per_row) * 8;
   float v[8] = {};
   for (int s = 0; s < splits; ++s) {
-    const float4* src = reinterpret_cast<const float4*>(slots + (s * rows + i) * d + col);
-    const float4 a = src[0], b = src[1];
-    v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
-    v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
+    float x[8];
+    load_piece(slots + (s * rows + i) * ld_slot, col, ld_slot, true, x);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] += x[k];
   }
-  const int64_t off = (ids != nullptr ? static_cast<int64_t>(ids[i]) : i) * ld_out + col;
+  const int64_t row = (ids != nullptr ? static_cast<int64_t>(ids[i]) : i);
   if (out_fp32) {
-    float4* dst = reinterpret_cast<float4*>(static_cast<float*>(out) + off);
-    float4 a = make_float4(v[0], v[1], v[2], v[3]), b = make_float4(v[4], v[5], v[6], v[7]);
+    float* dst = static_cast<float*>(out) + row * ld_out;
     if (add) {
-      const float4 a0 = dst[0], b0 = dst[1];
-      a.x += a0.x; a.y += a0.y; a.z += a0.z; a.w += a0.w;
-      b.x += b0.x; b.y += b0.y; b.z += b0.z; b.w += b0.w;
+      float old[8];
+      load_piece(dst, col, d, out_vec != 0, old);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] += old[k];
     }
-    dst[0] = a;
-    dst[1] = b;
+    store_piece(dst, col, d, out_vec != 0, v);
   } else {
-    *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + off) =
+    *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + row * ld_out + col) =
         make_uint4(Elem<T>::pack2(v[0], v[1]), Elem<T>::pack2(v[2], v[3]), Elem<T>::pack2(v[4], v[5]), Elem<T>::pack2(v[6], v[7]));
   }
 }
@@ -449,12 +589,12 @@ static int64_t split_stages(int64_t stages, int splits) { return (stages + split
 // product tile (64 steps of 256 x 256; 1.65 us where all units are busy): the dz tiles in rounds of all units, d / 64
 // stages each, then the product items as they are handed out.  An item of a cut reduction leaves 256 KB of fp32 (and
 // takes them in first, where slots are carried): up to 6 stages of time where every unit does so at once.
-static double launch_cost(int64_t rows, int64_t cls, int64_t d, int de_splits, int dc_splits, bool carried) {
+static double launch_cost(int64_t rows, int64_t cls, int64_t d, int de_splits, int dc_splits, bool carried, int terms = 1) {
   const int64_t cus = compute_units();
   const int64_t tr = (rows + 255) / 256, tc = (cls + 255) / 256, tn = (d + 255) / 256;
-  const int64_t dz = (tr * tc + cus - 1) / cus * tn * 4;
+  const int64_t dz = (tr * tc + cus - 1) / cus * tn * 4 * terms;
   auto item = [&](int64_t total, int splits, int64_t tiles) {
-    const int64_t len = split_stages((total + 63) / 64, splits);
+    const int64_t len = split_stages((total + 63) / 64, splits) * terms;
     if (splits == 1) return len;
     const int64_t items = tiles * splits;
     return len + (4 + 6 * (items < cus ? items : cus) / cus) * (carried ? 2 : 1);
@@ -579,6 +719,104 @@ static DensePlan dense_plan(int64_t b, int64_t v, int64_t d, bool g16, int64_t m
   return answer;
 }
 
+// ---- the products of one chunk of classes with operands and dz in bf16 parts (cce_fp32.hip) ---------------------
+// The walk over the classes for a dz of `dz_bytes_per_class` and a copy of C of `c_bytes_per_class`, either at most
+// `most_bytes`, in chunks that are multiples of 256 classes; the reductions are cut as in cce_backward_dense.
+TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class, int64_t c_bytes_per_class,
+                     int64_t most_bytes, bool cut_dc) {
+  TermsPlan pl = {256, 1, 1};
+  static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+  const int64_t v_pad = (v + 255) / 256 * 256;
+  int64_t most = most_bytes / std::max(dz_bytes_per_class, c_bytes_per_class) / 256 * 256;
+  most = std::min(std::max<int64_t>(most, 256), v_pad);
+  const int64_t least = (v_pad + most - 1) / most;
+  double best = 1e300;
+  for (int64_t n = least; n <= least + 2; ++n) {
+    const int64_t unit = ((v_pad + n - 1) / n + 255) / 256 * 256;
+    const int64_t launches = (v + unit - 1) / unit;
+    for (int se : kSplits) {
+      if (se > 1 && ((unit + 63) / 64 * terms < se * kMinSplitStages || se * b * d * 4 > most_bytes || unit / 64 < se)) break;
+      for (int sc : kSplits) {
+        if (sc > 1 && (!cut_dc || launches > 1 || (b + 63) / 64 * terms < sc * kMinSplitStages || sc * v * d * 4 > most_bytes ||
+                       b / 64 < sc))
+          break;
+        const int64_t rest = v - (launches - 1) * unit;
+        double cost = static_cast<double>(launches - 1) * (1.0 + launch_cost(b, unit, d, se, sc, launches > 1, terms)) + 1.0 +
+                      launch_cost(b, rest, d, se, sc, launches > 1, terms);
+        cost += split_sum_cost(b, d, se) + split_sum_cost(v, d, sc);
+        if (se > 1 || sc > 1) cost *= 1.03;
+        if (cost < best * (1.0 - 1e-9)) {
+          best = cost;
+          pl.unit = unit;
+          pl.de_splits = se;
+          pl.dc_splits = sc;
+        }
+      }
+    }
+  }
+  return pl;
+}
+
+int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t* c_parts, int64_t ld_c, const uint16_t* e_parts,
+                          int64_t ld_e, const int32_t* valids, float* d_e, int64_t ld_de, bool de_by_number, bool de_init,
+                          int64_t de_slot, int de_len, float* d_c, int64_t ld_dc, bool dc_add, int64_t dc_slot, int dc_len,
+                          bool out_vec, int64_t b, int64_t b_pad, int64_t cls, int64_t cls_pad, int64_t d, int64_t part_d, int terms,
+                          int parts, hipStream_t stream) {
+  ProductParams p = {};
+  p.dz = dz_parts;
+  p.ldz = parts * ldz;
+  p.dz_part = static_cast<int>(ldz);
+  p.c = c_parts;
+  p.stride_cv = ld_c;
+  p.e = e_parts;
+  p.stride_e = ld_e;
+  p.valids = valids;
+  p.de_f32 = d_e;
+  p.ld_de = ld_de;
+  p.de_rows_by_number = de_by_number ? 1 : 0;
+  p.de_init = de_init ? 1 : 0;
+  p.d_c = d_c;
+  p.ld_dc = ld_dc;
+  p.dc_accumulate = dc_add ? 1 : 0;
+  p.b = b_pad;
+  p.rows_out = b;
+  p.n_cls = static_cast<int>(cls_pad);
+  p.cls_out = static_cast<int>(cls);
+  p.d = static_cast<int>(d);
+  p.part_d = static_cast<int>(part_d);
+  p.terms = terms;
+  p.out_vec = out_vec ? 1 : 0;
+  p.de_len = de_len;
+  p.dc_len = dc_len;
+  p.de_slot = de_slot;
+  p.dc_slot = dc_slot;
+  p.de_splits = static_cast<int>((cls_pad + de_len - 1) / de_len);
+  p.dc_splits = static_cast<int>((b_pad + dc_len - 1) / dc_len);
+  p.tiles_n = static_cast<int>((d + 255) / 256);
+  p.dc_tiles = d_c != nullptr ? static_cast<int>((cls + 255) / 256) * p.tiles_n * p.dc_splits : 0;
+  p.de_tiles = d_e != nullptr ? static_cast<int>((b + 255) / 256) * p.tiles_n * p.de_splits : 0;
+  p.dc_per_xcd = (p.dc_tiles + 7) / 8;
+  p.de_per_xcd = (p.de_tiles + 7) / 8;
+  p.de_first = std::min<int64_t>(de_len, cls_pad) > std::min<int64_t>(dc_len, b_pad) ? 1 : 0;
+  const int blocks = (p.dc_per_xcd + p.de_per_xcd) * 8;
+  if (blocks == 0) return CCE_OK;
+  const int lds = Tile4<BF16, true, true>::LDS_BYTES;
+  auto kern = terms_products_kernel;
+  static LdsLimitOnce lds_limit;
+  const hipError_t err = lds_limit.set(kern, lds);
+  if (err != hipSuccess) return status_from_hip(err);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kProdThreads), lds, stream, p);
+  return status_from_hip(hipGetLastError());
+}
+
+int split_sum_launch(const float* slots, int count, int64_t rows, int64_t d, int64_t ld_slot, const int32_t* ids, float* out,
+                     int64_t ld, bool add, bool out_vec, hipStream_t stream) {
+  const unsigned blocks = static_cast<unsigned>((rows * ((d + 7) / 8) + 255) / 256);
+  hipLaunchKernelGGL(split_sum_kernel<BF16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d),
+                     static_cast<int>(ld_slot), ids, out, ld, 1, add ? 1 : 0, out_vec ? 1 : 0);
+  return status_from_hip(hipGetLastError());
+}
+
 }  // namespace cce
 
 using namespace cce;
@@ -655,7 +893,7 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
   const bool dc_cut = d_c != nullptr && plan.dc_splits > 1;
   const bool pair_de = split_de && !de_cut;  // dE leaves the products as 16-bit numbers
 
-  ProductParams p;
+  ProductParams p = {};
   p.dz = dz;
   p.ldz = ldz;
   p.stride_cv = stride_cv;
@@ -788,11 +1026,11 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
   auto sum_slots = [&](const float* slots, int count, int64_t rows, const int32_t* ids, void* out, int64_t ld, int fp32, int add) {
     const unsigned blocks = static_cast<unsigned>((rows * (d / 8) + 255) / 256);
     if (dtype == CCE_DTYPE_BF16)
-      hipLaunchKernelGGL(split_sum_kernel<BF16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d), ids, out,
-                         ld, fp32, add);
+      hipLaunchKernelGGL(split_sum_kernel<BF16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d),
+                         static_cast<int>(d), ids, out, ld, fp32, add, 1);
     else
-      hipLaunchKernelGGL(split_sum_kernel<F16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d), ids, out,
-                         ld, fp32, add);
+      hipLaunchKernelGGL(split_sum_kernel<F16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d),
+                         static_cast<int>(d), ids, out, ld, fp32, add, 1);
   };
   if (de_cut) sum_slots(de_slots, de_nslots, b, valids, d_e, stride_e, d_e_is_fp32, 1);
   if (dc_cut) sum_slots(dc_slots, dc_nslots, v, nullptr, d_c, stride_cv, d_c_is_fp32, 0);
@@ -819,7 +1057,7 @@ extern "C" int cce_backward_products(const void* dz, int64_t ldz, const void* c,
   if (d_c != nullptr && (!aligned16(e) || stride_e % 8 != 0 || !aligned16(d_c) || ld_dc % 4 != 0 || ld_dc < d))
     return CCE_ERR_MISALIGNED;
 
-  ProductParams p;
+  ProductParams p = {};
   p.dz = static_cast<const uint16_t*>(dz);
   p.ldz = ldz;
   p.c = static_cast<const uint16_t*>(c);

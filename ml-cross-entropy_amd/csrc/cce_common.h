@@ -553,8 +553,22 @@ struct DmaLogitTile {
 // first two stages of the NEXT tile (next_tile() swaps the class pointers), so that nothing is fetched that is
 // not consumed and the next main loop starts with its data in LDS, whatever the epilogue in between does.
 // `buf` carries the ring stage the next tile starts in (it alternates when D / 64 is odd).
+//
+// TERMS: the operands are fp32 values split into 16-bit parts, [hi | mid | lo] side by side in a row, D columns each, and
+// the reduction runs over the cross terms of the parts one after the other (term_part() below): the stages of a
+// tile walk columns 0 .. D of the two parts of term 0, then of term 1, and so on, so that a part is stored once however
+// many terms it takes part in.
 // ---------------------------------------------------------------------------------------------
-template <typename T, int WV, int WT, int NWV, int NWT>
+// Which part (0 hi, 1 mid, 2 lo) of the first and of the second operand meets in term t, smallest terms first, so that
+// the accumulator is rounded at its full size only while the last one is added:
+//   hi lo, lo hi, mid mid, hi mid, mid hi, hi hi          (two bits per term; the last three are the 16-bit product)
+constexpr int kTermsAll = 6;
+constexpr unsigned kTermsFirst = 0x118u, kTermsSecond = 0x052u;
+__host__ __device__ __forceinline__ int term_part(unsigned table, int term) {
+  return static_cast<int>((table >> (2 * term)) & 3u);
+}
+
+template <typename T, int WV, int WT, int NWV, int NWT, bool TERMS = false>
 struct DmaLogitTile16 {
   static_assert(WV % 2 == 0 && WT % 2 == 0, "the ring is addressed in blocks of 32 rows");
   using Base = DmaLogitTile<T, WV / 2, WT / 2, NWV, NWT>;
@@ -585,11 +599,41 @@ struct DmaLogitTile16 {
     unsigned c_stride_bytes;
     unsigned row_in_block;  // lane >> 3
     unsigned chunk_bytes;   // byte offset of this lane's 16-byte chunk inside a 128-byte row segment
+    int terms;              // TERMS only: 3 or 6
   };
+
+  // Where a stage starts in the rows of either operand (elements), stage after stage.
+  struct Walk {
+    int col, term;   // TERMS only
+    int off_c, off_e;
+  };
+  static __device__ __forceinline__ void walk_offsets(Walk& w, int D) {
+    w.off_e = term_part(kTermsFirst, w.term) * D + w.col;
+    w.off_c = term_part(kTermsSecond, w.term) * D + w.col;
+  }
+  static __device__ __forceinline__ void walk_next(Walk& w, int D, int terms) {
+    w.col += kDmaBK;
+    if (w.col == D) {
+      w.col = 0;
+      w.term = (w.term + 1 == kTermsAll) ? kTermsAll - terms : w.term + 1;
+    }
+    walk_offsets(w, D);
+  }
+  static __device__ __forceinline__ Walk walk_start(int D, int terms) {
+    Walk w = {0, TERMS ? kTermsAll - terms : 0, 0, 0};
+    if constexpr (TERMS) walk_offsets(w, D);
+    return w;
+  }
 
   // Points the class loads of `src` at the tile whose first class row is `tile` and which has `left` >= 1 classes
   // inside the matrix (256 or more: a whole tile).
+  // (TERMS: the parts live in a workspace whose rows go on to the end of the last tile, so nothing is clamped and the
+  // blocks of a tile are one base and a step: a dozen scalar registers, which the walk over the terms needs)
   static __device__ __forceinline__ void set_class_tile(Source& src, const unsigned char* tile, int left, int wave) {
+    if constexpr (TERMS) {
+      src.c_blk[0] = tile + static_cast<int64_t>(8 * wave) * src.c_stride_bytes;
+      return;
+    }
 #pragma unroll
     for (int q = 0; q < NQC; ++q) {
       const int first = 8 * (q * NW + wave);
@@ -603,15 +647,18 @@ struct DmaLogitTile16 {
     return __builtin_bit_cast(vec8, *reinterpret_cast<const uint4*>(p));
   }
 
-  // Load q of one stage, columns [k0, k0 + 64), into ring stage `stage_off`.
-  static __device__ __forceinline__ void issue_one(const Source& src, int q, int k0, unsigned lds_base, int stage_off,
+  // Load q of one stage, 64 columns from kc (class rows) and ke (token rows) on, into ring stage `stage_off`.
+  static __device__ __forceinline__ void issue_one(const Source& src, int q, int kc, int ke, unsigned lds_base, int stage_off,
                                                    int wave) {
-    if (q < NQC) {
+    if (TERMS && q < NQC) {
+      lds_dma16_sbase(src.c_blk[0] + (2 * kc + static_cast<uint64_t>(q * 8 * NW) * src.c_stride_bytes),
+                      src.row_in_block * src.c_stride_bytes + src.chunk_bytes, lds_base + stage_off + (q * NW + wave) * 1024);
+    } else if (q < NQC) {
       const unsigned row = min(src.row_in_block, static_cast<unsigned>(src.c_lim[q]));
-      lds_dma16_sbase(src.c_blk[q] + 2 * k0, row * src.c_stride_bytes + src.chunk_bytes,
+      lds_dma16_sbase(src.c_blk[q] + 2 * kc, row * src.c_stride_bytes + src.chunk_bytes,
                       lds_base + stage_off + (q * NW + wave) * 1024);
     } else {
-      lds_dma16_sbase(src.e_base + 2 * k0, src.e_off[q - NQC],
+      lds_dma16_sbase(src.e_base + 2 * ke, src.e_off[q - NQC],
                       lds_base + stage_off + (TILE_V / 8 + (q - NQC) * NW + wave) * 1024);
     }
   }
@@ -620,7 +667,7 @@ struct DmaLogitTile16 {
   // memory instruction after each MFMA:
   //   READ  the fragments of the next step from rd_c / rd_e (ring stage + this lane's chunk): class fragment vi
   //         into a[vi] once the last MFMA that uses the old one is issued, the token fragments into bn[];
-  //   LOAD  all loads of a later stage (columns koff ..) into ring stage `ld_stage`.
+  //   LOAD  all loads of a later stage (columns kc .. / ke ..) into ring stage `ld_stage`.
   // SYNC (the step on the second half of a stage): after the first WT MFMAs, which need nothing new, this wave
   // waits for its own loads of the next stage and for the fragment reads it still has in flight, then the
   // barrier: from there on the next stage may be read and the stage this step computes on (every wave holds
@@ -645,7 +692,7 @@ struct DmaLogitTile16 {
   template <bool READ, bool LOAD, bool SYNC, bool ZERO = false>
   static __device__ __forceinline__ void step(f32x4 (&acc)[WV][WT], vec8 (&a)[WV], const vec8 (&bc)[WT], vec8 (&bn)[WT],
                                               const unsigned char* rd_c, const unsigned char* rd_e, const Source& src,
-                                              int koff, unsigned lds_base, int ld_stage, int wave) {
+                                              int kc, int ke, unsigned lds_base, int ld_stage, int wave) {
     static_for<WV * WT>([&](auto idx_c) {
       constexpr int idx = decltype(idx_c)::value;
       constexpr int vi = idx / WT, ti = idx % WT;
@@ -668,7 +715,7 @@ struct DmaLogitTile16 {
       if (LOAD) {
         static_for<NQ>([&](auto j_c) {
           constexpr int j = decltype(j_c)::value;
-          if (idx == load_slot(j)) issue_one(src, j, koff, lds_base, ld_stage, wave);
+          if (idx == load_slot(j)) issue_one(src, j, kc, ke, lds_base, ld_stage, wave);
         });
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -676,16 +723,19 @@ struct DmaLogitTile16 {
   }
 
   // Start the ring for the first tile of a span: its first two stages, into ring stages 0 and 1.
-  static __device__ __forceinline__ void prefetch(const Source& src, unsigned char* lds) {
+  static __device__ __forceinline__ void prefetch(const Source& src, unsigned char* lds, int D) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
+    Walk w = walk_start(D, src.terms);
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) issue_one(src, q, 0, lds_base, 0, wave);
+    for (int q = 0; q < NQ; ++q) issue_one(src, q, w.off_c, w.off_e, lds_base, 0, wave);
+    if constexpr (TERMS) walk_next(w, D, src.terms);
+    else w.off_c = w.off_e = kDmaBK;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) issue_one(src, q, kDmaBK, lds_base, STAGE_BYTES, wave);
+    for (int q = 0; q < NQ; ++q) issue_one(src, q, w.off_c, w.off_e, lds_base, STAGE_BYTES, wave);
   }
 
-  // D must be a multiple of 64 and at least 128.  The first two stages of this tile must be in flight or landed in
+  // D must be a multiple of 64 and, without TERMS, at least 128.  The first two stages of this tile must be in flight or landed in
   // ring stages buf, 1 - buf (prefetch() for the first tile of a span: first_tile; else the previous run()), and
   // nothing else may have touched the ring.
   // next_tile() is called once, when the class rows of this tile have been fetched for the last time: it points
@@ -707,7 +757,20 @@ struct DmaLogitTile16 {
     const unsigned char* e_row = lds + (TILE_V + wt * WT * 16 + r16) * kDmaRowBytes;
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
 
-    const int nk = D / kDmaBK;
+    const int nk = TERMS ? src.terms * (D / kDmaBK) : D / kDmaBK;  // >= 2
+    Walk w = walk_start(D, src.terms);
+    if constexpr (TERMS) {
+      walk_next(w, D, src.terms);
+      walk_next(w, D, src.terms);
+    }
+    // columns of the stage two ahead of stage s (a stage of the next tile under the last two)
+    auto ahead = [&](int s) {
+      if constexpr (TERMS) {
+        if (s > 0) walk_next(w, D, src.terms);
+      } else {
+        w.off_c = w.off_e = (s + 2 < nk) ? (s + 2) * kDmaBK : (s + 2 - nk) * kDmaBK;
+      }
+    };
     int cur = buf * STAGE_BYTES;
     if (first_tile) {
       wait_vmcnt<NQ>();  // the first stage has landed for this wave (the second may be in flight) ...
@@ -721,28 +784,31 @@ struct DmaLogitTile16 {
 #pragma unroll
     for (int vi = 0; vi < WV; ++vi) a[vi] = frag(c_row + cur + chunk0 + vi * 16 * kDmaRowBytes);
 
-    // first stage (never the last: D >= 128)
+    // first stage (never the last: there are at least two)
     {
       const int nxt = STAGE_BYTES - cur;
-      step<true, false, false, true>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, lds_base, 0, wave);
+      step<true, false, false, true>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, 0, lds_base, 0, wave);
       if (nk == 2) next_tile();
-      step<true, true, true>(acc, a, b1, b0, c_row + nxt + chunk0, e_row + nxt + chunk0, src, (2 < nk) ? 2 * kDmaBK : 0,
-                             lds_base, cur, wave);
+      ahead(0);
+      step<true, true, true>(acc, a, b1, b0, c_row + nxt + chunk0, e_row + nxt + chunk0, src, w.off_c, w.off_e, lds_base, cur,
+                             wave);
       cur = nxt;
     }
 #pragma unroll 1
     for (int s = 1; s < nk - 1; ++s) {
       const int nxt = STAGE_BYTES - cur;
-      step<true, false, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, lds_base, 0, wave);
+      step<true, false, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, 0, lds_base, 0, wave);
       if (s == nk - 2) next_tile();
-      const int koff = (s + 2 < nk) ? (s + 2) * kDmaBK : 0;
-      step<true, true, true>(acc, a, b1, b0, c_row + nxt + chunk0, e_row + nxt + chunk0, src, koff, lds_base, cur, wave);
+      ahead(s);
+      step<true, true, true>(acc, a, b1, b0, c_row + nxt + chunk0, e_row + nxt + chunk0, src, w.off_c, w.off_e, lds_base, cur,
+                             wave);
       cur = nxt;
     }
     // the last stage: its second step reads nothing (the next tile's first fragments would sit in registers
     // through the epilogue) and fetches the second stage of the next tile
-    step<true, false, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, lds_base, 0, wave);
-    step<false, true, true>(acc, a, b1, b0, c_row, e_row, src, kDmaBK, lds_base, cur, wave);
+    step<true, false, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, 0, lds_base, 0, wave);
+    ahead(nk - 1);
+    step<false, true, true>(acc, a, b1, b0, c_row, e_row, src, w.off_c, w.off_e, lds_base, cur, wave);
     buf = 1 - cur / STAGE_BYTES;
   }
 };

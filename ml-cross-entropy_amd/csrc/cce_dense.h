@@ -16,4 +16,43 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
                     float grad_scale, int64_t shift, int64_t target_offset,
                     float softcap, int dtype, hipStream_t stream);
 
+// ---- fp32 operands as 16-bit parts (cce_fp32.hip) ---------------------------------------------------------------
+// A row of e_parts / c_parts holds its parts [hi | mid | lo] side by side, part_d (a multiple of 64) columns each;
+// ld_e / ld_c elements from row to row, a multiple of 8.  terms: 6 cross terms of three parts, or 3 of two.
+
+// Spans per row block that lse_terms_launch makes of v classes: the float2 partials [spans][b] it writes.
+int lse_terms_splits(int64_t b, int64_t v);
+int lse_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
+                     float2* partial, int64_t b, int64_t v, int64_t part_d, int terms, float softcap, hipStream_t stream);
+// lse[b] of partials [nsplit][b]
+int lse_merge_launch(const float2* partial, float* lse, int64_t b, int nsplit, hipStream_t stream);
+
+// dz of v classes as bf16 parts [b_store][parts][ldz], ldz = v rounded up to 64; columns past v and rows b .. b_store
+// (b rounded up to 64) are zeros.  valids: the rows of the batch that the (compact) rows of e_parts are.
+int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
+                    const float* lse, const float* d_out, int d_out_is_scalar, const float* d_lse,
+                    const int32_t* valids, const int64_t* targets, uint16_t* dz_parts, int64_t ldz,
+                    int64_t n_rows, int64_t b, int64_t b_store, int64_t v, int64_t part_d, int terms, int parts,
+                    float grad_scale, int64_t shift, int64_t target_offset, float softcap, hipStream_t stream);
+
+// Chunks of classes and cuts of the reductions of dE and dC for terms_products_launch.
+struct TermsPlan {
+  int64_t unit;
+  int de_splits, dc_splits;
+};
+TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class, int64_t c_bytes_per_class,
+                     int64_t most_bytes, bool cut_dc);
+
+// dE (+)= dz . C and dC (+)= dz^T . E of one chunk, fp32 results.  dz_parts as written by dz_terms_launch, c_parts and
+// e_parts with zero rows up to cls_pad and b_pad (multiples of 64).  Range s of a reduction (de_len classes, dc_len rows,
+// multiples of 64) goes to d_e + s * de_slot / d_c + s * dc_slot.  d_e is indexed by row number, or through valids.
+int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t* c_parts, int64_t ld_c, const uint16_t* e_parts,
+                          int64_t ld_e, const int32_t* valids, float* d_e, int64_t ld_de, bool de_by_number, bool de_init,
+                          int64_t de_slot, int de_len, float* d_c, int64_t ld_dc, bool dc_add, int64_t dc_slot, int dc_len,
+                          bool out_vec, int64_t b, int64_t b_pad, int64_t cls, int64_t cls_pad, int64_t d, int64_t part_d, int terms,
+                          int parts, hipStream_t stream);
+// out[row(i)][0 .. d) (+)= sum over the slots [count][rows][ld_slot]
+int split_sum_launch(const float* slots, int count, int64_t rows, int64_t d, int64_t ld_slot, const int32_t* ids, float* out,
+                     int64_t ld, bool add, bool out_vec, hipStream_t stream);
+
 }  // namespace cce

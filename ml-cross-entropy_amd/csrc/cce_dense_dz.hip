@@ -32,7 +32,15 @@ struct DzParams {
                   // up to column ldz: the product kernels read dz in whole 64-class stages
   int nrb, nvt, nsplit, nitems, items_per_xcd;
   Softcap sc;
+  // operands and dz in 16-bit parts (kDzParts): d is the width of a part, rows of e are compact (valids only says which
+  // targets and upstream gradients they belong to), dz is [b_store][parts][ldz], rows past b zeros
+  const float* bias32;
+  int terms, parts;
+  int64_t b_store;
 };
+
+// How dz leaves: in the input type, as fp32, or as an fp32 value in two or three bf16 parts
+enum DzOut { kDz16Bit, kDzFp32, kDzParts };
 
 constexpr int kDzWV = 4, kDzWT = 2, kDzNWV = 2, kDzNWT = 4;  // the forward kernel's wave tiling
 constexpr int kDzThreads = 64 * kDzNWV * kDzNWT;
@@ -255,9 +263,11 @@ struct DzRow {
   int tgt;
 };
 
-template <typename T, bool GENERAL, bool OUT32>
+template <typename T, bool GENERAL, DzOut OUT>
 __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
-  using Fast = DmaLogitTile16<T, kDz16WV, kDz16WT, kDzNWV, kDzNWT>;
+  constexpr bool OUT32 = OUT == kDzFp32;
+  constexpr bool PARTS = OUT == kDzParts;
+  using Fast = DmaLogitTile16<T, kDz16WV, kDz16WT, kDzNWV, kDzNWT, PARTS>;
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_addend = reinterpret_cast<float*>(smem + Fast::LDS_BYTES);                                   // [2][256]
   DzRow* s_rows = reinterpret_cast<DzRow*>(smem + Fast::LDS_BYTES + 2 * kDzTile * 4);                    // [256]
@@ -288,11 +298,12 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   src.chunk_bytes = 2u * static_cast<unsigned>(Fast::chunk_elems(wave, lane));
   src.row_in_block = static_cast<unsigned>(lane >> 3);
   src.c_stride_bytes = static_cast<unsigned>(p.stride_cv * 2);
+  src.terms = PARTS ? p.terms : 1;
 #pragma unroll
   for (int q = Fast::NQC; q < Fast::NQ; ++q) {
     int64_t i = t0 + Fast::row_of(q, wave, lane);
     i = (i < p.b) ? i : p.b - 1;  // rows past the end repeat the last one; their results are dropped
-    const int64_t row = p.valids ? static_cast<int64_t>(p.valids[i]) : i;
+    const int64_t row = (!PARTS && p.valids) ? static_cast<int64_t>(p.valids[i]) : i;
     src.e_off[q - Fast::NQC] = static_cast<unsigned>(row * p.stride_e * 2) + src.chunk_bytes;
   }
   auto set_class_tile = [&](int vt) {
@@ -304,7 +315,7 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   unsigned char* stage = s_stage + wave * kDz16StageBytes;
   int buf = 0;
   set_class_tile(vt_begin);
-  Fast::prefetch(src, smem);
+  Fast::prefetch(src, smem, static_cast<int>(p.d));
   // What the rows of this workgroup need, fixed for the whole item (published by the first barrier of the main loop;
   // fetched behind the first stages of the ring, so that the two latencies overlap).
   if (tid < kDzTile) {
@@ -331,7 +342,10 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
       if (tid < kDzTile) {  // published by the barriers of the main loop
         const int64_t vg = v0 + tid;
         float a = -INFINITY;
-        if (vg < p.v) a = (p.bias != nullptr) ? Elem<T>::to_float(p.bias[vg]) : 0.0f;
+        if (vg < p.v) {
+          if (PARTS) a = (p.bias32 != nullptr) ? p.bias32[vg] : 0.0f;
+          else a = (p.bias != nullptr) ? Elem<T>::to_float(p.bias[vg]) : 0.0f;
+        }
         addend[tid] = a;
       }
     }
@@ -357,6 +371,7 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
       const DzRow rr = s_rows[wt * (16 * kDz16WT) + ti * 16 + r16];
 #pragma unroll
       for (int vh = 0; vh < kParts; ++vh) {
+        float rest[PARTS ? kViPer : 1][4];  // PARTS: what the parts stored so far leave of the gradients
         // The gradients of one staged block.  One copy of the arithmetic per answer to "soft-capped?".
         auto stage_block = [&](auto capped) {
 #pragma unroll
@@ -390,7 +405,10 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
             }
             const int col = (vj * 16 + 4 * kq) * kEs;  // byte inside the staged row
             unsigned char* dst = stage + r16 * kDzStageRow + ((((col >> 4) ^ sw) << 4) | (col & 15));
-            if (OUT32) {
+            if (PARTS) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r) rest[vj][r] = dzv[r];
+            } else if (OUT32) {
               *reinterpret_cast<float4*>(dst) = make_float4(dzv[0], dzv[1], dzv[2], dzv[3]);
             } else {
               uint2 pk;
@@ -405,34 +423,61 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
         } else {
           stage_block(std::false_type{});
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the block is private to this wave: no barrier
         // 16 rows x 128 bytes leave as 16-byte pieces: one instruction covers 8 rows of 128 contiguous bytes
+        auto store_block = [&](int part) {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the block is private to this wave: no barrier
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int j = lane + 64 * k;
-          const int row = j >> 3;
-          const int pc = j & 7;
-          const uint4 val = *reinterpret_cast<const uint4*>(stage + row * kDzStageRow + ((pc ^ ((row >> 1) & 7)) << 4));
-          const int64_t gi = wrow0 + ti * 16 + row;
-          const int64_t gcol = static_cast<int64_t>(cls0) + vh * (16 * kViPer) + pc * kPieceElems;
-          if (gi < p.b) {
-            unsigned char* dst = static_cast<unsigned char*>(p.dz) + (gi * p.ldz + gcol) * kEs;
-            if (!GENERAL || gcol + kPieceElems <= p.v || (p.pad_store && gcol + kPieceElems <= p.ldz)) {
-              *reinterpret_cast<uint4*>(dst) = val;
-            } else if (OUT32) {
-              const uint32_t w[4] = {val.x, val.y, val.z, val.w};
+          for (int k = 0; k < 2; ++k) {
+            const int j = lane + 64 * k;
+            const int row = j >> 3;
+            const int pc = j & 7;
+            const uint4 val = *reinterpret_cast<const uint4*>(stage + row * kDzStageRow + ((pc ^ ((row >> 1) & 7)) << 4));
+            const int64_t gi = wrow0 + ti * 16 + row;
+            const int64_t gcol = static_cast<int64_t>(cls0) + vh * (16 * kViPer) + pc * kPieceElems;
+            if constexpr (PARTS) {
+              if (gi < p.b_store && gcol < p.ldz)
+                *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.dz) + (gi * p.parts + part) * p.ldz + gcol) = val;
+            } else if (gi < p.b) {
+              unsigned char* dst = static_cast<unsigned char*>(p.dz) + (gi * p.ldz + gcol) * kEs;
+              if (!GENERAL || gcol + kPieceElems <= p.v || (p.pad_store && gcol + kPieceElems <= p.ldz)) {
+                *reinterpret_cast<uint4*>(dst) = val;
+              } else if (OUT32) {
+                const uint32_t w[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (gcol + i < p.v) reinterpret_cast<uint32_t*>(dst)[i] = w[i];
-            } else {
-              const uint32_t w[4] = {val.x, val.y, val.z, val.w};
+                for (int i = 0; i < 4; ++i)
+                  if (gcol + i < p.v) reinterpret_cast<uint32_t*>(dst)[i] = w[i];
+              } else {
+                const uint32_t w[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll
-              for (int i = 0; i < 8; ++i)
-                if (gcol + i < p.v) reinterpret_cast<uint16_t*>(dst)[i] = static_cast<uint16_t>(w[i >> 1] >> ((i & 1) * 16));
+                for (int i = 0; i < 8; ++i)
+                  if (gcol + i < p.v) reinterpret_cast<uint16_t*>(dst)[i] = static_cast<uint16_t>(w[i >> 1] >> ((i & 1) * 16));
+              }
             }
           }
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // reads done before the next block is staged
+        };
+        if constexpr (PARTS) {
+          // x = hi + mid + lo, each the bf16 nearest to what the ones before it leave; one staged block per part
+#pragma unroll
+          for (int part = 0; part < 3; ++part) {
+            if (part >= p.parts) break;
+#pragma unroll
+            for (int vj = 0; vj < kViPer; ++vj) {
+              uint2 pk;
+              pk.x = Elem<T>::pack2(rest[vj][0], rest[vj][1]);
+              pk.y = Elem<T>::pack2(rest[vj][2], rest[vj][3]);
+              rest[vj][0] -= Elem<T>::to_float(static_cast<uint16_t>(pk.x));
+              rest[vj][1] -= Elem<T>::to_float(static_cast<uint16_t>(pk.x >> 16));
+              rest[vj][2] -= Elem<T>::to_float(static_cast<uint16_t>(pk.y));
+              rest[vj][3] -= Elem<T>::to_float(static_cast<uint16_t>(pk.y >> 16));
+              const int col = (vj * 16 + 4 * kq) * 2;
+              *reinterpret_cast<uint2*>(stage + r16 * kDzStageRow + ((((col >> 4) ^ sw) << 4) | (col & 15))) = pk;
+            }
+            store_block(part);
+          }
+        } else {
+          store_block(0);
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // reads done before the next block is staged
       }
     }
   }
@@ -460,7 +505,7 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
       stride_cv % 8 != 0 || stride_cd != 1 || ldz % (dz_is_fp32 ? 4 : 8) != 0)
     return CCE_ERR_MISALIGNED;
 
-  DzParams p;
+  DzParams p = {};
   p.e = static_cast<const uint16_t*>(e);
   p.c = static_cast<const uint16_t*>(c);
   p.bias = static_cast<const uint16_t*>(bias);
@@ -501,7 +546,7 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
 #define CCE_LAUNCH_DZ2(TT, GE, O32)                                                               \
   do {                                                                                            \
     if (k16) {                                                                                    \
-      auto kern = dense_dz16_kernel<TT, GE, O32>;                                                 \
+      auto kern = dense_dz16_kernel<TT, GE, (O32) ? kDzFp32 : kDz16Bit>;                          \
       static LdsLimitOnce lds_limit;                                                              \
       err = lds_limit.set(kern, lds16);                                                           \
       if (err != hipSuccess) return status_from_hip(err);                                         \
@@ -525,6 +570,62 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
   }
 #undef CCE_LAUNCH_DZ
 #undef CCE_LAUNCH_DZ2
+  return status_from_hip(hipGetLastError());
+}
+
+// ---- dz of one chunk of classes with operands and result in bf16 parts (cce_fp32.hip) --------------------------
+int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
+                    const float* lse, const float* d_out, int d_out_is_scalar, const float* d_lse,
+                    const int32_t* valids, const int64_t* targets, uint16_t* dz_parts, int64_t ldz,
+                    int64_t n_rows, int64_t b, int64_t b_store, int64_t v, int64_t part_d, int terms, int parts,
+                    float grad_scale, int64_t shift, int64_t target_offset, float softcap, hipStream_t stream) {
+  DzParams p = {};
+  p.e = e_parts;
+  p.c = c_parts;
+  p.bias32 = bias;
+  p.terms = terms;
+  p.parts = parts;
+  p.b_store = b_store;
+  p.valids = valids;
+  p.lse = lse;
+  p.d_out = d_out;
+  p.d_lse = d_lse;
+  p.targets = targets;
+  p.dz = dz_parts;
+  p.ldz = ldz;
+  p.n_rows = n_rows;
+  p.b = b;
+  p.v = v;
+  p.d = part_d;
+  p.stride_e = ld_e;
+  p.stride_cv = ld_c;
+  p.shift = shift;
+  p.target_offset = target_offset;
+  p.grad_scale = grad_scale;
+  p.d_out_is_scalar = d_out_is_scalar;
+  p.nrb = static_cast<int>((b + kDzTile - 1) / kDzTile);
+  p.nvt = static_cast<int>((v + kDzTile - 1) / kDzTile);
+  p.nsplit = choose_span_count(p.nrb, p.nvt);
+  p.nitems = p.nrb * p.nsplit;
+  p.items_per_xcd = (p.nitems + 7) / 8;
+  p.sc = make_softcap(softcap);
+  using Fast = DmaLogitTile16<BF16, kDz16WV, kDz16WT, kDzNWV, kDzNWT, true>;
+  const int lds = Fast::LDS_BYTES + 2 * kDzTile * 4 + kDzTile * static_cast<int>(sizeof(DzRow)) + kDzNWV * kDzNWT * kDz16StageBytes;
+  const int grid = p.items_per_xcd * 8;
+  hipError_t err;
+  if (bias != nullptr || v % kDzTile != 0) {
+    auto kern = dense_dz16_kernel<BF16, true, kDzParts>;
+    static LdsLimitOnce lds_limit;
+    err = lds_limit.set(kern, lds);
+    if (err != hipSuccess) return status_from_hip(err);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kDzThreads), lds, stream, p);
+  } else {
+    auto kern = dense_dz16_kernel<BF16, false, kDzParts>;
+    static LdsLimitOnce lds_limit;
+    err = lds_limit.set(kern, lds);
+    if (err != hipSuccess) return status_from_hip(err);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kDzThreads), lds, stream, p);
+  }
   return status_from_hip(hipGetLastError());
 }
 

@@ -14,7 +14,7 @@
 // several row blocks.
 #include <atomic>
 
-#include "cce_common.h"
+#include "cce_dense.h"
 
 namespace cce {
 
@@ -33,6 +33,9 @@ struct LseFwdParams {
   Softcap sc;
   float avg_scale;  // ln 2 / b: turns a column sum in log2 units into its share of logit_avg
   float cap_inv;    // 1 / (-2 cap log2(e)) (soft-capping on), for the fixed-reference epilogue
+  // operands in 16-bit parts (TERMS): d is the width of a part, rows of e are taken as they lie
+  const float* bias32;
+  int terms;
 };
 
 // 8 waves (two per SIMD, so that one wave's LDS and global traffic issues in the shadow of the
@@ -382,9 +385,9 @@ __device__ __forceinline__ void row_block(const Softcap& sc, float cap_inv, bool
   else row_block_impl<GENERAL, false, false, WANT_S2>(sc, cap_inv, acc, ti, addend, kq, run, bm, s2);
 }
 
-template <typename T, bool GENERAL, bool WANT_LA>
+template <typename T, bool GENERAL, bool WANT_LA, bool TERMS = false>
 __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdParams p) {
-  using Fast = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT>;
+  using Fast = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, TERMS>;
   static_assert(!WANT_LA || GENERAL, "the column average uses the general epilogue");
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_addend = reinterpret_cast<float*>(smem + Fast::LDS_BYTES);  // [2][256]
@@ -425,11 +428,12 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   src.chunk_bytes = 2u * static_cast<unsigned>(Fast::chunk_elems(wave, lane));
   src.row_in_block = static_cast<unsigned>(lane >> 3);
   src.c_stride_bytes = static_cast<unsigned>(p.stride_cv * 2);
+  src.terms = TERMS ? p.terms : 1;
 #pragma unroll
   for (int q = Fast::NQC; q < Fast::NQ; ++q) {
     int64_t i = t0 + Fast::row_of(q, wave, lane);
     i = (i < p.b) ? i : p.b - 1;  // rows past the end repeat the last one; their results are dropped
-    const int64_t row = p.valids ? static_cast<int64_t>(p.valids[i]) : i;
+    const int64_t row = (!TERMS && p.valids) ? static_cast<int64_t>(p.valids[i]) : i;
     src.e_off[q - Fast::NQC] = static_cast<unsigned>(row * p.stride_e * 2) + src.chunk_bytes;
   }
   auto set_class_tile = [&](int64_t v0) {
@@ -459,7 +463,7 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   float stat = 0.0f;  // statistic cells waiting to be written (see the epilogue)
   int buf = 0;
   set_class_tile(static_cast<int64_t>(vt_begin) * kFwdTile);
-  Fast::prefetch(src, smem);
+  Fast::prefetch(src, smem, static_cast<int>(p.d));
 
   for (int vt = vt_begin; vt < vt_end; ++vt) {
     const int64_t v0 = static_cast<int64_t>(vt) * kFwdTile;
@@ -470,7 +474,10 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
       if (tid < kFwdTile) {
         const int64_t vg = v0 + tid;
         float a = -INFINITY;
-        if (vg < p.v) a = (p.bias != nullptr) ? Elem<T>::to_float(p.bias[vg]) : 0.0f;
+        if (vg < p.v) {
+          if (TERMS) a = (p.bias32 != nullptr) ? p.bias32[vg] : 0.0f;
+          else a = (p.bias != nullptr) ? Elem<T>::to_float(p.bias[vg]) : 0.0f;
+        }
         addend[tid] = a;
       }
     }
@@ -483,7 +490,7 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
     const float* wave_addend = addend + wv * (16 * kF16WV);
     // A tile with no bias and no class past the end of the vocabulary has nothing to add and nothing to mask: of a
     // vocabulary that is no multiple of 256 only the last tile pays for the per-class addend.
-    const bool plain_tile = GENERAL && p.bias == nullptr && v0 + kFwdTile <= p.v;
+    const bool plain_tile = GENERAL && (TERMS ? p.bias32 == nullptr : p.bias == nullptr) && v0 + kFwdTile <= p.v;
     float la[WANT_LA ? kF16WV : 1][4];  // this lane's sums over its four rows of the tile, log2 units
     if (WANT_LA) {
       if (vt > vt_begin) flush_colsum(v0 - kFwdTile, (vt - 1) & 1);
@@ -687,6 +694,59 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
   return status_from_hip(hipGetLastError());
 }
 
+// ---- the forward over one chunk of classes with operands in 16-bit parts (cce_fp32.hip) ------------------------
+int lse_terms_splits(int64_t b, int64_t v) {
+  return choose_nsplit(static_cast<int>((b + 255) / 256), static_cast<int>((v + 255) / 256));
+}
+
+int lse_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
+                     float2* partial, int64_t b, int64_t v, int64_t part_d, int terms, float softcap, hipStream_t stream) {
+  LseFwdParams p = {};
+  p.e = e_parts;
+  p.c = c_parts;
+  p.bias32 = bias;
+  p.terms = terms;
+  p.partial = partial;
+  p.b = b;
+  p.v = v;
+  p.d = part_d;
+  p.n_rows = b;
+  p.stride_e = ld_e;
+  p.stride_cv = ld_c;
+  p.stride_cd = 1;
+  p.nrb = static_cast<int>((b + 255) / 256);
+  p.nvt = static_cast<int>((v + 255) / 256);
+  p.nsplit = choose_nsplit(p.nrb, p.nvt);
+  p.nitems = p.nrb * p.nsplit;
+  p.items_per_xcd = (p.nitems + 7) / 8;
+  p.sc = make_softcap(softcap);
+  p.cap_inv = p.sc.on ? 1.0f / (-2.0f * p.sc.out_scale) : 0.0f;
+  using Fast = DmaLogitTile16<BF16, kF16WV, kF16WT, kFwdNWV, kFwdNWT, true>;
+  const int bytes = Fast::LDS_BYTES + kFwdBiasBytes + kF16RunBytes;
+  const int grid = p.items_per_xcd * 8;
+  hipError_t err;
+  if (bias != nullptr || v % kFwdTile != 0) {
+    auto kern = lse_forward16_kernel<BF16, true, false, true>;
+    static LdsLimitOnce lds_limit;
+    err = lds_limit.set(kern, bytes);
+    if (err != hipSuccess) return status_from_hip(err);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), bytes, stream, p);
+  } else {
+    auto kern = lse_forward16_kernel<BF16, false, false, true>;
+    static LdsLimitOnce lds_limit;
+    err = lds_limit.set(kern, bytes);
+    if (err != hipSuccess) return status_from_hip(err);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), bytes, stream, p);
+  }
+  return status_from_hip(hipGetLastError());
+}
+
+int lse_merge_launch(const float2* partial, float* lse, int64_t b, int nsplit, hipStream_t stream) {
+  hipLaunchKernelGGL(lse_merge_kernel, dim3(static_cast<unsigned>((b + kMergeRows - 1) / kMergeRows)),
+                     dim3(kMergeRows * kMergeParts), 0, stream, partial, lse, b, nsplit);
+  return status_from_hip(hipGetLastError());
+}
+
 }  // namespace cce
 
 using namespace cce;
@@ -715,7 +775,7 @@ static int lse_forward_impl(const void* e, const void* c, const void* bias, cons
   if (workspace == nullptr || workspace_bytes < need) return CCE_ERR_WORKSPACE_TOO_SMALL;
   if ((reinterpret_cast<uintptr_t>(workspace) & 7u) != 0) return CCE_ERR_MISALIGNED;
 
-  LseFwdParams p;
+  LseFwdParams p = {};
   p.e = static_cast<const uint16_t*>(e);
   p.c = static_cast<const uint16_t*>(c);
   p.bias = static_cast<const uint16_t*>(bias);
@@ -750,9 +810,7 @@ static int lse_forward_impl(const void* e, const void* c, const void* bias, cons
   int st = (dtype == CCE_DTYPE_BF16) ? launch_lse_forward<BF16>(p, aligned, logit_avg != nullptr, stream)
                                      : launch_lse_forward<F16>(p, aligned, logit_avg != nullptr, stream);
   if (st != CCE_OK) return st;
-  hipLaunchKernelGGL(lse_merge_kernel, dim3(static_cast<unsigned>((b + kMergeRows - 1) / kMergeRows)),
-                     dim3(kMergeRows * kMergeParts), 0, stream, p.partial, lse, b, p.nsplit);
-  return status_from_hip(hipGetLastError());
+  return lse_merge_launch(p.partial, lse, b, p.nsplit, stream);
 }
 
 // Argument checks shared by the two entry points; CCE_OK with *done set means "nothing to do".

@@ -27,6 +27,10 @@
 // only, and what it fetches past the end of the reduction (its loads run two stages ahead) is the last whole
 // stage again, never consumed.
 //
+// TERMS: the operands are fp32 values in 16-bit parts, a_part / b_part elements from part to part, and the reduction
+// runs over the cross terms of the parts one after the other (kTermsFirst / kTermsSecond of cce_common.h: A is the
+// first operand), whole stages only.
+//
 // A stage is 64 reduction steps (32 KB per operand), two stages per operand in LDS (operand-major: A0 A1 B0 B1,
 // so that every read offset fits the 16-bit immediate), one barrier per stage.  The loads of a stage are
 // issued in two groups of 8, one load after every second MFMA: A under the last 16-step of the stage before last,
@@ -44,9 +48,10 @@ static __device__ __align__(256) uint16_t g_zero_line[128];  // never written
 
 typedef short tr_short4_t __attribute__((ext_vector_type(4)));
 
-template <typename T, bool A_KM, bool B_KM, bool B_GATHER = false>
+template <typename T, bool A_KM, bool B_KM, bool B_GATHER = false, bool TERMS = false>
 struct Tile4 {
   static_assert(!B_GATHER || B_KM, "only the rows of a KMajor operand are gathered");
+  static_assert(!B_GATHER || !TERMS, "parts are compact");
   static constexpr int WM = 4, WN = 4;   // accumulator blocks per wave
   static constexpr int NW = 4;           // waves, 2 (m) x 2 (n)
   static constexpr int NT = 64 * NW;
@@ -79,7 +84,9 @@ struct Tile4 {
     int64_t a_stride;       // KMajor: elements between consecutive k rows (< 2^30)
     int64_t b_stride;
     const int32_t* b_rows;  // B_GATHER: the k rows of B (k_total entries)
-    int k_total;            // length of the reduction
+    int k_total;            // length of the reduction (TERMS: of one term, a multiple of 64)
+    int64_t a_part, b_part; // TERMS: elements from one part to the next
+    int terms;              // TERMS: 3 or 6
   };
 
   // What the loads inside the main loop work from (built by plan()).  With no whole stage in the reduction the
@@ -138,8 +145,8 @@ struct Tile4 {
   static __device__ __forceinline__ Loop plan(const Source& s, const Geometry& g) {
     Loop l;
     const int whole = s.k_total / BK;
-    l.partial = (s.k_total % BK) != 0;
-    l.nk = whole + l.partial;
+    l.partial = TERMS ? 0 : (s.k_total % BK) != 0;
+    l.nk = TERMS ? s.terms * whole : whole + l.partial;
     l.k_first = l.partial ? whole * BK : 0;
     l.k_clamp = whole > 0 ? (whole - 1) * BK : 0;
     const bool any = whole > 0;
@@ -154,6 +161,39 @@ struct Tile4 {
   }
   // Where stage t >= 1 starts; past the end of the reduction: the last whole stage again.
   static __device__ __forceinline__ int k_of(const Loop& l, int t) { return min((t - l.partial) * BK, l.k_clamp); }
+
+  // A stage of the reduction: its first step and, with TERMS, how far into the rows of A and B its parts lie.
+  struct Pos {
+    int k, term;
+    int64_t a, b;
+  };
+  static __device__ __forceinline__ void set_parts(Pos& p, const Source& s) {
+    p.a = term_part(kTermsFirst, p.term) * s.a_part;
+    p.b = term_part(kTermsSecond, p.term) * s.b_part;
+  }
+  static __device__ __forceinline__ Pos first_pos(const Source& s, const Loop& l) {
+    Pos p = {l.k_first, 0, 0, 0};
+    if constexpr (TERMS) {
+      p.term = kTermsAll - s.terms;
+      set_parts(p, s);
+    }
+    return p;
+  }
+  // Stage t + 1 from stage t (with TERMS; past the end the walk starts over, and what it fetches is not consumed).
+  static __device__ __forceinline__ Pos pos_of(const Source& s, const Loop& l, const Pos& before, int t) {
+    Pos p = before;
+    if constexpr (TERMS) {
+      p.k += BK;
+      if (p.k == s.k_total) {
+        p.k = 0;
+        p.term = (p.term + 1 == kTermsAll) ? kTermsAll - s.terms : p.term + 1;
+      }
+      set_parts(p, s);
+    } else {
+      p.k = k_of(l, t);
+    }
+    return p;
+  }
 
   // The row numbers and load addresses of a gathered B, formed a step ahead of their use.
   struct Ids {
@@ -175,34 +215,35 @@ struct Tile4 {
   }
   // Load q of the stage that starts at k0 (a whole stage) into LDS stage STAGE.
   template <int STAGE>
-  static __device__ __forceinline__ void issue_a(int q, const Source& s, const Loop& l, int k0, const Geometry& g) {
+  static __device__ __forceinline__ void issue_a(int q, const Source& s, const Loop& l, const Pos& at, const Geometry& g) {
     const uint16_t* src;
     if (A_KM) {
-      const uint32_t r = static_cast<uint32_t>(k0 + row_kmajor(q, g.wave));  // uniform
-      src = l.a_lane + static_cast<uint64_t>(r) * l.a_stride;
+      const uint32_t r = static_cast<uint32_t>(at.k + row_kmajor(q, g.wave));  // uniform
+      src = l.a_lane + (static_cast<uint64_t>(r) * l.a_stride + (TERMS ? at.a : 0));
     } else {
-      src = s.a_row[A_KM ? 0 : q] + k0;
+      src = s.a_row[A_KM ? 0 : q] + (at.k + (TERMS ? at.a : 0));
     }
     lds_dma16(src, g.lds_base + STAGE * OP_BYTES + (q * NW + g.wave) * 1024);
   }
   template <int STAGE>
-  static __device__ __forceinline__ void issue_b(const Ptrs& p, int q, const Source& s, const Loop& l, int k0,
+  static __device__ __forceinline__ void issue_b(const Ptrs& p, int q, const Source& s, const Loop& l, const Pos& at,
                                                 const Geometry& g) {
     const uint16_t* src;
     if (B_GATHER) {
       src = p.b[B_GATHER ? q : 0];
     } else if (B_KM) {
-      const uint32_t r = static_cast<uint32_t>(k0 + row_kmajor(q, g.wave));  // uniform
-      src = l.b_lane + static_cast<uint64_t>(r) * l.b_stride;
+      const uint32_t r = static_cast<uint32_t>(at.k + row_kmajor(q, g.wave));  // uniform
+      src = l.b_lane + (static_cast<uint64_t>(r) * l.b_stride + (TERMS ? at.b : 0));
     } else {
-      src = s.b_row[B_KM ? 0 : q] + k0;
+      src = s.b_row[B_KM ? 0 : q] + (at.k + (TERMS ? at.b : 0));
     }
     lds_dma16(src, g.lds_base + B_BASE + STAGE * OP_BYTES + (q * NW + g.wave) * 1024);
   }
 
   // ---- loads of stage 0 (the partial stage when there is one): every row is asked for --------------------
-  static __device__ __forceinline__ void issue_first_a(int q, const Source& s, int k0, const Geometry& g) {
+  static __device__ __forceinline__ void issue_first_a(int q, const Source& s, const Pos& at, const Geometry& g) {
     const uint16_t* src;
+    const int k0 = at.k;
     if (A_KM) {
       const int row = k0 + row_kmajor(q, g.wave) + g.half;
       src = s.a_km + static_cast<uint64_t>(static_cast<uint32_t>(row)) * static_cast<uint32_t>(s.a_stride);
@@ -210,6 +251,7 @@ struct Tile4 {
     } else {
       src = s.a_row[A_KM ? 0 : q] + k0;
     }
+    if constexpr (TERMS) src += at.a;  // (whole stages: no row is missing)
     lds_dma16(src, g.lds_base + (q * NW + g.wave) * 1024);
   }
   // (the row numbers of a gathered B are looked up for all loads first: the lookups and the loads share a queue)
@@ -220,14 +262,15 @@ struct Tile4 {
     if (row < s.k_total) id = B_GATHER ? s.b_rows[row] : row;
     return id;
   }
-  static __device__ __forceinline__ void issue_first_b(int q, int id, const Source& s, int k0, const Geometry& g) {
+  static __device__ __forceinline__ void issue_first_b(int q, int id, const Source& s, const Pos& at, const Geometry& g) {
     const uint16_t* src;
     if (B_KM) {
       src = s.b_km + static_cast<uint64_t>(static_cast<uint32_t>(id)) * static_cast<uint32_t>(s.b_stride);
       if (id < 0) src = zero_line(g);
     } else {
-      src = s.b_row[B_KM ? 0 : q] + k0;
+      src = s.b_row[B_KM ? 0 : q] + at.k;
     }
+    if constexpr (TERMS) src += at.b;
     lds_dma16(src, g.lds_base + B_BASE + (q * NW + g.wave) * 1024);
   }
 
@@ -294,16 +337,16 @@ struct Tile4 {
   }
 
   // What a 16-step does between its MFMAs besides the fragment reads of the next step:
-  //   kIssueB  + loads of B for the stage at kl into LDS stage LSTAGE, one after every odd MFMA
+  //   kIssueB  + loads of B for the stage `at` into LDS stage LSTAGE, one after every odd MFMA
   //   kPrepIds + row numbers of a gathered B for the stage at k0, one pair after every even MFMA
-  //   kIssueAPrepB  loads of A for the stage at kl into LDS stage LSTAGE after the odd MFMAs, addresses of the
+  //   kIssueAPrepB  loads of A for the stage `at` into LDS stage LSTAGE after the odd MFMAs, addresses of the
   //                 loads of a gathered B (from `ids`) after the even ones
   enum Extra { kNone, kIssueB, kPrepIds, kIssueAPrepB };
 
   // The 16 MFMAs on `cur`; between them the reads of fragment set `nxt` (step RKK of stage RSTAGE) and EXTRA.
   template <int RSTAGE, int RKK, Extra EXTRA, int LSTAGE>
   static __device__ __forceinline__ void step(f32x16 (&acc)[WM][WN], const Frags& cur, Frags& nxt, const unsigned char* lds,
-                                              const Source& s, const Loop& l, int kl, int k0, Ptrs& ptrs, Ids& ids,
+                                              const Source& s, const Loop& l, const Pos& at, int k0, Ptrs& ptrs, Ids& ids,
                                               const Geometry& g) {
     constexpr int kMfmas = WM * WN;
     Half ha[WM], hb[WN];
@@ -319,8 +362,8 @@ struct Tile4 {
           read_op<RSTAGE, RKK>(r, nxt, ha, hb, lds, g);
         const int q = idx >> 1;
         if (idx & 1) {
-          if (EXTRA == kIssueB) issue_b<LSTAGE>(ptrs, q, s, l, kl, g);
-          if (EXTRA == kIssueAPrepB) issue_a<LSTAGE>(q, s, l, kl, g);
+          if (EXTRA == kIssueB) issue_b<LSTAGE>(ptrs, q, s, l, at, g);
+          if (EXTRA == kIssueAPrepB) issue_a<LSTAGE>(q, s, l, at, g);
         } else {
           if (EXTRA == kPrepIds) prep_b_id(ids, q, l, k0, g);
           if (EXTRA == kIssueAPrepB) prep_b(ptrs, q, ids, l, g);
@@ -333,18 +376,19 @@ struct Tile4 {
   // the addresses of a gathered B for stage 1.  A caller with work between two tiles (an epilogue) calls this
   // first, so that the next main loop starts with data in LDS.
   static __device__ __forceinline__ void prefetch(const Source& s, const Loop& l, Ptrs& ptrs, Ids& ids, const Geometry& g) {
+    const Pos at0 = first_pos(s, l);
     int first[NQ1];
 #pragma unroll
     for (int q = 0; q < NQ1; ++q) first[q] = first_b_id(q, s, l.k_first, g);
 #pragma unroll
-    for (int q = 0; q < NQ1; ++q) issue_first_a(q, s, l.k_first, g);
+    for (int q = 0; q < NQ1; ++q) issue_first_a(q, s, at0, g);
 #pragma unroll
-    for (int q = 0; q < NQ1; ++q) issue_first_b(q, first[q], s, l.k_first, g);
-    const int k1 = k_of(l, 1);
+    for (int q = 0; q < NQ1; ++q) issue_first_b(q, first[q], s, at0, g);
+    const Pos at1 = pos_of(s, l, first_pos(s, l), 1);
 #pragma unroll
-    for (int q = 0; q < NQ1; ++q) prep_b_id(ids, q, l, k1, g);
+    for (int q = 0; q < NQ1; ++q) prep_b_id(ids, q, l, at1.k, g);
 #pragma unroll
-    for (int q = 0; q < NQ1; ++q) issue_a<1>(q, s, l, k1, g);
+    for (int q = 0; q < NQ1; ++q) issue_a<1>(q, s, l, at1, g);
 #pragma unroll
     for (int q = 0; q < NQ1; ++q) prep_b(ptrs, q, ids, l, g);
   }
@@ -353,14 +397,14 @@ struct Tile4 {
   // that of the next stage on exit.
   template <int CUR>
   static __device__ __forceinline__ void stage(f32x16 (&acc)[WM][WN], Frags& fa, Frags& fb, const unsigned char* lds,
-                                               const Source& s, const Loop& l, int st, Ptrs& ptrs, Ids& ids,
+                                               const Source& s, const Loop& l, int st, Pos& at1, Ptrs& ptrs, Ids& ids,
                                                const Geometry& g) {
     constexpr int NXT = 1 - CUR;
-    const int k1 = k_of(l, st + 1);
-    const int k2 = k_of(l, st + 2);
-    step<CUR, 1, kIssueB, NXT>(acc, fa, fb, lds, s, l, k1, k2, ptrs, ids, g);    // the B loads of stage st + 1
-    step<CUR, 2, kPrepIds, NXT>(acc, fb, fa, lds, s, l, k1, k2, ptrs, ids, g);   // rows of B for stage st + 2
-    step<CUR, 3, kNone, NXT>(acc, fa, fb, lds, s, l, k1, k2, ptrs, ids, g);
+    if constexpr (!TERMS) at1 = pos_of(s, l, at1, st + 1);  // (TERMS: carried from stage to stage)
+    const Pos at2 = pos_of(s, l, at1, st + 2);
+    step<CUR, 1, kIssueB, NXT>(acc, fa, fb, lds, s, l, at1, at2.k, ptrs, ids, g);    // the B loads of stage st + 1
+    step<CUR, 2, kPrepIds, NXT>(acc, fb, fa, lds, s, l, at1, at2.k, ptrs, ids, g);   // rows of B for stage st + 2
+    step<CUR, 3, kNone, NXT>(acc, fa, fb, lds, s, l, at1, at2.k, ptrs, ids, g);
     // Stage st + 1 has landed for this wave; after the barrier for every wave, and every wave holds its last
     // fragments of stage st in registers: that LDS stage is free for stage st + 2.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -371,7 +415,8 @@ struct Tile4 {
       for (int q = 0; q < NQ1; ++q) asm volatile("" : "+v"(ids.v[q]));
     }
     __syncthreads();
-    step<NXT, 0, kIssueAPrepB, CUR>(acc, fb, fa, lds, s, l, k2, k2, ptrs, ids, g);  // the A loads of stage st + 2
+    step<NXT, 0, kIssueAPrepB, CUR>(acc, fb, fa, lds, s, l, at2, at2.k, ptrs, ids, g);  // the A loads of stage st + 2
+    if constexpr (TERMS) at1 = at2;
   }
 
   // Every per-lane value the main loop reads, marked as used: should the compiler have parked one of them in
@@ -412,12 +457,13 @@ struct Tile4 {
 
     // two stages per trip, so that every LDS address is a lane constant plus an immediate; an odd last stage
     // stands outside the loop (a branch inside it costs the register allocator its footing)
+    Pos at1 = pos_of(s, l, first_pos(s, l), 1);
 #pragma unroll 1
     for (int st = 0; st + 1 < nk; st += 2) {
-      stage<0>(acc, fa, fb, lds, s, l, st, ptrs, ids, g);
-      stage<1>(acc, fa, fb, lds, s, l, st + 1, ptrs, ids, g);
+      stage<0>(acc, fa, fb, lds, s, l, st, at1, ptrs, ids, g);
+      stage<1>(acc, fa, fb, lds, s, l, st + 1, at1, ptrs, ids, g);
     }
-    if (nk & 1) stage<0>(acc, fa, fb, lds, s, l, nk - 1, ptrs, ids, g);
+    if (nk & 1) stage<0>(acc, fa, fb, lds, s, l, nk - 1, at1, ptrs, ids, g);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last, unused prefetch
     __syncthreads();
   }

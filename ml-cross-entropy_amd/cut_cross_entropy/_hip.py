@@ -16,7 +16,7 @@ _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "li
 _lib: Optional[ctypes.CDLL] = None
 _lock = threading.Lock()
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1}
 STAT_ROWS = 32
 STAT_COLS = 32
@@ -64,6 +64,13 @@ _SIGNATURES = {
     "cce_backward_products": (
         _i32,
         [_ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _ptr, _i64, _i32, _i64, _i64, _i64, _i32, _ptr],
+    ),
+    "cce_fp32_forward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
+    "cce_fp32_forward": (_i32, [_ptr] * 8 + [_i64] + [_i64] * 4 + [_i64] * 3 + [_i64, _i64, _f32, _i32, _ptr]),
+    "cce_fp32_backward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
+    "cce_fp32_backward": (
+        _i32,
+        [_ptr] * 5 + [_i32] + [_ptr] * 7 + [_i64] + [_i64] * 4 + [_i64] * 5 + [_f32, _i64, _i64, _f32, _i32, _ptr],
     ),
     "cce_backward_dz": (
         _i32,

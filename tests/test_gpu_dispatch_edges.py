@@ -90,3 +90,95 @@ def test_backward_dense_cuts_long_reductions(shape, fp32_out, gathered, budget):
         scale = want.abs().amax(dim=1, keepdim=True)
         assert ((got.double() - want).abs() <= 1e-2 * scale + 1e-2 * want.abs() + 1e-6).all()
         assert (got.double() - want).norm() <= 6e-3 * want.norm()
+
+
+def _fp32_case(N, V, D, keep, seed, softcap=None, bias=False, d_lse=False, strided=False):
+    """(inputs, results in fp64) of one fp32 call, everything made on the GPU."""
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(seed)
+    e = torch.randn((N, D), generator=g, device=dev)
+    c = torch.randn((V, D + 4), generator=g, device=dev)[:, :D] if strided else torch.randn((V, D), generator=g, device=dev)
+    c = c * (0.5 / D**0.5) if not strided else c.mul_(0.5 / D**0.5)
+    t = torch.randint(0, V, (N,), generator=g, device=dev)
+    b = torch.randn((V,), generator=g, device=dev) if bias else None
+    w = torch.rand((N,), generator=g, device=dev) + 0.5
+    h = torch.randn((N,), generator=g, device=dev) * 0.1 if d_lse else None
+    rows = torch.arange(N, device=dev)
+    valids = None
+    if keep < 1.0:
+        rows = rows[torch.rand((N,), generator=g, device=dev) < keep]
+        valids = rows.to(torch.int32)
+    return e, c, t, b, w, h, rows, valids
+
+
+@pytest.mark.parametrize("shape,keep,extra", [
+    ((1, 3, 1), 1.0, {}), ((65, 257, 65), 1.0, {"softcap": 5.0}), ((300, 9001, 123), 0.7, {"bias": True, "d_lse": True}),
+    ((64, 256, 64), 1.0, {}), ((130, 600, 1000), 0.5, {"strided": True}), ((40, 33000, 2048), 1.0, {"bias": True}),
+    ((6000, 300, 200), 0.9, {"d_lse": True, "softcap": 20.0}), ((1500, 1400, 96), 1.0, {"strided": True, "bias": True}),
+    ((176000, 70, 4096), 1.0, {}), ((180000, 70, 4096), 0.98, {}),
+])
+@pytest.mark.parametrize("terms", [6, 3])
+def test_fp32_passes_abi(shape, keep, extra, terms):
+    """cce_fp32_forward / cce_fp32_backward against fp64: widths that are no multiple of anything, one and several chunks
+    of classes (33000 x 2048), cut reductions of dE and of dC, rows gathered or taken as they lie, more rows than 32-bit
+    offsets reach in one copy (two blocks of rows), a classifier with gaps between its rows."""
+    lib = _lib()
+    dev = torch.device("cuda:0")
+    N, V, D = shape
+    e, c, t, bias, w, h, rows, valids = _fp32_case(N, V, D, keep, 21, **extra)
+    B, cap = rows.numel(), extra.get("softcap")
+    p = lambda x: x.data_ptr() if x is not None else None
+    lse = torch.full((B,), float("nan"), device=dev)
+    dot = torch.full((B,), float("nan"), device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def workspace(nbytes):
+        buf = torch.full((nbytes // 4 + 64,), float("nan"), device=dev)
+        return buf, (buf.data_ptr() + 255) // 256 * 256
+
+    n_ws = lib.cce_fp32_forward_workspace_bytes(B, V, D, terms)
+    buf, ws = workspace(n_ws)
+    st = lib.cce_fp32_forward(p(e), p(c), p(bias), p(valids), p(t), p(lse), p(dot), ws, n_ws, N, B, V, D, e.stride(0), c.stride(0),
+                              1, 0, 0, cap or 0.0, terms, stream)
+    assert st == 0, lib.cce_error_string(st)
+    x = e.double()[rows] @ c.double().T + (bias.double() if bias is not None else 0.0)
+    damp = 1.0
+    if cap:
+        th = torch.tanh(x / cap)
+        x, damp = cap * th, 1.0 - th * th
+    want_lse = torch.logsumexp(x, dim=1)
+    # six terms: 2^-24 per product, fp32 sums of D of them and of V exponentials; three: 2^-16 of |e| |c| ~ sqrt(D) / 2
+    # per logit (before the cap), of random sign over D
+    tol = 4e-6 if terms == 6 else 4e-5
+    assert torch.allclose(lse.double(), want_lse, atol=tol, rtol=2e-6)
+    # plain fp32 whatever the number of terms: D roundings of terms of up to 1
+    assert torch.allclose(dot.double(), -x[torch.arange(B, device=dev), t[rows]], atol=2e-5, rtol=2e-6)
+    dz = torch.exp(x - want_lse[:, None]) * (w.double()[rows] + (h.double()[rows] if h is not None else 0.0))[:, None]
+    dz[torch.arange(B, device=dev), t[rows]] -= w.double()[rows]
+    dz *= damp
+    del x
+    want_de = torch.zeros((N, D), dtype=torch.float64, device=dev)
+    want_de[rows] = dz @ c.double()
+    want_dc, want_db = dz.T @ e.double()[rows], dz.sum(0)
+    del dz, buf
+    de = torch.zeros((N, D), device=dev)
+    dc = torch.full((V, D), float("nan"), device=dev)
+    db = torch.zeros((V,), device=dev)
+    n_ws = lib.cce_fp32_backward_workspace_bytes(B, V, D, terms)
+    buf, ws = workspace(n_ws)
+    lse32 = want_lse.float()
+    st = lib.cce_fp32_backward(p(e), p(c), p(bias), p(lse32), p(w), 0, p(h), p(valids), p(t), p(de), p(dc), p(db), ws, n_ws,
+                               N, B, V, D, e.stride(0), c.stride(0), 1, D, D, 1.0, 0, 0, cap or 0.0, terms, stream)
+    assert st == 0, lib.cce_error_string(st)
+    torch.cuda.synchronize()
+    # relative to the norm: 2^-24 per term of the sums (2^-16 with three terms), a few times that for what dz inherits
+    # from the logits and from the rounding of lse to fp32
+    # (dC sums up to 180000 rows in fp32, 16 per rounding: sqrt(11000) 2^-24)
+    rel = 8e-6 if terms == 6 else 2e-4
+    for name, got, want in (("dE", de, want_de), ("dC", dc, want_dc), ("dBias", db, want_db)):
+        assert torch.isfinite(got).all(), name
+        err = (got.double() - want).norm().item()
+        assert err <= rel * want.norm().item() + 1e-6 * want.numel() ** 0.5 * 1e-2, (name, err, want.norm().item())
+    ignored = torch.ones(N, dtype=torch.bool, device=dev)
+    ignored[rows] = False
+    assert (de[ignored] == 0).all()
