@@ -286,12 +286,31 @@ int cce_backward_products(const void* dz, int64_t ldz, const void* c, int64_t st
                           int64_t b, int64_t n_cls, int64_t d, int dtype, void* stream);
 
 /*
+ * rows[0 .. *count) = the positions p of labels[n], in increasing order, that enter the loss: sequences of `steps` labels
+ * (n a multiple of it), p scored against labels[p + shift] of the same sequence, which is not `ignored`.  Restates
+ * cut_cross_entropy/utils.py:28-49.  `rows` has room for n; `count` is host memory that the device can write (pinned), to be
+ * read once the stream has come past this call.
+ */
+int cce_valid_rows(const int64_t* labels, int64_t n, int64_t steps, int64_t shift, int64_t ignored, int32_t* rows,
+                   int64_t* count, void* stream);
+
+/*
+ * cce_lse_forward (without logit_avg) and cce_indexed_neg_dot in one call: lse[b], and nll[b] = lse + neg_dot, the loss of
+ * every valid row (cut_cross_entropy/cce.py:87-131).  tile_max may be NULL; workspace as for cce_lse_forward.
+ */
+int cce_loss_forward(const void* e, const void* c, const void* bias, const int32_t* valids, const int64_t* targets,
+                     float* lse, float* nll, float* tile_max, void* workspace, int64_t workspace_bytes,
+                     int64_t n_rows, int64_t b, int64_t v, int64_t d,
+                     int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
+                     int64_t shift, int64_t target_offset, float softcap, int dtype, void* stream);
+
+/*
  * fp32 inputs.  The matrix cores multiply 16-bit numbers: every value is split into bf16 parts, x = hi + mid + lo, and a
  * product is taken as its leading cross terms (`terms`: 6, what is left is below 2^-24 relative; or 3 of two parts,
  * 16 bits), all in fp32 accumulators.  The reference gives this dtype to tl.dot (cut_cross_entropy/cce_lse_forward.py:81,
  * cce_backward.py:170-302).
  *
- * cce_fp32_forward: lse[b] and neg_dot[b] as cce_lse_forward and cce_indexed_neg_dot define them; bias [v] float or NULL.
+ * cce_fp32_forward: lse[b] and nll[b] as cce_loss_forward defines them; bias [v] float or NULL.
  * cce_fp32_backward: the unfiltered gradients, arguments as for cce_backward_dense: d_e [n_rows, d] is added to (row
  * stride ld_de), d_c [v, d] written (row stride ld_dc), d_bias [v] added to.
  * Any alignment and width; stride_cd must be 1, else CCE_ERR_MISALIGNED.  `workspace` 256-byte aligned, of at least the
@@ -299,7 +318,7 @@ int cce_backward_products(const void* dz, int64_t ldz, const void* c, int64_t st
  */
 int64_t cce_fp32_forward_workspace_bytes(int64_t b, int64_t v, int64_t d, int terms);
 int cce_fp32_forward(const float* e, const float* c, const float* bias, const int32_t* valids, const int64_t* targets,
-                     float* lse, float* neg_dot, void* workspace, int64_t workspace_bytes,
+                     float* lse, float* nll, void* workspace, int64_t workspace_bytes,
                      int64_t n_rows, int64_t b, int64_t v, int64_t d,
                      int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
                      int64_t shift, int64_t target_offset, float softcap, int terms, void* stream);

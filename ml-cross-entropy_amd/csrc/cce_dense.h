@@ -24,8 +24,6 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
 int lse_terms_splits(int64_t b, int64_t v);
 int lse_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
                      float2* partial, int64_t b, int64_t v, int64_t part_d, int terms, float softcap, hipStream_t stream);
-// lse[b] of partials [nsplit][b]
-int lse_merge_launch(const float2* partial, float* lse, int64_t b, int nsplit, hipStream_t stream);
 
 // dz of v classes as bf16 parts [b_store][parts][ldz], ldz = v rounded up to 64; columns past v and rows b .. b_store
 // (b rounded up to 64) are zeros.  valids: the rows of the batch that the (compact) rows of e_parts are.
@@ -54,5 +52,22 @@ int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t*
 // out[row(i)][0 .. d) (+)= sum over the slots [count][rows][ld_slot]
 int split_sum_launch(const float* slots, int count, int64_t rows, int64_t d, int64_t ld_slot, const int32_t* ids, float* out,
                      int64_t ld, bool add, bool out_vec, hipStream_t stream);
+
+// ---- the loss of every valid row (cce_rows.hip) -------------------------------------------------------------------
+constexpr int kLossRowsFp32 = -1;  // beside CCE_DTYPE_*
+struct LossRowsParams {
+  const void* e;
+  const void* c;
+  const void* bias;
+  const int32_t* valids;
+  const int64_t* targets;
+  const float2* partial;  // [nsplit][b]
+  float* lse;
+  float* nll;
+  int nsplit;
+  int64_t n_rows, b, v, d, stride_e, stride_cv, stride_cd, shift, target_offset;
+  float softcap;
+};
+int loss_rows_launch(const LossRowsParams& p, int dtype, hipStream_t stream);
 
 }  // namespace cce

@@ -77,44 +77,6 @@ static int split_parts(const float* x, int64_t stride, const int32_t* ids, int64
   return status_from_hip(hipGetLastError());
 }
 
-// out[i] = softcap(-(e[row_i] . c[t_i]) - bias[t_i]), 0 where the target is not a class of c: a wave per row, plain fp32
-// arithmetic (the fp32 sibling of indexed_neg_dot_kernel, bound by the two rows it reads).
-struct Fp32DotParams {
-  const float* e;
-  const float* c;
-  const float* bias;
-  const int64_t* targets;
-  const int32_t* valids;
-  float* out;
-  int64_t n_rows, b, v, d, stride_e, stride_cv, shift, target_offset;
-  float softcap;
-};
-__global__ __launch_bounds__(256) void fp32_indexed_neg_dot_kernel(Fp32DotParams p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (i >= p.b) return;
-  const int64_t row = p.valids ? static_cast<int64_t>(p.valids[i]) : i;
-  const int64_t ti = row + p.shift;
-  int64_t t = -1;
-  if (ti < p.n_rows) t = p.targets[ti] - p.target_offset;
-  if (t < 0 || t >= p.v) {
-    if (lane == 0) p.out[i] = 0.0f;
-    return;
-  }
-  const float* er = p.e + row * p.stride_e;
-  const float* cr = p.c + t * p.stride_cv;
-  float acc = 0.0f;
-  for (int64_t k = lane; k < p.d; k += 64) acc = fmaf(er[k], cr[k], acc);
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
-  if (lane == 0) {
-    float r = -acc;
-    if (p.bias != nullptr) r -= p.bias[t];
-    if (p.softcap > 0.0f) r = tanhf(r / p.softcap) * p.softcap;
-    p.out[i] = r;
-  }
-}
-
 // d_bias[class] += sum over the rows of the parts of dz: 1024 threads = 16 row lanes x 64 classes, fixed order.
 __global__ __launch_bounds__(1024) void dz_parts_colsum_kernel(const uint16_t* dz, int64_t ldz, int parts, int64_t b, int n_cls,
                                                                float* d_bias) {
@@ -227,14 +189,14 @@ extern "C" int64_t cce_fp32_forward_workspace_bytes(int64_t b, int64_t v, int64_
 }
 
 extern "C" int cce_fp32_forward(const float* e, const float* c, const float* bias, const int32_t* valids, const int64_t* targets,
-                                float* lse, float* neg_dot, void* workspace, int64_t workspace_bytes,
+                                float* lse, float* nll, void* workspace, int64_t workspace_bytes,
                                 int64_t n_rows, int64_t b, int64_t v, int64_t d,
                                 int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
                                 int64_t shift, int64_t target_offset, float softcap, int terms, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   int st = check(e, c, targets, n_rows, b, v, d, valids, stride_cd, shift, terms);
   if (st != CCE_OK || b == 0) return st;
-  if (lse == nullptr || neg_dot == nullptr) return CCE_ERR_INVALID_ARGUMENT;
+  if (lse == nullptr || nll == nullptr) return CCE_ERR_INVALID_ARGUMENT;
   const Fp32Forward f = plan_forward(b, v, d, terms);
   if (workspace == nullptr || workspace_bytes < f.e_bytes + f.c_bytes + f.partial_bytes) return CCE_ERR_WORKSPACE_TOO_SMALL;
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return CCE_ERR_MISALIGNED;
@@ -259,12 +221,13 @@ extern "C" int cce_fp32_forward(const float* e, const float* c, const float* bia
       if (st != CCE_OK) return st;
       nsplit += lse_terms_splits(rows, cls);
     }
-    st = lse_merge_launch(partial, lse + r0, rows, nsplit, stream);
+    const int64_t moved = valids == nullptr ? r0 : 0;
+    const LossRowsParams p = {e + moved * stride_e, c, bias, ids, targets + moved, partial, lse + r0, nll + r0, nsplit, n_rows - moved,
+                              rows, v, d, stride_e, stride_cv, stride_cd, shift, target_offset, softcap};
+    st = loss_rows_launch(p, kLossRowsFp32, stream);
     if (st != CCE_OK) return st;
   }
-  Fp32DotParams p = {e, c, bias, targets, valids, neg_dot, n_rows, b, v, d, stride_e, stride_cv, shift, target_offset, softcap};
-  hipLaunchKernelGGL(fp32_indexed_neg_dot_kernel, dim3(static_cast<unsigned>((b + 3) / 4)), dim3(256), 0, stream, p);
-  return status_from_hip(hipGetLastError());
+  return CCE_OK;
 }
 
 extern "C" int64_t cce_fp32_backward_workspace_bytes(int64_t b, int64_t v, int64_t d, int terms) {

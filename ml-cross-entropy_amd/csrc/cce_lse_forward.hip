@@ -741,7 +741,7 @@ int lse_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_pa
   return status_from_hip(hipGetLastError());
 }
 
-int lse_merge_launch(const float2* partial, float* lse, int64_t b, int nsplit, hipStream_t stream) {
+static int lse_merge_launch(const float2* partial, float* lse, int64_t b, int nsplit, hipStream_t stream) {
   hipLaunchKernelGGL(lse_merge_kernel, dim3(static_cast<unsigned>((b + kMergeRows - 1) / kMergeRows)),
                      dim3(kMergeRows * kMergeParts), 0, stream, partial, lse, b, nsplit);
   return status_from_hip(hipGetLastError());
@@ -765,8 +765,9 @@ extern "C" int64_t cce_lse_forward_workspace_bytes(int64_t b, int64_t v, int64_t
   return static_cast<int64_t>(nsplit) * b * static_cast<int64_t>(sizeof(float2));
 }
 
+// (lse == nullptr: the partials stay in the workspace, and *nsplit_out says how many spans they are of)
 static int lse_forward_impl(const void* e, const void* c, const void* bias, const int32_t* valids,
-                            float* lse, float* logit_avg, float* tile_max,
+                            float* lse, int* nsplit_out, float* logit_avg, float* tile_max,
                             void* workspace, int64_t workspace_bytes,
                             int64_t n_rows, int64_t b, int64_t v, int64_t d,
                             int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
@@ -810,6 +811,10 @@ static int lse_forward_impl(const void* e, const void* c, const void* bias, cons
   int st = (dtype == CCE_DTYPE_BF16) ? launch_lse_forward<BF16>(p, aligned, logit_avg != nullptr, stream)
                                      : launch_lse_forward<F16>(p, aligned, logit_avg != nullptr, stream);
   if (st != CCE_OK) return st;
+  if (lse == nullptr) {
+    *nsplit_out = p.nsplit;
+    return CCE_OK;
+  }
   return lse_merge_launch(p.partial, lse, b, p.nsplit, stream);
 }
 
@@ -838,8 +843,27 @@ extern "C" int cce_lse_forward(const void* e, const void* c, const void* bias, c
   bool done;
   const int st = lse_forward_check(e, c, lse, valids, n_rows, b, v, d, dtype, &done);
   if (st != CCE_OK || done) return st;
-  return lse_forward_impl(e, c, bias, valids, lse, logit_avg, tile_max, workspace, workspace_bytes, n_rows, b, v, d,
+  return lse_forward_impl(e, c, bias, valids, lse, nullptr, logit_avg, tile_max, workspace, workspace_bytes, n_rows, b, v, d,
                           stride_e, stride_cv, stride_cd, softcap, dtype, static_cast<hipStream_t>(stream_));
+}
+
+extern "C" int cce_loss_forward(const void* e, const void* c, const void* bias, const int32_t* valids, const int64_t* targets,
+                                float* lse, float* nll, float* tile_max, void* workspace, int64_t workspace_bytes,
+                                int64_t n_rows, int64_t b, int64_t v, int64_t d,
+                                int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
+                                int64_t shift, int64_t target_offset, float softcap, int dtype, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  bool done;
+  int st = lse_forward_check(e, c, lse, valids, n_rows, b, v, d, dtype, &done);
+  if (st != CCE_OK || done) return st;
+  if (nll == nullptr || targets == nullptr || shift < 0) return CCE_ERR_INVALID_ARGUMENT;
+  int nsplit = 0;
+  st = lse_forward_impl(e, c, bias, valids, nullptr, &nsplit, nullptr, tile_max, workspace, workspace_bytes, n_rows, b, v, d,
+                        stride_e, stride_cv, stride_cd, softcap, dtype, stream);
+  if (st != CCE_OK) return st;
+  const LossRowsParams p = {e, c, bias, valids, targets, static_cast<const float2*>(workspace), lse, nll, nsplit, n_rows, b, v, d,
+                            stride_e, stride_cv, stride_cd, shift, target_offset, softcap};
+  return loss_rows_launch(p, dtype, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -891,6 +915,6 @@ extern "C" int cce_lse_forward_static(const void* e, const void* c, const void* 
   void* ws = nullptr;
   st = static_scratch_for_current_device(&ws);
   if (st != CCE_OK) return st;
-  return lse_forward_impl(e, c, bias, valids, lse, logit_avg, tile_max, ws, CCE_STATIC_SCRATCH_BYTES, n_rows, b, v, d,
+  return lse_forward_impl(e, c, bias, valids, lse, nullptr, logit_avg, tile_max, ws, CCE_STATIC_SCRATCH_BYTES, n_rows, b, v, d,
                           stride_e, stride_cv, stride_cd, softcap, dtype, static_cast<hipStream_t>(stream_));
 }

@@ -65,6 +65,8 @@ _SIGNATURES = {
         _i32,
         [_ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _ptr, _i64, _i32, _i64, _i64, _i64, _i32, _ptr],
     ),
+    "cce_valid_rows": (_i32, [_ptr, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr]),
+    "cce_loss_forward": (_i32, [_ptr] * 9 + [_i64] + [_i64] * 4 + [_i64] * 3 + [_i64, _i64, _f32, _i32, _ptr]),
     "cce_fp32_forward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "cce_fp32_forward": (_i32, [_ptr] * 8 + [_i64] + [_i64] * 4 + [_i64] * 3 + [_i64, _i64, _f32, _i32, _ptr]),
     "cce_fp32_backward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
@@ -167,7 +169,29 @@ def require_gpu_tensor(name: str, t: torch.Tensor) -> None:
 
 
 def current_stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw handle of the current stream (what ``torch.cuda.current_stream(device).cuda_stream`` builds a Stream
+    object to answer: 2 us where a small call has some fifty)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+class on_device:
+    """``with on_device(dev): lib.call(...)``: makes the tensors' device the current one, which it nearly always is."""
+
+    def __init__(self, device: torch.device):
+        self.index = device.index
+        self.before = None
+
+    def __enter__(self):
+        if self.index is not None and torch._C._cuda_getDevice() != self.index:
+            self.before = torch.cuda.device(self.index)
+            self.before.__enter__()
+        return self
+
+    def __exit__(self, *exc):
+        if self.before is not None:
+            self.before.__exit__(*exc)
+        return False
 
 
 # Device timings for a benchmark: while a dict is set here, every launcher brackets its library calls with a

@@ -91,7 +91,7 @@ class _FlaggedMonitor:
 
     def measure(self, lib, tile_max, lse, B: int, V: int, filter_eps: float, dev: torch.device) -> None:
         self.counter.zero_()
-        with torch.cuda.device(dev):
+        with _hip.on_device(dev):
             status = lib.cce_count_flagged_cells(tile_max.data_ptr(), lse.data_ptr(), B, V, float(filter_eps),
                                                  self.counter.data_ptr(), _hip.current_stream_ptr(dev))
         _hip.check(status, "cce_count_flagged_cells")
@@ -180,7 +180,7 @@ def _dense_backward(lib, code, dev, e, c, bias, lse, do, dlse, valids, targets, 
     ws_bytes = lib.cce_backward_dense_workspace_bytes(B, V, D, 1 if de_in_ws else 0, int(dz_budget))
     workspace = torch.empty((ws_bytes + 256,), dtype=torch.uint8, device=dev)
     ws_ptr = (workspace.data_ptr() + 255) // 256 * 256
-    with torch.cuda.device(dev), _hip.timed("backward_dense", dev):
+    with _hip.on_device(dev), _hip.timed("backward_dense", dev):
         status = lib.cce_backward_dense(
             e.data_ptr(), c.data_ptr(), _hip.ptr(bias),
             lse.data_ptr(), do.data_ptr(), 1 if do.numel() == 1 else 0, _hip.ptr(dlse),
@@ -356,7 +356,7 @@ def cce_backward_kernel(
     if B > 0 and (de_sparse or dc_sparse):
         ws_bytes = lib.cce_backward_workspace_bytes(B, c.size(0), e.size(1))
         workspace = torch.empty((max(ws_bytes, 8) // 8 + 1,), dtype=torch.int64, device=dev)
-        with torch.cuda.device(dev), _hip.timed("backward_sparse", dev):
+        with _hip.on_device(dev), _hip.timed("backward_sparse", dev):
             status = lib.cce_backward(
                 e.data_ptr(), c.data_ptr(), _hip.ptr(bias),
                 lse.data_ptr(), do.data_ptr(), 1 if do.numel() == 1 else 0, _hip.ptr(dlse),

@@ -53,7 +53,7 @@ def lse_forward(
 
     ws_bytes = lib.cce_lse_forward_workspace_bytes(B, V, D)
     workspace = torch.empty((max(ws_bytes, 8) // 8,), dtype=torch.int64, device=e.device)
-    with torch.cuda.device(e.device), _hip.timed("lse_forward", e.device):
+    with _hip.on_device(e.device), _hip.timed("lse_forward", e.device):
         status = lib.cce_lse_forward(
             e.data_ptr(), c.data_ptr(), _hip.ptr(bias), _hip.ptr(valids),
             lse.data_ptr(), _hip.ptr(logit_avg), _hip.ptr(tile_max),
@@ -65,6 +65,53 @@ def lse_forward(
         )
     _hip.check(status, "cce_lse_forward")
     return lse, logit_avg, tile_max
+
+
+def loss_forward(
+    e: torch.Tensor,
+    c: torch.Tensor,
+    bias: Optional[torch.Tensor],
+    targets: torch.Tensor,
+    valids: Optional[torch.Tensor],
+    shift: int,
+    softcap: Optional[float],
+    target_offset: int,
+    want_tile_max: bool,
+) -> Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
+    """``(lse, nll, tile_max | None)`` of the valid rows in one library call: ``lse_forward`` plus the logit of each
+    row's target (``indexed_neg_dot_forward_kernel``), merged and added up by one kernel."""
+    assert e.ndim == 2 and c.ndim == 2 and e.is_contiguous()
+    assert e.shape[1] == c.shape[1], "Incompatible dimensions"
+    _hip.require_gpu_tensor("e", e)
+    dev = e.device
+    assert c.device == dev and c.dtype == e.dtype
+    V, D = c.shape
+    code = _hip.dtype_code(e.dtype)
+    lib = _hip.load()
+    B = valids.numel() if valids is not None else e.shape[0]
+    if bias is not None:
+        assert bias.ndim == 1 and bias.shape[0] == V
+        bias = bias.to(e.dtype).contiguous()
+    targets = targets.to(torch.int64).contiguous()
+    lse = torch.empty((B,), dtype=torch.float32, device=dev)
+    nll = torch.empty((B,), dtype=torch.float32, device=dev)
+    tile_max = None
+    if want_tile_max:
+        tile_max = torch.empty((lib.cce_tile_stat_elems(B, V),), dtype=torch.float32, device=dev)
+    if B == 0:
+        return lse, nll, tile_max
+    ws_bytes = lib.cce_lse_forward_workspace_bytes(B, V, D)
+    workspace = torch.empty((max(ws_bytes, 8) // 8,), dtype=torch.int64, device=dev)
+    with _hip.on_device(dev), _hip.timed("lse_forward", dev):
+        status = lib.cce_loss_forward(
+            e.data_ptr(), c.data_ptr(), _hip.ptr(bias), _hip.ptr(valids), targets.data_ptr(),
+            lse.data_ptr(), nll.data_ptr(), _hip.ptr(tile_max), workspace.data_ptr(), workspace.numel() * 8,
+            e.shape[0], B, V, D, e.stride(0), c.stride(0), c.stride(1),
+            int(shift), int(target_offset), float(softcap) if softcap is not None else 0.0, code,
+            _hip.current_stream_ptr(dev),
+        )
+    _hip.check(status, "cce_loss_forward")
+    return lse, nll, tile_max
 
 
 def cce_lse_forward_kernel(

@@ -39,28 +39,28 @@ def _as_fp32(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
 
 
 def fp32_forward(e, c, bias, targets, valids, shift, softcap, target_offset) -> Tuple[torch.Tensor, torch.Tensor]:
-    """``(lse, neg_dot)`` of the valid rows: the log-sum-exp over the whole vocabulary, and minus the (soft-capped)
-    logit of the target, 0 where the target is not a class of this shard."""
+    """``(lse, nll)`` of the valid rows: the log-sum-exp over the whole vocabulary, and what is left of it when the
+    (soft-capped) logit of the target is taken off (all of it where the target is not a class of this shard)."""
     lib = _hip.load()
     dev = e.device
     b = valids.numel() if valids is not None else e.size(0)
     lse = torch.empty((b,), dtype=torch.float32, device=dev)
-    neg_dot = torch.empty((b,), dtype=torch.float32, device=dev)
+    nll = torch.empty((b,), dtype=torch.float32, device=dev)
     if b == 0:
-        return lse, neg_dot
+        return lse, nll
     terms = n_terms()
     bias, targets = _as_fp32(bias), targets.to(torch.int64).contiguous()
     ws_bytes = lib.cce_fp32_forward_workspace_bytes(b, c.size(0), c.size(1), terms)
     _buf, ws = _workspace(ws_bytes, dev)
-    with torch.cuda.device(dev):
+    with _hip.on_device(dev):
         status = lib.cce_fp32_forward(
             e.data_ptr(), c.data_ptr(), _hip.ptr(bias), _hip.ptr(valids), targets.data_ptr(),
-            lse.data_ptr(), neg_dot.data_ptr(), ws, ws_bytes,
+            lse.data_ptr(), nll.data_ptr(), ws, ws_bytes,
             e.size(0), b, c.size(0), c.size(1), e.stride(0), c.stride(0), c.stride(1),
             int(shift), int(target_offset), float(softcap) if softcap is not None else 0.0, terms,
             _hip.current_stream_ptr(dev))
     _hip.check(status, "cce_fp32_forward")
-    return lse, neg_dot
+    return lse, nll
 
 
 def fp32_backward(e, c, bias, lse, do, dlse, valids, targets, shift, target_offset, softcap, grad_scale,
@@ -88,7 +88,7 @@ def fp32_backward(e, c, bias, lse, do, dlse, valids, targets, shift, target_offs
     dlse = dlse.to(torch.float32).contiguous().view(-1) if dlse is not None else None
     ws_bytes = lib.cce_fp32_backward_workspace_bytes(b, v, d, terms)
     _buf, ws = _workspace(ws_bytes, dev)
-    with torch.cuda.device(dev):
+    with _hip.on_device(dev):
         status = lib.cce_fp32_backward(
             e.data_ptr(), c.data_ptr(), _hip.ptr(bias), lse.data_ptr(), do.data_ptr(), 1 if do.numel() == 1 else 0,
             _hip.ptr(dlse), _hip.ptr(valids), targets.data_ptr(), _hip.ptr(de), _hip.ptr(dc), _hip.ptr(dbias), ws, ws_bytes,

@@ -48,7 +48,7 @@ def indexed_neg_dot_forward_kernel(
 
     out = torch.empty((B,), dtype=torch.float32, device=e.device)
     if B > 0:
-        with torch.cuda.device(e.device):
+        with _hip.on_device(e.device):
             status = lib.cce_indexed_neg_dot(
                 e.data_ptr(), c.data_ptr(), inds.data_ptr(), _hip.ptr(bias), _hip.ptr(valids),
                 out.data_ptr(),

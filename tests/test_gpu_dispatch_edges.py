@@ -129,7 +129,7 @@ def test_fp32_passes_abi(shape, keep, extra, terms):
     B, cap = rows.numel(), extra.get("softcap")
     p = lambda x: x.data_ptr() if x is not None else None
     lse = torch.full((B,), float("nan"), device=dev)
-    dot = torch.full((B,), float("nan"), device=dev)
+    nll = torch.full((B,), float("nan"), device=dev)
     stream = torch.cuda.current_stream().cuda_stream
 
     def workspace(nbytes):
@@ -138,7 +138,7 @@ def test_fp32_passes_abi(shape, keep, extra, terms):
 
     n_ws = lib.cce_fp32_forward_workspace_bytes(B, V, D, terms)
     buf, ws = workspace(n_ws)
-    st = lib.cce_fp32_forward(p(e), p(c), p(bias), p(valids), p(t), p(lse), p(dot), ws, n_ws, N, B, V, D, e.stride(0), c.stride(0),
+    st = lib.cce_fp32_forward(p(e), p(c), p(bias), p(valids), p(t), p(lse), p(nll), ws, n_ws, N, B, V, D, e.stride(0), c.stride(0),
                               1, 0, 0, cap or 0.0, terms, stream)
     assert st == 0, lib.cce_error_string(st)
     x = e.double()[rows] @ c.double().T + (bias.double() if bias is not None else 0.0)
@@ -152,7 +152,7 @@ def test_fp32_passes_abi(shape, keep, extra, terms):
     tol = 4e-6 if terms == 6 else 4e-5
     assert torch.allclose(lse.double(), want_lse, atol=tol, rtol=2e-6)
     # plain fp32 whatever the number of terms: D roundings of terms of up to 1
-    assert torch.allclose(dot.double(), -x[torch.arange(B, device=dev), t[rows]], atol=2e-5, rtol=2e-6)
+    assert torch.allclose(nll.double(), want_lse - x[torch.arange(B, device=dev), t[rows]], atol=2e-5 + tol, rtol=2e-6)
     dz = torch.exp(x - want_lse[:, None]) * (w.double()[rows] + (h.double()[rows] if h is not None else 0.0))[:, None]
     dz[torch.arange(B, device=dev), t[rows]] -= w.double()[rows]
     dz *= damp
@@ -182,3 +182,43 @@ def test_fp32_passes_abi(shape, keep, extra, terms):
     ignored = torch.ones(N, dtype=torch.bool, device=dev)
     ignored[rows] = False
     assert (de[ignored] == 0).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 64), (3, 21), (1, 8192), (1, 8193), (7, 1171), (5, 5000)])
+@pytest.mark.parametrize("keep", [0.0, 0.4, 1.0])
+def test_valid_rows_kernel_matches_the_host(shape, keep):
+    """One trip of 8192 positions and its edges, sequences that end inside a wave, nothing and everything ignored."""
+    from cut_cross_entropy.utils import _build_flat_valids
+
+    t = torch.randint(0, 50, shape, generator=torch.Generator().manual_seed(1))
+    t[torch.rand(shape, generator=torch.Generator().manual_seed(2)) >= keep] = -100
+    for shift in (0, 1, 3):
+        if shift >= shape[1]:
+            continue
+        want = _build_flat_valids(t, -100, shift)
+        got = _build_flat_valids(t.cuda(), -100, shift)
+        assert (want is None) == (got is None)
+        if want is not None:
+            assert got.dtype == torch.int32 and torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(2, 3, 8), (5, 256 * 70, 128), (130, 700, 123), (1000, 2000, 192)])
+@pytest.mark.parametrize("softcap,bias,shift", [(None, False, 0), (15.0, True, 1)])
+def test_loss_forward_matches_its_two_halves(dtype, shape, softcap, bias, shift):
+    """cce_loss_forward against cce_lse_forward and cce_indexed_neg_dot on the same inputs: more spans than lanes, one
+    span, a width the vector loads cannot take, targets that are no class of the shard."""
+    from cut_cross_entropy.cce_lse_forward import cce_lse_forward_kernel, loss_forward
+    from cut_cross_entropy.indexed_dot import indexed_neg_dot_forward_kernel
+
+    N, V, D = shape
+    e, c, t, b = make_inputs(N, V, D, dtype, seed=8, bias=bias)
+    t = t * 2 - V // 2  # half of them outside [0, V)
+    valids = torch.arange(0, N - shift, 3, dtype=torch.int32).cuda() if shift else None
+    e, c, t, b = e.cuda(), c.cuda(), t.cuda(), b.cuda() if b is not None else None
+    lse, nll, _ = loss_forward(e, c, b, t, valids, shift, softcap, 0, False)
+    want = cce_lse_forward_kernel(e, c, b, valids, softcap)
+    dot = indexed_neg_dot_forward_kernel(e, c, t, b, shift, valids, softcap, torch.float32)
+    # the same sums in another order: fp32 rounding of quantities of up to 20
+    assert torch.allclose(lse, want, atol=4e-6, rtol=4e-7)
+    assert torch.allclose(nll, dot + want, atol=8e-6, rtol=1e-6)
