@@ -1282,9 +1282,11 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
 }
 
 // Number of cells of the forward statistic (32 rows x 32 classes) whose bound exp(max logit - min lse of the 32
-// rows) reaches eps: the cells the ownership kernels have to recompute.  One workgroup per row group.
+// rows) reaches eps: the cells the ownership kernels have to recompute.  One workgroup per row group.  With `answer` the
+// last workgroup to finish moves the total there and leaves count[0] (the sum) and count[1] (workgroups done) at zero for
+// the next launch on the same stream: one launch in place of a fill, the count and a copy.
 __global__ __launch_bounds__(256) void flagged_cells_kernel(const float* tile_max, const float* lse, int64_t b, int stat_cols,
-                                                            float log_eps, unsigned long long* count) {
+                                                            float log_eps, unsigned long long* count, unsigned long long* answer) {
   __shared__ float s_min;
   __shared__ unsigned int s_part[4];
   const int tg = blockIdx.x;
@@ -1303,25 +1305,45 @@ __global__ __launch_bounds__(256) void flagged_cells_kernel(const float* tile_ma
   for (int off = 32; off >= 1; off >>= 1) n += __shfl_xor(n, off, 64);
   if (lane == 0) s_part[wave] = n;
   __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(count, static_cast<unsigned long long>(s_part[0] + s_part[1] + s_part[2] + s_part[3]));
+  if (threadIdx.x == 0) {
+    atomicAdd(count, static_cast<unsigned long long>(s_part[0] + s_part[1] + s_part[2] + s_part[3]));
+    if (answer != nullptr) {
+      __threadfence();  // this workgroup's share is in the sum before it is counted as done
+      if (atomicAdd(count + 1, 1ull) == gridDim.x - 1ull) {
+        *answer = atomicExch(count, 0ull);
+        count[1] = 0ull;
+      }
+    }
+  }
 }
 
 }  // namespace cce
 
 using namespace cce;
 
-extern "C" int cce_count_flagged_cells(const float* tile_max, const float* lse, int64_t b, int64_t v, float filter_eps,
-                                       uint64_t* count, void* stream_) {
+static int count_flagged_cells(const float* tile_max, const float* lse, int64_t b, int64_t v, float filter_eps, uint64_t* count,
+                               uint64_t* answer, void* stream) {
   if (b < 0 || v <= 0 || !(filter_eps > 0.0f)) return CCE_ERR_INVALID_ARGUMENT;
   if (b == 0) return CCE_OK;
   if (tile_max == nullptr || lse == nullptr || count == nullptr) return CCE_ERR_INVALID_ARGUMENT;
   const int64_t ntg = (b + CCE_STAT_ROWS - 1) / CCE_STAT_ROWS;
   if (ntg >= (int64_t(1) << 31) || v >= (int64_t(1) << 31) - 512) return CCE_ERR_INVALID_ARGUMENT;
   const int stat_cols = static_cast<int>((v + CCE_STAT_COLS - 1) / CCE_STAT_COLS);
-  hipLaunchKernelGGL(flagged_cells_kernel, dim3(static_cast<unsigned>(ntg)), dim3(256), 0, static_cast<hipStream_t>(stream_),
+  hipLaunchKernelGGL(flagged_cells_kernel, dim3(static_cast<unsigned>(ntg)), dim3(256), 0, static_cast<hipStream_t>(stream),
                      tile_max, lse, b, stat_cols, logf(filter_eps) - 0.01f,
-                     reinterpret_cast<unsigned long long*>(count));
+                     reinterpret_cast<unsigned long long*>(count), reinterpret_cast<unsigned long long*>(answer));
   return status_from_hip(hipGetLastError());
+}
+
+extern "C" int cce_count_flagged_cells(const float* tile_max, const float* lse, int64_t b, int64_t v, float filter_eps,
+                                       uint64_t* count, void* stream) {
+  return count_flagged_cells(tile_max, lse, b, v, filter_eps, count, nullptr, stream);
+}
+
+extern "C" int cce_measure_flagged_cells(const float* tile_max, const float* lse, int64_t b, int64_t v, float filter_eps,
+                                         uint64_t* scratch, uint64_t* answer, void* stream) {
+  if (answer == nullptr || b <= 0) return CCE_ERR_INVALID_ARGUMENT;
+  return count_flagged_cells(tile_max, lse, b, v, filter_eps, scratch, answer, stream);
 }
 
 static int64_t bit_words_for(int64_t v) { return ((v + 31) / 32 + 31) / 32; }

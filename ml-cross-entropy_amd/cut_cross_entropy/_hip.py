@@ -53,6 +53,7 @@ _SIGNATURES = {
         + [_i64] * 4 + [_i64] * 3 + [_f32, _f32, _i32, _i32, _i32, _i32, _i64, _i64, _f32, _i32, _ptr],
     ),
     "cce_count_flagged_cells": (_i32, [_ptr, _ptr, _i64, _i64, _f32, _ptr, _ptr]),
+    "cce_measure_flagged_cells": (_i32, [_ptr, _ptr, _i64, _i64, _f32, _ptr, _ptr, _ptr]),
     "cce_backward_dense_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32, _i64]),
     "cce_backward_dense_fixed_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "cce_backward_dense_dz_bytes": (_i64, [_i64, _i64, _i64, _i32, _i64]),

@@ -74,7 +74,7 @@ class _FlaggedMonitor:
     """Fraction of flagged cells of the latest backward of one (device, V, D, dtype), and the path it chose."""
 
     def __init__(self, device: torch.device):
-        self.counter = torch.zeros((1,), dtype=torch.int64, device=device)
+        self.scratch: dict = {}  # stream -> the two words its measurements count in
         self.host = torch.zeros((1,), dtype=torch.int64, pin_memory=True)
         self.event = torch.cuda.Event()
         self.pending_cells = 0   # cells of the measurement in flight (0: none)
@@ -90,13 +90,17 @@ class _FlaggedMonitor:
             self.pending_cells = 0
 
     def measure(self, lib, tile_max, lse, B: int, V: int, filter_eps: float, dev: torch.device) -> None:
-        self.counter.zero_()
+        stream = torch.cuda.current_stream(dev)
+        scratch = self.scratch.get(stream.cuda_stream)
+        if scratch is None:
+            if len(self.scratch) >= 16:  # streams come and go; whatever of theirs is still running holds its own memory
+                self.scratch.clear()
+            scratch = self.scratch[stream.cuda_stream] = torch.zeros((2,), dtype=torch.int64, device=dev)
         with _hip.on_device(dev):
-            status = lib.cce_count_flagged_cells(tile_max.data_ptr(), lse.data_ptr(), B, V, float(filter_eps),
-                                                 self.counter.data_ptr(), _hip.current_stream_ptr(dev))
-        _hip.check(status, "cce_count_flagged_cells")
-        self.host.copy_(self.counter, non_blocking=True)
-        self.event.record(torch.cuda.current_stream(dev))
+            status = lib.cce_measure_flagged_cells(tile_max.data_ptr(), lse.data_ptr(), B, V, float(filter_eps),
+                                                   scratch.data_ptr(), self.host.data_ptr(), stream.cuda_stream)
+        _hip.check(status, "cce_measure_flagged_cells")
+        self.event.record(stream)
         self.pending_cells = lib.cce_tile_stat_elems(B, V)
 
 
