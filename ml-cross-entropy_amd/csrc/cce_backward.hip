@@ -54,6 +54,11 @@ struct BwdParams {
   int* heavy_list;  // [1 + nvg]: count, then the class groups the light variant leaves to the full one
   int ntg, nvc, nvg, bit_words, nslices, dslice, stat_cols;
   int vec_e, vec_c;  // 4-element vector stores are legal for dE / dC
+  // dE pass of the fast kernels with few row groups: the trips of a row group are dealt to `parts` workgroups, each with
+  // an fp32 slot [32 ntg][d] and a set of survivor bits of its own (owner_merge_kernel puts them together); 1: none
+  int parts;
+  float* slots;
+  uint32_t* part_bits;  // [parts][ntg][bit_words]
   Softcap sc;
 };
 
@@ -723,8 +728,10 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int half = lane >> 5;
-  int own = blockIdx.x / p.nslices;
-  const int slice = blockIdx.x % p.nslices;
+  const int parts = IS_DE ? p.parts : 1;
+  const int part = IS_DE ? static_cast<int>(blockIdx.x) % parts : 0;
+  int own = blockIdx.x / (p.nslices * parts);
+  const int slice = (blockIdx.x / parts) % p.nslices;
   if (IS_DE && blockIdx.x == 0 && threadIdx.x == 0 && p.heavy_list != nullptr) p.heavy_list[0] = 0;  // for the dC passes
   if (!IS_DE && !LIGHT && p.light_on) {
     // the full dC pass after the light one: only the class groups that one listed
@@ -810,6 +817,7 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   const int seg_units = IS_DE ? kFSegCells : kFListCap;
 
   int carry = 0;  // listed entries a segment left over for the next one (trips are filled four at a time)
+  int trip = 0;   // of the row group, counted by all of its workgroups alike
   for (int seg = 0; seg < n_units; seg += seg_units) {
     const int seg_n = min(seg_units, n_units - seg);
     if (use_list) {
@@ -887,6 +895,7 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
     const int run_n = keep_rest ? (list_n & ~3) : list_n;
 
     for (int li = 0; li < run_n; li += 4) {
+      if (IS_DE && trip++ % parts != part) continue;
       if (IS_DE) {
         if (tid < 128) {
           const int k = li + (tid >> 5);
@@ -1188,7 +1197,8 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   }
 
   mfma_drain_all();  // the last product MFMAs, before anything else reads the accumulators
-  const bool out_fp32 = IS_DE ? (p.de_fp32 != 0) : (p.dc_fp32 != 0);
+  const bool to_slot = IS_DE && parts > 1;
+  const bool out_fp32 = IS_DE ? (p.de_fp32 != 0 || to_slot) : (p.dc_fp32 != 0);
   if constexpr (LIGHT) {
     if (write_out && !touched) {
       // Nothing survived for this class group: its rows are zeros, written as whole 16-byte pieces, a wave
@@ -1203,11 +1213,16 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
                                     (j - row * ppr) * 8) = zero;
       }
     }
-  } else if (write_out && (touched || !IS_DE)) {  // dC rows are always written; the launcher guarantees 16-byte aligned rows
+  } else if (write_out && (touched || !IS_DE || to_slot)) {  // dC rows and slots are always written; the launcher guarantees 16-byte aligned rows
     // The accumulators hold the tile transposed (lane = own row, registers = columns): stored as they
     // are, one instruction would touch 32 rows with 16 bytes each.  Four chunks at a time go through
     // LDS instead and leave as whole rows, 16 bytes per lane and 1 KB per row and instruction.
     unsigned char* out_base = static_cast<unsigned char*>(IS_DE ? p.d_e : p.d_c);
+    int64_t out_sr = own_sr;
+    if (to_slot) {
+      out_base = reinterpret_cast<unsigned char*>(p.slots + (static_cast<int64_t>(part) * p.ntg + own) * 32 * p.d);
+      out_sr = p.d;
+    }
     auto store_tile = [&](auto fp32_tag) {
       constexpr bool FP32 = decltype(fp32_tag)::value;
       constexpr int es = FP32 ? 4 : 2;
@@ -1247,14 +1262,14 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
             const int ja = j, jb = j + kBwdThreads;
             const int rowa = ja / ppr, rowb = jb / ppr;
             const int pca = ja - rowa * ppr, pcb = jb - rowb * ppr;
-            const int ida = own_ids[rowa], idb = own_ids[rowb];
+            const int ida = to_slot ? rowa : own_ids[rowa], idb = to_slot ? rowb : own_ids[rowb];
             const uint4 va = *reinterpret_cast<const uint4*>(smem + rowa * pitch + pca * 16);
             const uint4 vb = *reinterpret_cast<const uint4*>(smem + rowb * pitch + pcb * 16);
             const int64_t col_bytes = static_cast<int64_t>(d_begin + g * 4 * kFCols) * es;
             if (ida >= 0)
-              *reinterpret_cast<uint4*>(out_base + static_cast<int64_t>(ida) * own_sr * es + col_bytes + pca * 16) = va;
+              *reinterpret_cast<uint4*>(out_base + static_cast<int64_t>(ida) * out_sr * es + col_bytes + pca * 16) = va;
             if (idb >= 0)
-              *reinterpret_cast<uint4*>(out_base + static_cast<int64_t>(idb) * own_sr * es + col_bytes + pcb * 16) = vb;
+              *reinterpret_cast<uint4*>(out_base + static_cast<int64_t>(idb) * out_sr * es + col_bytes + pcb * 16) = vb;
           }
         }
       }
@@ -1264,9 +1279,10 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   }
   if (slice == 0) {
     if (IS_DE) {
-      if (p.kept_bits != nullptr)
-        for (int w = tid; w < p.bit_words; w += kBwdThreads)
-          p.kept_bits[static_cast<int64_t>(own) * p.bit_words + w] = sBits[w];
+      if (p.kept_bits != nullptr) {
+        uint32_t* bits = to_slot ? p.part_bits + static_cast<int64_t>(part) * p.ntg * p.bit_words : p.kept_bits;
+        for (int w = tid; w < p.bit_words; w += kBwdThreads) bits[static_cast<int64_t>(own) * p.bit_words + w] = sBits[w];
+      }
       if (p.counters != nullptr) {
         if (lane == 0 && n_recomputed) atomicAdd(p.counters + 1, n_recomputed);
         if (tid == 0 && n_product) atomicAdd(p.counters + 2, n_product);
@@ -1279,6 +1295,42 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
       if (p.counters != nullptr && tid == 0 && n_product) atomicAdd(p.counters + 3, n_product);
     }
   }
+}
+
+// The slots and survivor bits of a dE pass whose row groups were dealt to several workgroups: dE rows = sum of the slots
+// in their order, bits = union.  Eight columns of a row per thread, then a word of bits per thread.
+template <typename T>
+__global__ __launch_bounds__(256) void owner_merge_kernel(BwdParams p) {
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int per_row = static_cast<int>(p.d / 8);
+  const int64_t pieces = p.d_e != nullptr ? p.b * per_row : 0;
+  if (item < pieces) {
+    const int64_t i = item / per_row;
+    const int col = static_cast<int>(item - i * per_row) * 8;
+    float v[8] = {};
+    for (int s = 0; s < p.parts; ++s) {
+      const float* src = p.slots + (static_cast<int64_t>(s) * p.ntg * 32 + i) * p.d + col;
+      const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
+      v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
+      v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
+    }
+    const int64_t off = (p.valids ? static_cast<int64_t>(p.valids[i]) : i) * p.stride_e + col;
+    if (p.de_fp32) {
+      float4* dst = reinterpret_cast<float4*>(static_cast<float*>(p.d_e) + off);
+      dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+      dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+    } else {
+      *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.d_e) + off) =
+          make_uint4(Elem<T>::pack2(v[0], v[1]), Elem<T>::pack2(v[2], v[3]), Elem<T>::pack2(v[4], v[5]), Elem<T>::pack2(v[6], v[7]));
+    }
+    return;
+  }
+  const int64_t words = static_cast<int64_t>(p.ntg) * p.bit_words;
+  const int64_t w = item - pieces;
+  if (p.kept_bits == nullptr || w >= words) return;
+  uint32_t bits = 0u;
+  for (int s = 0; s < p.parts; ++s) bits |= p.part_bits[s * words + w];
+  p.kept_bits[w] = bits;
 }
 
 // Number of cells of the forward statistic (32 rows x 32 classes) whose bound exp(max logit - min lse of the 32
@@ -1351,10 +1403,28 @@ static int64_t bit_words_for(int64_t v) { return ((v + 31) / 32 + 31) / 32; }
 // survivor bits, then the list of class groups for the full dC pass (a count and up to one id per group)
 static int64_t kept_bits_bytes(int64_t b, int64_t v) { return ((b + 31) / 32) * bit_words_for(v) * 4; }
 
+static int owner_slices(int64_t d) { return static_cast<int>((d + kMaxChunks * kStageCols - 1) / (kMaxChunks * kStageCols)); }
+
+// Workgroups per row group (and slice of D) of the dE pass: as many as fill the chip, at most 16 (a row group has 8 trips
+// and more: its 32 rows have that many labels), and no more slots than half of C takes (E [307, 5120] x C [131072, 5120]:
+// 30 workgroups took 745 us, 240 take 174 and 11 to put the slots together).
+static int owner_parts(int64_t b, int64_t v, int64_t d) {
+  const int64_t groups = (b + 31) / 32 * owner_slices(d);
+  int64_t n = compute_units() / groups;
+  if (n > 16) n = 16;
+  if (n > v / (4 * b)) n = v / (4 * b);
+  return n < 1 ? 1 : static_cast<int>(n);
+}
+static int64_t round16(int64_t x) { return (x + 15) / 16 * 16; }
+// what the parts keep behind the lists: bits, then slots
+static int64_t part_bits_bytes(int64_t b, int64_t v, int parts) { return parts > 1 ? round16(parts * kept_bits_bytes(b, v)) : 0; }
+static int64_t lists_bytes(int64_t b, int64_t v) { return kept_bits_bytes(b, v) + (1 + (v + 31) / 32) * 4; }
+
 extern "C" int64_t cce_backward_workspace_bytes(int64_t b, int64_t v, int64_t d) {
-  (void)d;
   if (b <= 0 || v <= 0) return 0;
-  return kept_bits_bytes(b, v) + (1 + (v + 31) / 32) * 4;
+  const int parts = owner_parts(b, v, d);
+  if (parts == 1) return lists_bytes(b, v);
+  return round16(lists_bytes(b, v)) + part_bits_bytes(b, v, parts) + parts * ((b + 31) / 32 * 32) * d * 4;
 }
 
 extern "C" int cce_backward(const void* e, const void* c, const void* bias,
@@ -1418,7 +1488,7 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
   p.nvc = static_cast<int>((v + 127) / 128);
   p.nvg = static_cast<int>((v + 31) / 32);
   p.bit_words = static_cast<int>(bit_words_for(v));
-  p.nslices = static_cast<int>((d + kMaxChunks * kStageCols - 1) / (kMaxChunks * kStageCols));
+  p.nslices = owner_slices(d);
   const int64_t per = (d + p.nslices - 1) / p.nslices;
   p.dslice = static_cast<int>((per + kStageCols - 1) / kStageCols * kStageCols);
   p.stat_cols = static_cast<int>((v + CCE_STAT_COLS - 1) / CCE_STAT_COLS);
@@ -1434,9 +1504,11 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
   const bool need_bits = need_dc_pass && p.filter_c;
   const bool need_de_pass = (d_e != nullptr) || need_bits;
   p.kept_bits = nullptr;
+  p.parts = 1;
+  p.slots = nullptr;
+  p.part_bits = nullptr;
   if (need_bits) {
-    const int64_t need = cce_backward_workspace_bytes(b, v, d);
-    if (workspace == nullptr || workspace_bytes < need) return CCE_ERR_WORKSPACE_TOO_SMALL;
+    if (workspace == nullptr || workspace_bytes < lists_bytes(b, v)) return CCE_ERR_WORKSPACE_TOO_SMALL;
     if ((reinterpret_cast<uintptr_t>(workspace) & 3u) != 0) return CCE_ERR_MISALIGNED;
     p.kept_bits = static_cast<uint32_t*>(workspace);
     p.heavy_list = reinterpret_cast<int*>(static_cast<unsigned char*>(workspace) + kept_bits_bytes(b, v));
@@ -1474,10 +1546,27 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
   const int full_slices = p.nslices;
   if (need_de_pass) {
     p.nslices = (d_e != nullptr) ? full_slices : 1;
-    const unsigned grid = static_cast<unsigned>(p.ntg) * static_cast<unsigned>(p.nslices);
+    // (a caller who brings less workspace than the size query names gets one workgroup per row group)
+    const int parts = owner_parts(b, v, d);
+    if (fast && parts > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
+        workspace_bytes >= cce_backward_workspace_bytes(b, v, d)) {
+      unsigned char* const ws = static_cast<unsigned char*>(workspace) + round16(lists_bytes(b, v));
+      p.parts = parts;
+      p.part_bits = reinterpret_cast<uint32_t*>(ws);
+      p.slots = reinterpret_cast<float*>(ws + part_bits_bytes(b, v, parts));
+    }
+    const unsigned grid = static_cast<unsigned>(p.ntg) * static_cast<unsigned>(p.nslices) * static_cast<unsigned>(p.parts);
     CCE_LAUNCH_OWNER(true, grid);
     err = hipGetLastError();
     if (err != hipSuccess) return status_from_hip(err);
+    if (p.parts > 1) {
+      const int64_t items = (d_e != nullptr ? b * (d / 8) : 0) + (p.kept_bits != nullptr ? static_cast<int64_t>(p.ntg) * p.bit_words : 0);
+      const dim3 blocks(static_cast<unsigned>((items + 255) / 256));
+      if (dtype == CCE_DTYPE_BF16) hipLaunchKernelGGL(owner_merge_kernel<BF16>, blocks, dim3(256), 0, stream, p);
+      else hipLaunchKernelGGL(owner_merge_kernel<F16>, blocks, dim3(256), 0, stream, p);
+      err = hipGetLastError();
+      if (err != hipSuccess) return status_from_hip(err);
+    }
   }
   if (need_dc_pass) {
     // Class groups with at most two surviving entries (most of them when rows are few against the classes) go to a

@@ -222,3 +222,60 @@ def test_loss_forward_matches_its_two_halves(dtype, shape, softcap, bias, shift)
     # the same sums in another order: fp32 rounding of quantities of up to 20
     assert torch.allclose(lse, want, atol=4e-6, rtol=4e-7)
     assert torch.allclose(nll, dot + want, atol=8e-6, rtol=1e-6)
+
+
+@pytest.mark.parametrize("shape", [(1, 4000, 128), (33, 20000, 256), (200, 9000, 2432), (500, 40000, 128), (90, 30000, 4736)])
+@pytest.mark.parametrize("fp32_out", [False, True])
+@pytest.mark.parametrize("with_dlse,gathered", [(False, False), (True, True)])
+def test_filtered_backward_of_few_rows_deals_its_trips(shape, fp32_out, with_dlse, gathered):
+    """Few row groups: their trips are dealt to several workgroups with a slot each.  One row group (16 parts), parts that
+    get no trip, one to three slices of D.  The same call with less workspace runs one workgroup per row group: the same
+    sub-tiles survive, so dC has the same bits, and dE is the same sum in another order."""
+    lib = _lib()
+    dev = torch.device("cuda:0")
+    N, V, D = shape
+    g = torch.Generator(device=dev).manual_seed(17)
+    c = torch.randn((V, D), generator=g, device=dev).mul_(0.02).bfloat16()
+    t = torch.randint(0, V, (N,), generator=g, device=dev)
+    other = torch.randint(0, V, (N,), generator=g, device=dev)
+    gain = (30.0 / D) ** 0.5 / 0.02
+    e = (gain * (c[t].float() + 0.9 * c[other].float()) * 0.2 + torch.randn((N, D), generator=g, device=dev) * 0.1).bfloat16()
+    rows = torch.arange(N, device=dev)
+    valids = None
+    if gathered:
+        rows = rows[torch.arange(N, device=dev) % 5 != 3]
+        valids = rows.to(torch.int32)
+    B = rows.numel()
+    w = torch.rand((N,), generator=g, device=dev) + 0.5
+    h = torch.randn((N,), generator=g, device=dev) * 0.1 if with_dlse else None
+    p = lambda x: x.data_ptr() if x is not None else None
+    stream = torch.cuda.current_stream().cuda_stream
+    lse = torch.empty((B,), device=dev)
+    tile_max = torch.empty((lib.cce_tile_stat_elems(B, V),), device=dev)
+    n_ws = lib.cce_lse_forward_workspace_bytes(B, V, D)
+    ws = torch.empty((n_ws // 8 + 1,), dtype=torch.int64, device=dev)
+    st = lib.cce_lse_forward(p(e), p(c), None, p(valids), p(lse), None, p(tile_max), p(ws), n_ws, N, B, V, D, D, D, 1, 0.0, 0, stream)
+    assert st == 0, lib.cce_error_string(st)
+    most = lib.cce_backward_workspace_bytes(B, V, D)
+    # (a row group's survivor bits, then the count and ids of the class groups left to the second dC pass)
+    least = (B + 31) // 32 * (((V + 31) // 32 + 31) // 32) * 4 + (1 + (V + 31) // 32) * 4
+    assert most > least  # this shape is dealt out
+    gdt = torch.float32 if fp32_out else torch.bfloat16
+    got = []
+    for n_ws in (most, least):
+        ws = torch.full((most // 4 + 1,), float("nan"), device=dev)
+        de = torch.zeros((N, D), dtype=gdt, device=dev)
+        dc = torch.full((V, D), float("nan"), dtype=gdt, device=dev)
+        st = lib.cce_backward(
+            p(e), p(c), None, p(lse), p(w), 0, p(h), p(valids), None, p(t), p(tile_max), p(de), p(dc), None, p(ws), n_ws, None,
+            N, B, V, D, D, D, 1, 1.0, 2.0**-12, 1, 1, int(fp32_out), int(fp32_out), 0, 0, 0.0, 0, stream)
+        assert st == 0, lib.cce_error_string(st)
+        got.append((de, dc))
+    torch.cuda.synchronize()
+    assert torch.isfinite(got[0][0]).all() and torch.isfinite(got[0][1]).all() and got[0][0].abs().max() > 0
+    assert torch.equal(got[0][1], got[1][1])
+    # the slots are fp32 sums of the same products, 1e-6 of the row's largest apart; two such values on either side of a
+    # rounding boundary of bf16 come out one unit in the last place apart, 2^-7 of the value at most
+    a, b = got[0][0].double(), got[1][0].double()
+    scale = b.abs().amax(dim=1, keepdim=True)
+    assert ((a - b).abs() <= (2e-6 if fp32_out else 2.0**-7) * b.abs() + 4e-6 * scale).all()
