@@ -501,25 +501,75 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* slots, int 
   }
 }
 
-// dBias[class] = sum_row dz[row][class] over the chunk: 1024 threads = 16 row lanes x 64 classes.
-template <typename T>
-__global__ __launch_bounds__(1024) void dz_colsum_kernel(const uint16_t* dz, int64_t ldz, int64_t b, int n_cls, float* d_bias) {
-  __shared__ float part[16][64];
-  const int cl = threadIdx.x & 63;
-  const int rl = threadIdx.x >> 6;
-  const int cls = blockIdx.x * 64 + cl;
-  float sum = 0.0f;
-  if (cls < n_cls) {
-    for (int64_t i = rl; i < b; i += 16) sum += Elem<T>::to_float(dz[i * ldz + cls]);
-  }
-  part[rl][cl] = sum;
-  __syncthreads();
-  if (rl == 0 && cls < n_cls) {
-    float t = 0.0f;
+// d_bias[class] += sum over the rows of dz[row][class] (of the parts of it, where dz comes in parts).  A thread reads 16
+// bytes of a row, LANES threads side by side cover 8 LANES classes, and the 1024 / LANES row lanes of a workgroup are
+// added up in LDS in a fixed order.  Bound by reading dz; fewer classes per workgroup (down to a 16-byte column) where
+// there are few classes, so that they make enough workgroups: [54888 rows] x 1088 classes in three parts took 8.1 ms in
+// 17 workgroups of 64 classes and 2-byte reads.
+template <typename T, int LANES>
+__global__ __launch_bounds__(1024) void dz_colsum_kernel(const uint16_t* dz, int64_t ldz, int parts, int64_t b, int n_cls, float* d_bias) {
+  constexpr int kRowLanes = 1024 / LANES;
+  __shared__ float s_sum[kRowLanes][LANES * 8 + 1];
+  const int cl = threadIdx.x % LANES, rl = threadIdx.x / LANES;
+  const int cls = (blockIdx.x * LANES + cl) * 8;
+  float sum[8] = {};
+  if (cls < n_cls) {  // (a row of dz goes on in whole 16-byte pieces)
+    auto value = [&](int64_t i, float (&x)[8]) {
+      for (int part = parts - 1; part >= 0; --part) {
+        const uint4 v = *reinterpret_cast<const uint4*>(dz + (i * parts + part) * ldz + cls);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int j = 0; j < 16; ++j) t += part[j][cl];  // fixed order: deterministic
-    d_bias[cls] += t;
+        for (int k = 0; k < 8; ++k) x[k] += Elem<T>::to_float(static_cast<uint16_t>(w[k >> 1] >> (16 * (k & 1))));
+      }
+    };
+    int64_t i = rl;
+    for (; i + 3 * kRowLanes < b; i += 4 * kRowLanes) {  // four rows in flight
+      float x[4][8] = {};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) value(i + u * kRowLanes, x[u]);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum[k] += (x[0][k] + x[1][k]) + (x[2][k] + x[3][k]);
+    }
+    for (; i < b; i += kRowLanes) {
+      float x[8] = {};
+      value(i, x);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum[k] += x[k];
+    }
   }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) s_sum[rl][cl * 8 + k] = sum[k];
+  __syncthreads();
+  for (int half = kRowLanes / 2; half >= 1; half /= 2) {
+    for (int j = threadIdx.x; j < half * LANES * 8; j += 1024) s_sum[j / (LANES * 8)][j % (LANES * 8)] += s_sum[j / (LANES * 8) + half][j % (LANES * 8)];
+    __syncthreads();
+  }
+  if (threadIdx.x < LANES * 8) {
+    const int c = blockIdx.x * LANES * 8 + threadIdx.x;
+    if (c < n_cls) d_bias[c] += s_sum[0][threadIdx.x];
+  }
+}
+
+int dz_colsum_launch(const uint16_t* dz, int64_t ldz, int parts, int64_t b, int64_t n_cls, float* d_bias, int dtype, hipStream_t stream) {
+  const int pieces = static_cast<int>((n_cls + 7) / 8);
+  // 64 classes (whole lines) per workgroup from 256 workgroups on, else down to 8
+  int lanes = 8;
+  while (lanes > 1 && (pieces + lanes - 1) / lanes < compute_units()) lanes /= 2;
+  const dim3 blocks(static_cast<unsigned>((pieces + lanes - 1) / lanes));
+#define CCE_COLSUM(TT, L)                                                                                            \
+  hipLaunchKernelGGL((dz_colsum_kernel<TT, L>), blocks, dim3(1024), 0, stream, dz, ldz, parts, b, static_cast<int>(n_cls), d_bias)
+#define CCE_COLSUM_LANES(TT)                                                                                         \
+  do {                                                                                                               \
+    if (lanes == 8) CCE_COLSUM(TT, 8);                                                                               \
+    else if (lanes == 4) CCE_COLSUM(TT, 4);                                                                          \
+    else if (lanes == 2) CCE_COLSUM(TT, 2);                                                                          \
+    else CCE_COLSUM(TT, 1);                                                                                          \
+  } while (0)
+  if (dtype == CCE_DTYPE_BF16) CCE_COLSUM_LANES(BF16);
+  else CCE_COLSUM_LANES(F16);
+#undef CCE_COLSUM_LANES
+#undef CCE_COLSUM
+  return status_from_hip(hipGetLastError());
 }
 
 static int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
@@ -566,9 +616,9 @@ static int64_t product_makespan(int64_t n1, int64_t l1, int64_t n2, int64_t l2) 
 // rows outnumber the classes two to one (measured, E [65536, 3584] x C [19008, 3584]: 36.1 ms and 581 MB by classes
 // with 1024-class chunks, against the same 130 MB of dz by rows).  Only with 16-bit gradients: an fp32 dE is its own
 // accumulator.  unit == 0: not even the smallest plan (256 classes / rows) fits.
-//   splits      into how many ranges the reductions of dE and dC are cut.  The gradient that is carried may be cut in any
-//               walk (its slots are then what is carried, in place of the pair and its compensation term), the other one
-//               only where a single launch completes it.
+//   splits      into how many ranges the reductions of dE and dC are cut.  The slots of the gradient that is carried are
+//               then what is carried, in place of the pair and its compensation term; those of the other one are added up
+//               after every launch.
 struct DensePlan {
   bool by_rows;
   int64_t unit;
@@ -589,18 +639,19 @@ static int64_t split_stages(int64_t stages, int splits) { return (stages + split
 // product tile (64 steps of 256 x 256; 1.65 us where all units are busy): the dz tiles in rounds of all units, d / 64
 // stages each, then the product items as they are handed out.  An item of a cut reduction leaves 256 KB of fp32 (and
 // takes them in first, where slots are carried): up to 6 stages of time where every unit does so at once.
-static double launch_cost(int64_t rows, int64_t cls, int64_t d, int de_splits, int dc_splits, bool carried, int terms = 1) {
+static double launch_cost(int64_t rows, int64_t cls, int64_t d, int de_splits, int dc_splits, bool de_carried, bool dc_carried,
+                          int terms = 1) {
   const int64_t cus = compute_units();
   const int64_t tr = (rows + 255) / 256, tc = (cls + 255) / 256, tn = (d + 255) / 256;
   const int64_t dz = (tr * tc + cus - 1) / cus * tn * 4 * terms;
-  auto item = [&](int64_t total, int splits, int64_t tiles) {
+  auto item = [&](int64_t total, int splits, int64_t tiles, bool carried) {
     const int64_t len = split_stages((total + 63) / 64, splits) * terms;
     if (splits == 1) return len;
     const int64_t items = tiles * splits;
     return len + (4 + 6 * (items < cus ? items : cus) / cus) * (carried ? 2 : 1);
   };
-  return static_cast<double>(dz + product_makespan(tc * tn * dc_splits, item(rows, dc_splits, tc * tn),
-                                                   tr * tn * de_splits, item(cls, de_splits, tr * tn)));
+  return static_cast<double>(dz + product_makespan(tc * tn * dc_splits, item(rows, dc_splits, tc * tn, dc_carried),
+                                                   tr * tn * de_splits, item(cls, de_splits, tr * tn, de_carried)));
 }
 
 // Adding the slots up at the end: a launch, and reading them at 4 TB/s (6.6 MB in the time of a stage).
@@ -627,22 +678,21 @@ static DensePlan dense_plan_uncached(int64_t b, int64_t v, int64_t d, bool g16, 
     const bool cut = de_splits > 1 || dc_splits > 1;
     const bool carried_cut = pl.by_rows ? dc_splits > 1 : de_splits > 1;
     const int64_t launches = pl.by_rows ? (b + unit - 1) / unit : (v + unit - 1) / unit;
-    if (launches > 1 && (pl.by_rows ? de_splits : dc_splits) > 1) return;
     const int64_t comp = carried_cut ? 0 : pl.fixed_bytes;
     const int64_t dz = align256((pl.by_rows ? unit * v_pad : b * unit) * 2);
-    const int64_t slots = align256((de_splits > 1 ? de_splits * b * d * 4 : 0)) + align256(dc_splits > 1 ? dc_splits * v * d * 4 : 0);
+    const int64_t slot_rows = pl.by_rows ? std::min(unit, b) : b, slot_cls = pl.by_rows ? v : std::min(unit, v);
+    const int64_t slots = align256(de_splits > 1 ? de_splits * slot_rows * d * 4 : 0) + align256(dc_splits > 1 ? dc_splits * slot_cls * d * 4 : 0);
     if (comp + dz + slots > budget) return;
+    auto launch = [&](int64_t n) {
+      const int64_t rows = pl.by_rows ? n : b, cls = pl.by_rows ? v : n;
+      double cost = 1.0 + launch_cost(rows, cls, d, de_splits, dc_splits, launches > 1 && !pl.by_rows, launches > 1 && pl.by_rows);
+      return cost + (pl.by_rows ? split_sum_cost(rows, d, de_splits) : split_sum_cost(cls, d, dc_splits));
+    };
     const int64_t whole = pl.by_rows ? b / unit : v / unit;
     const int64_t rest = pl.by_rows ? b - whole * unit : v - whole * unit;
-    const bool carried = launches > 1;
-    double cost = 0.0;
-    if (whole > 0)
-      cost += whole * (1.0 + (pl.by_rows ? launch_cost(unit, v, d, de_splits, dc_splits, carried)
-                                         : launch_cost(b, unit, d, de_splits, dc_splits, carried)));
-    if (rest > 0)
-      cost += 1.0 + (pl.by_rows ? launch_cost(rest, v, d, de_splits, dc_splits, carried)
-                                : launch_cost(b, rest, d, de_splits, dc_splits, carried));
-    cost += split_sum_cost(b, d, de_splits) + split_sum_cost(v, d, dc_splits);
+    double cost = pl.by_rows ? split_sum_cost(v, d, dc_splits) : split_sum_cost(b, d, de_splits);
+    if (whole > 0) cost += whole * launch(unit);
+    if (rest > 0) cost += launch(rest);
     if (cost * (cut ? 1.03 : 1.0) >= best * (1.0 - 1e-9)) return;
     best = cost * (cut ? 1.03 : 1.0);
     pl.unit = unit;
@@ -734,16 +784,17 @@ TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_byte
   for (int64_t n = least; n <= least + 2; ++n) {
     const int64_t unit = ((v_pad + n - 1) / n + 255) / 256 * 256;
     const int64_t launches = (v + unit - 1) / unit;
+    const int64_t rest = v - (launches - 1) * unit;
     for (int se : kSplits) {
       if (se > 1 && ((unit + 63) / 64 * terms < se * kMinSplitStages || se * b * d * 4 > most_bytes || unit / 64 < se)) break;
       for (int sc : kSplits) {
-        if (sc > 1 && (!cut_dc || launches > 1 || (b + 63) / 64 * terms < sc * kMinSplitStages || sc * v * d * 4 > most_bytes ||
+        if (sc > 1 && (!cut_dc || (b + 63) / 64 * terms < sc * kMinSplitStages || sc * std::min(unit, v) * d * 4 > most_bytes ||
                        b / 64 < sc))
           break;
-        const int64_t rest = v - (launches - 1) * unit;
-        double cost = static_cast<double>(launches - 1) * (1.0 + launch_cost(b, unit, d, se, sc, launches > 1, terms)) + 1.0 +
-                      launch_cost(b, rest, d, se, sc, launches > 1, terms);
-        cost += split_sum_cost(b, d, se) + split_sum_cost(v, d, sc);
+        auto launch = [&](int64_t cls) {
+          return 1.0 + launch_cost(b, cls, d, se, sc, launches > 1, false, terms) + split_sum_cost(cls, d, sc);
+        };
+        double cost = static_cast<double>(launches - 1) * launch(unit) + launch(rest) + split_sum_cost(b, d, se);
         if (se > 1 || sc > 1) cost *= 1.03;
         if (cost < best * (1.0 - 1e-9)) {
           best = cost;
@@ -886,7 +937,8 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
   uint16_t* dz = reinterpret_cast<uint16_t*>(ws + plan.comp_bytes);
   float* const de_slots = reinterpret_cast<float*>(ws + plan.comp_bytes + plan.dz_bytes);
   float* const dc_slots =
-      reinterpret_cast<float*>(ws + plan.comp_bytes + plan.dz_bytes + (plan.de_splits > 1 ? align256(plan.de_splits * b * d * 4) : 0));
+      reinterpret_cast<float*>(ws + plan.comp_bytes + plan.dz_bytes +
+                               (plan.de_splits > 1 ? align256(plan.de_splits * (by_rows ? std::min(plan.unit, b) : b) * d * 4) : 0));
   const int64_t vc = by_rows ? (v + 255) / 256 * 256 : plan.unit;
   const int64_t ldz = vc;
   const bool de_cut = d_e != nullptr && plan.de_splits > 1;
@@ -913,10 +965,8 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
   p.de_init = 0;
   p.b = b;
   p.d = static_cast<int>(d);
-  p.de_slot = b * d;
-  p.dc_slot = v * d;
   // Ranges of the reductions, fixed by the first launch, which is the largest: it fills every slot there is (seven stages
-  // cut in five make four ranges of two, the last of them short), a later one adds to as many of them as it has ranges.
+  // cut in five make four ranges of two, the last of them short), a later one has as many of them or fewer.
   const int64_t first_rows = by_rows ? std::min(plan.unit, b) : b, first_cls = by_rows ? v : std::min(vc, v);
   p.de_len = static_cast<int>(split_stages((first_cls + 63) / 64, de_cut ? plan.de_splits : 1) * 64);
   p.dc_len = static_cast<int>(split_stages((first_rows + 63) / 64, dc_cut ? plan.dc_splits : 1) * 64);
@@ -928,6 +978,8 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
     p.n_cls = static_cast<int>(cls);
     p.de_splits = static_cast<int>((cls + p.de_len - 1) / p.de_len);
     p.dc_splits = static_cast<int>((rows + p.dc_len - 1) / p.dc_len);
+    p.de_slot = rows * d;  // slots are packed for what they hold: all rows or classes where they are carried
+    p.dc_slot = cls * d;
     p.dc_tiles = (d_c != nullptr) ? static_cast<int>((cls + 255) / 256) * p.tiles_n * p.dc_splits : 0;
     p.de_tiles = (d_e != nullptr) ? static_cast<int>((rows + 255) / 256) * p.tiles_n * p.de_splits : 0;
     p.dc_per_xcd = (p.dc_tiles + 7) / 8;
@@ -958,18 +1010,20 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
         else CCE_LAUNCH_PRODUCT((dense_products_kernel<F16, false>), blocks);
       }
     }
-    if (bias_out != nullptr) {
-      const unsigned cblocks = static_cast<unsigned>((cls + 63) / 64);
-      if (dtype == CCE_DTYPE_BF16)
-        hipLaunchKernelGGL(dz_colsum_kernel<BF16>, dim3(cblocks), dim3(1024), 0, stream, dz, ldz, rows, static_cast<int>(cls),
-                           bias_out);
-      else
-        hipLaunchKernelGGL(dz_colsum_kernel<F16>, dim3(cblocks), dim3(1024), 0, stream, dz, ldz, rows, static_cast<int>(cls),
-                           bias_out);
-    }
+    if (bias_out != nullptr) return dz_colsum_launch(dz, ldz, 1, rows, cls, bias_out, dtype, stream);
     return status_from_hip(hipGetLastError());
   };
 #undef CCE_LAUNCH_PRODUCT
+
+  auto sum_slots = [&](const float* slots, int count, int64_t rows, const int32_t* ids, void* out, int64_t ld, int fp32, int add) {
+    const unsigned blocks = static_cast<unsigned>((rows * (d / 8) + 255) / 256);
+    if (dtype == CCE_DTYPE_BF16)
+      hipLaunchKernelGGL(split_sum_kernel<BF16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d),
+                         static_cast<int>(d), ids, out, ld, fp32, add, 1);
+    else
+      hipLaunchKernelGGL(split_sum_kernel<F16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d),
+                         static_cast<int>(d), ids, out, ld, fp32, add, 1);
+  };
 
   const size_t es = 2;
   if (by_rows) {
@@ -1001,6 +1055,7 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
       set_items(n, v);
       st = products(n, v, d_bias);
       if (st != CCE_OK) return st;
+      if (de_cut) sum_slots(de_slots, p.de_splits, n, valids_blk, static_cast<uint16_t*>(d_e) + shift_rows * stride_e, stride_e, 0, 0);
     }
   } else {
     for (int64_t v0 = 0; v0 < v; v0 += vc) {
@@ -1020,20 +1075,14 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
       set_items(b, n);
       st = products(b, n, d_bias != nullptr ? d_bias + v0 : nullptr);
       if (st != CCE_OK) return st;
+      if (dc_cut)
+        sum_slots(dc_slots, p.dc_splits, n, nullptr, static_cast<unsigned char*>(d_c) + v0 * stride_cv * (d_c_is_fp32 ? 4 : 2), stride_cv,
+                  d_c_is_fp32, 0);
     }
   }
 
-  auto sum_slots = [&](const float* slots, int count, int64_t rows, const int32_t* ids, void* out, int64_t ld, int fp32, int add) {
-    const unsigned blocks = static_cast<unsigned>((rows * (d / 8) + 255) / 256);
-    if (dtype == CCE_DTYPE_BF16)
-      hipLaunchKernelGGL(split_sum_kernel<BF16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d),
-                         static_cast<int>(d), ids, out, ld, fp32, add, 1);
-    else
-      hipLaunchKernelGGL(split_sum_kernel<F16>, dim3(blocks), dim3(256), 0, stream, slots, count, rows, static_cast<int>(d),
-                         static_cast<int>(d), ids, out, ld, fp32, add, 1);
-  };
-  if (de_cut) sum_slots(de_slots, de_nslots, b, valids, d_e, stride_e, d_e_is_fp32, 1);
-  if (dc_cut) sum_slots(dc_slots, dc_nslots, v, nullptr, d_c, stride_cv, d_c_is_fp32, 0);
+  if (de_cut && !by_rows) sum_slots(de_slots, de_nslots, b, valids, d_e, stride_e, d_e_is_fp32, 1);
+  if (dc_cut && by_rows) sum_slots(dc_slots, dc_nslots, v, nullptr, d_c, stride_cv, d_c_is_fp32, 0);
   return status_from_hip(hipGetLastError());
 }
 

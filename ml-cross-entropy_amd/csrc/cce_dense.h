@@ -49,6 +49,8 @@ int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t*
                           int64_t de_slot, int de_len, float* d_c, int64_t ld_dc, bool dc_add, int64_t dc_slot, int dc_len,
                           bool out_vec, int64_t b, int64_t b_pad, int64_t cls, int64_t cls_pad, int64_t d, int64_t part_d, int terms,
                           int parts, hipStream_t stream);
+// d_bias[class] += column sums of dz [b][parts][ldz] in dtype
+int dz_colsum_launch(const uint16_t* dz, int64_t ldz, int parts, int64_t b, int64_t n_cls, float* d_bias, int dtype, hipStream_t stream);
 // out[row(i)][0 .. d) (+)= sum over the slots [count][rows][ld_slot]
 int split_sum_launch(const float* slots, int count, int64_t rows, int64_t d, int64_t ld_slot, const int32_t* ids, float* out,
                      int64_t ld, bool add, bool out_vec, hipStream_t stream);

@@ -77,31 +77,6 @@ static int split_parts(const float* x, int64_t stride, const int32_t* ids, int64
   return status_from_hip(hipGetLastError());
 }
 
-// d_bias[class] += sum over the rows of the parts of dz: 1024 threads = 16 row lanes x 64 classes, fixed order.
-__global__ __launch_bounds__(1024) void dz_parts_colsum_kernel(const uint16_t* dz, int64_t ldz, int parts, int64_t b, int n_cls,
-                                                               float* d_bias) {
-  __shared__ float part_sum[16][64];
-  const int cl = threadIdx.x & 63;
-  const int rl = threadIdx.x >> 6;
-  const int cls = blockIdx.x * 64 + cl;
-  float sum = 0.0f;
-  if (cls < n_cls) {
-    for (int64_t i = rl; i < b; i += 16) {
-      float x = 0.0f;
-      for (int part = parts - 1; part >= 0; --part) x += Elem<BF16>::to_float(dz[(i * parts + part) * ldz + cls]);
-      sum += x;
-    }
-  }
-  part_sum[rl][cl] = sum;
-  __syncthreads();
-  if (rl == 0 && cls < n_cls) {
-    float t = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) t += part_sum[j][cl];
-    d_bias[cls] += t;
-  }
-}
-
 // Rows of e per pass: all of them, or as many as 32-bit offsets reach.
 static int64_t row_block(int64_t b, int64_t part_d, int parts) {
   const int64_t most = kRowBlockBytes / (parts * part_d * 2) / 256 * 256;
@@ -162,7 +137,7 @@ static Fp32Backward plan_backward(int64_t b, int64_t v, int64_t d, int terms) {
   f.c_bytes = align256(round_up(std::min(f.unit, v), 256) * row_bytes);
   f.dz_bytes = align256(f.rows_pad * f.parts * cls * 2);
   f.de_slot_bytes = f.de_slots > 1 ? align256(f.de_slots * f.rows * f.part_d * 4) : 0;
-  f.dc_slot_bytes = f.dc_slots > 1 ? align256(f.dc_slots * v * f.part_d * 4) : 0;
+  f.dc_slot_bytes = f.dc_slots > 1 ? align256(f.dc_slots * std::min(f.unit, v) * f.part_d * 4) : 0;
   return f;
 }
 
@@ -289,12 +264,15 @@ extern "C" int cce_fp32_backward(const float* e, const float* c, const float* bi
       float* const dc = d_c == nullptr ? nullptr : (dc_cut ? dc_slots : d_c + v0 * ld_dc);
       st = terms_products_launch(dz_parts, cls_pad, c_parts, ld, e_parts, ld, de_cut ? nullptr : ids, de, de_cut ? f.part_d : ld_de,
                                  de_cut, de_cut && v0 == 0, rows * f.part_d, de_len, dc, dc_cut ? f.part_d : ld_dc, r0 > 0,
-                                 v * f.part_d, dc_len, out_vec, rows, rows_pad, cls, cls_pad, d, f.part_d, terms, f.parts, stream);
+                                 cls * f.part_d, dc_len, out_vec, rows, rows_pad, cls, cls_pad, d, f.part_d, terms, f.parts, stream);
       if (st != CCE_OK) return st;
+      if (dc_cut) {
+        const int ranges = static_cast<int>((rows_pad + dc_len - 1) / dc_len);
+        st = split_sum_launch(dc_slots, ranges, cls, d, f.part_d, nullptr, d_c + v0 * ld_dc, ld_dc, false, out_vec, stream);
+        if (st != CCE_OK) return st;
+      }
       if (d_bias != nullptr) {
-        hipLaunchKernelGGL(dz_parts_colsum_kernel, dim3(static_cast<unsigned>((cls + 63) / 64)), dim3(1024), 0, stream, dz_parts,
-                           cls_pad, f.parts, rows, static_cast<int>(cls), d_bias + v0);
-        st = status_from_hip(hipGetLastError());
+        st = dz_colsum_launch(dz_parts, cls_pad, f.parts, rows, cls, d_bias + v0, CCE_DTYPE_BF16, stream);
         if (st != CCE_OK) return st;
       }
     }
@@ -303,6 +281,5 @@ extern "C" int cce_fp32_backward(const float* e, const float* c, const float* bi
       if (st != CCE_OK) return st;
     }
   }
-  if (dc_cut) return split_sum_launch(dc_slots, f.dc_slots, v, d, f.part_d, nullptr, d_c, ld_dc, false, out_vec, stream);
   return CCE_OK;
 }

@@ -39,7 +39,8 @@ def test_lse_forward_of_few_rows_fills_the_chip(shape):
 
 @pytest.mark.parametrize("shape,fp32_out", [((300, 9000, 128), False), ((300, 9000, 128), True), ((70, 20011, 192), False),
                                             ((1100, 33000, 320), False), ((9001, 200, 128), False), ((5000, 520, 64), False),
-                                            ((2100, 2500, 64), False), ((2100, 2500, 64), True)])
+                                            ((2100, 2500, 64), False), ((2100, 2500, 64), True), ((9000, 9000, 64), False),
+                                            ((9000, 70, 64), True)])
 @pytest.mark.parametrize("gathered", [False, True])
 @pytest.mark.parametrize("budget", [1 << 28, 0])
 def test_backward_dense_cuts_long_reductions(shape, fp32_out, gathered, budget):
@@ -71,12 +72,13 @@ def test_backward_dense_cuts_long_reductions(shape, fp32_out, gathered, budget):
     if fp32_out:
         de += 1.0
     dc = torch.full((V, D), float("nan"), dtype=gdt, device=dev)
+    db = torch.full((V,), 0.5, device=dev)
     smallest = lib.cce_backward_dense_workspace_bytes(B, V, D, 0 if fp32_out else 1, 0)
     ws_bytes = lib.cce_backward_dense_workspace_bytes(B, V, D, 0 if fp32_out else 1, budget or 3 * smallest)
     ws = torch.full((ws_bytes // 4 + 64,), float("nan"), device=dev)
     p = lambda x: x.data_ptr() if x is not None else None
     st = lib.cce_backward_dense(
-        p(ed), p(cd), None, p(lse.float()), p(g), 0, None, p(valids), p(td), p(de), p(dc), None,
+        p(ed), p(cd), None, p(lse.float()), p(g), 0, None, p(valids), p(td), p(de), p(dc), p(db),
         (ws.data_ptr() + 255) // 256 * 256, ws_bytes, N, B, V, D, D, D, 1, 1.0, int(fp32_out), int(fp32_out), 0, 0, 0.0, 0,
         torch.cuda.current_stream().cuda_stream)
     assert st == 0, lib.cce_error_string(st)
@@ -90,6 +92,9 @@ def test_backward_dense_cuts_long_reductions(shape, fp32_out, gathered, budget):
         scale = want.abs().amax(dim=1, keepdim=True)
         assert ((got.double() - want).abs() <= 1e-2 * scale + 1e-2 * want.abs() + 1e-6).all()
         assert (got.double() - want).norm() <= 6e-3 * want.norm()
+    # the column sums of dz, rounded to 8 significant bits before: each term off by half a unit in the last place, 2^-8 of it
+    want_db, size = dz.sum(0), dz.abs().sum(0)
+    assert ((db.double() - 0.5 - want_db).abs() <= 2.0**-8 * size + 1e-6).all()
 
 
 def _fp32_case(N, V, D, keep, seed, softcap=None, bias=False, d_lse=False, strided=False):
@@ -116,6 +121,7 @@ def _fp32_case(N, V, D, keep, seed, softcap=None, bias=False, d_lse=False, strid
     ((64, 256, 64), 1.0, {}), ((130, 600, 1000), 0.5, {"strided": True}), ((40, 33000, 2048), 1.0, {"bias": True}),
     ((6000, 300, 200), 0.9, {"d_lse": True, "softcap": 20.0}), ((1500, 1400, 96), 1.0, {"strided": True, "bias": True}),
     ((176000, 70, 4096), 1.0, {}), ((180000, 70, 4096), 0.98, {}),
+    ((30000, 5000, 64), 1.0, {"bias": True}),
 ])
 @pytest.mark.parametrize("terms", [6, 3])
 def test_fp32_passes_abi(shape, keep, extra, terms):
