@@ -257,7 +257,8 @@ int64_t cce_backward_dense_dz_bytes(int64_t b, int64_t v, int64_t d, int d_e_in_
  * d_c in place).  The same number of launches for the same dz buffer, with the smaller matrix as the one that is
  * read and written once per launch.
  * Layout requirements as for cce_backward_dz (16-byte aligned e, c and d_e, unit stride_cd, row strides that
- * are multiples of 8, d a multiple of 64), else CCE_ERR_MISALIGNED and the caller uses cce_backward.
+ * are multiples of 8), d a multiple of 64, or of 8 and above 64 where n_rows * stride_e and 256 * stride_cv are below
+ * 2^31; else CCE_ERR_MISALIGNED and the caller uses cce_backward.
  */
 int cce_backward_dense(const void* e, const void* c, const void* bias,
                        const float* lse, const float* d_out, int d_out_is_scalar, const float* d_lse,

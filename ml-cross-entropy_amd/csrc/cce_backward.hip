@@ -15,7 +15,7 @@
 //             logits, and accumulates dC^T (D x 32 classes) += E_cell^T . dz; dBias is the row sum of the
 //             same dz.  Rows are written once at the end.
 // Both passes are one kernel template with the roles of E and C swapped: bwd_owner_kernel for any layout,
-// bwd_owner_fast_kernel (direct-to-LDS loads, D % 128 == 0, 16-byte aligned rows) for the common one.
+// bwd_owner_fast_kernel (direct-to-LDS loads, D % 8 == 0, 16-byte aligned rows) for the common one.
 //
 // Which sub-blocks can matter: the forward pass left, per 32 rows x 32 classes, the largest
 // soft-capped logit.  If the bound exp(cell_max - min_row lse) of a sub-block is below filter_eps, every
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(kBwdThreads, 1) void bwd_owner_kernel(BwdParams p) 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Fast variant of the ownership kernel (16-byte aligned rows, unit column stride, D % 128 == 0):
+// Fast variant of the ownership kernel (16-byte aligned rows, unit column stride, D % 8 == 0):
 // the same algorithm with direct global -> LDS loads (no staging registers, no LDS stores) through a
 // ring of 128-column stages.  Both phases of a trip are bound by memory latency and gather
 // bandwidth, not by the MFMAs, so what matters is how much is in flight and how little is fetched:
@@ -616,7 +616,9 @@ __global__ __launch_bounds__(kBwdThreads, 1) void bwd_owner_kernel(BwdParams p) 
 // block b = q * 4 + wave holds rows [4 b, 4 b + 4) of the 128-row virtual cell; own-side likewise for
 // its 32 rows.  A row id of -1 (no row: past the last valid row or the last class) is fetched from a
 // line of zeros, whatever the stage: its products are exactly zero and no non-finite value of another
-// row of the matrices can leak into real rows through it.
+// row of the matrices can leak into real rows through it.  TAIL (D no multiple of 128): so is every 16-byte piece past
+// the end of a row, and the gradient is stored up to there; a variant of its own because the question costs each load
+// three vector instructions.
 // ---------------------------------------------------------------------------------------------
 static __device__ __align__(256) uint16_t g_owner_zero_line[128];  // never written
 
@@ -702,7 +704,7 @@ __device__ __forceinline__ void wait_vmcnt_upto_wide(int n) {
   }
 }
 
-template <typename T, bool IS_DE, bool LIGHT = false>
+template <typename T, bool IS_DE, bool LIGHT = false, bool TAIL = false>
 __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_kernel(BwdParams p) {
   static_assert(!(LIGHT && IS_DE), "the light variant is a dC pass");
   using Lds = FastLds<LIGHT>;
@@ -740,9 +742,9 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   }
   const int d_begin = slice * p.dslice;
   const int d_end = min(static_cast<int>(p.d), d_begin + p.dslice);
-  const int nchunks = (d_end - d_begin) / kFCols;
+  const int nchunks = (d_end - d_begin + (TAIL ? kFCols - 1 : 0)) / kFCols;
   const int D = static_cast<int>(p.d);
-  const int nstages = D / kFCols;
+  const int nstages = (D + (TAIL ? kFCols - 1 : 0)) / kFCols;
   const bool write_out = IS_DE ? (p.d_e != nullptr) : (p.d_c != nullptr);
 
   const uint16_t* other_base = IS_DE ? p.c : p.e;
@@ -751,6 +753,12 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   const int64_t own_sr = IS_DE ? p.stride_e : p.stride_cv;
   // element offset of the chunk this lane fetches inside a 128-column stage
   const int lane_chunk = ((lane & 15) ^ ((4 * wave + (lane >> 4)) & 15)) * 8;
+  const int lane_cols = D - lane_chunk;  // TAIL: the stages that hold a piece for this lane start below this column
+  // where a lane fetches the piece of the stage at col0 (`row`: its piece of stage 0, or of the line of zeros)
+  auto piece = [&](const uint16_t* row, bool live, int col0, const uint16_t* zeros) {
+    const uint16_t* at = row + (live ? col0 : 0);
+    return (TAIL && col0 >= lane_cols) ? zeros : at;
+  };
 
   float my_lse = INFINITY;
   if (IS_DE) {
@@ -798,11 +806,14 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   auto store_chunk_direct = [&](int ci, const f32x16& a) {
     const int id = own_ids[l32];
     if (id < 0) return;
-    uint16_t* dst = static_cast<uint16_t*>(p.d_c) + static_cast<int64_t>(id) * own_sr + d_begin + ci * kFCols + wave * 32 + 4 * half;
+    const int col = d_begin + ci * kFCols + wave * 32 + 4 * half;
+    uint16_t* dst = static_cast<uint16_t*>(p.d_c) + static_cast<int64_t>(id) * own_sr + col;
     // exactly kLightStores store instructions per wave and chunk (the product loop below counts them: stores share
-    // the counter its loads are awaited on), whatever the compiler would make of four plain assignments
+    // the counter its loads are awaited on), whatever the compiler would make of four plain assignments; fewer in a
+    // partial chunk, which is the last one: nothing is counted after it
 #pragma unroll
     for (int r4 = 0; r4 < kLightStores; ++r4) {
+      if (TAIL && col + 8 * r4 >= D) break;
       uint2 pk;
       pk.x = Elem<T>::pack2(a[r4 * 4 + 0], a[r4 * 4 + 1]);
       pk.y = Elem<T>::pack2(a[r4 * 4 + 2], a[r4 * 4 + 3]);
@@ -952,7 +963,8 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
       // product phase: load q of this wave (rows of entry q / 2) for the stage that starts at column col0
       auto issue_load = [&](int q, int col0, int slot, uint32_t entries) {
         if ((entries >> (q >> 1)) & 1u)
-          lds_dma16(other_ptr[q] + (((other_live >> q) & 1u) ? col0 : 0), lds_base + slot * slot_bytes + (q * 4 + wave) * 1024);
+          lds_dma16(piece(other_ptr[q], (other_live >> q) & 1u, col0, zero_chunk),
+                    lds_base + slot * slot_bytes + (q * 4 + wave) * 1024);
       };
       auto issue_stage = [&](int col0, int slot, uint32_t entries) {
 #pragma unroll
@@ -978,9 +990,10 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
         auto issue = [&](auto q_tag, int col0, unsigned base) {
           constexpr int Q = decltype(q_tag)::value;
           if constexpr (Q < 2 * NENT) {
-            lds_dma16(other_ptr[Q] + (((other_live >> Q) & 1u) ? col0 : 0), base + (Q * 4 + wave) * 1024);
+            lds_dma16(piece(other_ptr[Q], (other_live >> Q) & 1u, col0, zero_chunk), base + (Q * 4 + wave) * 1024);
           } else if constexpr (Q >= 8) {
-            lds_dma16(own_ptr[Q - 8] + (own_step[Q - 8] ? col0 : 0), base + OWN_OFF + ((Q - 8) * 4 + wave) * 1024);
+            lds_dma16(piece(own_ptr[Q - 8], own_step[Q - 8] != 0, col0, zero_chunk),
+                      base + OWN_OFF + ((Q - 8) * 4 + wave) * 1024);
           }
         };
         // the MFMAs of stage `slot`; with ISSUE the loads of column block next_col go out among them
@@ -1202,7 +1215,7 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   if constexpr (LIGHT) {
     if (write_out && !touched) {
       // Nothing survived for this class group: its rows are zeros, written as whole 16-byte pieces, a wave
-      // instruction inside one row (the launcher guarantees 16-byte aligned rows and D a multiple of 128).
+      // instruction inside one row (the launcher guarantees 16-byte aligned rows and D a multiple of 8).
       const int ppr = (d_end - d_begin) / 8;  // 16-byte pieces per row
       const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
       for (int j = tid; j < 32 * ppr; j += kBwdThreads) {
@@ -1266,9 +1279,10 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
             const uint4 va = *reinterpret_cast<const uint4*>(smem + rowa * pitch + pca * 16);
             const uint4 vb = *reinterpret_cast<const uint4*>(smem + rowb * pitch + pcb * 16);
             const int64_t col_bytes = static_cast<int64_t>(d_begin + g * 4 * kFCols) * es;
-            if (ida >= 0)
+            const int row_bytes = TAIL ? (d_end - d_begin - g * 4 * kFCols) * es : 0;  // of this group, inside the slice
+            if (ida >= 0 && (!TAIL || pca * 16 < row_bytes))
               *reinterpret_cast<uint4*>(out_base + static_cast<int64_t>(ida) * out_sr * es + col_bytes + pca * 16) = va;
-            if (idb >= 0)
+            if (idb >= 0 && (!TAIL || pcb * 16 < row_bytes))
               *reinterpret_cast<uint4*>(out_base + static_cast<int64_t>(idb) * out_sr * es + col_bytes + pcb * 16) = vb;
           }
         }
@@ -1519,9 +1533,10 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
 
   const bool aligned = aligned16(e) && aligned16(c) && (d % 8 == 0) && (stride_e % 8 == 0) &&
                        (stride_cv % 8 == 0) && (stride_cd == 1);
-  // The fast kernels want whole 128-column stages, also inside every slice of D.
-  // ... and they store whole 16-byte pieces of the output rows.
-  const bool fast = aligned && (d % kFCols == 0) && (d_e == nullptr || p.vec_e) && (d_c == nullptr || p.vec_c);
+  // The fast kernels store whole 16-byte pieces of the output rows.  A width of less than one stage stays with the general
+  // kernel, as a width that is mostly padding would.
+  const bool fast = aligned && d >= kFCols / 2 + 8 && (d_e == nullptr || p.vec_e) && (d_c == nullptr || p.vec_c);
+  const bool tail = d % kFCols != 0;
   hipError_t err;
 #define CCE_LAUNCH(KERN, LDS, GRID)                                                                 \
   do {                                                                                              \
@@ -1534,11 +1549,13 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
 #define CCE_LAUNCH_OWNER(IS_DE_, GRID)                                                              \
   do {                                                                                              \
     if (dtype == CCE_DTYPE_BF16) {                                                                  \
-      if (fast) CCE_LAUNCH((bwd_owner_fast_kernel<BF16, IS_DE_>), kFLdsBytes, GRID);                \
+      if (fast && tail) CCE_LAUNCH((bwd_owner_fast_kernel<BF16, IS_DE_, false, true>), kFLdsBytes, GRID); \
+      else if (fast) CCE_LAUNCH((bwd_owner_fast_kernel<BF16, IS_DE_>), kFLdsBytes, GRID);           \
       else if (aligned) CCE_LAUNCH((bwd_owner_kernel<BF16, true, IS_DE_>), kBwdLdsBytes, GRID);     \
       else CCE_LAUNCH((bwd_owner_kernel<BF16, false, IS_DE_>), kBwdLdsBytes, GRID);                 \
     } else {                                                                                        \
-      if (fast) CCE_LAUNCH((bwd_owner_fast_kernel<F16, IS_DE_>), kFLdsBytes, GRID);                 \
+      if (fast && tail) CCE_LAUNCH((bwd_owner_fast_kernel<F16, IS_DE_, false, true>), kFLdsBytes, GRID); \
+      else if (fast) CCE_LAUNCH((bwd_owner_fast_kernel<F16, IS_DE_>), kFLdsBytes, GRID);            \
       else if (aligned) CCE_LAUNCH((bwd_owner_kernel<F16, true, IS_DE_>), kBwdLdsBytes, GRID);      \
       else CCE_LAUNCH((bwd_owner_kernel<F16, false, IS_DE_>), kBwdLdsBytes, GRID);                  \
     }                                                                                               \
@@ -1579,20 +1596,20 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
       q.nslices = 1;
       q.dslice = static_cast<int>(d);
       const unsigned grid = static_cast<unsigned>(q.nvg);
+      auto launch = [&](auto kern, LdsLimitOnce& lds_limit) {
+        const hipError_t e0 = lds_limit.set(kern, kFLightLdsBytes);
+        if (e0 != hipSuccess) return e0;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(kBwdThreads), kFLightLdsBytes, stream, q);
+        return hipGetLastError();
+      };
+      static LdsLimitOnce limits[4];
       if (dtype == CCE_DTYPE_BF16) {
-        auto kern = bwd_owner_fast_kernel<BF16, false, true>;
-        static LdsLimitOnce lds_limit;
-        err = lds_limit.set(kern, kFLightLdsBytes);
-        if (err != hipSuccess) return status_from_hip(err);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(kBwdThreads), kFLightLdsBytes, stream, q);
+        err = tail ? launch(bwd_owner_fast_kernel<BF16, false, true, true>, limits[0])
+                   : launch(bwd_owner_fast_kernel<BF16, false, true>, limits[1]);
       } else {
-        auto kern = bwd_owner_fast_kernel<F16, false, true>;
-        static LdsLimitOnce lds_limit;
-        err = lds_limit.set(kern, kFLightLdsBytes);
-        if (err != hipSuccess) return status_from_hip(err);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(kBwdThreads), kFLightLdsBytes, stream, q);
+        err = tail ? launch(bwd_owner_fast_kernel<F16, false, true, true>, limits[2])
+                   : launch(bwd_owner_fast_kernel<F16, false, true>, limits[3]);
       }
-      err = hipGetLastError();
       if (err != hipSuccess) return status_from_hip(err);
       p.light_on = 1;
     }

@@ -918,7 +918,7 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
     return CCE_ERR_INVALID_ARGUMENT;
   if (dtype != CCE_DTYPE_BF16 && dtype != CCE_DTYPE_F16) return CCE_ERR_UNSUPPORTED_DTYPE;
   if (d_e == nullptr && d_c == nullptr && d_bias == nullptr) return CCE_OK;
-  if (!aligned16(e) || !aligned16(c) || d % kDmaBK != 0 || stride_e % 8 != 0 || stride_cv % 8 != 0 || stride_cd != 1)
+  if (!aligned16(e) || !aligned16(c) || !dense_width_ok(n_rows, d, stride_e, stride_cv) || stride_e % 8 != 0 || stride_cv % 8 != 0 || stride_cd != 1)
     return CCE_ERR_MISALIGNED;
   if (stride_e >= (int64_t(1) << 30) || stride_cv >= (int64_t(1) << 30)) return CCE_ERR_INVALID_ARGUMENT;
   if ((d_e != nullptr && !aligned16(d_e)) || (d_c != nullptr && !aligned16(d_c))) return CCE_ERR_MISALIGNED;

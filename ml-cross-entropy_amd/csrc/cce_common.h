@@ -350,7 +350,35 @@ __device__ __forceinline__ void lds_dma16_sbase(const void* sbase, unsigned voff
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr)
                : "memory", "m0");
 }
+// ... of which only the lanes whose byte offset inside the 128-byte row segment lies below `valid` read their row when
+// `k` is `k_tail`; the others then read zeros, from a line that every wave finds in its cache.  One scalar comparison
+// per load on whole stages; a partial one issues two loads, each under its part of the mask (a lane's place in LDS goes by
+// its number, whichever lanes are on).  For whole waves: all 64 lanes are on before and after.
+__device__ __forceinline__ void lds_dma16_sbase_tail(const void* sbase, unsigned voff, unsigned lds_addr, int k, int k_tail,
+                                                     unsigned chunk_bytes, unsigned valid, const void* zeros) {
+  asm volatile(
+      "s_mov_b32 m0, %[lds]\n\t"
+      "s_cmp_lg_u32 %[k], %[kt]\n\t"
+      "s_cbranch_scc1 .Lwhole%=\n\t"
+      "v_cmp_gt_u32 vcc, %[valid], %[chunk]\n\t"
+      "s_mov_b64 exec, vcc\n\t"
+      "global_load_lds_dwordx4 %[voff], %[base]\n\t"
+      "s_not_b64 exec, vcc\n\t"
+      "global_load_lds_dwordx4 %[chunk], %[zeros]\n\t"
+      "s_mov_b64 exec, -1\n\t"
+      "s_branch .Ldone%=\n"
+      ".Lwhole%=:\n\t"
+      "global_load_lds_dwordx4 %[voff], %[base]\n"
+      ".Ldone%=:"
+      :
+      : [base] "s"(sbase), [voff] "v"(voff), [lds] "s"(lds_addr), [k] "s"(k), [kt] "s"(k_tail), [chunk] "v"(chunk_bytes),
+        [valid] "s"(valid), [zeros] "s"(zeros)
+      : "memory", "m0", "vcc", "scc");
+}
 #pragma clang diagnostic pop
+
+// What loads read in place of a row or a column that does not exist.
+static __device__ __align__(256) uint16_t g_zero_line[128];  // never written
 
 template <typename F, int... Is>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>) {
@@ -558,6 +586,11 @@ struct DmaLogitTile {
 // the reduction runs over the cross terms of the parts one after the other (term_part() below): the stages of a
 // tile walk columns 0 .. D of the two parts of term 0, then of term 1, and so on, so that a part is stored once however
 // many terms it takes part in.
+//
+// TAIL: D is a multiple of 8 and not of 64.  The last stage of a tile is a partial one: what lies past the end of a row is
+// fetched from a line of zeros, for both operands, so that nothing of another row (a non-finite value least of all) meets
+// the product.  A variant of its own, since the question costs every load two scalar instructions: such widths were
+// padded to a multiple of 128 before, a pass over E and C and one over each of their gradients.
 // ---------------------------------------------------------------------------------------------
 // Which part (0 hi, 1 mid, 2 lo) of the first and of the second operand meets in term t, smallest terms first, so that
 // the accumulator is rounded at its full size only while the last one is added:
@@ -568,8 +601,9 @@ __host__ __device__ __forceinline__ int term_part(unsigned table, int term) {
   return static_cast<int>((table >> (2 * term)) & 3u);
 }
 
-template <typename T, int WV, int WT, int NWV, int NWT, bool TERMS = false>
+template <typename T, int WV, int WT, int NWV, int NWT, bool TERMS = false, bool TAIL = false>
 struct DmaLogitTile16 {
+  static_assert(!TERMS || !TAIL, "parts are whole stages");
   static_assert(WV % 2 == 0 && WT % 2 == 0, "the ring is addressed in blocks of 32 rows");
   using Base = DmaLogitTile<T, WV / 2, WT / 2, NWV, NWT>;
   static constexpr int TILE_V = Base::TILE_V;
@@ -600,7 +634,14 @@ struct DmaLogitTile16 {
     unsigned row_in_block;  // lane >> 3
     unsigned chunk_bytes;   // byte offset of this lane's 16-byte chunk inside a 128-byte row segment
     int terms;              // TERMS only: 3 or 6
+    // TAIL only: where the partial stage starts and how many bytes of a row it holds
+    int k_tail;
+    unsigned tail_bytes;
   };
+  static __device__ __forceinline__ void set_tail(Source& src, int D) {
+    src.k_tail = D / kDmaBK * kDmaBK;
+    src.tail_bytes = 2u * static_cast<unsigned>(D - src.k_tail);
+  }
 
   // Where a stage starts in the rows of either operand (elements), stage after stage.
   struct Walk {
@@ -653,6 +694,13 @@ struct DmaLogitTile16 {
     if (TERMS && q < NQC) {
       lds_dma16_sbase(src.c_blk[0] + (2 * kc + static_cast<uint64_t>(q * 8 * NW) * src.c_stride_bytes),
                       src.row_in_block * src.c_stride_bytes + src.chunk_bytes, lds_base + stage_off + (q * NW + wave) * 1024);
+    } else if (TAIL) {
+      const bool cls = q < NQC;
+      const unsigned row = cls ? min(src.row_in_block, static_cast<unsigned>(src.c_lim[cls ? q : 0])) : 0u;
+      lds_dma16_sbase_tail((cls ? src.c_blk[cls ? q : 0] : src.e_base) + 2 * kc,
+                           cls ? row * src.c_stride_bytes + src.chunk_bytes : src.e_off[cls ? 0 : q - NQC],
+                           lds_base + stage_off + ((cls ? 0 : TILE_V / 8) + (cls ? q : q - NQC) * NW + wave) * 1024, kc,
+                           src.k_tail, src.chunk_bytes, src.tail_bytes, g_zero_line);
     } else if (q < NQC) {
       const unsigned row = min(src.row_in_block, static_cast<unsigned>(src.c_lim[q]));
       lds_dma16_sbase(src.c_blk[q] + 2 * kc, row * src.c_stride_bytes + src.chunk_bytes,
@@ -735,7 +783,7 @@ struct DmaLogitTile16 {
     for (int q = 0; q < NQ; ++q) issue_one(src, q, w.off_c, w.off_e, lds_base, STAGE_BYTES, wave);
   }
 
-  // D must be a multiple of 64 and, without TERMS, at least 128.  The first two stages of this tile must be in flight or landed in
+  // D must be a multiple of 64 (TAIL: of 8) and, without TERMS, make at least two stages.  The first two stages of this tile must be in flight or landed in
   // ring stages buf, 1 - buf (prefetch() for the first tile of a span: first_tile; else the previous run()), and
   // nothing else may have touched the ring.
   // next_tile() is called once, when the class rows of this tile have been fetched for the last time: it points
@@ -757,7 +805,7 @@ struct DmaLogitTile16 {
     const unsigned char* e_row = lds + (TILE_V + wt * WT * 16 + r16) * kDmaRowBytes;
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
 
-    const int nk = TERMS ? src.terms * (D / kDmaBK) : D / kDmaBK;  // >= 2
+    const int nk = TERMS ? src.terms * (D / kDmaBK) : (D + (TAIL ? kDmaBK - 1 : 0)) / kDmaBK;  // >= 2
     Walk w = walk_start(D, src.terms);
     if constexpr (TERMS) {
       walk_next(w, D, src.terms);
@@ -773,7 +821,7 @@ struct DmaLogitTile16 {
     };
     int cur = buf * STAGE_BYTES;
     if (first_tile) {
-      wait_vmcnt<NQ>();  // the first stage has landed for this wave (the second may be in flight) ...
+      wait_vmcnt<NQ>();  // the first stage has landed for this wave (the second, NQ loads or twice that, may be in flight) ...
       __syncthreads();   // ... and for all of them
     }
     // (a later tile's first stage was awaited by every wave before the last barrier of the tile before it: no

@@ -5,6 +5,16 @@
 
 namespace cce {
 
+// The 16 x 16 x 32 kernels address rows by 32-bit byte offsets and stream at least two stages per tile.
+inline bool dense_k16(int64_t n_rows, int64_t d, int64_t stride_e, int64_t stride_cv) {
+  return d > kDmaBK && n_rows * stride_e * 2 < (int64_t(1) << 32) && 256 * stride_cv * 2 < (int64_t(1) << 32);
+}
+// Widths the logits of the unfiltered backward can be streamed at: whole stages, or (16 x 16 x 32 kernel only) whole
+// 16-byte pieces.  The products take any multiple of 8.
+inline bool dense_width_ok(int64_t n_rows, int64_t d, int64_t stride_e, int64_t stride_cv) {
+  return d % kDmaBK == 0 || (d % 8 == 0 && dense_k16(n_rows, d, stride_e, stride_cv));
+}
+
 // dz of one vocabulary chunk (cce_dense_dz.hip); the arguments of cce_backward_dz plus `pad_store`: also store
 // the zero gradients of the columns between v and ldz.
 int dense_dz_launch(const void* e, const void* c, const void* bias,

@@ -263,11 +263,11 @@ struct DzRow {
   int tgt;
 };
 
-template <typename T, bool GENERAL, DzOut OUT>
+template <typename T, bool GENERAL, DzOut OUT, bool TAIL = false>
 __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   constexpr bool OUT32 = OUT == kDzFp32;
   constexpr bool PARTS = OUT == kDzParts;
-  using Fast = DmaLogitTile16<T, kDz16WV, kDz16WT, kDzNWV, kDzNWT, PARTS>;
+  using Fast = DmaLogitTile16<T, kDz16WV, kDz16WT, kDzNWV, kDzNWT, PARTS, TAIL>;
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_addend = reinterpret_cast<float*>(smem + Fast::LDS_BYTES);                                   // [2][256]
   DzRow* s_rows = reinterpret_cast<DzRow*>(smem + Fast::LDS_BYTES + 2 * kDzTile * 4);                    // [256]
@@ -299,6 +299,7 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   src.row_in_block = static_cast<unsigned>(lane >> 3);
   src.c_stride_bytes = static_cast<unsigned>(p.stride_cv * 2);
   src.terms = PARTS ? p.terms : 1;
+  if constexpr (TAIL) Fast::set_tail(src, static_cast<int>(p.d));
 #pragma unroll
   for (int q = Fast::NQC; q < Fast::NQ; ++q) {
     int64_t i = t0 + Fast::row_of(q, wave, lane);
@@ -501,8 +502,9 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
   if (d > (1 << 30) || v > (int64_t(1) << 31) - 512) return CCE_ERR_INVALID_ARGUMENT;
   if (dtype != CCE_DTYPE_BF16 && dtype != CCE_DTYPE_F16) return CCE_ERR_UNSUPPORTED_DTYPE;
   // direct-to-LDS main loop and 16-byte stores only
-  if (!aligned16(e) || !aligned16(c) || !aligned16(dz) || d % kDmaBK != 0 || stride_e % 8 != 0 ||
-      stride_cv % 8 != 0 || stride_cd != 1 || ldz % (dz_is_fp32 ? 4 : 8) != 0)
+  const bool tail = d % kDmaBK != 0;
+  if (!aligned16(e) || !aligned16(c) || !aligned16(dz) || !dense_width_ok(n_rows, d, stride_e, stride_cv) || (tail && dz_is_fp32) ||
+      stride_e % 8 != 0 || stride_cv % 8 != 0 || stride_cd != 1 || ldz % (dz_is_fp32 ? 4 : 8) != 0)
     return CCE_ERR_MISALIGNED;
 
   DzParams p = {};
@@ -539,13 +541,18 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
   const int lds16 = lds + kDzTile * static_cast<int>(sizeof(DzRow)) + kDzNWV * kDzNWT * kDz16StageBytes;
   const bool general = (bias != nullptr) || (v % kDzTile != 0);
   // the 16 x 16 x 32 kernel addresses rows by 32-bit byte offsets and streams at least two stages per tile
-  const bool k16 = (d >= 2 * kDmaBK) && (n_rows * stride_e * 2 < (int64_t(1) << 32)) &&
-                   (256 * stride_cv * 2 < (int64_t(1) << 32));
+  const bool k16 = dense_k16(n_rows, d, stride_e, stride_cv);
   const int grid = p.items_per_xcd * 8;
   hipError_t err;
 #define CCE_LAUNCH_DZ2(TT, GE, O32)                                                               \
   do {                                                                                            \
-    if (k16) {                                                                                    \
+    if (k16 && tail) {                                                                            \
+      auto kern = dense_dz16_kernel<TT, GE, kDz16Bit, true>;                                      \
+      static LdsLimitOnce lds_limit;                                                              \
+      err = lds_limit.set(kern, lds16);                                                           \
+      if (err != hipSuccess) return status_from_hip(err);                                         \
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(kDzThreads), lds16, stream, p);                   \
+    } else if (k16) {                                                                             \
       auto kern = dense_dz16_kernel<TT, GE, (O32) ? kDzFp32 : kDz16Bit>;                          \
       static LdsLimitOnce lds_limit;                                                              \
       err = lds_limit.set(kern, lds16);                                                           \
@@ -639,6 +646,7 @@ extern "C" int cce_backward_dz(const void* e, const void* c, const void* bias,
                                int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
                                float grad_scale, int64_t shift, int64_t target_offset,
                                float softcap, int dtype, void* stream) {
+  if (b > 0 && d > 0 && d % cce::kDmaBK != 0) return CCE_ERR_MISALIGNED;
   return cce::dense_dz_launch(e, c, bias, lse, d_out, d_out_is_scalar, d_lse, valids, targets, dz, ldz, dz_is_fp32, 0,
                               n_rows, b, v, d, stride_e, stride_cv, stride_cd, grad_scale, shift, target_offset, softcap,
                               dtype, static_cast<hipStream_t>(stream));

@@ -385,9 +385,9 @@ __device__ __forceinline__ void row_block(const Softcap& sc, float cap_inv, bool
   else row_block_impl<GENERAL, false, false, WANT_S2>(sc, cap_inv, acc, ti, addend, kq, run, bm, s2);
 }
 
-template <typename T, bool GENERAL, bool WANT_LA, bool TERMS = false>
+template <typename T, bool GENERAL, bool WANT_LA, bool TERMS = false, bool TAIL = false>
 __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdParams p) {
-  using Fast = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, TERMS>;
+  using Fast = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, TERMS, TAIL>;
   static_assert(!WANT_LA || GENERAL, "the column average uses the general epilogue");
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_addend = reinterpret_cast<float*>(smem + Fast::LDS_BYTES);  // [2][256]
@@ -429,6 +429,7 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   src.row_in_block = static_cast<unsigned>(lane >> 3);
   src.c_stride_bytes = static_cast<unsigned>(p.stride_cv * 2);
   src.terms = TERMS ? p.terms : 1;
+  if constexpr (TAIL) Fast::set_tail(src, static_cast<int>(p.d));
 #pragma unroll
   for (int q = Fast::NQC; q < Fast::NQ; ++q) {
     int64_t i = t0 + Fast::row_of(q, wave, lane);
@@ -652,10 +653,12 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
   const int lds = Tile::LDS_BYTES + kFwdBiasBytes;
   const int lds16 = lds + kF16RunBytes;  // + the running (max, sum) pairs
   // the 16 x 16 x 32 kernel addresses token rows by 32-bit byte offsets from e and class rows by offsets from the
-  // first class of a tile; shapes beyond that, and a D of one stage, take the 32 x 32 x 16 kernel
+  // first class of a tile; shapes beyond that, and a D of one stage, take the 32 x 32 x 16 kernel, which knows whole
+  // stages only
   const bool fast = aligned && (p.d % kDmaBK == 0);
-  const bool fast16 = fast && (p.d >= 2 * kDmaBK) && (p.n_rows * p.stride_e * 2 < (int64_t(1) << 32)) &&
+  const bool fast16 = aligned && (p.d > kDmaBK) && (p.n_rows * p.stride_e * 2 < (int64_t(1) << 32)) &&
                       (256 * p.stride_cv * 2 < (int64_t(1) << 32));
+  const bool tail = p.d % kDmaBK != 0;
   const bool general = want_la || (p.bias != nullptr) || (p.v % Tile::TILE_V != 0);
   const int grid = p.items_per_xcd * 8;
   hipError_t err;
@@ -667,19 +670,23 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
     if (err != hipSuccess) return status_from_hip(err);                                           \
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), lds, stream, p);                           \
   } while (0)
-#define CCE_LAUNCH_FWD16(GE, LA)                                                                  \
+#define CCE_LAUNCH_FWD16(GE, LA, TAIL)                                                            \
   do {                                                                                            \
-    auto kern = lse_forward16_kernel<T, GE, LA>;                                                  \
+    auto kern = lse_forward16_kernel<T, GE, LA, false, TAIL>;                                     \
     static LdsLimitOnce lds_limit;                                                            \
     const int bytes = lds16 + ((LA) ? kF16ColsumBytes : 0);                                       \
     err = lds_limit.set(kern, bytes);                                                             \
     if (err != hipSuccess) return status_from_hip(err);                                           \
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), bytes, stream, p);                    \
   } while (0)
-  if (fast16) {
-    if (want_la) CCE_LAUNCH_FWD16(true, true);
-    else if (general) CCE_LAUNCH_FWD16(true, false);
-    else CCE_LAUNCH_FWD16(false, false);
+  if (fast16 && tail) {
+    if (want_la) CCE_LAUNCH_FWD16(true, true, true);
+    else if (general) CCE_LAUNCH_FWD16(true, false, true);
+    else CCE_LAUNCH_FWD16(false, false, true);
+  } else if (fast16) {
+    if (want_la) CCE_LAUNCH_FWD16(true, true, false);
+    else if (general) CCE_LAUNCH_FWD16(true, false, false);
+    else CCE_LAUNCH_FWD16(false, false, false);
   } else if (fast) {
     if (want_la) CCE_LAUNCH_FWD(true, true, true, true);
     else if (general) CCE_LAUNCH_FWD(true, true, true, false);

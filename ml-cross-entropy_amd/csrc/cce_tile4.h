@@ -44,8 +44,6 @@
 
 namespace cce {
 
-static __device__ __align__(256) uint16_t g_zero_line[128];  // never written
-
 typedef short tr_short4_t __attribute__((ext_vector_type(4)));
 
 template <typename T, bool A_KM, bool B_KM, bool B_GATHER = false, bool TERMS = false>

@@ -162,8 +162,11 @@ def _filtered_backward_runs_dense(lib, tile_max, lse, B: int, V: int, D: int, fi
 def _dense_layout_ok(e, c) -> bool:
     """Whether the layout suits the direct-to-LDS kernels of the unfiltered backward (cce_backward_dense: dz chunks
     and the two products as MFMA kernels)."""
+    width_ok = e.size(1) % 64 == 0 or (
+        e.size(1) % 8 == 0 and e.size(1) > 64 and e.size(0) * e.stride(0) * 2 < 1 << 32 and c.stride(0) * 512 < 1 << 32
+    )
     return (
-        e.size(1) % 64 == 0
+        width_ok
         and e.stride(0) % 8 == 0
         and c.stride(1) == 1
         and c.stride(0) % 8 == 0

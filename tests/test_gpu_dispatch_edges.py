@@ -285,3 +285,102 @@ def test_filtered_backward_of_few_rows_deals_its_trips(shape, fp32_out, with_dls
     a, b = got[0][0].double(), got[1][0].double()
     scale = b.abs().amax(dim=1, keepdim=True)
     assert ((a - b).abs() <= (2e-6 if fp32_out else 2.0**-7) * b.abs() + 4e-6 * scale).all()
+
+
+def _columns_with_rubbish_behind(x, gap):
+    """The same matrix as a view whose rows are followed by ``gap`` columns of NaN."""
+    wide = torch.full((x.size(0), x.size(1) + gap), float("nan"), dtype=x.dtype, device=x.device)
+    wide[:, : x.size(1)] = x
+    return wide[:, : x.size(1)]
+
+
+# One 16-byte piece past a whole stage of the logits (64) or of the ownership kernels (128), one short of it, both sides of
+# the halves in between, and a width of two slices of the ownership kernels whose second one ends in a partial stage.
+@pytest.mark.parametrize("width", [72, 120, 136, 184, 192, 200, 248, 264, 1000, 2312, 4664])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("path", ["sparse", "dense"])
+def test_widths_of_whole_pieces_are_streamed_as_they_lie(monkeypatch, width, dtype, path):
+    """A width that is a multiple of 8 gives, bit for bit, what the same matrices with zero columns up to a multiple of 128
+    give (the unfiltered backward: within the rounding of its 16-bit results, since the plan of its reductions goes by the
+    width), whatever stands behind the rows and in rows that do not count."""
+    from cut_cross_entropy import cce_backward as bw
+    from cut_cross_entropy import linear_cross_entropy
+
+    monkeypatch.setattr(bw, "FILTERED_BACKWARD_PATH", path)
+    N, V = 330, 1300
+    e, c, t, bias = make_inputs(N, V, width, dtype, seed=width, invalid_frac=0.2, bias=True)
+    e, c, t, bias = e.cuda(), c.cuda(), t.cuda(), bias.cuda()
+    ep = torch.nn.functional.pad(e, (0, -width % 128)).requires_grad_(True)
+    cp = torch.nn.functional.pad(c, (0, -width % 128)).requires_grad_(True)
+    e = torch.where((t == -100)[:, None], torch.full_like(e, float("inf")), e).requires_grad_(True)
+    c = _columns_with_rubbish_behind(c, 16).requires_grad_(True)
+
+    def run(e, c):
+        return linear_cross_entropy(e, c, t, bias=bias, softcap=20.0, reduction="sum", return_lse=True, impl="cce")
+
+    (got, lse), (want, want_lse) = run(e, c), run(ep, cp)
+    assert torch.equal(lse, want_lse)
+    # (the target's logit is summed by another kernel, in the order of the width)
+    assert abs(got.item() - want.item()) <= 1e-5 * abs(want.item())
+    (got + 0.1 * lse.sum()).backward()
+    (want + 0.1 * want_lse.sum()).backward()
+    if path == "sparse":
+        assert torch.equal(e.grad, ep.grad[:, :width]) and torch.equal(c.grad, cp.grad[:, :width])
+    else:
+        for a, b in ((e.grad, ep.grad), (c.grad, cp.grad)):
+            b = b[:, :width].float()
+            # both round sums of the same 16-bit dz: two roundings to the type, and fp32 sums in another order
+            eps = torch.finfo(dtype).eps
+            assert ((a.float() - b).abs() <= 2 * eps * b.abs() + 1e-3 * eps * b.abs().max()).all()
+    assert (e.grad[t == -100] == 0).all()
+
+
+@pytest.mark.parametrize("rows", [2048, 2049])
+@pytest.mark.parametrize("moved", ["e", "c", "both"])
+def test_packed_matrices_off_a_boundary_are_copied(rows, moved):
+    """e or c packed, but starting off a 16-byte boundary, on both sides of the number of rows up to which a ragged
+    width is streamed as it lies: the results of aligned matrices, bit for bit."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    e, c, t, _ = make_inputs(rows, 300, 136, torch.bfloat16, seed=2)
+
+    def off(x):
+        flat = torch.empty((x.numel() + 1,), dtype=x.dtype, device="cuda")
+        flat[1:] = x.flatten().cuda()
+        return flat[1:].view(x.shape)
+
+    results = []
+    for which in ("", moved):
+        ed = (off(e) if which in ("e", "both") else e.cuda()).requires_grad_(True)
+        cd = (off(c) if which in ("c", "both") else c.cuda()).requires_grad_(True)
+        loss = linear_cross_entropy(ed, cd, t.cuda(), impl="cce_exact")
+        loss.backward()
+        results.append((loss.detach(), ed.grad, cd.grad))
+    # (the target's logit alone is summed by whatever kernel the alignment allows)
+    assert abs(results[0][0] - results[1][0]) <= 1e-5 * abs(results[0][0])
+    assert torch.equal(results[0][1], results[1][1]) and torch.equal(results[0][2], results[1][2])
+
+
+@pytest.mark.parametrize("width", [1, 63, 64, 65, 123, 129, 1001])
+@pytest.mark.parametrize("autocast", [False, True])
+def test_other_widths_get_zero_columns(width, autocast):
+    """Widths that are no multiple of 8 (or at most one stage) against the formulas in fp64; under autocast fp32 inputs are
+    rounded and padded in one pass and their gradients come back in fp32, packed."""
+    from cut_cross_entropy import linear_cross_entropy
+    from oracle import dense_lce
+
+    N, V = 140, 700
+    e, c, t, _ = make_inputs(N, V, width, torch.bfloat16, seed=width, invalid_frac=0.2)
+    given = torch.float32 if autocast else torch.bfloat16
+    ed, cd = (x.to("cuda", given).requires_grad_(True) for x in (e, c))
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        loss = linear_cross_entropy(ed, cd, t.cuda(), reduction="sum", impl="cce_exact")
+    loss.backward()
+    eo, co = e.double().requires_grad_(True), c.double().requires_grad_(True)
+    want, _ = dense_lce.dense_linear_cross_entropy(eo, co, t, reduction="sum")
+    want.backward()
+    assert abs(loss.item() - want.item()) <= 1e-5 * abs(want.item())
+    for got, ref in ((ed.grad, eo.grad), (cd.grad, co.grad)):
+        assert got.dtype == given and got.is_contiguous() and got.shape == ref.shape
+        # dz and the result are rounded to bf16: 2^-9 of every product and of the sum
+        assert (got.cpu().double() - ref).norm() <= 4e-3 * ref.norm()
