@@ -511,7 +511,10 @@ __global__ __launch_bounds__(1024) void dz_colsum_kernel(const uint16_t* dz, int
   constexpr int kRowLanes = 1024 / LANES;
   __shared__ float s_sum[kRowLanes][LANES * 8 + 1];
   const int cl = threadIdx.x % LANES, rl = threadIdx.x / LANES;
-  const int cls = (blockIdx.x * LANES + cl) * 8;
+  // the 8 / LANES workgroups that read the same lines follow one another on one XCD
+  const int per_xcd = (gridDim.x + 7) / 8;
+  const int block = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int cls = (block * LANES + cl) * 8;
   float sum[8] = {};
   if (cls < n_cls) {  // (a row of dz goes on in whole 16-byte pieces)
     auto value = [&](int64_t i, float (&x)[8]) {
@@ -545,7 +548,7 @@ __global__ __launch_bounds__(1024) void dz_colsum_kernel(const uint16_t* dz, int
     __syncthreads();
   }
   if (threadIdx.x < LANES * 8) {
-    const int c = blockIdx.x * LANES * 8 + threadIdx.x;
+    const int c = block * LANES * 8 + threadIdx.x;
     if (c < n_cls) d_bias[c] += s_sum[0][threadIdx.x];
   }
 }
@@ -555,7 +558,7 @@ int dz_colsum_launch(const uint16_t* dz, int64_t ldz, int parts, int64_t b, int6
   // 64 classes (whole lines) per workgroup from 256 workgroups on, else down to 8
   int lanes = 8;
   while (lanes > 1 && (pieces + lanes - 1) / lanes < compute_units()) lanes /= 2;
-  const dim3 blocks(static_cast<unsigned>((pieces + lanes - 1) / lanes));
+  const dim3 blocks(static_cast<unsigned>(((pieces + lanes - 1) / lanes + 7) / 8 * 8));
 #define CCE_COLSUM(TT, L)                                                                                            \
   hipLaunchKernelGGL((dz_colsum_kernel<TT, L>), blocks, dim3(1024), 0, stream, dz, ldz, parts, b, static_cast<int>(n_cls), d_bias)
 #define CCE_COLSUM_LANES(TT)                                                                                         \
