@@ -300,6 +300,12 @@ int cce_valid_rows(const int64_t* labels, int64_t n, int64_t steps, int64_t shif
                    int64_t* count, void* stream);
 
 /*
+ * out[n]: values[r] at position rows[r] + shift, zeros elsewhere (cut_cross_entropy/utils.py:52-61).  rows[count] in
+ * increasing order, as cce_valid_rows writes them.
+ */
+int cce_rows_to_batch(const float* values, const int32_t* rows, int64_t count, int64_t n, int64_t shift, float* out, void* stream);
+
+/*
  * cce_lse_forward (without logit_avg) and cce_indexed_neg_dot in one call: lse[b], and nll[b] = lse + neg_dot, the loss of
  * every valid row (cut_cross_entropy/cce.py:87-131).  tile_max may be NULL; workspace as for cce_lse_forward.
  */

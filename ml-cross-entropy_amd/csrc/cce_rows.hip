@@ -52,6 +52,22 @@ __global__ __launch_bounds__(kRowThreads) void valid_rows_kernel(const int64_t* 
   if (tid == 0) *count = base;
 }
 
+// out[p] = values[r] where rows[r] + shift == p, 0 where there is no such r: the values of the valid rows (rows as
+// valid_rows_kernel leaves them, in increasing order) at their places in the batch.  A search per position, all of it in
+// cache; one launch in place of a fill, a widening, an addition and a scatter.
+__global__ __launch_bounds__(256) void rows_to_batch_kernel(const float* values, const int32_t* rows, int count, int n, int shift,
+                                                            float* out) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= n) return;
+  int lo = 0, hi = count;  // the first r with rows[r] >= p - shift
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (rows[mid] < p - shift) lo = mid + 1;
+    else hi = mid;
+  }
+  out[p] = (lo < count && rows[lo] == p - shift) ? values[lo] : 0.0f;
+}
+
 // The loss of one valid row per wave: its log-sum-exp from the partial (max, sum) pairs of the vocabulary spans, and minus
 // the soft-capped logit of its target, by a dot product of the two rows (0 where the target is no class of c), added up.
 // Bound by the rows it reads; one launch in place of a merge, a dot product and an addition (12 - 25 us of a short call).
@@ -186,5 +202,17 @@ extern "C" int cce_valid_rows(const int64_t* labels, int64_t n, int64_t steps, i
   if (shift >= steps && n > 0) shift = steps;  // no position has a label that far on
   hipLaunchKernelGGL(valid_rows_kernel, dim3(1), dim3(kRowThreads), 0, static_cast<hipStream_t>(stream), labels, static_cast<int>(n),
                      static_cast<int>(steps), static_cast<int>(shift), ignored, rows, count);
+  return status_from_hip(hipGetLastError());
+}
+
+extern "C" int cce_rows_to_batch(const float* values, const int32_t* rows, int64_t count, int64_t n, int64_t shift, float* out,
+                                 void* stream) {
+  if (n < 0 || n >= (int64_t(1) << 31) - 8192 || count < 0 || count > n || shift < 0) return CCE_ERR_INVALID_ARGUMENT;
+  if (n == 0) return CCE_OK;
+  if (out == nullptr || (count > 0 && (values == nullptr || rows == nullptr))) return CCE_ERR_INVALID_ARGUMENT;
+  if (shift > n) count = 0;  // no position is that far on
+  hipLaunchKernelGGL(rows_to_batch_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), values, rows, static_cast<int>(count), static_cast<int>(n),
+                     static_cast<int>(shift > n ? 0 : shift), out);
   return status_from_hip(hipGetLastError());
 }

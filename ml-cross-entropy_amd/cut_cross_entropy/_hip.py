@@ -66,6 +66,7 @@ _SIGNATURES = {
         _i32,
         [_ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _i64, _ptr, _i64, _i32, _i64, _i64, _i64, _i32, _ptr],
     ),
+    "cce_rows_to_batch": (_i32, [_ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr]),
     "cce_valid_rows": (_i32, [_ptr, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr]),
     "cce_loss_forward": (_i32, [_ptr] * 9 + [_i64] + [_i64] * 4 + [_i64] * 3 + [_i64, _i64, _f32, _i32, _ptr]),
     "cce_fp32_forward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),

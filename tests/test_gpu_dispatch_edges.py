@@ -384,3 +384,22 @@ def test_other_widths_get_zero_columns(width, autocast):
         assert got.dtype == given and got.is_contiguous() and got.shape == ref.shape
         # dz and the result are rounded to bf16: 2^-9 of every product and of the sum
         assert (got.cpu().double() - ref).norm() <= 4e-3 * ref.norm()
+
+
+@pytest.mark.parametrize("shape,shift", [((1, 1), 0), ((1, 1), 1), ((3, 85), 0), ((3, 85), 2), ((1, 257), 1), ((4, 64), 70), ((2, 5000), 1)])
+@pytest.mark.parametrize("keep", [0.0, 0.5, 1.0])
+def test_rows_to_batch_matches_the_library_chain(shape, shift, keep):
+    from cut_cross_entropy.utils import _build_flat_valids, handle_reduction_none, rows_to_batch
+
+    g = torch.Generator().manual_seed(sum(shape) + shift)
+    t = torch.randint(0, 9, shape, generator=g)
+    t[torch.rand(shape, generator=g) >= keep] = -100
+    if shift >= shape[1]:
+        valids = torch.empty((0,), dtype=torch.int32)
+    else:
+        valids = _build_flat_valids(t, -100, shift)
+        if valids is None:
+            valids = torch.arange(t.numel(), dtype=torch.int32)
+    values = torch.randn((valids.numel(),), generator=g)
+    got = rows_to_batch(t.size(), valids.cuda(), shift, values.cuda())
+    assert torch.equal(got.cpu(), handle_reduction_none(t.size(), valids, shift, values))
