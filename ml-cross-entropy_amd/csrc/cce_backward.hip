@@ -1533,9 +1533,9 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
 
   const bool aligned = aligned16(e) && aligned16(c) && (d % 8 == 0) && (stride_e % 8 == 0) &&
                        (stride_cv % 8 == 0) && (stride_cd == 1);
-  // The fast kernels store whole 16-byte pieces of the output rows.  A width of less than one stage stays with the general
-  // kernel, as a width that is mostly padding would.
-  const bool fast = aligned && d >= kFCols / 2 + 8 && (d_e == nullptr || p.vec_e) && (d_c == nullptr || p.vec_c);
+  // The fast kernels store whole 16-byte pieces of the output rows.  A width that would be mostly padding of their one
+  // stage stays with the general kernel.
+  const bool fast = aligned && d >= kFCols / 2 && (d_e == nullptr || p.vec_e) && (d_c == nullptr || p.vec_c);
   const bool tail = d % kFCols != 0;
   hipError_t err;
 #define CCE_LAUNCH(KERN, LDS, GRID)                                                                 \
