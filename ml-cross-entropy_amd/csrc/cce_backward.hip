@@ -1423,6 +1423,7 @@ static int owner_slices(int64_t d) { return static_cast<int>((d + kMaxChunks * k
 // and more: its 32 rows have that many labels), and no more slots than half of C takes (E [307, 5120] x C [131072, 5120]:
 // 30 workgroups took 745 us, 240 take 174 and 11 to put the slots together).
 static int owner_parts(int64_t b, int64_t v, int64_t d) {
+  if (b <= 0 || d <= 0) return 1;
   const int64_t groups = (b + 31) / 32 * owner_slices(d);
   int64_t n = compute_units() / groups;
   if (n > 16) n = 16;

@@ -102,3 +102,16 @@ def test_dense_backward_plans_by_classes_or_by_rows():
         assert dz % (256 * v_pad * 2) == 0 and dz >= 256 * v_pad * 2
         assert dz <= max(budget, 256 * v_pad * 2)
         assert dz <= a256(B) * v_pad * 2
+
+
+@pytest.mark.parametrize("sizes", [(0, 10, 64), (10, 0, 64), (10, 10, 0), (0, 0, 0)])
+def test_size_queries_answer_for_empty_matrices(sizes):
+    """A query is asked before the call that refuses such sizes, so it has to answer."""
+    from cut_cross_entropy import _hip
+
+    lib = _hip.load()
+    assert lib.cce_lse_forward_workspace_bytes(*sizes) >= 0
+    assert 0 <= lib.cce_backward_workspace_bytes(*sizes) <= 12
+    assert lib.cce_backward_dense_workspace_bytes(*sizes, 1, 1 << 20) == 0
+    assert lib.cce_fp32_forward_workspace_bytes(*sizes, 6) == 0
+    assert lib.cce_fp32_backward_workspace_bytes(*sizes, 6) == 0
