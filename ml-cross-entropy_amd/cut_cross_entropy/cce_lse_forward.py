@@ -85,6 +85,7 @@ def loss_forward(
     _hip.require_gpu_tensor("e", e)
     dev = e.device
     assert c.device == dev and c.dtype == e.dtype
+    assert targets.device == dev and targets.numel() == e.shape[0]
     V, D = c.shape
     code = _hip.dtype_code(e.dtype)
     lib = _hip.load()

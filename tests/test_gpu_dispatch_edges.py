@@ -208,6 +208,16 @@ def test_valid_rows_kernel_matches_the_host(shape, keep):
             assert got.dtype == torch.int32 and torch.equal(got.cpu(), want)
 
 
+@pytest.mark.parametrize("shape,shift", [((2, 4), 4), ((2, 4), 5), ((0, 4), 4), ((2, 0), 1)])
+def test_a_shift_past_the_sequences_is_refused(shape, shift):
+    """With no label left to compare with there is no loss: an error on either device, and not a mean of nothing."""
+    from cut_cross_entropy.utils import _build_flat_valids
+
+    for device in ("cpu", "cuda"):
+        with pytest.raises(RuntimeError):
+            _build_flat_valids(torch.zeros(shape, dtype=torch.int64, device=device), -100, shift)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(2, 3, 8), (5, 256 * 70, 128), (130, 700, 123), (1000, 2000, 192)])
 @pytest.mark.parametrize("softcap,bias,shift", [(None, False, 0), (15.0, True, 1)])
