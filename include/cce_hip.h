@@ -183,8 +183,8 @@ int cce_backward(const void* e, const void* c, const void* bias,
  */
 int cce_count_flagged_cells(const float* tile_max, const float* lse, int64_t b, int64_t v, float filter_eps,
                             uint64_t* count, void* stream);
-/* The same count written to *answer, which may be pinned host memory, in one launch.  `scratch`: two words that are zero
- * before the first call and that every call leaves at zero; calls that share them must share a stream. */
+/* The same count written to *answer, which may be pinned host memory, in one launch.  `scratch`: a word that is zero
+ * before the first call and that every call leaves at zero; calls that share it must share a stream. */
 int cce_measure_flagged_cells(const float* tile_max, const float* lse, int64_t b, int64_t v, float filter_eps,
                               uint64_t* scratch, uint64_t* answer, void* stream);
 

@@ -1348,36 +1348,45 @@ __global__ __launch_bounds__(256) void owner_merge_kernel(BwdParams p) {
 }
 
 // Number of cells of the forward statistic (32 rows x 32 classes) whose bound exp(max logit - min lse of the 32
-// rows) reaches eps: the cells the ownership kernels have to recompute.  One workgroup per row group.  With `answer` the
-// last workgroup to finish moves the total there and leaves count[0] (the sum) and count[1] (workgroups done) at zero for
-// the next launch on the same stream: one launch in place of a fill, the count and a copy.
-__global__ __launch_bounds__(256) void flagged_cells_kernel(const float* tile_max, const float* lse, int64_t b, int stat_cols,
-                                                            float log_eps, unsigned long long* count, unsigned long long* answer) {
-  __shared__ float s_min;
+// rows) reaches eps: the cells the ownership kernels have to recompute.  With `answer` the last workgroup to finish
+// moves the total there and leaves *count at zero for the next launch on the same stream: one launch in place of a
+// fill, the count and a copy.
+// What bounds it is the word that all workgroups add to, one after the other (device-wide, some 15 ns each): at most two
+// workgroups per compute unit, which walk the row groups, eight cells in flight per thread, and with `answer` ONE addition
+// for cells and finished workgroups together, which needs no fence in between.  At 2048 row groups of 4752 cells a workgroup
+// per group took 36 us, 64 with an addition for each of the two; 22 us so.
+constexpr int kFlaggedCellBits = 37;  // 2^37 cells of 4 bytes are more than the card holds; 2^27 row groups more than 2^31 rows
+__global__ __launch_bounds__(256) void flagged_cells_kernel(const float* tile_max, const float* lse, int64_t b, int ntg,
+                                                            int stat_cols, float log_eps, unsigned long long* count,
+                                                            unsigned long long* answer) {
   __shared__ unsigned int s_part[4];
-  const int tg = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (wave == 0) {
-    const int64_t i = static_cast<int64_t>(tg) * 32 + lane;
-    const float mn = wave_min((lane < 32 && i < b) ? lse[i] : INFINITY);
-    if (lane == 0) s_min = mn;
-  }
-  __syncthreads();
-  const float min_lse = s_min;
-  const float* row = tile_max + static_cast<int64_t>(tg) * stat_cols;
   unsigned int n = 0;
-  for (int j = threadIdx.x; j < stat_cols; j += 256) n += (row[j] - min_lse >= log_eps) ? 1u : 0u;
+  for (int tg = blockIdx.x; tg < ntg; tg += gridDim.x) {
+    const int64_t i = static_cast<int64_t>(tg) * 32 + (lane & 31);
+    const float min_lse = wave_min(i < b ? lse[i] : INFINITY);  // by every wave for itself
+    const float* row = tile_max + static_cast<int64_t>(tg) * stat_cols;
+    for (int j0 = threadIdx.x; j0 < stat_cols; j0 += 8 * 256) {
+      float x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = (j0 + k * 256 < stat_cols) ? row[j0 + k * 256] : -INFINITY;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) n += (j0 + k * 256 < stat_cols && x[k] - min_lse >= log_eps) ? 1u : 0u;
+    }
+  }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) n += __shfl_xor(n, off, 64);
   if (lane == 0) s_part[wave] = n;
   __syncthreads();
   if (threadIdx.x == 0) {
-    atomicAdd(count, static_cast<unsigned long long>(s_part[0] + s_part[1] + s_part[2] + s_part[3]));
-    if (answer != nullptr) {
-      __threadfence();  // this workgroup's share is in the sum before it is counted as done
-      if (atomicAdd(count + 1, 1ull) == gridDim.x - 1ull) {
-        *answer = atomicExch(count, 0ull);
-        count[1] = 0ull;
+    const unsigned long long mine = static_cast<unsigned long long>(s_part[0]) + s_part[1] + s_part[2] + s_part[3];
+    if (answer == nullptr) {
+      atomicAdd(count, mine);
+    } else {
+      const unsigned long long before = atomicAdd(count, mine + (1ull << kFlaggedCellBits));
+      if (before >> kFlaggedCellBits == gridDim.x - 1ull) {
+        *answer = (before & ((1ull << kFlaggedCellBits) - 1ull)) + mine;
+        *count = 0ull;
       }
     }
   }
@@ -1393,10 +1402,11 @@ static int count_flagged_cells(const float* tile_max, const float* lse, int64_t 
   if (b == 0) return CCE_OK;
   if (tile_max == nullptr || lse == nullptr || count == nullptr) return CCE_ERR_INVALID_ARGUMENT;
   const int64_t ntg = (b + CCE_STAT_ROWS - 1) / CCE_STAT_ROWS;
-  if (ntg >= (int64_t(1) << 31) || v >= (int64_t(1) << 31) - 512) return CCE_ERR_INVALID_ARGUMENT;
+  if (ntg >= (int64_t(1) << 31) - 65536 || v >= (int64_t(1) << 31) - 512) return CCE_ERR_INVALID_ARGUMENT;
   const int stat_cols = static_cast<int>((v + CCE_STAT_COLS - 1) / CCE_STAT_COLS);
-  hipLaunchKernelGGL(flagged_cells_kernel, dim3(static_cast<unsigned>(ntg)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     tile_max, lse, b, stat_cols, logf(filter_eps) - 0.01f,
+  const int64_t most = 2 * static_cast<int64_t>(compute_units());
+  hipLaunchKernelGGL(flagged_cells_kernel, dim3(static_cast<unsigned>(ntg < most ? ntg : most)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), tile_max, lse, b, static_cast<int>(ntg), stat_cols, logf(filter_eps) - 0.01f,
                      reinterpret_cast<unsigned long long*>(count), reinterpret_cast<unsigned long long*>(answer));
   return status_from_hip(hipGetLastError());
 }

@@ -74,7 +74,7 @@ class _FlaggedMonitor:
     """Fraction of flagged cells of the latest backward of one (device, V, D, dtype), and the path it chose."""
 
     def __init__(self, device: torch.device):
-        self.scratch: dict = {}  # stream -> the two words its measurements count in
+        self.scratch: dict = {}  # stream -> the word its measurements count in
         self.host = torch.zeros((1,), dtype=torch.int64, pin_memory=True)
         self.event = torch.cuda.Event()
         self.pending_cells = 0   # cells of the measurement in flight (0: none)
@@ -95,7 +95,7 @@ class _FlaggedMonitor:
         if scratch is None:
             if len(self.scratch) >= 16:  # streams come and go; whatever of theirs is still running holds its own memory
                 self.scratch.clear()
-            scratch = self.scratch[stream.cuda_stream] = torch.zeros((2,), dtype=torch.int64, device=dev)
+            scratch = self.scratch[stream.cuda_stream] = torch.zeros((1,), dtype=torch.int64, device=dev)
         with _hip.on_device(dev):
             status = lib.cce_measure_flagged_cells(tile_max.data_ptr(), lse.data_ptr(), B, V, float(filter_eps),
                                                    scratch.data_ptr(), self.host.data_ptr(), stream.cuda_stream)

@@ -413,3 +413,35 @@ def test_rows_to_batch_matches_the_library_chain(shape, shift, keep):
     values = torch.randn((valids.numel(),), generator=g)
     got = rows_to_batch(t.size(), valids.cuda(), shift, values.cuda())
     assert torch.equal(got.cpu(), handle_reduction_none(t.size(), valids, shift, values))
+
+
+@pytest.mark.parametrize("rows,classes", [(1, 1), (31, 256 * 32), (32, 2049 * 32), (33, 2048 * 32 - 5), (512 * 32, 700), (512 * 32 + 1, 33), (40000, 5000)])
+def test_flagged_cells_are_counted_in_one_launch(rows, classes):
+    """One workgroup and several row groups per workgroup, cells of one trip of the loop and more; the word the workgroups
+    meet in is zero again for the next launch, and the form that adds to a caller's word counts the same."""
+    lib = _lib()
+    groups, cols = -(-rows // 32), -(-classes // 32)
+    assert lib.cce_tile_stat_elems(rows, classes) == groups * cols
+    g = torch.Generator().manual_seed(rows + classes)
+    cells = torch.randn((groups, cols), generator=g)
+    cells[:: 3, :: 5] = float("-inf")
+    lse = torch.randn((rows,), generator=g) + 3.0
+    eps = 0.05
+    padded = torch.full((groups * 32,), float("inf"))
+    padded[:rows] = lse
+    log_eps = (torch.tensor(eps).log() - 0.01).item()
+    margin = cells - padded.view(groups, 32).amin(1, keepdim=True) - log_eps
+    sure, open_ = int((margin > 1e-5).sum()), int((margin.abs() <= 1e-5).sum())  # fp32 rounding of values below 16
+    cells, lse = cells.cuda(), lse.cuda()
+    scratch = torch.zeros((2,), dtype=torch.int64, device="cuda")
+    answer = torch.full((1,), -1, dtype=torch.int64, pin_memory=True)
+    stream = torch.cuda.current_stream()
+    for _ in range(3):
+        answer.fill_(-1)
+        assert lib.cce_measure_flagged_cells(cells.data_ptr(), lse.data_ptr(), rows, classes, eps, scratch.data_ptr(),
+                                             answer.data_ptr(), stream.cuda_stream) == 0
+        stream.synchronize()
+        assert sure <= answer.item() <= sure + open_
+        assert scratch.tolist() == [0, 0]
+    assert lib.cce_count_flagged_cells(cells.data_ptr(), lse.data_ptr(), rows, classes, eps, scratch.data_ptr(), stream.cuda_stream) == 0
+    assert scratch[0].item() == answer.item()
