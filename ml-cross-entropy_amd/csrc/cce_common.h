@@ -591,6 +591,11 @@ struct DmaLogitTile {
 // fetched from a line of zeros, for both operands, so that nothing of another row (a non-finite value least of all) meets
 // the product.  A variant of its own, since the question costs every load two scalar instructions: such widths were
 // padded to a multiple of 128 before, a pass over E and C and one over each of their gradients.
+//
+// FEW: at most 128 token rows.  The read of C is then what takes the time, and with two stages of 64 KB only one of C (32 KB
+// per compute unit) is ever in flight.  Half of the token rows leave the ring and a third stage takes their place; the
+// waves are numbered so that those whose 64 rows exist sit on SIMDs of their own (wave / NWV instead of wave % NWT), and
+// the other waves only fetch (fetch_only).
 // ---------------------------------------------------------------------------------------------
 // Which part (0 hi, 1 mid, 2 lo) of the first and of the second operand meets in term t, smallest terms first, so that
 // the accumulator is rounded at its full size only while the last one is added:
@@ -601,19 +606,25 @@ __host__ __device__ __forceinline__ int term_part(unsigned table, int term) {
   return static_cast<int>((table >> (2 * term)) & 3u);
 }
 
-template <typename T, int WV, int WT, int NWV, int NWT, bool TERMS = false, bool TAIL = false>
+template <typename T, int WV, int WT, int NWV, int NWT, bool TERMS = false, bool TAIL = false, bool FEW = false>
 struct DmaLogitTile16 {
+  static_assert(!FEW || !TERMS, "parts take the ring of two stages");
   static_assert(!TERMS || !TAIL, "parts are whole stages");
   static_assert(WV % 2 == 0 && WT % 2 == 0, "the ring is addressed in blocks of 32 rows");
   using Base = DmaLogitTile<T, WV / 2, WT / 2, NWV, NWT>;
   static constexpr int TILE_V = Base::TILE_V;
   static constexpr int TILE_T = Base::TILE_T;
   static constexpr int NW = Base::NW;
-  static constexpr int STAGE_BYTES = Base::STAGE_BYTES;
-  static constexpr int LDS_BYTES = Base::LDS_BYTES;
   static constexpr int NQC = Base::NQC;
-  static constexpr int NQ = Base::NQ;
+  static constexpr int NQ = FEW ? NQC + (Base::NQ - NQC) / 2 : Base::NQ;
+  static constexpr int RING = FEW ? 3 : 2;
+  static constexpr int STAGE_BYTES = FEW ? (TILE_V + TILE_T / 2) * kDmaRowBytes : Base::STAGE_BYTES;
+  static constexpr int LDS_BYTES = RING * STAGE_BYTES;
+  static_assert(FEW || LDS_BYTES == Base::LDS_BYTES, "two stages");
   using vec8 = typename Elem<T>::vec8;
+
+  static __device__ __forceinline__ int wv_of(int wave) { return FEW ? wave % NWV : wave / NWT; }
+  static __device__ __forceinline__ int wt_of(int wave) { return FEW ? wave / NWV : wave % NWT; }
 
   static __device__ __forceinline__ int row_of(int q, int wave, int lane) { return Base::row_of(q, wave, lane); }
   static __device__ __forceinline__ int chunk_elems(int wave, int lane) { return Base::chunk_elems(wave, lane); }
@@ -732,7 +743,7 @@ struct DmaLogitTile16 {
     return sync ? kSyncAt + 5 + t * ((kSlots - kSyncAt - 8) / WT & ~1) : 1 + t * (kSlots / WT);
   }
   static constexpr int load_slot(int j) { return j < 6 ? kSyncAt + 2 + 4 * j : kSlots - 4 + 2 * (j - 6); }
-  static_assert(WV == 8 && WT == 4 && NQ == 8, "the slot tables above are laid out for 8 x 4 blocks and 8 loads");
+  static_assert(WV == 8 && WT == 4 && NQ <= 8, "the slot tables above are laid out for 8 x 4 blocks and 8 loads");
 
   // ZERO (the first step of a tile): the accumulators start from the instruction's constant zero instead of being
   // cleared beforehand (128 register writes per lane and tile; the copy of the first stage this takes costs a
@@ -745,7 +756,7 @@ struct DmaLogitTile16 {
       constexpr int idx = decltype(idx_c)::value;
       constexpr int vi = idx / WT, ti = idx % WT;
       if (SYNC && idx == kSyncAt) {
-        wait_vmcnt<0>();
+        wait_vmcnt<(RING - 2) * NQ>();
         __syncthreads();
       }
       acc[vi][ti] = Elem<T>::mfma16(a[vi], bc[ti], ZERO ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : acc[vi][ti]);
@@ -770,7 +781,7 @@ struct DmaLogitTile16 {
     });
   }
 
-  // Start the ring for the first tile of a span: its first two stages, into ring stages 0 and 1.
+  // Start the ring for the first tile of a span: its first RING stages.
   static __device__ __forceinline__ void prefetch(const Source& src, unsigned char* lds, int D) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
@@ -781,10 +792,44 @@ struct DmaLogitTile16 {
     else w.off_c = w.off_e = kDmaBK;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) issue_one(src, q, w.off_c, w.off_e, lds_base, STAGE_BYTES, wave);
+    if constexpr (FEW) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) issue_one(src, q, 2 * kDmaBK, 2 * kDmaBK, lds_base, 2 * STAGE_BYTES, wave);
+    }
   }
 
-  // D must be a multiple of 64 (TAIL: of 8) and, without TERMS, make at least two stages.  The first two stages of this tile must be in flight or landed in
-  // ring stages buf, 1 - buf (prefetch() for the first tile of a span: first_tile; else the previous run()), and
+  static __device__ __forceinline__ int next_stage(int cur) {
+    if constexpr (RING == 2) return STAGE_BYTES - cur;
+    return cur == (RING - 1) * STAGE_BYTES ? 0 : cur + STAGE_BYTES;
+  }
+
+  // run() for a wave that has no rows: its loads, and the barriers of the others.
+  template <typename NextTile>
+  static __device__ __forceinline__ void fetch_only(Source& src, unsigned char* lds, int D, int& buf, bool first_tile,
+                                                    NextTile&& next_tile) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
+    const int nk = (D + (TAIL ? kDmaBK - 1 : 0)) / kDmaBK;
+    int cur = buf * STAGE_BYTES;
+    if (first_tile) {
+      wait_vmcnt<(RING - 1) * NQ>();
+      __syncthreads();
+    }
+#pragma unroll 1
+    for (int s = 0; s < nk; ++s) {
+      if (s == nk - RING) next_tile();
+      const int col = ((s + RING < nk) ? s + RING : s + RING - nk) * kDmaBK;
+      wait_vmcnt<(RING - 2) * NQ>();
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) issue_one(src, q, col, col, lds_base, cur, wave);
+      cur = next_stage(cur);
+    }
+    buf = cur / STAGE_BYTES;
+  }
+
+  // D must be a multiple of 64 (TAIL: of 8) and, without TERMS, make at least RING stages.  The first RING stages of this tile must be in flight or landed in
+  // the ring, from stage buf on (prefetch() for the first tile of a span: first_tile; else the previous run()), and
   // nothing else may have touched the ring.
   // next_tile() is called once, when the class rows of this tile have been fetched for the last time: it points
   // `src` at the tile whose first stages the rest of this run fetches (or leaves it: those loads then repeat this
@@ -794,8 +839,8 @@ struct DmaLogitTile16 {
                                              bool first_tile, NextTile&& next_tile) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wv = wave / NWT;
-    const int wt = wave % NWT;
+    const int wv = wv_of(wave);
+    const int wt = wt_of(wave);
     const int r16 = lane & 15;
     // this lane's 16-byte chunk of a ring row: (l / 16) for the first half of a stage, + 4 for the second,
     // XOR-swizzled with (row >> 1) & 7 like the loads place them
@@ -805,23 +850,23 @@ struct DmaLogitTile16 {
     const unsigned char* e_row = lds + (TILE_V + wt * WT * 16 + r16) * kDmaRowBytes;
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
 
-    const int nk = TERMS ? src.terms * (D / kDmaBK) : (D + (TAIL ? kDmaBK - 1 : 0)) / kDmaBK;  // >= 2
+    const int nk = TERMS ? src.terms * (D / kDmaBK) : (D + (TAIL ? kDmaBK - 1 : 0)) / kDmaBK;  // >= RING
     Walk w = walk_start(D, src.terms);
     if constexpr (TERMS) {
       walk_next(w, D, src.terms);
       walk_next(w, D, src.terms);
     }
-    // columns of the stage two ahead of stage s (a stage of the next tile under the last two)
+    // columns of the stage RING ahead of stage s (a stage of the next tile under the last RING)
     auto ahead = [&](int s) {
       if constexpr (TERMS) {
         if (s > 0) walk_next(w, D, src.terms);
       } else {
-        w.off_c = w.off_e = (s + 2 < nk) ? (s + 2) * kDmaBK : (s + 2 - nk) * kDmaBK;
+        w.off_c = w.off_e = (s + RING < nk) ? (s + RING) * kDmaBK : (s + RING - nk) * kDmaBK;
       }
     };
     int cur = buf * STAGE_BYTES;
     if (first_tile) {
-      wait_vmcnt<NQ>();  // the first stage has landed for this wave (the second, NQ loads or twice that, may be in flight) ...
+      wait_vmcnt<(RING - 1) * NQ>();  // the first stage has landed for this wave (the others may be in flight) ...
       __syncthreads();   // ... and for all of them
     }
     // (a later tile's first stage was awaited by every wave before the last barrier of the tile before it: no
@@ -834,9 +879,9 @@ struct DmaLogitTile16 {
 
     // first stage (never the last: there are at least two)
     {
-      const int nxt = STAGE_BYTES - cur;
+      const int nxt = next_stage(cur);
       step<true, false, false, true>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, 0, lds_base, 0, wave);
-      if (nk == 2) next_tile();
+      if (nk == RING) next_tile();
       ahead(0);
       step<true, true, true>(acc, a, b1, b0, c_row + nxt + chunk0, e_row + nxt + chunk0, src, w.off_c, w.off_e, lds_base, cur,
                              wave);
@@ -844,9 +889,9 @@ struct DmaLogitTile16 {
     }
 #pragma unroll 1
     for (int s = 1; s < nk - 1; ++s) {
-      const int nxt = STAGE_BYTES - cur;
+      const int nxt = next_stage(cur);
       step<true, false, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, 0, lds_base, 0, wave);
-      if (s == nk - 2) next_tile();
+      if (s == nk - RING) next_tile();
       ahead(s);
       step<true, true, true>(acc, a, b1, b0, c_row + nxt + chunk0, e_row + nxt + chunk0, src, w.off_c, w.off_e, lds_base, cur,
                              wave);
@@ -857,7 +902,7 @@ struct DmaLogitTile16 {
     step<true, false, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, 0, 0, lds_base, 0, wave);
     ahead(nk - 1);
     step<false, true, true>(acc, a, b1, b0, c_row, e_row, src, w.off_c, w.off_e, lds_base, cur, wave);
-    buf = 1 - cur / STAGE_BYTES;
+    buf = next_stage(cur) / STAGE_BYTES;
   }
 };
 

@@ -385,10 +385,12 @@ __device__ __forceinline__ void row_block(const Softcap& sc, float cap_inv, bool
   else row_block_impl<GENERAL, false, false, WANT_S2>(sc, cap_inv, acc, ti, addend, kq, run, bm, s2);
 }
 
-template <typename T, bool GENERAL, bool WANT_LA, bool TERMS = false, bool TAIL = false>
+template <typename T, bool GENERAL, bool WANT_LA, bool TERMS = false, bool TAIL = false, bool FEW = false>
 __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdParams p) {
-  using Fast = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, TERMS, TAIL>;
+  using Fast = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, TERMS, TAIL, FEW>;
   static_assert(!WANT_LA || GENERAL, "the column average uses the general epilogue");
+  static_assert(!FEW || !WANT_LA, "all waves take part in the column average");
+  constexpr int kRunStride = FEW ? kFwdThreads / 2 : kFwdThreads;  // FEW: the waves without rows keep nothing
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_addend = reinterpret_cast<float*>(smem + Fast::LDS_BYTES);  // [2][256]
   // The running (max, sum-exp) of this lane's kF16WT token rows lives in LDS between the epilogues: [ti][thread].
@@ -415,12 +417,13 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   // wave-uniform, and known to the compiler as such: everything derived from it (row and class offsets of the
   // wave, addresses of the statistic cells) then lives in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wv = wave / kFwdNWT;
-  const int wt = wave % kFwdNWT;
+  const int wv = Fast::wv_of(wave);
+  const int wt = Fast::wt_of(wave);
   const int r16 = lane & 15;
   const int kq = lane >> 4;
   const int64_t t0 = static_cast<int64_t>(rb) * kFwdTile;
   const int64_t wrow0 = t0 + wt * (16 * kF16WT);  // first row of this wave
+  const bool live = !FEW || wrow0 < p.b;
 
   // Sources of the direct-to-LDS loads (the launcher has checked that the byte offsets fit 32 bits)
   typename Fast::Source src;
@@ -445,7 +448,8 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   // 2^(-2 cap log2(e)) must stay a normal float: cap log2(e) < 60, i.e. caps up to 41
   const bool fixed_ref = p.sc.on && p.sc.out_scale < 60.0f;
 #pragma unroll
-  for (int ti = 0; ti < kF16WT; ++ti) s_run[ti * kFwdThreads] = make_float2(-INFINITY, 0.0f);
+  for (int ti = 0; ti < kF16WT; ++ti)
+    if (live) s_run[ti * kRunStride] = make_float2(-INFINITY, 0.0f);
   if (WANT_LA) s_colsum[tid] = 0.0f;  // 512 threads, 2 x 256 sums; published by the barriers of the first main loop
   // the sums of the tile that starts at class `first` leave for the running average, and are cleared for the tile after next
   // (the scale comes as a kernel argument and the address is formed where it is used: a lane constant carried
@@ -482,10 +486,17 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
         addend[tid] = a;
       }
     }
-    f32x4 acc[kF16WV][kF16WT];
-    Fast::run(acc, src, smem, static_cast<int>(p.d), buf, vt == vt_begin, [&] {
+    auto next_tile = [&] {
       if (vt + 1 < vt_end) set_class_tile(v0 + kFwdTile);
-    });
+    };
+    if constexpr (FEW) {
+      if (!live) {
+        Fast::fetch_only(src, smem, static_cast<int>(p.d), buf, vt == vt_begin, next_tile);
+        continue;
+      }
+    }
+    f32x4 acc[kF16WV][kF16WT];
+    Fast::run(acc, src, smem, static_cast<int>(p.d), buf, vt == vt_begin, next_tile);
 
     // ---- epilogue: (bias, mask,) soft-cap, online max / sum-exp ---------------------------------
     const float* wave_addend = addend + wv * (16 * kF16WV);
@@ -510,10 +521,10 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
         const int ti = 2 * tp + u;
         __builtin_amdgcn_sched_barrier(0);  // keep each row block's register use to itself
         float s2[kF16WV][4];
-        float2 run = s_run[ti * kFwdThreads];
+        float2 run = s_run[ti * kRunStride];
         if (GENERAL && plain_tile) row_block<false, WANT_LA>(p.sc, p.cap_inv, fixed_ref, acc, ti, wave_addend, kq, run, bm, s2);
         else row_block<GENERAL, WANT_LA>(p.sc, p.cap_inv, fixed_ref, acc, ti, wave_addend, kq, run, bm, s2);
-        s_run[ti * kFwdThreads] = run;
+        s_run[ti * kRunStride] = run;
         if (WANT_LA) {
           const bool ok = wrow0 + ti * 16 + r16 < p.b;
 #pragma unroll
@@ -576,7 +587,7 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   float m2[kF16WT], sum[kF16WT];
 #pragma unroll
   for (int ti = 0; ti < kF16WT; ++ti) {
-    const float2 run = s_run[ti * kFwdThreads];
+    const float2 run = live ? s_run[ti * kRunStride] : make_float2(-INFINITY, 0.0f);
     m2[ti] = run.x;
     sum[ti] = run.y;
   }
@@ -652,6 +663,9 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
   static_assert(Fast::LDS_BYTES <= Tile::LDS_BYTES, "one LDS size serves both main loops");
   const int lds = Tile::LDS_BYTES + kFwdBiasBytes;
   const int lds16 = lds + kF16RunBytes;  // + the running (max, sum) pairs
+  using Few = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, false, false, true>;
+  constexpr int lds_few = Few::LDS_BYTES + kFwdBiasBytes + kF16RunBytes / 2;
+  static_assert(lds_few <= 160 * 1024, "three stages fit");
   // the 16 x 16 x 32 kernel addresses token rows by 32-bit byte offsets from e and class rows by offsets from the
   // first class of a tile; shapes beyond that, and a D of one stage, take the 32 x 32 x 16 kernel, which knows whole
   // stages only
@@ -659,6 +673,11 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
   const bool fast16 = aligned && (p.d > kDmaBK) && (p.n_rows * p.stride_e * 2 < (int64_t(1) << 32)) &&
                       (256 * p.stride_cv * 2 < (int64_t(1) << 32));
   const bool tail = p.d % kDmaBK != 0;
+  // Up to 128 rows the read of C is the larger part (at 256 rows the products are): the ring of three stages with half the
+  // token rows (FEW), which wants three stages of D.  Forward and loss of 64 rows, ring of two / three, us: 256000 classes x 2304 columns
+  // 290 / 210 (C at 5.6 TB/s), 131072 x 5120 334 / 251, 50257 x 1000 49 / 42, 4096 x 512 21 / 17.5, 512 x 192 17.5 / 17.5;
+  // 16 and 128 rows alike.
+  const bool few = fast16 && !want_la && p.b <= kFwdTile / 2 && p.d > 2 * kDmaBK;
   const bool general = want_la || (p.bias != nullptr) || (p.v % Tile::TILE_V != 0);
   const int grid = p.items_per_xcd * 8;
   hipError_t err;
@@ -670,23 +689,29 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
     if (err != hipSuccess) return status_from_hip(err);                                           \
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), lds, stream, p);                           \
   } while (0)
-#define CCE_LAUNCH_FWD16(GE, LA, TAIL)                                                            \
+#define CCE_LAUNCH_FWD16(GE, LA, TAIL, FEW)                                                       \
   do {                                                                                            \
-    auto kern = lse_forward16_kernel<T, GE, LA, false, TAIL>;                                     \
+    auto kern = lse_forward16_kernel<T, GE, LA, false, TAIL, FEW>;                                \
     static LdsLimitOnce lds_limit;                                                            \
-    const int bytes = lds16 + ((LA) ? kF16ColsumBytes : 0);                                       \
+    const int bytes = (FEW) ? lds_few : lds16 + ((LA) ? kF16ColsumBytes : 0);                     \
     err = lds_limit.set(kern, bytes);                                                             \
     if (err != hipSuccess) return status_from_hip(err);                                           \
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), bytes, stream, p);                    \
   } while (0)
-  if (fast16 && tail) {
-    if (want_la) CCE_LAUNCH_FWD16(true, true, true);
-    else if (general) CCE_LAUNCH_FWD16(true, false, true);
-    else CCE_LAUNCH_FWD16(false, false, true);
+  if (few && tail) {
+    if (general) CCE_LAUNCH_FWD16(true, false, true, true);
+    else CCE_LAUNCH_FWD16(false, false, true, true);
+  } else if (few) {
+    if (general) CCE_LAUNCH_FWD16(true, false, false, true);
+    else CCE_LAUNCH_FWD16(false, false, false, true);
+  } else if (fast16 && tail) {
+    if (want_la) CCE_LAUNCH_FWD16(true, true, true, false);
+    else if (general) CCE_LAUNCH_FWD16(true, false, true, false);
+    else CCE_LAUNCH_FWD16(false, false, true, false);
   } else if (fast16) {
-    if (want_la) CCE_LAUNCH_FWD16(true, true, false);
-    else if (general) CCE_LAUNCH_FWD16(true, false, false);
-    else CCE_LAUNCH_FWD16(false, false, false);
+    if (want_la) CCE_LAUNCH_FWD16(true, true, false, false);
+    else if (general) CCE_LAUNCH_FWD16(true, false, false, false);
+    else CCE_LAUNCH_FWD16(false, false, false, false);
   } else if (fast) {
     if (want_la) CCE_LAUNCH_FWD(true, true, true, true);
     else if (general) CCE_LAUNCH_FWD(true, true, true, false);

@@ -445,3 +445,35 @@ def test_flagged_cells_are_counted_in_one_launch(rows, classes):
         assert scratch.tolist() == [0, 0]
     assert lib.cce_count_flagged_cells(cells.data_ptr(), lse.data_ptr(), rows, classes, eps, scratch.data_ptr(), stream.cuda_stream) == 0
     assert scratch[0].item() == answer.item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("width,classes", [(128, 300), (136, 256 * 257), (192, 512), (200, 2000), (704, 256 * 600 + 1)])
+def test_forward_of_few_rows_keeps_three_stages(dtype, rows, width, classes):
+    """Up to 128 rows (waves with and without rows), the fewest stages of the ring of three and one less, partial last
+    stages, tiles of one span and of several, a cut last tile: log-sum-exp, losses and the cells' maxima."""
+    from cut_cross_entropy.cce_lse_forward import loss_forward
+
+    g = torch.Generator().manual_seed(rows + width)
+    e = torch.randn((rows + 5, width), generator=g).to(dtype).cuda()
+    c = (torch.randn((classes, width), generator=g) * 0.1).to(dtype).cuda()
+    t = torch.randint(0, classes, (rows + 5,), generator=g).cuda()
+    valids = torch.arange(5, rows + 5, dtype=torch.int32).cuda()
+    for softcap, bias in ((None, None), (20.0, None), (None, torch.randn((classes,), generator=g).to(dtype).cuda())):
+        for _ in range(2):
+            lse, nll, cells = loss_forward(e, c, bias, t, valids, 0, softcap, 0, True)
+        x = e[5:].float() @ c.float().T
+        if bias is not None:
+            x += bias.float()
+        if softcap is not None:
+            x = softcap * torch.tanh(x / softcap)
+        want = torch.logsumexp(x, 1)
+        # fp32 sums of `width` products of values around 1 and 0.1, then of the classes' exponentials
+        assert (lse - want).abs().max() < 2e-5 * max(1.0, want.abs().max().item())
+        assert (nll - (want - x.gather(1, t[5:, None])[:, 0])).abs().max() < 1e-4
+        rb, cb = -(-rows // 32), -(-classes // 32)
+        padded = torch.full((rb * 32, cb * 32), float("-inf"), device="cuda")
+        padded[:rows, :classes] = x
+        top = padded.view(rb, 32, cb, 32).amax((1, 3))
+        assert (cells.view(rb, cb) - top).abs().max() < 2e-4
