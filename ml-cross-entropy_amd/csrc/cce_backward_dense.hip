@@ -642,12 +642,14 @@ static int64_t split_stages(int64_t stages, int splits) { return (stages + split
 // product tile (64 steps of 256 x 256; 1.65 us where all units are busy): the dz tiles in rounds of all units, d / 64
 // stages each, then the product items as they are handed out.  An item of a cut reduction leaves 256 KB of fp32 (and
 // takes them in first, where slots are carried): up to 6 stages of time where every unit does so at once.
+// whole_tiles: reductions counted in whole tiles of 256 steps, as the chunks of whole reductions are chosen.
 static double launch_cost(int64_t rows, int64_t cls, int64_t d, int de_splits, int dc_splits, bool de_carried, bool dc_carried,
-                          int terms = 1) {
+                          int terms = 1, bool whole_tiles = false) {
   const int64_t cus = compute_units();
   const int64_t tr = (rows + 255) / 256, tc = (cls + 255) / 256, tn = (d + 255) / 256;
   const int64_t dz = (tr * tc + cus - 1) / cus * tn * 4 * terms;
   auto item = [&](int64_t total, int splits, int64_t tiles, bool carried) {
+    if (whole_tiles) return (total + 255) / 256 * 4;
     const int64_t len = split_stages((total + 63) / 64, splits) * terms;
     if (splits == 1) return len;
     const int64_t items = tiles * splits;
@@ -706,7 +708,11 @@ static DensePlan dense_plan_uncached(int64_t b, int64_t v, int64_t d, bool g16, 
     pl.slot_bytes = slots;
   };
 
-  // ---- whole reductions
+  // ---- whole reductions.  A carried 16-bit gradient is rounded once per launch, at places that go by the unit: the unit of
+  // a plan without cuts is chosen by the estimate in whole tiles alone, apart from what the cut plans below are weighed
+  // with, so that a shape which is not cut keeps the bits of its gradients whatever becomes of the other estimate, and by
+  // rows it takes no launch more than the buffer asks for (E [65536, 3584] x C [19008, 3584]: ten blocks of 6656 rows;
+  // twelve of 5632 take the same 28.9 ms, forward and backward, and round dC twice more).
   if (pl.by_rows) {
     int64_t rb = max_dz_bytes / (v_pad * 2) / 256 * 256;
     if (rb > b_pad) rb = b_pad;
@@ -718,9 +724,18 @@ static DensePlan dense_plan_uncached(int64_t b, int64_t v, int64_t d, bool g16, 
   } else {
     int64_t top = max_dz_bytes / (b * 2) / 256 * 256;
     if (top > kMaxChunkClasses) top = kMaxChunkClasses;
-    if (top >= v_pad) consider(v_pad, 1, 1);
-    else
-      for (int64_t vc = top; vc >= 256; vc -= 256) consider(vc, 1, 1);
+    int64_t unit = top >= v_pad ? v_pad : 0;
+    double least = 1e300;
+    for (int64_t vc = top; vc >= 256 && top < v_pad; vc -= 256) {
+      const int64_t whole = v / vc, rest = v - whole * vc;
+      double cost = static_cast<double>(whole) * (1.0 + launch_cost(b, vc, d, 1, 1, false, false, 1, true));
+      if (rest > 0) cost += 1.0 + launch_cost(b, rest, d, 1, 1, false, false, 1, true);
+      if (cost < least * (1.0 - 1e-9)) {
+        least = cost;
+        unit = vc;
+      }
+    }
+    if (unit > 0) consider(unit, 1, 1);
   }
 
   // ---- cut reductions, in as few launches as the budget allows (chunks past 16384 classes where the whole dz still
@@ -739,7 +754,7 @@ static DensePlan dense_plan_uncached(int64_t b, int64_t v, int64_t d, bool g16, 
         if (se > 1 && (cls + 63) / 64 < se * kMinSplitStages) break;
         for (int sc : kSplits) {
           if (sc > 1 && (rows + 63) / 64 < sc * kMinSplitStages) break;
-          consider(unit, se, sc);
+          if (se > 1 || sc > 1) consider(unit, se, sc);
         }
       }
     }

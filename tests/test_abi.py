@@ -115,3 +115,20 @@ def test_size_queries_answer_for_empty_matrices(sizes):
     assert lib.cce_backward_dense_workspace_bytes(*sizes, 1, 1 << 20) == 0
     assert lib.cce_fp32_forward_workspace_bytes(*sizes, 6) == 0
     assert lib.cce_fp32_backward_workspace_bytes(*sizes, 6) == 0
+
+
+@pytest.mark.parametrize("sizes,unit,budget", [
+    ((65536, 19008, 3584), 6656, 256 << 20), ((41192, 11918, 4864), 10496, 256 << 20), ((53256, 10706, 3200), 10752, 256 << 20),
+    ((5472, 148531, 1856), 11776, 256 << 20), ((3879, 33278, 3840), 12288, 256 << 20), ((3209, 48576, 4992), 15104, 256 << 20),
+    ((5824, 134912, 2688), 11264, 256 << 20), ((14400, 9131, 3840), 9216, 256 << 20)])
+def test_plans_of_whole_reductions_do_not_go_by_the_estimate_for_cut_ones(sizes, unit, budget):
+    """Rows per block (more than twice as many rows as classes) or classes per chunk of shapes whose reductions are not cut:
+    where the launches begin decides where the carried 16-bit gradient is rounded."""
+    lib = _lib()
+    a256 = lambda x: (x + 255) // 256 * 256
+    b, v, d = sizes
+    by_rows = b >= 2 * a256(v)
+    fixed = lib.cce_backward_dense_fixed_bytes(b, v, d, 1)
+    assert fixed == a256((v if by_rows else b) * d * 2)
+    dz = lib.cce_backward_dense_workspace_bytes(b, v, d, 1, budget) - fixed
+    assert dz == a256((unit * a256(v) if by_rows else unit * b) * 2)
