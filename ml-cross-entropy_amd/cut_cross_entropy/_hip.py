@@ -170,6 +170,14 @@ def require_gpu_tensor(name: str, t: torch.Tensor) -> None:
         )
 
 
+def require_device(device: torch.device, **tensors: Optional[torch.Tensor]) -> None:
+    """Every tensor lies on ``device``: asked before an address is handed on, since a kernel that reads another device's
+    memory, or the host's, faults."""
+    for name, t in tensors.items():
+        if t is not None and t.device != device:
+            raise RuntimeError(f"{name} is on {t.device}, e on {device}: all tensors have to be on one device")
+
+
 def current_stream_ptr(device: torch.device) -> int:
     """The raw handle of the current stream (what ``torch.cuda.current_stream(device).cuda_stream`` builds a Stream
     object to answer: 2 us where a small call has some fifty)."""

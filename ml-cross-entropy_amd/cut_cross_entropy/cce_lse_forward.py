@@ -84,8 +84,9 @@ def loss_forward(
     assert e.shape[1] == c.shape[1], "Incompatible dimensions"
     _hip.require_gpu_tensor("e", e)
     dev = e.device
-    assert c.device == dev and c.dtype == e.dtype
-    assert targets.device == dev and targets.numel() == e.shape[0]
+    _hip.require_device(dev, c=c, bias=bias, targets=targets, valids=valids)
+    assert c.dtype == e.dtype
+    assert targets.numel() == e.shape[0]
     V, D = c.shape
     code = _hip.dtype_code(e.dtype)
     lib = _hip.load()

@@ -34,6 +34,13 @@ def _workspace(nbytes: int, dev: torch.device) -> Tuple[torch.Tensor, int]:
     return buf, (buf.data_ptr() + 255) // 256 * 256
 
 
+def _check(e, c, bias, targets, valids) -> None:
+    _hip.require_gpu_tensor("e", e)
+    _hip.require_device(e.device, c=c, bias=bias, targets=targets, valids=valids)
+    assert targets.numel() == e.size(0)
+    assert bias is None or (bias.ndim == 1 and bias.size(0) == c.size(0))
+
+
 def _as_fp32(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     return None if bias is None else bias.to(torch.float32).contiguous()
 
@@ -41,6 +48,7 @@ def _as_fp32(bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
 def fp32_forward(e, c, bias, targets, valids, shift, softcap, target_offset) -> Tuple[torch.Tensor, torch.Tensor]:
     """``(lse, nll)`` of the valid rows: the log-sum-exp over the whole vocabulary, and what is left of it when the
     (soft-capped) logit of the target is taken off (all of it where the target is not a class of this shard)."""
+    _check(e, c, bias, targets, valids)
     lib = _hip.load()
     dev = e.device
     b = valids.numel() if valids is not None else e.size(0)
@@ -66,6 +74,8 @@ def fp32_forward(e, c, bias, targets, valids, shift, softcap, target_offset) -> 
 def fp32_backward(e, c, bias, lse, do, dlse, valids, targets, shift, target_offset, softcap, grad_scale,
                   want_de, want_dc, want_dbias):
     """(dE, dC, dBias) in fp32."""
+    _check(e, c, bias, targets, valids)
+    _hip.require_device(e.device, lse=lse, d_out=do, d_lse=dlse)
     lib = _hip.load()
     dev = e.device
     v, d = c.shape

@@ -766,3 +766,26 @@ def test_inside_a_compiled_function():
         outs.append((loss.detach(), x.grad, w.grad))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("on_host", ["c", "t", "bias"])
+def test_a_tensor_left_on_the_host_is_refused(dtype, on_host):
+    """With nothing ignored and with something, at the operator and at the launchers: an error before any launch."""
+    from cut_cross_entropy import fp32_path, linear_cross_entropy
+    from cut_cross_entropy.cce_lse_forward import loss_forward
+
+    e, c, t, bias = make_inputs(40, 96, 64, dtype, seed=3, bias=True)
+    for ignored in (False, True):
+        t = t.clone()
+        t[5] = IGNORE_INDEX if ignored else 0
+        x = {"c": c, "t": t, "bias": bias}
+        x = {k: v if k == on_host else v.cuda() for k, v in x.items()}
+        ed = e.cuda()
+        with pytest.raises(RuntimeError, match="on one device"):
+            linear_cross_entropy(ed, x["c"], x["t"], bias=x["bias"], impl="cce")
+        with pytest.raises(RuntimeError, match="on one device"):
+            if dtype == torch.float32:
+                fp32_path.fp32_forward(ed, x["c"], x["bias"], x["t"], None, 0, None, 0)
+            else:
+                loss_forward(ed, x["c"], x["bias"], x["t"], None, 0, None, 0, False)

@@ -68,6 +68,19 @@ def test_cce_without_gpu_fails_loudly():
         linear_cross_entropy(e, c, t, impl="cce")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("moved", ["c", "t", "bias"])
+def test_tensors_on_two_devices_are_refused_by_their_devices(dtype, moved):
+    """Before anything else is asked or launched: only the check on the devices says what is wrong."""
+    from cut_cross_entropy.cce import cce_linear_cross_entropy
+
+    e, c, t, bias = _small()
+    given = {"e": e.to(dtype), "c": c.to(dtype), "t": t, "bias": bias.to(dtype)}
+    given[moved] = given[moved].to("meta")
+    with pytest.raises(RuntimeError, match="on one device"):
+        cce_linear_cross_entropy(given["e"], given["c"], given["t"], bias=given["bias"])
+
+
 def test_shape_asserts():
     from cut_cross_entropy.torch_compile import torch_compile_linear_cross_entropy
 
