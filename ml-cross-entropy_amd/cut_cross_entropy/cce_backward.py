@@ -40,9 +40,9 @@ def _dz_budget(lib, B: int, V: int, D: int, de_16bit: bool) -> int:
 # recomputes its logits for each.  Above DENSE_WHEN_FLAGGED_ABOVE / slices a FILTERED backward runs unfiltered; an
 # unfiltered gradient is the exact one, so nothing is lost.  None switches the test off.
 #
-# The fraction is measured on the device (cce_count_flagged_cells over the forward's statistic) and the choice is
-# a function of the data alone, the same on every run: every filtered backward enqueues the count of ITS cells and
-# an asynchronous copy of it to pinned host memory; the FIRST backward of a (device, V, D, dtype) waits for its own
+# The fraction is measured on the device (cce_measure_flagged_cells over the forward's statistic) and the choice is
+# a function of the data alone, the same on every run: every filtered backward enqueues the count of ITS cells, which
+# the kernel leaves in pinned host memory; the FIRST backward of a (device, V, D, dtype) waits for its own
 # count (once per shape and process, as the reference's first call waits for its autotuner), every later one uses
 # the count of the backward before it, which has long arrived (a soft-max distribution moves slowly, so a decision
 # that lags one step is as good).  Identical inputs therefore take the same path, and give the same bits, on the
@@ -71,7 +71,12 @@ _OWNERSHIP_SLICE_COLS = 2304  # columns of D one ownership workgroup accumulates
 
 
 class _FlaggedMonitor:
-    """Fraction of flagged cells of the latest backward of one (device, V, D, dtype), and the path it chose."""
+    """Fraction of flagged cells of the latest backward of one (device, V, D, dtype), and the path it chose.
+
+    Kernels write ``host`` through its address, which the allocator of pinned memory does not hear of: a monitor lives as
+    long as the process, so that the word is nobody else's while a measurement is in flight."""
+
+    forgotten = False  # what was measured so far does not count any more
 
     def __init__(self, device: torch.device):
         self.scratch: dict = {}  # stream -> the word its measurements count in
@@ -88,6 +93,15 @@ class _FlaggedMonitor:
                 self.event.synchronize()
             self.fraction = int(self.host[0]) / self.pending_cells  # pinned host memory: a plain read
             self.pending_cells = 0
+
+    def forget(self) -> None:
+        self.fraction, self.dense, self.forgotten = None, False, True
+
+    def begin(self) -> None:
+        """Before a backward looks at the monitor: waits out a measurement from before a ``forget``, and drops it."""
+        if self.forgotten:
+            self.collect()
+            self.fraction, self.forgotten = None, False
 
     def measure(self, lib, tile_max, lse, B: int, V: int, filter_eps: float, dev: torch.device) -> None:
         stream = torch.cuda.current_stream(dev)
@@ -111,7 +125,8 @@ _monitors_lock = threading.Lock()
 def reset_backward_path_memory() -> None:
     """Forgets every measured fraction: the next filtered backward of each shape waits for its own count again."""
     with _monitors_lock:
-        _monitors.clear()
+        for mon in _monitors.values():
+            mon.forget()
 
 
 def _auto_dense_dz_budget(lib, B: int, V: int, D: int, de_16bit: bool, operand_bytes: int) -> Optional[int]:
@@ -149,6 +164,7 @@ def _filtered_backward_runs_dense(lib, tile_max, lse, B: int, V: int, D: int, fi
             return mon.dense if mon is not None else False
         if mon is None:
             mon = _monitors[key] = _FlaggedMonitor(dev)
+        mon.begin()
         first = mon.fraction is None and not mon.pending_cells
         if first:
             mon.measure(lib, tile_max, lse, B, V, filter_eps, dev)  # this backward's own cells ...

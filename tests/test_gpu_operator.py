@@ -789,3 +789,25 @@ def test_a_tensor_left_on_the_host_is_refused(dtype, on_host):
                 fp32_path.fp32_forward(ed, x["c"], x["bias"], x["t"], None, 0, None, 0)
             else:
                 loss_forward(ed, x["c"], x["bias"], x["t"], None, 0, None, 0, False)
+
+
+def test_forgetting_the_measured_fractions_starts_over(monkeypatch):
+    """After reset_backward_path_memory() the next filtered backward waits for the count of its own cells, as the first one
+    of a shape does, and takes the path that these ask for; the measurement that was in flight is not taken for it."""
+    from cut_cross_entropy import cce_backward as bw
+    from cut_cross_entropy import linear_cross_entropy
+
+    dense = []
+    real = bw._dense_backward
+    monkeypatch.setattr(bw, "_dense_backward", lambda *a, **k: (dense.append(1), real(*a, **k))[1])
+    g = torch.Generator().manual_seed(1)
+    flat = torch.randn((256, 192), generator=g).mul_(0.1).bfloat16().cuda()
+    c = torch.randn((16384, 192), generator=g).bfloat16().cuda().requires_grad_(True)
+    t = torch.randint(0, 16384, (256,), generator=g).cuda()
+    sure = c.detach()[t] * 4.0
+    for _ in range(3):
+        for e, want in ((flat, 1), (sure, 0)):
+            bw.reset_backward_path_memory()
+            dense.clear()
+            linear_cross_entropy(e.clone().requires_grad_(True), c, t, impl="cce").backward()
+            assert len(dense) == want

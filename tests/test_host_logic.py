@@ -157,3 +157,44 @@ def test_vocab_parallel_options_and_dtensor_message():
 
     o = VocabParallelOptions(3, 9)
     assert (o.start, o.stop, o.group, o.reduce_e_grad) == (3, 9, None, True)
+
+
+def test_forgotten_measurements_keep_their_word_until_it_has_been_written(monkeypatch):
+    """A kernel writes a monitor's pinned word by its address.  After reset_backward_path_memory() the word of a measurement
+    in flight stays held; the next backward waits for that measurement, drops it and takes its own."""
+    import gc
+    import weakref
+
+    from cut_cross_entropy import cce_backward as bw
+
+    class Event:
+        waited = 0
+
+        def query(self):
+            return False
+
+        def synchronize(self):
+            Event.waited += 1
+
+    def measure(mon, lib, tile_max, lse, B, V, filter_eps, dev):
+        assert Event.waited == (1 if not seen else Event.waited)  # the one in flight has been waited for
+        seen.append(1)
+        mon.host[0], mon.pending_cells = 1, 100
+
+    seen = []
+    monkeypatch.setattr(bw, "_monitors", {})
+    monkeypatch.setattr(bw, "FILTERED_BACKWARD_PATH", "auto")
+    monkeypatch.setattr(bw._FlaggedMonitor, "measure", measure)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    mon = object.__new__(bw._FlaggedMonitor)
+    mon.host, mon.event = torch.full((1,), 90, dtype=torch.int64), Event()
+    mon.pending_cells, mon.fraction, mon.dense, mon.scratch = 100, 0.9, True, {}
+    dev = torch.device("cuda", 0)
+    bw._monitors[(0, 512, 64, torch.bfloat16)] = mon
+    word = weakref.ref(mon.host)
+    del mon
+    bw.reset_backward_path_memory()
+    gc.collect()
+    assert word() is not None
+    assert bw._filtered_backward_runs_dense(None, None, None, 32, 512, 64, 1e-4, torch.bfloat16, dev) is False
+    assert len(seen) == 2 and Event.waited == 2  # its own cells, and those for the backward after it
