@@ -154,8 +154,9 @@ __global__ __launch_bounds__(256) void loss_rows_kernel(LossRowsParams p) {
   if (held)
     acc = RowDot<T, ALIGNED>::run(static_cast<const S*>(p.e) + row * p.stride_e, static_cast<const S*>(p.c) + t * p.stride_cv,
                                   p.stride_cd, p.d, lane);
+  // (a NaN row leaves (-inf, NaN) in its spans: the sum is scaled and never replaced, from a finite reference)
   const float top = wave_max(m);
-  sum = (m == -INFINITY) ? 0.0f : sum * exp2f(m - top);
+  sum *= exp2f(m - (top == -INFINITY ? 0.0f : top));
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     sum += __shfl_xor(sum, off, 64);

@@ -477,3 +477,29 @@ def test_forward_of_few_rows_keeps_three_stages(dtype, rows, width, classes):
         padded[:rows, :classes] = x
         top = padded.view(rb, 32, cb, 32).amax((1, 3))
         assert (cells.view(rb, cb) - top).abs().max() < 2e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("softcap", [None, 30.0, 50.0])
+@pytest.mark.parametrize("rows,width", [(40, 64), (70, 192), (300, 136), (300, 256), (130, 123)])
+def test_a_row_that_is_not_a_number_says_so(dtype, softcap, rows, width):
+    """A NaN in a row that counts: its log-sum-exp and its loss are NaN, also where its label is no class of the shard (the
+    loss is then the log-sum-exp alone); every other row has the values it has beside a row of zeros."""
+    from cut_cross_entropy import VocabParallelOptions, linear_cross_entropy
+
+    classes, bad = 3000, 33
+    e, c, t, _ = make_inputs(rows, classes, width, dtype, seed=rows)
+    e[bad] = 0.0
+    e, c, t = e.cuda(), c.cuda(), t.cuda()
+    spoilt = e.clone()
+    spoilt[bad, 7] = float("nan")
+    for shard in (None, VocabParallelOptions(0, classes)):
+        labels = t.clone()
+        if shard is not None:
+            labels[bad] = classes + 5
+        got, want = (linear_cross_entropy(x, c, labels, softcap=softcap, reduction="none", return_lse=True, impl="cce",
+                                          vocab_parallel_options=shard) for x in (spoilt, e))
+        others = torch.arange(rows, device="cuda") != bad
+        for x, y in zip(got, want):
+            assert torch.isfinite(y).all()
+            assert torch.isnan(x[bad]) and torch.equal(x[others], y[others])
