@@ -811,3 +811,26 @@ def test_forgetting_the_measured_fractions_starts_over(monkeypatch):
             dense.clear()
             linear_cross_entropy(e.clone().requires_grad_(True), c, t, impl="cce").backward()
             assert len(dense) == want
+
+
+@pytest.mark.parametrize("shift,ignored", [(0, 0.0), (0, 0.2), (1, 0.2)])
+def test_the_dense_implementation_needs_no_library(monkeypatch, shift, ignored):
+    """impl="torch_compile" on the GPU is made of tensor operations: it runs where the HIP library does not load, and under
+    function transforms, whose tensors have no storage."""
+    from cut_cross_entropy import _hip, linear_cross_entropy
+
+    def no_library():
+        raise AssertionError("the dense implementation asked for the HIP library")
+
+    monkeypatch.setattr(_hip, "load", no_library)
+    e, c, t, _ = make_inputs(48, 64, 32, torch.float32, seed=6, invalid_frac=ignored)
+    e, c, t = e.view(2, 24, 32).cuda().requires_grad_(True), c.cuda().requires_grad_(True), t.view(2, 24).cuda()
+
+    def loss_of(e, c, t):
+        return linear_cross_entropy(e, c, t, softcap=20.0, shift=shift, impl="torch_compile")
+
+    loss = loss_of(e, c, t)
+    loss.backward()
+    (g_e, g_c), value = torch.func.grad_and_value(loss_of, argnums=(0, 1))(e.detach(), c.detach(), t)
+    assert torch.allclose(value, loss.detach())
+    assert torch.allclose(g_e, e.grad, atol=1e-7) and torch.allclose(g_c, c.grad, atol=1e-7)
