@@ -323,7 +323,7 @@ int cce_loss_forward(const void* e, const void* c, const void* bias, const int32
  *
  * cce_fp32_forward: lse[b] and nll[b] as cce_loss_forward defines them; bias [v] float or NULL.
  * cce_fp32_backward: the unfiltered gradients, arguments as for cce_backward_dense: d_e [n_rows, d] is added to (row
- * stride ld_de), d_c [v, d] written (row stride ld_dc), d_bias [v] added to.
+ * stride ld_de), d_c [v, d] written (row stride ld_dc), d_bias [v] added to (sums of fp32 values whatever `terms` says).
  * Any alignment and width; stride_cd must be 1, else CCE_ERR_MISALIGNED.  `workspace` 256-byte aligned, of at least the
  * bytes that the size query names (copies of e and of a chunk of c in parts; dz of a chunk).
  */

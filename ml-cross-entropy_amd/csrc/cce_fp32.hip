@@ -112,6 +112,9 @@ static Fp32Forward plan_forward(int64_t b, int64_t v, int64_t d, int terms) {
 }
 
 // ---- backward
+// dz is stored in the parts that its products read; all three of them where its column sums are wanted, whatever `terms`
+// says, since those are sums of fp32 values and no products.  The workspace has room for that.
+constexpr int kDzParts = 3;
 struct Fp32Backward {
   int parts;
   int64_t part_d, rows, rows_pad, unit;
@@ -135,7 +138,7 @@ static Fp32Backward plan_backward(int64_t b, int64_t v, int64_t d, int terms) {
   f.dc_slots = static_cast<int>((f.rows_pad + f.dc_len - 1) / f.dc_len);
   f.e_bytes = align256(f.rows_pad * row_bytes);
   f.c_bytes = align256(round_up(std::min(f.unit, v), 256) * row_bytes);
-  f.dz_bytes = align256(f.rows_pad * f.parts * cls * 2);
+  f.dz_bytes = align256(f.rows_pad * kDzParts * cls * 2);
   f.de_slot_bytes = f.de_slots > 1 ? align256(f.de_slots * f.rows * f.part_d * 4) : 0;
   f.dc_slot_bytes = f.dc_slots > 1 ? align256(f.dc_slots * std::min(f.unit, v) * f.part_d * 4) : 0;
   return f;
@@ -239,6 +242,7 @@ extern "C" int cce_fp32_backward(const float* e, const float* c, const float* bi
   float* const de_slots = reinterpret_cast<float*>(take(f.de_slot_bytes));
   float* const dc_slots = reinterpret_cast<float*>(take(f.dc_slot_bytes));
   const int64_t ld = f.parts * f.part_d;
+  const int stored = d_bias != nullptr ? kDzParts : f.parts;
   const bool de_cut = d_e != nullptr && f.de_slots > 1, dc_cut = d_c != nullptr && f.dc_slots > 1;
   const bool out_vec = d % 8 == 0 && (d_e == nullptr || (aligned16(d_e) && ld_de % 4 == 0)) &&
                        (d_c == nullptr || (aligned16(d_c) && ld_dc % 4 == 0));
@@ -257,14 +261,14 @@ extern "C" int cce_fp32_backward(const float* e, const float* c, const float* bi
       if (st != CCE_OK) return st;
       st = dz_terms_launch(e_parts, ld, c_parts, ld, bias != nullptr ? bias + v0 : nullptr, lse + r0,
                            d_out_is_scalar ? d_out : d_out + moved, d_out_is_scalar, d_lse != nullptr ? d_lse + moved : nullptr, ids,
-                           targets + moved, dz_parts, cls_pad, n_rows - moved, rows, rows_pad, cls, f.part_d, terms, f.parts,
+                           targets + moved, dz_parts, cls_pad, n_rows - moved, rows, rows_pad, cls, f.part_d, terms, stored,
                            grad_scale, shift, target_offset + v0, softcap, stream);
       if (st != CCE_OK) return st;
       float* const de = d_e == nullptr ? nullptr : (de_cut ? de_slots : d_e + moved * ld_de);
       float* const dc = d_c == nullptr ? nullptr : (dc_cut ? dc_slots : d_c + v0 * ld_dc);
       st = terms_products_launch(dz_parts, cls_pad, c_parts, ld, e_parts, ld, de_cut ? nullptr : ids, de, de_cut ? f.part_d : ld_de,
                                  de_cut, de_cut && v0 == 0, rows * f.part_d, de_len, dc, dc_cut ? f.part_d : ld_dc, r0 > 0,
-                                 cls * f.part_d, dc_len, out_vec, rows, rows_pad, cls, cls_pad, d, f.part_d, terms, f.parts, stream);
+                                 cls * f.part_d, dc_len, out_vec, rows, rows_pad, cls, cls_pad, d, f.part_d, terms, stored, stream);
       if (st != CCE_OK) return st;
       if (dc_cut) {
         const int ranges = static_cast<int>((rows_pad + dc_len - 1) / dc_len);
@@ -272,7 +276,7 @@ extern "C" int cce_fp32_backward(const float* e, const float* c, const float* bi
         if (st != CCE_OK) return st;
       }
       if (d_bias != nullptr) {
-        st = dz_colsum_launch(dz_parts, cls_pad, f.parts, rows, cls, d_bias + v0, CCE_DTYPE_BF16, stream);
+        st = dz_colsum_launch(dz_parts, cls_pad, stored, rows, cls, d_bias + v0, CCE_DTYPE_BF16, stream);
         if (st != CCE_OK) return st;
       }
     }

@@ -503,3 +503,29 @@ def test_a_row_that_is_not_a_number_says_so(dtype, softcap, rows, width):
         for x, y in zip(got, want):
             assert torch.isfinite(y).all()
             assert torch.isnan(x[bad]) and torch.equal(x[others], y[others])
+
+
+@pytest.mark.parametrize("shape", [(1, 700, 64), (300, 2000, 200), (3000, 100, 72)])
+def test_fp32_column_sums_keep_their_bits_with_three_terms(shape):
+    """dBias is a sum of fp32 values and no product: with operands of 8 significant bits, whose logits three terms give
+    exactly, it is bit for bit what six terms give."""
+    lib = _lib()
+    N, V, D = shape
+    g = torch.Generator(device="cuda").manual_seed(N)
+    e = torch.randn((N, D), generator=g, device="cuda").bfloat16().float()
+    c = (torch.randn((V, D), generator=g, device="cuda") / D**0.5).bfloat16().float()
+    t = torch.randint(0, V, (N,), generator=g, device="cuda")
+    w = torch.rand((N,), generator=g, device="cuda") + 0.5
+    lse = torch.logsumexp((e.double() @ c.double().T), 1).float()
+    p = lambda x: x.data_ptr()
+    sums = []
+    for terms in (6, 3):
+        n_ws = lib.cce_fp32_backward_workspace_bytes(N, V, D, terms)
+        buf = torch.full((n_ws // 4 + 64,), float("nan"), device="cuda")
+        ws = (buf.data_ptr() + 255) // 256 * 256
+        de, dc, db = torch.zeros((N, D), device="cuda"), torch.empty((V, D), device="cuda"), torch.zeros((V,), device="cuda")
+        st = lib.cce_fp32_backward(p(e), p(c), None, p(lse), p(w), 0, None, None, p(t), p(de), p(dc), p(db), ws, n_ws, N, N, V, D,
+                                   D, D, 1, D, D, 1.0, 0, 0, 0.0, terms, torch.cuda.current_stream().cuda_stream)
+        assert st == 0, lib.cce_error_string(st)
+        sums.append(db)
+    assert torch.isfinite(sums[0]).all() and sums[0].abs().max() > 0 and torch.equal(*sums)
