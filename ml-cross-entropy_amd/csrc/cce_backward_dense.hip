@@ -790,8 +790,8 @@ static DensePlan dense_plan(int64_t b, int64_t v, int64_t d, bool g16, int64_t m
 // ---- the products of one chunk of classes with operands and dz in bf16 parts (cce_fp32.hip) ---------------------
 // The walk over the classes for a dz of `dz_bytes_per_class` and a copy of C of `c_bytes_per_class`, either at most
 // `most_bytes`, in chunks that are multiples of 256 classes; the reductions are cut as in cce_backward_dense.
-TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class, int64_t c_bytes_per_class,
-                     int64_t most_bytes, bool cut_dc) {
+static TermsPlan terms_plan_uncached(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class,
+                                     int64_t c_bytes_per_class, int64_t most_bytes, bool cut_dc) {
   TermsPlan pl = {256, 1, 1};
   static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   const int64_t v_pad = (v + 255) / 256 * 256;
@@ -824,6 +824,31 @@ TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_byte
     }
   }
   return pl;
+}
+
+// (asked by the size query and again by the call, with every step of a training loop, like dense_plan: 7 - 50 us each)
+TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class, int64_t c_bytes_per_class,
+                     int64_t most_bytes, bool cut_dc) {
+  struct Memo {
+    int64_t b, v, d, dz, c, most;
+    int terms, cus;
+    bool cut_dc;
+    TermsPlan answer;
+  };
+  constexpr int kMemos = 8;
+  static thread_local Memo memo[kMemos] = {};
+  static thread_local int next_slot = 0;
+  const int cus = compute_units();
+  for (int i = 0; i < kMemos; ++i) {
+    const Memo& m = memo[i];
+    if (m.b == b && m.v == v && m.d == d && m.dz == dz_bytes_per_class && m.c == c_bytes_per_class && m.most == most_bytes &&
+        m.terms == terms && m.cus == cus && m.cut_dc == cut_dc)
+      return m.answer;
+  }
+  const TermsPlan answer = terms_plan_uncached(b, v, d, terms, dz_bytes_per_class, c_bytes_per_class, most_bytes, cut_dc);
+  memo[next_slot] = {b, v, d, dz_bytes_per_class, c_bytes_per_class, most_bytes, terms, cus, cut_dc, answer};
+  next_slot = (next_slot + 1) % kMemos;
+  return answer;
 }
 
 int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t* c_parts, int64_t ld_c, const uint16_t* e_parts,

@@ -132,3 +132,29 @@ def test_plans_of_whole_reductions_do_not_go_by_the_estimate_for_cut_ones(sizes,
     assert fixed == a256((v if by_rows else b) * d * 2)
     dz = lib.cce_backward_dense_workspace_bytes(b, v, d, 1, budget) - fixed
     assert dz == a256((unit * a256(v) if by_rows else unit * b) * 2)
+
+
+def test_a_plan_of_the_fp32_backward_is_searched_once():
+    """The size query and the call ask for the plan of the same sizes, every step of a training loop again: the answer to a
+    question asked before costs a small part of a search."""
+    import time
+
+    lib = _lib()
+    b, v, d = 39665, 153856, 160
+
+    def seconds(sizes):
+        best = 1.0
+        for _ in range(5):
+            start = time.perf_counter()
+            for n in sizes:
+                lib.cce_fp32_backward_workspace_bytes(n, v, d, 6)
+            best = min(best, time.perf_counter() - start)
+        return best
+
+    searched, known = seconds(range(b, b + 200)), seconds([b] * 200)
+    assert known < searched / 4, (known, searched)
+    # ... and is the answer of a search of its own
+    answer = lib.cce_fp32_backward_workspace_bytes(b, v, d, 6)
+    for n in range(1, 20):
+        lib.cce_fp32_backward_workspace_bytes(b + n, v, d, 6)
+    assert lib.cce_fp32_backward_workspace_bytes(b, v, d, 6) == answer
