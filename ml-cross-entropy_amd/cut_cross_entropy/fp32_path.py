@@ -80,15 +80,11 @@ def fp32_backward(e, c, bias, lse, do, dlse, valids, targets, shift, target_offs
     dev = e.device
     v, d = c.shape
     b = lse.numel()
-    de = torch.zeros_like(e) if want_de else None  # added to; rows that do not count stay zeros
-    # written whole, unless there is no valid row; rows with gaps between them keep their layout
+    # packed, whatever the strides of e and c (those of a single row say nothing about where the next one would be)
+    de = torch.zeros(e.shape, dtype=e.dtype, device=dev) if want_de else None  # added to; rows that do not count stay zeros
     dc = None
-    if want_dc:
-        dc = torch.empty_like(c)
-        if dc.stride(1) != 1:
-            dc = torch.empty((v, d), dtype=c.dtype, device=dev)
-        if b == 0:
-            dc.zero_()
+    if want_dc:  # written whole, unless there is no valid row
+        dc = (torch.empty if b else torch.zeros)((v, d), dtype=c.dtype, device=dev)
     dbias = torch.zeros((v,), dtype=torch.float32, device=dev) if want_dbias else None
     if b == 0 or not (want_de or want_dc or want_dbias):
         return de, dc, dbias

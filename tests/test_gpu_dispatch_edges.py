@@ -529,3 +529,27 @@ def test_fp32_column_sums_keep_their_bits_with_three_terms(shape):
         assert st == 0, lib.cce_error_string(st)
         sums.append(db)
     assert torch.isfinite(sums[0]).all() and sums[0].abs().max() > 0 and torch.equal(*sums)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("which", ["e", "c", "both"])
+@pytest.mark.parametrize("width", [5, 8, 72, 128])
+def test_a_single_row_with_a_stride_of_its_own(dtype, which, width):
+    """One row of e, or one class, whose stride says nothing (the transpose of a [D, 1] column): as if it were packed."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    N, V = (1 if which in ("e", "both") else 9), (1 if which in ("c", "both") else 300)
+    e, c, _, _ = make_inputs(N, V, width, dtype, seed=width)
+    t = torch.randint(0, V, (N,), generator=torch.Generator().manual_seed(1)).cuda()
+
+    def column(x, moved):
+        return torch.as_strided(x.cuda().flatten().clone(), x.shape, (1, 1)) if moved else x.cuda()
+
+    results = []
+    for moved in (False, True):
+        ed, cd = column(e, moved and which != "c").requires_grad_(True), column(c, moved and which != "e").requires_grad_(True)
+        loss = linear_cross_entropy(ed, cd, t, impl="cce_exact")
+        loss.backward()
+        results.append((loss.detach(), ed.grad, cd.grad))
+    for a, b in zip(*results):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
