@@ -197,17 +197,16 @@ int cce_measure_flagged_cells(const float* tile_max, const float* lse, int64_t b
  * d_c += dz^T . e (:289-302), through atomics -- is not done here: with every dz in play they are dense
  * matrix products (d_e[rows] += dz . c, d_c = dz^T . e[rows], d_bias = column sums of dz) on the [b, v] matrix
  * this function fills, chunk of the vocabulary by chunk.  cce_backward_dense runs dz and products in one call,
- * cce_backward_products the products alone.
+ * cce_backward_products the products alone: these two stand by themselves, for callers of this library who put a step of
+ * their own between dz and its products; the Python operator calls cce_backward_dense and cce_fp32_backward.
  *
  *   c, bias    the chunk's rows: v classes starting at the caller's offset
  *   lse        [b] float, the LSE over the WHOLE vocabulary
- *   dz         [b, ldz] in `dtype`, or float when dz_is_fp32 (for callers that pass fp32 matrices split
- *              into 16-bit parts along d and want the gradient at that accuracy); row i = valid row i
+ *   dz         [b, ldz] in `dtype`, or float when dz_is_fp32 (not rounded to the input type); row i = valid row i
  *              (rows compacted through valids), ldz >= v
  *   target_offset  first class of the chunk (plus the shard start, if any)
  * Needs 16-byte aligned e, c, dz, unit stride_cd, row strides that are multiples of 8, ldz a multiple of 8
- * (4 when dz_is_fp32) and d a
- * multiple of 64; anything else returns CCE_ERR_MISALIGNED and the caller uses cce_backward.
+ * (4 when dz_is_fp32) and d a multiple of 64; anything else returns CCE_ERR_MISALIGNED and the caller uses cce_backward.
  */
 int cce_backward_dz(const void* e, const void* c, const void* bias,
                     const float* lse, const float* d_out, int d_out_is_scalar, const float* d_lse,
@@ -272,9 +271,8 @@ int cce_backward_dense(const void* e, const void* c, const void* bias,
                        float softcap, int dtype, void* stream);
 
 /*
- * The two matrix products of one vocabulary chunk on their own, for a caller that forms dz itself and wants
- * fp32 results: the fp32 path of the Python host splits dz, c and e into 16-bit parts and sums the cross terms
- * with one call per term.  The products of the reference's kernel (cut_cross_entropy/cce_backward.py:262-275
+ * The two matrix products of one vocabulary chunk on their own, for a caller that forms dz itself (or changes what
+ * cce_backward_dz wrote) and wants fp32 results.  The products of the reference's kernel (cut_cross_entropy/cce_backward.py:262-275
  * and :289-302) as 16-bit-in, fp32-accumulate matrix products on the tiles cce_backward_dense runs, both in one
  * launch:
  *     d_e[i, :] += sum_v dz[i, v] c[v, :]                    i < b   (d_e: a [b, d] float accumulator, row stride ld_de)

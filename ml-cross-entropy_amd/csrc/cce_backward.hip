@@ -1355,7 +1355,8 @@ __global__ __launch_bounds__(256) void owner_merge_kernel(BwdParams p) {
 // workgroups per compute unit, which walk the row groups, eight cells in flight per thread, and with `answer` ONE addition
 // for cells and finished workgroups together, which needs no fence in between.  At 2048 row groups of 4752 cells a workgroup
 // per group took 36 us, 64 with an addition for each of the two; 22 us so.
-constexpr int kFlaggedCellBits = 37;  // 2^37 cells of 4 bytes are more than the card holds; 2^27 row groups more than 2^31 rows
+// 2^37 cells of 4 bytes are more than the card holds; the bits above count workgroups, two per compute unit at most
+constexpr int kFlaggedCellBits = 37;
 __global__ __launch_bounds__(256) void flagged_cells_kernel(const float* tile_max, const float* lse, int64_t b, int ntg,
                                                             int stat_cols, float log_eps, unsigned long long* count,
                                                             unsigned long long* answer) {
@@ -1429,9 +1430,11 @@ static int64_t kept_bits_bytes(int64_t b, int64_t v) { return ((b + 31) / 32) * 
 
 static int owner_slices(int64_t d) { return static_cast<int>((d + kMaxChunks * kStageCols - 1) / (kMaxChunks * kStageCols)); }
 
-// Workgroups per row group (and slice of D) of the dE pass: as many as fill the chip, at most 16 (a row group has 8 trips
-// and more: its 32 rows have that many labels), and no more slots than half of C takes (E [307, 5120] x C [131072, 5120]:
-// 30 workgroups took 745 us, 240 take 174 and 11 to put the slots together).
+// Workgroups per row group (and slice of D) of the dE pass: as many as fill the chip, at most 16, and no more slots than half
+// of C takes (E [307, 5120] x C [131072, 5120]: 30 workgroups took 745 us, 240 take 174 and 11 to put the slots together).
+// 16, since 32 rows whose labels all lie in sub-tiles of their own make eight trips and what else survives makes more; equal
+// labels, labels side by side, a short last row group and labels of other shards make fewer, and a workgroup without a trip
+// walks the statistic and leaves a slot of zeros.
 static int owner_parts(int64_t b, int64_t v, int64_t d) {
   if (b <= 0 || d <= 0) return 1;
   const int64_t groups = (b + 31) / 32 * owner_slices(d);

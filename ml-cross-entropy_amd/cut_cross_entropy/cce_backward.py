@@ -55,7 +55,8 @@ FILTERED_BACKWARD_PATH = "auto"
 #     max(DENSE_WORKSPACE_LIMIT_BYTES, DENSE_WORKSPACE_LIMIT_OPERANDS x (bytes of E + bytes of C))
 # of workspace (the dz buffer, plus the 16-bit compensation buffer of the gradient that is carried between launches:
 # [B, D] for dE, or [V, D] for dC where rows outnumber classes two to one): the ownership kernels need well
-# under 16 MB, and a caller who picked a filtered preset did not ask for more.  The defaults, 256 MB and 1.0, say:
+# under 16 MB (with few rows up to half the bytes of C on top, fp32 slots for workgroups that share a row group: 53 MB at
+# 307 rows of 5120 columns against 131072 classes), and a caller who picked a filtered preset did not ask for more.  The defaults, 256 MB and 1.0, say:
 # never more than the operands the caller already holds take themselves, and 256 MB where they are smaller (the
 # second term matters when rows are many: at E [65536, 3584] x C [19008, 3584] the compensation buffer alone is
 # 448 MB and the operands are 578 MB; the ownership kernels take 167 ms there, the unfiltered path 22 - 30).  The dz chunk

@@ -13,7 +13,7 @@ produces, so the backward is the unfiltered one.
 ``torch.set_float32_matmul_precision``: "highest" (the default) takes the six terms above; with "high" or
 "medium" the caller has asked for fast fp32 products (the reference then lets Triton use tf32, 10 mantissa
 bits, cce_lse_forward.py:129-131) and logits and gradient products are formed from the three leading terms
-hi*hi + hi*mid + mid*hi (16 bits), half the work.
+hi*hi + hi*mid + mid*hi (16 bits), half the work.  dBias is no product: it is a sum of fp32 values either way.
 """
 
 from typing import Optional, Tuple
