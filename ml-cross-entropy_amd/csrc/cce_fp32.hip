@@ -114,7 +114,7 @@ static Fp32Forward plan_forward(int64_t b, int64_t v, int64_t d, int terms) {
 // ---- backward
 // dz is stored in the parts that its products read; all three of them where its column sums are wanted, whatever `terms`
 // says, since those are sums of fp32 values and no products.  The workspace has room for that.
-constexpr int kDzParts = 3;
+constexpr int kAllParts = 3;
 struct Fp32Backward {
   int parts;
   int64_t part_d, rows, rows_pad, unit;
@@ -138,7 +138,7 @@ static Fp32Backward plan_backward(int64_t b, int64_t v, int64_t d, int terms) {
   f.dc_slots = static_cast<int>((f.rows_pad + f.dc_len - 1) / f.dc_len);
   f.e_bytes = align256(f.rows_pad * row_bytes);
   f.c_bytes = align256(round_up(std::min(f.unit, v), 256) * row_bytes);
-  f.dz_bytes = align256(f.rows_pad * kDzParts * cls * 2);
+  f.dz_bytes = align256(f.rows_pad * kAllParts * cls * 2);
   f.de_slot_bytes = f.de_slots > 1 ? align256(f.de_slots * f.rows * f.part_d * 4) : 0;
   f.dc_slot_bytes = f.dc_slots > 1 ? align256(f.dc_slots * std::min(f.unit, v) * f.part_d * 4) : 0;
   return f;
@@ -242,7 +242,7 @@ extern "C" int cce_fp32_backward(const float* e, const float* c, const float* bi
   float* const de_slots = reinterpret_cast<float*>(take(f.de_slot_bytes));
   float* const dc_slots = reinterpret_cast<float*>(take(f.dc_slot_bytes));
   const int64_t ld = f.parts * f.part_d;
-  const int stored = d_bias != nullptr ? kDzParts : f.parts;
+  const int stored = d_bias != nullptr ? kAllParts : f.parts;
   const bool de_cut = d_e != nullptr && f.de_slots > 1, dc_cut = d_c != nullptr && f.dc_slots > 1;
   const bool out_vec = d % 8 == 0 && (d_e == nullptr || (aligned16(d_e) && ld_de % 4 == 0)) &&
                        (d_c == nullptr || (aligned16(d_c) && ld_dc % 4 == 0));
