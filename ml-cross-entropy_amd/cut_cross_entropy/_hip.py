@@ -170,12 +170,12 @@ def require_gpu_tensor(name: str, t: torch.Tensor) -> None:
         )
 
 
-def require_device(device: torch.device, **tensors: Optional[torch.Tensor]) -> None:
+def require_device(device: torch.device, *tensors: Optional[torch.Tensor]) -> None:
     """Every tensor lies on ``device``: asked before an address is handed on, since a kernel that reads another device's
     memory, or the host's, faults."""
-    for name, t in tensors.items():
+    for t in tensors:
         if t is not None and t.device != device:
-            raise RuntimeError(f"{name} is on {t.device}, e on {device}: all tensors have to be on one device")
+            raise RuntimeError(f"a tensor of shape {tuple(t.shape)} is on {t.device}, e on {device}: all have to be on one device")
 
 
 def current_stream_ptr(device: torch.device) -> int:

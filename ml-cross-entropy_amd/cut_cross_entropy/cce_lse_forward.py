@@ -82,9 +82,9 @@ def loss_forward(
     row's target (``indexed_neg_dot_forward_kernel``), merged and added up by one kernel."""
     assert e.ndim == 2 and c.ndim == 2 and e.is_contiguous()
     assert e.shape[1] == c.shape[1], "Incompatible dimensions"
-    _hip.require_gpu_tensor("e", e)
     dev = e.device
-    _hip.require_device(dev, c=c, bias=bias, targets=targets, valids=valids)
+    _hip.require_device(dev, c, bias, targets, valids)
+    _hip.require_gpu_tensor("e", e)
     assert c.dtype == e.dtype
     assert targets.numel() == e.shape[0]
     V, D = c.shape

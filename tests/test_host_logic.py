@@ -71,14 +71,19 @@ def test_cce_without_gpu_fails_loudly():
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("moved", ["c", "t", "bias"])
 def test_tensors_on_two_devices_are_refused_by_their_devices(dtype, moved):
-    """Before anything else is asked or launched: only the check on the devices says what is wrong."""
-    from cut_cross_entropy.cce import cce_linear_cross_entropy
+    """The launchers, which hand on addresses, ask for the devices before anything else: also where there is no GPU."""
+    from cut_cross_entropy.cce_lse_forward import loss_forward
+    from cut_cross_entropy.fp32_path import fp32_forward
 
     e, c, t, bias = _small()
-    given = {"e": e.to(dtype), "c": c.to(dtype), "t": t, "bias": bias.to(dtype)}
+    given = {"e": e.to(dtype).flatten(0, -2), "c": c.to(dtype), "t": t.flatten(), "bias": bias.to(dtype)}
     given[moved] = given[moved].to("meta")
+    e, c, t, bias = given.values()
     with pytest.raises(RuntimeError, match="on one device"):
-        cce_linear_cross_entropy(given["e"], given["c"], given["t"], bias=given["bias"])
+        if dtype == torch.float32:
+            fp32_forward(e, c, bias, t, None, 0, None, 0)
+        else:
+            loss_forward(e, c, bias, t, None, 0, None, 0, False)
 
 
 def test_shape_asserts():
