@@ -170,12 +170,20 @@ def require_gpu_tensor(name: str, t: torch.Tensor) -> None:
         )
 
 
-def require_device(device: torch.device, *tensors: Optional[torch.Tensor]) -> None:
-    """Every tensor lies on ``device``: asked before an address is handed on, since a kernel that reads another device's
-    memory, or the host's, faults."""
-    for t in tensors:
-        if t is not None and t.device != device:
-            raise RuntimeError(f"a tensor of shape {tuple(t.shape)} is on {t.device}, e on {device}: all have to be on one device")
+def require_one_gpu(e: torch.Tensor, *others: Optional[torch.Tensor]) -> None:
+    """``e`` lies on a GPU and every other tensor on the same one: asked before an address is handed on, since a kernel that
+    reads another device's memory, or the host's, faults."""
+    index = e.get_device()  # (an index compares in half the time of a device; -1: not on a GPU)
+    if index >= 0:
+        for t in others:
+            if t is not None and t.get_device() != index:
+                break
+        else:
+            return
+    for t in others:
+        if t is not None and t.device != e.device:
+            raise RuntimeError(f"a tensor of shape {tuple(t.shape)} is on {t.device}, e on {e.device}: all have to be on one device")
+    require_gpu_tensor("e", e)
 
 
 def current_stream_ptr(device: torch.device) -> int:

@@ -83,8 +83,7 @@ def loss_forward(
     assert e.ndim == 2 and c.ndim == 2 and e.is_contiguous()
     assert e.shape[1] == c.shape[1], "Incompatible dimensions"
     dev = e.device
-    _hip.require_device(dev, c, bias, targets, valids)
-    _hip.require_gpu_tensor("e", e)
+    _hip.require_one_gpu(e, c, bias, targets, valids)
     assert c.dtype == e.dtype
     assert targets.numel() == e.shape[0]
     V, D = c.shape

@@ -35,8 +35,7 @@ def _workspace(nbytes: int, dev: torch.device) -> Tuple[torch.Tensor, int]:
 
 
 def _check(e, c, bias, targets, valids) -> None:
-    _hip.require_device(e.device, c, bias, targets, valids)
-    _hip.require_gpu_tensor("e", e)
+    _hip.require_one_gpu(e, c, bias, targets, valids)
     assert targets.numel() == e.size(0)
     assert bias is None or (bias.ndim == 1 and bias.size(0) == c.size(0))
 
@@ -75,7 +74,7 @@ def fp32_backward(e, c, bias, lse, do, dlse, valids, targets, shift, target_offs
                   want_de, want_dc, want_dbias):
     """(dE, dC, dBias) in fp32."""
     _check(e, c, bias, targets, valids)
-    _hip.require_device(e.device, lse, do, dlse)
+    _hip.require_one_gpu(e, lse, do, dlse)
     lib = _hip.load()
     dev = e.device
     v, d = c.shape
