@@ -156,7 +156,10 @@ __global__ __launch_bounds__(256) void loss_rows_kernel(LossRowsParams p) {
                                   p.stride_cd, p.d, lane);
   // (a NaN row leaves (-inf, NaN) in its spans: the sum is scaled and never replaced, from a finite reference)
   const float top = wave_max(m);
-  sum *= exp2f(m - (top == -INFINITY ? 0.0f : top));
+  {
+#pragma clang fp contract(off)  // rounded like the sums of the other lanes that it is added to
+    sum = sum * exp2f(m - (top == -INFINITY ? 0.0f : top));
+  }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     sum += __shfl_xor(sum, off, 64);
