@@ -64,7 +64,8 @@ const char* cce_error_string(int status);
  * ceil(b / CCE_STAT_ROWS) * ceil(v / CCE_STAT_COLS). */
 int64_t cce_tile_stat_elems(int64_t b, int64_t v);
 
-/* Scratch bytes cce_lse_forward needs (split-vocabulary partial max / sum-exp). */
+/* Scratch bytes for cce_lse_forward (split-vocabulary partial max / sum-exp).  With a little less it may still run, in
+ * larger blocks of rows. */
 int64_t cce_lse_forward_workspace_bytes(int64_t b, int64_t v, int64_t d);
 
 /*

@@ -620,7 +620,6 @@ struct DmaLogitTile16 {
   static constexpr int RING = FEW ? 3 : 2;
   static constexpr int STAGE_BYTES = FEW ? (TILE_V + TILE_T / 2) * kDmaRowBytes : Base::STAGE_BYTES;
   static constexpr int LDS_BYTES = RING * STAGE_BYTES;
-  static_assert(FEW || LDS_BYTES == Base::LDS_BYTES, "two stages");
   using vec8 = typename Elem<T>::vec8;
 
   static __device__ __forceinline__ int wv_of(int wave) { return FEW ? wave % NWV : wave / NWT; }
@@ -727,23 +726,29 @@ struct DmaLogitTile16 {
   //   READ  the fragments of the next step from rd_c / rd_e (ring stage + this lane's chunk): class fragment vi
   //         into a[vi] once the last MFMA that uses the old one is issued, the token fragments into bn[];
   //   LOAD  all loads of a later stage (columns kc .. / ke ..) into ring stage `ld_stage`.
-  // SYNC (the step on the second half of a stage): after the first WT MFMAs, which need nothing new, this wave
+  // SYNC (the step on the second half of a stage): after the first four MFMAs, which need nothing new, this wave
   // waits for its own loads of the next stage and for the fragment reads it still has in flight, then the
   // barrier: from there on the next stage may be read and the stage this step computes on (every wave holds
   // its last fragments of it) may be overwritten.  Reads and loads of such a step all come after the barrier.
   // (With the barrier between the steps instead, every wave met it with its last fragment read just issued and
   // the compute units idled a sixth of the time.)
-  static constexpr int kSyncAt = WT;  // MFMAs of a SYNC step issued before the barrier
+  static constexpr int kSyncAt = 4;  // MFMAs of a SYNC step issued before the barrier
   static constexpr int kSlots = WV * WT;
   static constexpr int a_slot(bool sync, int vi) {
     const int natural = vi * WT + WT - 1;  // the last MFMA that reads a[vi]
+    if (WV == 4) return natural;           // 5, 11, 17, 23
     return (sync && natural < kSyncAt + 1 + 2 * vi) ? kSyncAt + 1 + 2 * vi : natural;
   }
   static constexpr int b_slot(bool sync, int t) {
+    if (WV == 4) return (sync ? 7 : 1) + 6 * (t / 2) + 2 * (t % 2);  // 7, 9, 13, 15, 19, 21 or 1, 3, 7, 9, 13, 15
     return sync ? kSyncAt + 5 + t * ((kSlots - kSyncAt - 8) / WT & ~1) : 1 + t * (kSlots / WT);
   }
-  static constexpr int load_slot(int j) { return j < 6 ? kSyncAt + 2 + 4 * j : kSlots - 4 + 2 * (j - 6); }
-  static_assert(WV == 8 && WT == 4 && NQ <= 8, "the slot tables above are laid out for 8 x 4 blocks and 8 loads");
+  static constexpr int load_slot(int j) {
+    if (WV == 4) return kSyncAt + 2 + 2 * j;  // 6, 8, .. 18
+    return j < 6 ? kSyncAt + 2 + 4 * j : kSlots - 4 + 2 * (j - 6);
+  }
+  static_assert((WV == 8 && WT == 4 && NQ <= 8) || (WV == 4 && WT == 6 && NQ <= 7 && !FEW),
+                "the slot tables above are laid out for 8 x 4 blocks and 8 loads, or 4 x 6 and 7");
 
   // ZERO (the first step of a tile): the accumulators start from the instruction's constant zero instead of being
   // cleared beforehand (128 register writes per lane and tile; the copy of the first stage this takes costs a
@@ -947,7 +952,11 @@ inline int compute_units() {
 // E [65536, 3584] x C [152064, 3584] (1, 2, 4, 8, 16 spans: 70.8, 62.5, 53.9, 56.8, 59.4 ms).
 // Up to 64 spans are weighed, and as many as fill the chip where the row blocks are fewer than that takes: one row
 // block against 256000 classes of 2304 columns is 847 us in 64 spans (a quarter of the compute units) and 262 us in 250 (4.5 TB/s).
-inline int choose_span_count(int nrb, int nvt) {
+struct SpanChoice {
+  int count;
+  double cost;  // of the launch, in times of one tile
+};
+inline SpanChoice choose_spans(int nrb, int nvt) {
   const int num_cu = compute_units();  // (the size query and the launch must see the same device)
   int best = 1;
   double best_cost = 1e300;
@@ -965,8 +974,9 @@ inline int choose_span_count(int nrb, int nvt) {
       best = s;
     }
   }
-  return best;
+  return {best, best_cost};
 }
+inline int choose_span_count(int nrb, int nvt) { return choose_spans(nrb, nvt).count; }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -1,7 +1,7 @@
 // cce_lse_forward: fused (E . C^T) -> soft-cap -> online log-sum-exp for gfx950.
 //
 // Work decomposition.  The (row-block, vocabulary) plane is cut into items: one item is a block
-// of 256 valid rows times a contiguous span of 256-wide vocabulary tiles.  A workgroup (8 waves,
+// of 256 valid rows (or 192: best_blocks) times a contiguous span of 256-wide vocabulary tiles.  A workgroup (8 waves,
 // 2 x 4, each wave 128 classes x 64 rows of accumulators) owns one item, walks its span tile by
 // tile and keeps, per row, a running (max, sum-exp) pair in registers in the log2 domain.  At the
 // end the pairs of the two lane halves and of the two wave rows are merged and written as one
@@ -12,6 +12,7 @@
 // into (xcd, slot) and items are numbered so that one XCD works on neighbouring spans of the
 // same few row blocks: its L2 then serves each E block to several workgroups and each C tile to
 // several row blocks.
+#include <algorithm>
 #include <atomic>
 
 #include "cce_dense.h"
@@ -300,6 +301,16 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward_kernel(LseFwdParam
 // ---------------------------------------------------------------------------------------------
 constexpr int kF16WV = 8, kF16WT = 4;  // 16-row blocks per wave: 128 classes x 64 rows
 constexpr int kF16RunBytes = kF16WT * kFwdThreads * static_cast<int>(sizeof(float2));  // running (max, sum) pairs
+constexpr int kFwdMidRows = 192;
+// Who holds what of a tile of ROWS x 256: 2 x 4 waves of 128 classes x 64 rows, or 4 x 2 of 64 x 96.
+template <int ROWS>
+struct Fwd16Shape {
+  static_assert(ROWS == kFwdTile || ROWS == kFwdMidRows, "rows of a tile");
+  static constexpr bool MID = ROWS == kFwdMidRows;
+  static constexpr int WV = MID ? 4 : kF16WV, WT = MID ? 6 : kF16WT;
+  static constexpr int NWV = MID ? 4 : kFwdNWV, NWT = MID ? 2 : kFwdNWT;
+  static constexpr int RUN_BYTES = WT * kFwdThreads * static_cast<int>(sizeof(float2));
+};
 constexpr int kF16ColsumBytes = 2 * kFwdTile * static_cast<int>(sizeof(float));       // column sums (logit_avg only)
 static_assert(16 * kF16WV * kFwdNWV == kFwdTile && 16 * kF16WT * kFwdNWT == kFwdTile, "tile is 256 x 256");
 
@@ -312,15 +323,15 @@ static_assert(16 * kF16WV * kFwdNWV == kFwdTile && 16 * kF16WT * kFwdNWT == kFwd
 // 2^(-2 cap log2(e) w): two instructions fewer per logit than soft-cap, subtract, exponentiate.  The cell maxima are
 // taken on the raw logits (soft-capping is monotone) and soft-capped once per cell.  The running pair then holds
 // (cap log2(e), sum) and merges with the other spans' pairs like any other.
-template <bool GENERAL, bool CAP, bool FIXED, bool WANT_S2>
-__device__ __forceinline__ void row_block_impl(const Softcap& sc, float cap_inv, const f32x4 (&acc)[kF16WV][kF16WT], int ti,
-                                               const float* addend, int kq, float2& run, float (&bm)[kF16WV / 2],
-                                               float (&s2)[kF16WV][4]) {
-  float y[kF16WV][4];
+template <bool GENERAL, bool CAP, bool FIXED, bool WANT_S2, int WV, int WT>
+__device__ __forceinline__ void row_block_impl(const Softcap& sc, float cap_inv, const f32x4 (&acc)[WV][WT], int ti,
+                                               const float* addend, int kq, float2& run, float (&bm)[WV / 2],
+                                               float (&s2)[WV][4]) {
+  float y[WV][4];
   float tm = -INFINITY;
   float part = 0.0f;
 #pragma unroll
-  for (int vi = 0; vi < kF16WV; ++vi) {
+  for (int vi = 0; vi < WV; ++vi) {
     float gm = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -366,7 +377,7 @@ __device__ __forceinline__ void row_block_impl(const Softcap& sc, float cap_inv,
     const float mn = fmaxf(run.x, tm);
     const float ms = (mn == -INFINITY) ? 0.0f : mn;
 #pragma unroll
-    for (int vi = 0; vi < kF16WV; ++vi)
+    for (int vi = 0; vi < WV; ++vi)
 #pragma unroll
       for (int r = 0; r < 4; ++r) part += __builtin_amdgcn_exp2f(CAP ? y[vi][r] - ms : fmaf(y[vi][r], kLog2e, -ms));
     run.y = run.y * __builtin_amdgcn_exp2f(run.x - ms) + part;
@@ -374,33 +385,35 @@ __device__ __forceinline__ void row_block_impl(const Softcap& sc, float cap_inv,
   }
 }
 
-// One uniform branch per row block: each arm is straight-line code over all 32 values.
-template <bool GENERAL, bool WANT_S2>
-__device__ __forceinline__ void row_block(const Softcap& sc, float cap_inv, bool fixed_ref,
-                                          const f32x4 (&acc)[kF16WV][kF16WT], int ti,
-                                          const float* addend, int kq, float2& run, float (&bm)[kF16WV / 2],
-                                          float (&s2)[kF16WV][4]) {
+// One uniform branch per row block: each arm is straight-line code over all values of the block.
+template <bool GENERAL, bool WANT_S2, int WV, int WT>
+__device__ __forceinline__ void row_block(const Softcap& sc, float cap_inv, bool fixed_ref, const f32x4 (&acc)[WV][WT], int ti,
+                                          const float* addend, int kq, float2& run, float (&bm)[WV / 2],
+                                          float (&s2)[WV][4]) {
   if (fixed_ref) row_block_impl<GENERAL, true, true, WANT_S2>(sc, cap_inv, acc, ti, addend, kq, run, bm, s2);
   else if (sc.on) row_block_impl<GENERAL, true, false, WANT_S2>(sc, cap_inv, acc, ti, addend, kq, run, bm, s2);
   else row_block_impl<GENERAL, false, false, WANT_S2>(sc, cap_inv, acc, ti, addend, kq, run, bm, s2);
 }
 
-template <typename T, bool GENERAL, bool WANT_LA, bool TERMS = false, bool TAIL = false, bool FEW = false>
+template <typename T, bool GENERAL, bool WANT_LA, bool TERMS = false, bool TAIL = false, bool FEW = false, int ROWS = kFwdTile>
 __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdParams p) {
-  using Fast = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, TERMS, TAIL, FEW>;
-  static_assert(!WANT_LA || GENERAL, "the column average uses the general epilogue");
+  using Shape = Fwd16Shape<ROWS>;
+  constexpr int WV = Shape::WV, WT = Shape::WT;
+  using Fast = DmaLogitTile16<T, WV, WT, Shape::NWV, Shape::NWT, TERMS, TAIL, FEW>;
+  static_assert(Fast::TILE_T == ROWS && Fast::TILE_V == kFwdTile, "256 classes x ROWS rows");
+  static_assert(!WANT_LA || (GENERAL && ROWS == kFwdTile), "the column average uses the general epilogue of 256 rows");
   static_assert(!FEW || !WANT_LA, "all waves take part in the column average");
   constexpr int kRunStride = FEW ? kFwdThreads / 2 : kFwdThreads;  // FEW: the waves without rows keep nothing
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_addend = reinterpret_cast<float*>(smem + Fast::LDS_BYTES);  // [2][256]
-  // The running (max, sum-exp) of this lane's kF16WT token rows lives in LDS between the epilogues: [ti][thread].
+  // The running (max, sum-exp) of this lane's WT token rows lives in LDS between the epilogues: [ti][thread].
   // Eight registers fewer across the main loop, which is what lets the loop and the epilogue go without spills
   // (a reload from scratch memory makes the compiler wait for ALL loads in flight, the ring's included).
   float2* s_run = reinterpret_cast<float2*>(smem + Fast::LDS_BYTES + kFwdBiasBytes) + threadIdx.x;
   // WANT_LA: the sums of the soft-capped logits of a tile over its 256 rows, per class: [2][256], by tile parity.
   // The waves add their shares while they are in the epilogue of tile t; the sums leave for memory in the epilogue of
   // tile t + 1 (or after the last tile): the barriers of the main loop in between order the two.
-  float* s_colsum = reinterpret_cast<float*>(smem + Fast::LDS_BYTES + kFwdBiasBytes + kF16RunBytes);
+  float* s_colsum = reinterpret_cast<float*>(smem + Fast::LDS_BYTES + kFwdBiasBytes + Shape::RUN_BYTES);
 
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
@@ -421,8 +434,8 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   const int wt = Fast::wt_of(wave);
   const int r16 = lane & 15;
   const int kq = lane >> 4;
-  const int64_t t0 = static_cast<int64_t>(rb) * kFwdTile;
-  const int64_t wrow0 = t0 + wt * (16 * kF16WT);  // first row of this wave
+  const int64_t t0 = static_cast<int64_t>(rb) * ROWS;
+  const int64_t wrow0 = t0 + wt * (16 * WT);  // first row of this wave
   const bool live = !FEW || wrow0 < p.b;
 
   // Sources of the direct-to-LDS loads (the launcher has checked that the byte offsets fit 32 bits)
@@ -448,7 +461,7 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   // 2^(-2 cap log2(e)) must stay a normal float: cap log2(e) < 60, i.e. caps up to 41
   const bool fixed_ref = p.sc.on && p.sc.out_scale < 60.0f;
 #pragma unroll
-  for (int ti = 0; ti < kF16WT; ++ti)
+  for (int ti = 0; ti < WT; ++ti)
     if (live) s_run[ti * kRunStride] = make_float2(-INFINITY, 0.0f);
   if (WANT_LA) s_colsum[tid] = 0.0f;  // 512 threads, 2 x 256 sums; published by the barriers of the first main loop
   // the sums of the tile that starts at class `first` leave for the running average, and are cleared for the tile after next
@@ -495,32 +508,32 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
         continue;
       }
     }
-    f32x4 acc[kF16WV][kF16WT];
+    f32x4 acc[WV][WT];
     Fast::run(acc, src, smem, static_cast<int>(p.d), buf, vt == vt_begin, next_tile);
 
     // ---- epilogue: (bias, mask,) soft-cap, online max / sum-exp ---------------------------------
-    const float* wave_addend = addend + wv * (16 * kF16WV);
+    const float* wave_addend = addend + wv * (16 * WV);
     // A tile with no bias and no class past the end of the vocabulary has nothing to add and nothing to mask: of a
     // vocabulary that is no multiple of 256 only the last tile pays for the per-class addend.
     const bool plain_tile = GENERAL && (TERMS ? p.bias32 == nullptr : p.bias == nullptr) && v0 + kFwdTile <= p.v;
-    float la[WANT_LA ? kF16WV : 1][4];  // this lane's sums over its four rows of the tile, log2 units
+    float la[WANT_LA ? WV : 1][4];  // this lane's sums over its four rows of the tile, log2 units
     if (WANT_LA) {
       if (vt > vt_begin) flush_colsum(v0 - kFwdTile, (vt - 1) & 1);
 #pragma unroll
-      for (int vi = 0; vi < kF16WV; ++vi)
+      for (int vi = 0; vi < WV; ++vi)
 #pragma unroll
         for (int r = 0; r < 4; ++r) la[vi][r] = 0.0f;
     }
 #pragma unroll
-    for (int tp = 0; tp < kF16WT / 2; ++tp) {
-      float bm[kF16WV / 2];  // this lane's maxima in the four statistic cells of this row pair
+    for (int tp = 0; tp < WT / 2; ++tp) {
+      float bm[WV / 2];  // this lane's maxima in the statistic cells of this row pair
 #pragma unroll
-      for (int j = 0; j < kF16WV / 2; ++j) bm[j] = -INFINITY;
+      for (int j = 0; j < WV / 2; ++j) bm[j] = -INFINITY;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const int ti = 2 * tp + u;
         __builtin_amdgcn_sched_barrier(0);  // keep each row block's register use to itself
-        float s2[kF16WV][4];
+        float s2[WV][4];
         float2 run = s_run[ti * kRunStride];
         if (GENERAL && plain_tile) row_block<false, WANT_LA>(p.sc, p.cap_inv, fixed_ref, acc, ti, wave_addend, kq, run, bm, s2);
         else row_block<GENERAL, WANT_LA>(p.sc, p.cap_inv, fixed_ref, acc, ti, wave_addend, kq, run, bm, s2);
@@ -528,31 +541,31 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
         if (WANT_LA) {
           const bool ok = wrow0 + ti * 16 + r16 < p.b;
 #pragma unroll
-          for (int vi = 0; vi < kF16WV; ++vi)
+          for (int vi = 0; vi < WV; ++vi)
 #pragma unroll
             for (int r = 0; r < 4; ++r) la[vi][r] += (ok && s2[vi][r] != -INFINITY) ? s2[vi][r] : 0.0f;
         }
       }
 
       if (p.tile_max != nullptr) {
-        // Maxima over the 32 rows x 32 classes of the four statistic cells of this (wave, row pair): wave-uniform
-        // values, parked in one register across the lanes -- lane 8 k + 4 tp + j holds cell (row pair tp, class
+        // Maxima over the 32 rows x 32 classes of the statistic cells of this (wave, row pair): wave-uniform
+        // values, parked in one register across the lanes -- lane 8 k + (WV / 2) tp + j holds cell (row pair tp, class
         // group j) of the k-th tile of a run of eight -- and written out once per eight tiles: a store after every
         // tile would have the next tile's first wait for its loads wait for the store's acknowledgement as well.
         const int slot = (vt - vt_begin) & 7;
 #pragma unroll
-        for (int j = 0; j < kF16WV / 2; ++j) {
+        for (int j = 0; j < WV / 2; ++j) {
           const float cell = wave_max_uniform(bm[j]);
-          stat = (lane == 8 * slot + 4 * tp + j) ? cell : stat;
+          stat = (lane == 8 * slot + (WV / 2) * tp + j) ? cell : stat;
         }
       }
     }
     if (WANT_LA) {
       // Over the 16 lanes that hold the 16 rows of a block (rotations on the vector unit), then one LDS add per class
       // from the first lane of each group of 16: the four waves that share these classes meet there.
-      float* cs = s_colsum + (vt & 1) * kFwdTile + wv * (16 * kF16WV) + 4 * kq;
+      float* cs = s_colsum + (vt & 1) * kFwdTile + wv * (16 * WV) + 4 * kq;
 #pragma unroll
-      for (int vi = 0; vi < kF16WV; ++vi)
+      for (int vi = 0; vi < WV; ++vi)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float sum = row16_sum(la[vi][r]);
@@ -564,9 +577,10 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
       if constexpr (WANT_LA) asm volatile("" : "+v"(ln));  // the cell address is formed here, not carried through the loop
       const int first_vt = vt - ((vt - vt_begin) & 7);
       const int my_vt = first_vt + (ln >> 3);
-      const int64_t row = wrow0 + ((ln >> 2) & 1) * 32;
-      const int64_t cls = static_cast<int64_t>(my_vt) * kFwdTile + wv * (16 * kF16WV) + (ln & 3) * 32;
-      if (my_vt <= vt && row < p.b && cls < p.v) {
+      const int pair = (ln & 7) / (WV / 2);
+      const int64_t row = wrow0 + pair * 32;
+      const int64_t cls = static_cast<int64_t>(my_vt) * kFwdTile + wv * (16 * WV) + (ln & (WV / 2 - 1)) * 32;
+      if (my_vt <= vt && pair < WT / 2 && row < p.b && cls < p.v) {
         float mine = stat;
         if (fixed_ref) {  // the maximum was taken over raw logits
           const float t = __builtin_amdgcn_exp2f(mine * p.sc.in_scale);
@@ -582,17 +596,17 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   __syncthreads();
   if (WANT_LA && vt_end > vt_begin) flush_colsum(static_cast<int64_t>(vt_end - 1) * kFwdTile, (vt_end - 1) & 1);
 
-  // ---- merge the four lane groups, then the two wave rows, and emit one partial per row -------
-  float2* stage = reinterpret_cast<float2*>(smem);  // [NWT][WT][16]
-  float m2[kF16WT], sum[kF16WT];
+  // ---- merge the four lane groups, then the wave rows, and emit one partial per row -------
+  float2* stage = reinterpret_cast<float2*>(smem);  // [NWV - 1][ROWS]
+  float m2[WT], sum[WT];
 #pragma unroll
-  for (int ti = 0; ti < kF16WT; ++ti) {
+  for (int ti = 0; ti < WT; ++ti) {
     const float2 run = live ? s_run[ti * kRunStride] : make_float2(-INFINITY, 0.0f);
     m2[ti] = run.x;
     sum[ti] = run.y;
   }
 #pragma unroll
-  for (int ti = 0; ti < kF16WT; ++ti) {
+  for (int ti = 0; ti < WT; ++ti) {
 #pragma unroll
     for (int off = 16; off <= 32; off <<= 1) {
       const float om = __shfl_xor(m2[ti], off, 64);
@@ -603,18 +617,23 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
       m2[ti] = mn;
     }
   }
-  if (wv == 1 && kq == 0) {
+  if (wv != 0 && kq == 0) {
 #pragma unroll
-    for (int ti = 0; ti < kF16WT; ++ti) stage[(wt * kF16WT + ti) * 16 + r16] = make_float2(m2[ti], sum[ti]);
+    for (int ti = 0; ti < WT; ++ti) stage[(wv - 1) * ROWS + (wt * WT + ti) * 16 + r16] = make_float2(m2[ti], sum[ti]);
   }
   __syncthreads();
   if (wv == 0 && kq == 0) {
 #pragma unroll
-    for (int ti = 0; ti < kF16WT; ++ti) {
-      const float2 o = stage[(wt * kF16WT + ti) * 16 + r16];
-      const float mn = fmaxf(m2[ti], o.x);
-      const float ms = (mn == -INFINITY) ? 0.0f : mn;
-      const float s = sum[ti] * __builtin_amdgcn_exp2f(m2[ti] - ms) + o.y * __builtin_amdgcn_exp2f(o.x - ms);
+    for (int ti = 0; ti < WT; ++ti) {
+      float mn = m2[ti], s = sum[ti];
+#pragma unroll
+      for (int w = 0; w < Shape::NWV - 1; ++w) {
+        const float2 o = stage[w * ROWS + (wt * WT + ti) * 16 + r16];
+        const float m1 = fmaxf(mn, o.x);
+        const float ms = (m1 == -INFINITY) ? 0.0f : m1;
+        s = s * __builtin_amdgcn_exp2f(mn - ms) + o.y * __builtin_amdgcn_exp2f(o.x - ms);
+        mn = m1;
+      }
       const int64_t i = wrow0 + ti * 16 + r16;
       if (i < p.b) p.partial[static_cast<int64_t>(split) * p.b + i] = make_float2(mn, s);
     }
@@ -656,8 +675,33 @@ __global__ void fill_zero_kernel(float* p, int64_t n) {
 
 static int choose_nsplit(int nrb, int nvt) { return choose_span_count(nrb, nvt); }
 
+struct RowBlocks {
+  int rows, nrb, nvt, nsplit;
+  int64_t partial_bytes(int64_t b) const { return static_cast<int64_t>(nsplit) * b * static_cast<int64_t>(sizeof(float2)); }
+};
+static RowBlocks blocks_of(int rows, int64_t b, int64_t v, double* cost = nullptr) {
+  RowBlocks r = {rows, static_cast<int>((b + rows - 1) / rows), static_cast<int>((v + kFwdTile - 1) / kFwdTile), 0};
+  const SpanChoice s = choose_spans(r.nrb, r.nvt);
+  r.nsplit = s.count;
+  if (cost != nullptr) *cost = s.cost;
+  return r;
+}
+// Rows per block of the 16 x 16 x 32 kernel: 256, or 192 where that leaves fewer rows of padding or an emptier last round
+// less work.  A tile of 192 rows has three quarters of the products but 56 of the 64 KB of loads per stage, and more
+// fragment reads per product (10 for 24 instead of 12 for 32), so that it costs 0.82 - 0.94 of a whole one; at equal
+// rounds it wins, for one round more in ten it does not.  Forward of R rows, blocks of 256 / 192, us: 307 x 5120 x 131072 633 / 521,
+// 192 x 2048 x 32000 52 / 46, 900 x 1024 x 50257 104 / 97.5, 900 x 1000 x 50257 (soft-cap, bias) 147 / 142, 600 x 640 x 8000
+// 24.8 / 23.5; and 960 x 4096 x 128256 854 / 948, 3891 x 1024 x 32000 215 / 229, 8192 x 2304 x 256000 6979 / 8811.
+constexpr double kMidTileCost = 0.92;
+static RowBlocks best_blocks(int64_t b, int64_t v) {
+  double whole, mid;
+  const RowBlocks w = blocks_of(kFwdTile, b, v, &whole);
+  const RowBlocks m = blocks_of(kFwdMidRows, b, v, &mid);
+  return mid * kMidTileCost < whole ? m : w;
+}
+
 template <typename T>
-static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipStream_t stream) {
+static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64_t workspace_bytes, hipStream_t stream) {
   using Tile = LogitTile<T, kFwdWV, kFwdWT, kFwdNWV, kFwdNWT, true>;
   using Fast = DmaLogitTile<T, kFwdWV, kFwdWT, kFwdNWV, kFwdNWT>;
   static_assert(Fast::LDS_BYTES <= Tile::LDS_BYTES, "one LDS size serves both main loops");
@@ -666,6 +710,9 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
   using Few = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, false, false, true>;
   constexpr int lds_few = Few::LDS_BYTES + kFwdBiasBytes + kF16RunBytes / 2;
   static_assert(lds_few <= 160 * 1024, "three stages fit");
+  using MidShape = Fwd16Shape<kFwdMidRows>;
+  constexpr int lds_mid = DmaLogitTile16<T, MidShape::WV, MidShape::WT, MidShape::NWV, MidShape::NWT>::LDS_BYTES + kFwdBiasBytes +
+                          MidShape::RUN_BYTES;
   // the 16 x 16 x 32 kernel addresses token rows by 32-bit byte offsets from e and class rows by offsets from the
   // first class of a tile; shapes beyond that, and a D of one stage, take the 32 x 32 x 16 kernel, which knows whole
   // stages only
@@ -678,6 +725,17 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
   // 290 / 210 (C at 5.6 TB/s), 131072 x 5120 334 / 251, 50257 x 1000 49 / 42, 4096 x 512 21 / 17.5, 512 x 192 17.5 / 17.5;
   // 16 and 128 rows alike.
   const bool few = fast16 && !want_la && p.b <= kFwdTile / 2 && p.d > 2 * kDmaBK;
+  RowBlocks blocks = blocks_of(kFwdTile, p.b, p.v);
+  if (fast16 && !want_la && !few) {
+    const RowBlocks best = best_blocks(p.b, p.v);
+    if (best.partial_bytes(p.b) <= workspace_bytes) blocks = best;
+  }
+  const bool mid = blocks.rows == kFwdMidRows;
+  p.nrb = blocks.nrb;
+  p.nvt = blocks.nvt;
+  p.nsplit = blocks.nsplit;
+  p.nitems = p.nrb * p.nsplit;
+  p.items_per_xcd = (p.nitems + 7) / 8;
   const bool general = want_la || (p.bias != nullptr) || (p.v % Tile::TILE_V != 0);
   const int grid = p.items_per_xcd * 8;
   hipError_t err;
@@ -689,29 +747,35 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, hipSt
     if (err != hipSuccess) return status_from_hip(err);                                           \
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), lds, stream, p);                           \
   } while (0)
-#define CCE_LAUNCH_FWD16(GE, LA, TAIL, FEW)                                                       \
+#define CCE_LAUNCH_FWD16(GE, LA, TAIL, FEW, ROWS)                                                 \
   do {                                                                                            \
-    auto kern = lse_forward16_kernel<T, GE, LA, false, TAIL, FEW>;                                \
-    static LdsLimitOnce lds_limit;                                                            \
-    const int bytes = (FEW) ? lds_few : lds16 + ((LA) ? kF16ColsumBytes : 0);                     \
+    auto kern = lse_forward16_kernel<T, GE, LA, false, TAIL, FEW, ROWS>;                          \
+    static LdsLimitOnce lds_limit;                                                                \
+    const int bytes = (ROWS) != kFwdTile ? lds_mid : (FEW) ? lds_few : lds16 + ((LA) ? kF16ColsumBytes : 0); \
     err = lds_limit.set(kern, bytes);                                                             \
     if (err != hipSuccess) return status_from_hip(err);                                           \
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kFwdThreads), bytes, stream, p);                    \
   } while (0)
   if (few && tail) {
-    if (general) CCE_LAUNCH_FWD16(true, false, true, true);
-    else CCE_LAUNCH_FWD16(false, false, true, true);
+    if (general) CCE_LAUNCH_FWD16(true, false, true, true, kFwdTile);
+    else CCE_LAUNCH_FWD16(false, false, true, true, kFwdTile);
   } else if (few) {
-    if (general) CCE_LAUNCH_FWD16(true, false, false, true);
-    else CCE_LAUNCH_FWD16(false, false, false, true);
+    if (general) CCE_LAUNCH_FWD16(true, false, false, true, kFwdTile);
+    else CCE_LAUNCH_FWD16(false, false, false, true, kFwdTile);
+  } else if (mid && tail) {
+    if (general) CCE_LAUNCH_FWD16(true, false, true, false, kFwdMidRows);
+    else CCE_LAUNCH_FWD16(false, false, true, false, kFwdMidRows);
+  } else if (mid) {
+    if (general) CCE_LAUNCH_FWD16(true, false, false, false, kFwdMidRows);
+    else CCE_LAUNCH_FWD16(false, false, false, false, kFwdMidRows);
   } else if (fast16 && tail) {
-    if (want_la) CCE_LAUNCH_FWD16(true, true, true, false);
-    else if (general) CCE_LAUNCH_FWD16(true, false, true, false);
-    else CCE_LAUNCH_FWD16(false, false, true, false);
+    if (want_la) CCE_LAUNCH_FWD16(true, true, true, false, kFwdTile);
+    else if (general) CCE_LAUNCH_FWD16(true, false, true, false, kFwdTile);
+    else CCE_LAUNCH_FWD16(false, false, true, false, kFwdTile);
   } else if (fast16) {
-    if (want_la) CCE_LAUNCH_FWD16(true, true, false, false);
-    else if (general) CCE_LAUNCH_FWD16(true, false, false, false);
-    else CCE_LAUNCH_FWD16(false, false, false, false);
+    if (want_la) CCE_LAUNCH_FWD16(true, true, false, false, kFwdTile);
+    else if (general) CCE_LAUNCH_FWD16(true, false, false, false, kFwdTile);
+    else CCE_LAUNCH_FWD16(false, false, false, false, kFwdTile);
   } else if (fast) {
     if (want_la) CCE_LAUNCH_FWD(true, true, true, true);
     else if (general) CCE_LAUNCH_FWD(true, true, true, false);
@@ -791,10 +855,7 @@ extern "C" int64_t cce_tile_stat_elems(int64_t b, int64_t v) {
 extern "C" int64_t cce_lse_forward_workspace_bytes(int64_t b, int64_t v, int64_t d) {
   (void)d;
   if (b <= 0 || v <= 0) return 0;
-  const int nrb = static_cast<int>((b + 255) / 256);
-  const int nvt = static_cast<int>((v + 255) / 256);
-  const int nsplit = choose_nsplit(nrb, nvt);
-  return static_cast<int64_t>(nsplit) * b * static_cast<int64_t>(sizeof(float2));
+  return std::max(blocks_of(kFwdTile, b, v).partial_bytes(b), best_blocks(b, v).partial_bytes(b));
 }
 
 // (lse == nullptr: the partials stay in the workspace, and *nsplit_out says how many spans they are of)
@@ -804,7 +865,7 @@ static int lse_forward_impl(const void* e, const void* c, const void* bias, cons
                             int64_t n_rows, int64_t b, int64_t v, int64_t d,
                             int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
                             float softcap, int dtype, hipStream_t stream) {
-  const int64_t need = cce_lse_forward_workspace_bytes(b, v, d);
+  const int64_t need = blocks_of(kFwdTile, b, v).partial_bytes(b);  // other row blocks are taken where their spans fit
   if (workspace == nullptr || workspace_bytes < need) return CCE_ERR_WORKSPACE_TOO_SMALL;
   if ((reinterpret_cast<uintptr_t>(workspace) & 7u) != 0) return CCE_ERR_MISALIGNED;
 
@@ -823,11 +884,6 @@ static int lse_forward_impl(const void* e, const void* c, const void* bias, cons
   p.stride_e = stride_e;
   p.stride_cv = stride_cv;
   p.stride_cd = stride_cd;
-  p.nrb = static_cast<int>((b + 255) / 256);
-  p.nvt = static_cast<int>((v + 255) / 256);
-  p.nsplit = choose_nsplit(p.nrb, p.nvt);
-  p.nitems = p.nrb * p.nsplit;
-  p.items_per_xcd = (p.nitems + 7) / 8;
   p.stat_cols = static_cast<int>((v + CCE_STAT_COLS - 1) / CCE_STAT_COLS);
   p.avg_scale = kLn2 / static_cast<float>(b);
   p.sc = make_softcap(softcap);
@@ -840,8 +896,8 @@ static int lse_forward_impl(const void* e, const void* c, const void* bias, cons
     hipLaunchKernelGGL(fill_zero_kernel, dim3(static_cast<unsigned>((v + 255) / 256)), dim3(256), 0, stream,
                        logit_avg, v);
   }
-  int st = (dtype == CCE_DTYPE_BF16) ? launch_lse_forward<BF16>(p, aligned, logit_avg != nullptr, stream)
-                                     : launch_lse_forward<F16>(p, aligned, logit_avg != nullptr, stream);
+  int st = (dtype == CCE_DTYPE_BF16) ? launch_lse_forward<BF16>(p, aligned, logit_avg != nullptr, workspace_bytes, stream)
+                                     : launch_lse_forward<F16>(p, aligned, logit_avg != nullptr, workspace_bytes, stream);
   if (st != CCE_OK) return st;
   if (lse == nullptr) {
     *nsplit_out = p.nsplit;
@@ -943,7 +999,7 @@ extern "C" int cce_lse_forward_static(const void* e, const void* c, const void* 
   bool done;
   int st = lse_forward_check(e, c, lse, valids, n_rows, b, v, d, dtype, &done);
   if (st != CCE_OK || done) return st;
-  if (cce_lse_forward_workspace_bytes(b, v, d) > CCE_STATIC_SCRATCH_BYTES) return CCE_ERR_STATIC_SCRATCH_LIMIT;
+  if (blocks_of(kFwdTile, b, v).partial_bytes(b) > CCE_STATIC_SCRATCH_BYTES) return CCE_ERR_STATIC_SCRATCH_LIMIT;
   void* ws = nullptr;
   st = static_scratch_for_current_device(&ws);
   if (st != CCE_OK) return st;

@@ -553,3 +553,34 @@ def test_a_single_row_with_a_stride_of_its_own(dtype, which, width):
         results.append((loss.detach(), ed.grad, cd.grad))
     for a, b in zip(*results):
         assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [129, 191, 192, 193, 300, 384, 385, 576])
+@pytest.mark.parametrize("width,classes", [(128, 256), (136, 1000), (192, 256 * 40 + 1), (704, 256 * 130)])
+def test_forward_in_blocks_of_192_rows(dtype, rows, width, classes):
+    """Blocks of 192 rows where 256 would be padding or an emptier last round: the edges of the blocks and of the cells in them, gathered
+    rows, partial stages, cut tiles, several tiles per span; log-sum-exp, losses and the cells' maxima."""
+    from cut_cross_entropy.cce_lse_forward import loss_forward
+
+    g = torch.Generator().manual_seed(rows + width)
+    e = torch.randn((rows + 5, width), generator=g).to(dtype).cuda()
+    c = (torch.randn((classes, width), generator=g) * 0.1).to(dtype).cuda()
+    t = torch.randint(0, classes, (rows + 5,), generator=g).cuda()
+    valids = torch.arange(5, rows + 5, dtype=torch.int32).cuda()
+    for softcap, bias in ((None, None), (20.0, None), (50.0, torch.randn((classes,), generator=g).to(dtype).cuda())):
+        lse, nll, cells = loss_forward(e, c, bias, t, valids, 0, softcap, 0, True)
+        x = e[5:].float() @ c.float().T
+        if bias is not None:
+            x += bias.float()
+        if softcap is not None:
+            x = softcap * torch.tanh(x / softcap)
+        want = torch.logsumexp(x, 1)
+        # the bounds of test_forward_of_few_rows_keeps_three_stages: the same sums in fp32
+        assert (lse - want).abs().max() < 2e-5 * max(1.0, want.abs().max().item())
+        assert (nll - (want - x.gather(1, t[5:, None])[:, 0])).abs().max() < 1e-4
+        rb, cb = -(-rows // 32), -(-classes // 32)
+        padded = torch.full((rb * 32, cb * 32), float("-inf"), device="cuda")
+        padded[:rows, :classes] = x
+        top = padded.view(rb, 32, cb, 32).amax((1, 3))
+        assert (cells.view(rb, cb) - top).abs().max() < 2e-4
