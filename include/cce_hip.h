@@ -305,6 +305,32 @@ int cce_valid_rows(const int64_t* labels, int64_t n, int64_t steps, int64_t shif
 int cce_rows_to_batch(const float* values, const int32_t* rows, int64_t count, int64_t n, int64_t shift, float* out, void* stream);
 
 /*
+ * The same for sequences of `steps` positions (n a multiple) without the first `shift` steps of each, for up to two sets of values
+ * (out NULL: not wanted): out[n / steps][steps - shift], [s][j] the value of row s * steps + j.  And the way back, zeros in the
+ * first `shift` steps: in[n / steps][steps - shift] to out[n / steps][steps].
+ */
+int cce_rows_to_steps(const float* first, const float* second, const int32_t* rows, int64_t count, int64_t n, int64_t steps,
+                      int64_t shift, float* out_first, float* out_second, void* stream);
+int cce_steps_to_batch(const float* first, const float* second, int64_t n, int64_t steps, int64_t shift, float* out_first,
+                       float* out_second, void* stream);
+
+/*
+ * The z-loss (cut_cross_entropy/utils.py:64-102): squares of lse[rows][cols], zero where labels[rows][cols] (NULL: nowhere) is
+ * `ignored`; CCE_REDUCTION_NONE writes out[rows * cols], the others one value, and how many positions count to *count where
+ * that is not NULL.  The strides lead from row to row.  Backward: d_lse[rows * cols] from the upstream gradient (one value, or one
+ * per position), divided by *count where that is not NULL (the mean).
+ */
+#define CCE_REDUCTION_NONE 0
+#define CCE_REDUCTION_SUM 1
+#define CCE_REDUCTION_MEAN 2
+int64_t cce_z_loss_workspace_bytes(int64_t rows, int64_t cols);
+int cce_z_loss_forward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows, int64_t cols,
+                       int64_t ignored, int reduction, float* out, float* count, void* workspace, int64_t workspace_bytes,
+                       void* stream);
+int cce_z_loss_backward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows, int64_t cols,
+                        int64_t ignored, const float* grad, int grad_is_scalar, const float* count, float* d_lse, void* stream);
+
+/*
  * cce_lse_forward (without logit_avg) and cce_indexed_neg_dot in one call: lse[b], and nll[b] = lse + neg_dot, the loss of
  * every valid row (cut_cross_entropy/cce.py:87-131).  tile_max may be NULL; workspace as for cce_lse_forward.
  */

@@ -1,6 +1,6 @@
-// The per-row work around the two big kernels: which rows of a batch count (cce_valid_rows), and the loss of a row from
-// the forward's partial sums (loss_rows_kernel).  Both are small and come with every call, so what they cost is launches:
-// each replaces a chain of library kernels or of kernels of ours.
+// The per-row work around the two big kernels: which rows of a batch count (cce_valid_rows), the loss of a row from the
+// forward's partial sums (loss_rows_kernel), per-row values at their places in the batch and back, and the z-loss.  All are
+// small and come with every call, so what they cost is launches: each replaces a chain of library kernels or of kernels of ours.
 #include "cce_dense.h"
 
 namespace cce {
@@ -66,6 +66,123 @@ __global__ __launch_bounds__(256) void rows_to_batch_kernel(const float* values,
     else hi = mid;
   }
   out[p] = (lo < count && rows[lo] == p - shift) ? values[lo] : 0.0f;
+}
+
+// Up to two sets of values at once, and the first `shift` steps of every sequence left out: out[s][j] of [n / steps][steps -
+// shift] is the value of row s * steps + j.  With the z-loss's log-sum-exp beside a loss per token this is one launch of four (two
+// searches, and autograd's zeros and copy for either slice on the way back, which steps_to_batch_kernel does in one).
+struct TwoSets {
+  const float* in[2];
+  float* out[2];
+};
+__global__ __launch_bounds__(256) void rows_to_steps_kernel(TwoSets sets, const int32_t* rows, int count, int n_out, int steps, int kept) {
+  const int q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= n_out) return;
+  const int row = q / kept * steps + q % kept;
+  int lo = 0, hi = count;  // the first r with rows[r] >= row
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (rows[mid] < row) lo = mid + 1;
+    else hi = mid;
+  }
+  const bool found = lo < count && rows[lo] == row;
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (sets.out[k] != nullptr) sets.out[k][q] = found ? sets.in[k][lo] : 0.0f;
+}
+
+// The way back: out[s][j + shift] of [n / steps][steps] = in[s][j], zeros in the first `shift` steps.
+__global__ __launch_bounds__(256) void steps_to_batch_kernel(TwoSets sets, int n, int steps, int shift) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= n) return;
+  const int s = p / steps, j = p - s * steps - shift;
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (sets.out[k] != nullptr) sets.out[k][p] = j >= 0 ? sets.in[k][s * (steps - shift) + j] : 0.0f;
+}
+
+// The squares of log-sum-exps, zero where a label is ignored; as they are, or their sum or mean over what counts.  `rows`
+// sequences of `cols` steps, either operand with a stride of its own from sequence to sequence (a slice of longer ones).
+// Sums in fp64: one workgroup up to 16384 values, else partial sums of one workgroup each and another launch for them
+// (fixed order, no atomics).  Launches are what it costs: with its gradient two of them, where the library's chain takes
+// twelve (square, comparison, copy, fill, sum, count and division, and the same backwards).
+struct ZLossParams {
+  const float* lse;
+  const int64_t* labels;  // nullptr: everything counts
+  int64_t lse_stride, label_stride, ignored;
+  int n, cols;
+};
+__device__ __forceinline__ bool z_loss_counts(const ZLossParams& p, int r, int c) {
+  return p.labels == nullptr || p.labels[r * p.label_stride + c] != p.ignored;
+}
+
+constexpr int kZThreads = 1024, kZPerBlock = 16384, kZBlocks = 256;
+struct ZPartial {
+  double sum;
+  int64_t count;
+};
+__device__ __forceinline__ ZPartial z_block_sum(ZPartial mine, ZPartial* s_part) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    mine.sum += __shfl_xor(mine.sum, off, 64);
+    mine.count += __shfl_xor(static_cast<long long>(mine.count), off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = mine;
+  __syncthreads();
+  ZPartial all = {0.0, 0};
+  if (threadIdx.x == 0) {
+    for (int w = 0; w < kZThreads / 64; ++w) {
+      all.sum += s_part[w].sum;
+      all.count += s_part[w].count;
+    }
+  }
+  return all;  // in thread 0
+}
+__device__ __forceinline__ void z_loss_result(const ZPartial& all, bool mean, float* out, float* count) {
+  const float total = static_cast<float>(all.sum);
+  *out = mean ? total / static_cast<float>(all.count) : total;
+  if (count != nullptr) *count = static_cast<float>(all.count);
+}
+
+__global__ __launch_bounds__(kZThreads) void z_loss_sum_kernel(ZLossParams p, bool mean, ZPartial* partial, float* out, float* count) {
+  __shared__ ZPartial s_part[kZThreads / 64];
+  ZPartial mine = {0.0, 0};
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kZThreads + threadIdx.x; i < p.n; i += static_cast<int64_t>(gridDim.x) * kZThreads) {
+    const int r = static_cast<int>(i) / p.cols, c = static_cast<int>(i) - r * p.cols;
+    if (z_loss_counts(p, r, c)) {
+      const float x = p.lse[r * p.lse_stride + c];
+      mine.sum += static_cast<double>(x * x);
+      ++mine.count;
+    }
+  }
+  const ZPartial all = z_block_sum(mine, s_part);
+  if (threadIdx.x != 0) return;
+  if (gridDim.x == 1) z_loss_result(all, mean, out, count);
+  else partial[blockIdx.x] = all;
+}
+__global__ __launch_bounds__(kZThreads) void z_loss_total_kernel(const ZPartial* partial, int blocks, bool mean, float* out, float* count) {
+  __shared__ ZPartial s_part[kZThreads / 64];
+  ZPartial mine = {0.0, 0};
+  if (static_cast<int>(threadIdx.x) < blocks) mine = partial[threadIdx.x];
+  const ZPartial all = z_block_sum(mine, s_part);
+  if (threadIdx.x == 0) z_loss_result(all, mean, out, count);
+}
+
+// GRAD: the gradient of either, g the upstream value (one for a sum or mean, which divides by its count, or one per position)
+template <bool GRAD>
+__global__ __launch_bounds__(256) void z_loss_map_kernel(ZLossParams p, const float* grad, bool one_grad, const float* count, float* out) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= p.n) return;
+  const int r = static_cast<int>(i) / p.cols, c = static_cast<int>(i) - r * p.cols;
+  const bool counts = z_loss_counts(p, r, c);
+  const float x = p.lse[r * p.lse_stride + c];
+  if (!GRAD) {
+    out[i] = counts ? x * x : 0.0f;
+    return;
+  }
+  float g = one_grad ? grad[0] : grad[i];
+  if (count != nullptr) g /= count[0];
+  out[i] = (counts ? g : 0.0f) * (2.0f * x);
 }
 
 // The loss of one valid row per wave: its log-sum-exp from the partial (max, sum) pairs of the vocabulary spans, and minus
@@ -218,5 +335,84 @@ extern "C" int cce_rows_to_batch(const float* values, const int32_t* rows, int64
   hipLaunchKernelGGL(rows_to_batch_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), values, rows, static_cast<int>(count), static_cast<int>(n),
                      static_cast<int>(shift > n ? 0 : shift), out);
+  return status_from_hip(hipGetLastError());
+}
+
+extern "C" int cce_rows_to_steps(const float* first, const float* second, const int32_t* rows, int64_t count, int64_t n, int64_t steps,
+                                 int64_t shift, float* out_first, float* out_second, void* stream) {
+  if (n < 0 || n >= (int64_t(1) << 31) - 8192 || count < 0 || count > n || steps <= 0 || shift < 0) return CCE_ERR_INVALID_ARGUMENT;
+  if (n == 0 || shift >= steps) return CCE_OK;
+  if (n % steps != 0 || (count > 0 && rows == nullptr)) return CCE_ERR_INVALID_ARGUMENT;
+  if (count > 0 && ((out_first != nullptr && first == nullptr) || (out_second != nullptr && second == nullptr)))
+    return CCE_ERR_INVALID_ARGUMENT;
+  const int n_out = static_cast<int>(n / steps * (steps - shift));
+  const TwoSets sets = {{first, second}, {out_first, out_second}};
+  hipLaunchKernelGGL(rows_to_steps_kernel, dim3((n_out + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), sets, rows,
+                     static_cast<int>(count), n_out, static_cast<int>(steps), static_cast<int>(steps - shift));
+  return status_from_hip(hipGetLastError());
+}
+
+extern "C" int cce_steps_to_batch(const float* first, const float* second, int64_t n, int64_t steps, int64_t shift, float* out_first,
+                                  float* out_second, void* stream) {
+  if (n < 0 || n >= (int64_t(1) << 31) - 8192 || steps <= 0 || shift < 0 || shift > steps) return CCE_ERR_INVALID_ARGUMENT;
+  if (n == 0) return CCE_OK;
+  if (n % steps != 0 || (out_first != nullptr && first == nullptr) || (out_second != nullptr && second == nullptr))
+    return CCE_ERR_INVALID_ARGUMENT;
+  const TwoSets sets = {{first, second}, {out_first, out_second}};
+  hipLaunchKernelGGL(steps_to_batch_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), sets, static_cast<int>(n), static_cast<int>(steps), static_cast<int>(shift));
+  return status_from_hip(hipGetLastError());
+}
+
+static int z_loss_check(const float* lse, int64_t rows, int64_t cols, int64_t* n) {
+  if (rows < 0 || cols < 0) return CCE_ERR_INVALID_ARGUMENT;
+  if (cols > 0 && rows > ((int64_t(1) << 31) - 8192) / cols) return CCE_ERR_INVALID_ARGUMENT;
+  *n = rows * cols;
+  return (*n > 0 && lse == nullptr) ? CCE_ERR_INVALID_ARGUMENT : CCE_OK;
+}
+
+extern "C" int64_t cce_z_loss_workspace_bytes(int64_t rows, int64_t cols) {
+  return rows > 0 && cols > 0 && rows * cols > kZPerBlock ? kZBlocks * static_cast<int64_t>(sizeof(ZPartial)) : 0;
+}
+
+extern "C" int cce_z_loss_forward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows,
+                                  int64_t cols, int64_t ignored, int reduction, float* out, float* count, void* workspace,
+                                  int64_t workspace_bytes, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  int64_t n = 0;
+  const int st = z_loss_check(lse, rows, cols, &n);
+  if (st != CCE_OK) return st;
+  if (reduction < CCE_REDUCTION_NONE || reduction > CCE_REDUCTION_MEAN) return CCE_ERR_INVALID_ARGUMENT;
+  if (out == nullptr && (n > 0 || reduction != CCE_REDUCTION_NONE)) return CCE_ERR_INVALID_ARGUMENT;
+  const ZLossParams p = {lse, labels, lse_stride, label_stride, ignored, static_cast<int>(n), static_cast<int>(cols > 0 ? cols : 1)};
+  if (reduction == CCE_REDUCTION_NONE) {
+    if (n == 0) return CCE_OK;
+    hipLaunchKernelGGL(z_loss_map_kernel<false>, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream, p, nullptr, false,
+                       nullptr, out);
+    return status_from_hip(hipGetLastError());
+  }
+  const bool mean = reduction == CCE_REDUCTION_MEAN;
+  const int64_t wanted = (n + kZPerBlock - 1) / kZPerBlock;
+  const int blocks = static_cast<int>(wanted < 1 ? 1 : wanted > kZBlocks ? kZBlocks : wanted);
+  if (blocks > 1 && (workspace == nullptr || workspace_bytes < cce_z_loss_workspace_bytes(rows, cols)))
+    return CCE_ERR_WORKSPACE_TOO_SMALL;
+  if ((reinterpret_cast<uintptr_t>(workspace) & 7u) != 0) return CCE_ERR_MISALIGNED;
+  ZPartial* const partial = static_cast<ZPartial*>(workspace);
+  hipLaunchKernelGGL(z_loss_sum_kernel, dim3(blocks), dim3(kZThreads), 0, stream, p, mean, partial, out, count);
+  if (blocks > 1)
+    hipLaunchKernelGGL(z_loss_total_kernel, dim3(1), dim3(kZThreads), 0, stream, partial, blocks, mean, out, count);
+  return status_from_hip(hipGetLastError());
+}
+
+extern "C" int cce_z_loss_backward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows,
+                                   int64_t cols, int64_t ignored, const float* grad, int grad_is_scalar, const float* count,
+                                   float* d_lse, void* stream) {
+  int64_t n = 0;
+  const int st = z_loss_check(lse, rows, cols, &n);
+  if (st != CCE_OK || n == 0) return st;
+  if (grad == nullptr || d_lse == nullptr) return CCE_ERR_INVALID_ARGUMENT;
+  const ZLossParams p = {lse, labels, lse_stride, label_stride, ignored, static_cast<int>(n), static_cast<int>(cols)};
+  hipLaunchKernelGGL(z_loss_map_kernel<true>, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), p, grad, grad_is_scalar != 0, count, d_lse);
   return status_from_hip(hipGetLastError());
 }

@@ -584,3 +584,97 @@ def test_forward_in_blocks_of_192_rows(dtype, rows, width, classes):
         padded[:rows, :classes] = x
         top = padded.view(rb, 32, cb, 32).amax((1, 3))
         assert (cells.view(rb, cb) - top).abs().max() < 2e-4
+
+
+@pytest.mark.parametrize("shape,shift", [((1, 1), 0), ((3, 85), 0), ((3, 85), 2), ((1, 257), 1), ((2, 2, 5), 4), ((2, 5000), 1)])
+@pytest.mark.parametrize("keep", [0.0, 0.5, 1.0])
+def test_rows_to_steps_and_back(shape, shift, keep):
+    """Per-row values laid out without the first steps of each sequence, and their gradients padded with zeros again: what slicing
+    the whole batch and autograd's way back through the slice give."""
+    from cut_cross_entropy.utils import flat_valids, handle_reduction_none, rows_to_steps, steps_to_batch
+
+    g = torch.Generator().manual_seed(sum(shape) + shift)
+    t = torch.randint(0, 9, shape, generator=g)
+    t[torch.rand(shape, generator=g) >= keep] = -100
+    valids = flat_valids(t, -100, shift)
+    if valids is None:
+        valids = torch.arange(t.numel(), dtype=torch.int32)
+    for sets in (1, 2, 3):
+        values = [torch.randn((valids.numel(),), generator=g) if sets >> k & 1 else None for k in range(2)]
+        got = rows_to_steps(t.size(), valids.cuda(), shift, *(None if v is None else v.cuda() for v in values))
+        for v, out in zip(values, got):
+            assert (v is None) == (out is None)
+            if v is not None:
+                assert torch.equal(out.cpu(), handle_reduction_none(t.size(), valids, shift, v)[..., shift:])
+        back = steps_to_batch(t.size(), shift, *got)
+        for out, flat in zip(got, back):
+            if out is not None:
+                want = torch.zeros(shape)
+                want[..., shift:] = out.cpu()
+                assert torch.equal(flat.cpu(), want.view(-1))
+
+
+@pytest.mark.parametrize("shape,shift", [((1,), 0), ((2, 1), 0), ((70,), 3), ((3, 85), 2), ((2, 3, 50), 1), ((1, 16384), 0), ((1, 16385), 0),
+                                         ((5, 3277), 1), ((3, 1400001), 1)])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+@pytest.mark.parametrize("labels", ["some", "none", "all ignored", "not given"])
+def test_z_loss_kernels_against_tensor_operations(shape, shift, reduction, labels):
+    """One value, one workgroup, one value more than that, and more values than the workgroups take once; slices of longer sequences;
+    what a masked position holds (NaN, infinities) stays out of the value.  Bits of the single squares and gradients; sums in
+    fp64 rounded once, which is as near as fp32 gets."""
+    from cut_cross_entropy import utils
+
+    g = torch.Generator().manual_seed(sum(shape) + shift)
+    whole = (torch.randn(shape, generator=g) * 3 + 9).cuda()
+    t = torch.randint(0, 50, shape, generator=g)
+    t[torch.rand(shape, generator=g) < 0.3] = -100
+    if labels == "all ignored":
+        t[...] = -100
+    elif labels == "none":
+        t.clamp_(min=0)
+    t = None if labels == "not given" else t.cuda()
+    n_masked = 0
+    if labels == "some" and whole[..., shift:].numel() > 2:
+        masked = (t[..., shift:] == -100).nonzero()
+        n_masked = len(masked)
+        if n_masked:
+            whole[..., shift:][tuple(masked[0])] = float("inf")
+            whole[..., shift:][tuple(masked[-1])] = float("nan")
+    lse = whole[..., shift:].detach().requires_grad_(True)
+    assert utils._z_loss_has_kernels(lse.detach(), t, shift, -100)
+    out = utils.compute_z_loss(lse, t, shift, reduction=reduction)
+    up = torch.rand(out.shape, generator=g).cuda() + 0.5
+    (grad,) = torch.autograd.grad(out, lse, up, retain_graph=True)
+
+    ref = lse.detach().requires_grad_(True)
+    sq = ref.square()
+    if t is not None:
+        sq = sq.masked_fill(t[..., shift:] == -100, 0.0)
+    if reduction == "none":
+        assert torch.equal(out, sq) and out.shape == sq.shape
+        want = sq
+    else:
+        total = sq.double().sum()
+        counted = sq.numel() if t is None else (t[..., shift:] != -100).sum()
+        want = total if reduction == "sum" else total.float() / counted
+        assert torch.allclose(out.double(), want.double(), rtol=2e-7, atol=0, equal_nan=True) and out.shape == ()
+    (want_grad,) = torch.autograd.grad(want.float(), ref, up)
+    # (the reference divides where the kernel does; NaN under a mask stays NaN in a gradient: 0 x NaN)
+    assert grad.shape == want_grad.shape and torch.allclose(grad, want_grad, rtol=2e-7, atol=0, equal_nan=True)
+
+    # a graph of the gradient, and what the kernels are not for: the same function by tensor operations
+    if whole.numel() < 1000 and not n_masked and labels != "all ignored":  # (0 / 0 has no tangent)
+        (g1,) = torch.autograd.grad(out, lse, up, create_graph=True)
+        assert torch.allclose(g1, want_grad, rtol=2e-7, atol=0, equal_nan=True)
+        (g2,) = torch.autograd.grad(g1.sum(), lse)
+        assert torch.allclose(g2 * lse.detach(), want_grad, rtol=1e-6, atol=0)
+        plain = lse.detach()
+        import torch.autograd.forward_ad as fwAD
+
+        with fwAD.dual_level():
+            dual = utils.compute_z_loss(fwAD.make_dual(plain, torch.ones_like(plain)), t, shift, reduction=reduction)
+            tangent = fwAD.unpack_dual(dual).tangent
+        (all_ones,) = torch.autograd.grad(utils.compute_z_loss(lse, t, shift, reduction=reduction).sum(), lse)
+        assert torch.allclose(tangent.sum(), all_ones.sum(), rtol=1e-5, atol=1e-5, equal_nan=True)
+        pair = torch.vmap(lambda x: utils.compute_z_loss(x, t, shift, reduction=reduction))(torch.stack([plain, plain]))
+        assert torch.allclose(pair[1], out.detach(), rtol=1e-6, atol=0, equal_nan=True)
