@@ -3,7 +3,8 @@
  *
  * Every entry point is stream-ordered (work is enqueued on `stream`, a
  * hipStream_t passed as void*), takes plain device pointers and sizes, never
- * allocates device memory, never synchronises, and returns 0 on success or a
+ * allocates device memory, never synchronises (but for cce_loss_call, which
+ * waits for one number), and returns 0 on success or a
  * non-zero status (a hipError_t value, or one of the CCE_ERR_* codes below).
  * All scratch memory comes in through the `workspace` argument, sized by the
  * matching *_workspace_bytes() query, so that a caller's allocator sees every
@@ -39,6 +40,7 @@ extern "C" {
 
 #define CCE_DTYPE_BF16 0
 #define CCE_DTYPE_F16 1
+#define CCE_DTYPE_F32 2 /* cce_loss_call only */
 
 /* Granularity of the forward tile statistic (rows x vocabulary entries per cell). */
 #define CCE_STAT_ROWS 32
@@ -339,6 +341,22 @@ int cce_loss_forward(const void* e, const void* c, const void* bias, const int32
                      int64_t n_rows, int64_t b, int64_t v, int64_t d,
                      int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
                      int64_t shift, int64_t target_offset, float softcap, int dtype, void* stream);
+
+/*
+ * The whole forward of the operator (cut_cross_entropy/cce.py:48-137, 261-319): cce_valid_rows of labels[n], then, as soon as
+ * the number of rows that count is known (*count, pinned host memory, waited for), cce_loss_forward or cce_fp32_forward
+ * (CCE_DTYPE_F32, with `terms`) over them, and what the operator returns: `loss`, the sum or mean or, for CCE_REDUCTION_NONE, one value
+ * per position without the first `shift` steps, and lse_out (may be NULL) like that, which is left alone where it would be lse:
+ * no shift and *count == n.  rows[n], lse[n] (the first *count
+ * are written) and tile_max (may be NULL; cce_tile_stat_elems(n, v) floats) are kept for a backward.  `workspace` 256-byte
+ * aligned.  CCE_ERR_WORKSPACE_TOO_SMALL after a wait (*count >= 0): rows and *count are written, the rest is for the single calls.
+ * Refuses a stream that is being captured.
+ */
+int64_t cce_loss_call_workspace_bytes(int64_t n, int64_t v, int64_t d, int dtype, int terms);
+int cce_loss_call(const void* e, const void* c, const void* bias, const int64_t* labels, int32_t* rows, int64_t* count,
+                  float* lse, float* tile_max, float* loss, float* lse_out, void* workspace, int64_t workspace_bytes,
+                  int64_t n, int64_t steps, int64_t v, int64_t d, int64_t stride_e, int64_t stride_cv, int64_t stride_cd,
+                  int64_t shift, int64_t ignored, int64_t target_offset, float softcap, int reduction, int dtype, int terms, void* stream);
 
 /*
  * fp32 inputs.  The matrix cores multiply 16-bit numbers: every value is split into bf16 parts, x = hi + mid + lo, and a

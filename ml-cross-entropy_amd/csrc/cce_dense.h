@@ -81,5 +81,8 @@ struct LossRowsParams {
   float softcap;
 };
 int loss_rows_launch(const LossRowsParams& p, int dtype, hipStream_t stream);
+// *out = the sum or mean of values[n] (n == 0: 0 or NaN), added up in fp64
+int64_t row_total_workspace_bytes(int64_t n);
+int row_total_launch(const float* values, int64_t n, bool mean, float* out, void* workspace, hipStream_t stream);
 
 }  // namespace cce

@@ -49,7 +49,8 @@ __global__ __launch_bounds__(kRowThreads) void valid_rows_kernel(const int64_t* 
     base += s_total;
     __syncthreads();  // the counts are read before the next trip writes them
   }
-  if (tid == 0) *count = base;
+  // (a store that the host sees when it is made, not when the kernel has ended: cce_loss_call looks for it)
+  if (tid == 0) __hip_atomic_store(count, static_cast<int64_t>(base), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // out[p] = values[r] where rows[r] + shift == p, 0 where there is no such r: the values of the valid rows (rows as
@@ -144,6 +145,8 @@ __device__ __forceinline__ void z_loss_result(const ZPartial& all, bool mean, fl
   if (count != nullptr) *count = static_cast<float>(all.count);
 }
 
+// SQUARE: the z-loss; else plain values, all of which count (the reduction of the loss itself)
+template <bool SQUARE>
 __global__ __launch_bounds__(kZThreads) void z_loss_sum_kernel(ZLossParams p, bool mean, ZPartial* partial, float* out, float* count) {
   __shared__ ZPartial s_part[kZThreads / 64];
   ZPartial mine = {0.0, 0};
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(kZThreads) void z_loss_sum_kernel(ZLossParams p, bo
     const int r = static_cast<int>(i) / p.cols, c = static_cast<int>(i) - r * p.cols;
     if (z_loss_counts(p, r, c)) {
       const float x = p.lse[r * p.lse_stride + c];
-      mine.sum += static_cast<double>(x * x);
+      mine.sum += static_cast<double>(SQUARE ? x * x : x);
       ++mine.count;
     }
   }
@@ -312,6 +315,24 @@ int loss_rows_launch(const LossRowsParams& p, int dtype, hipStream_t stream) {
   return status_from_hip(hipGetLastError());
 }
 
+static int sum_blocks(int64_t n) {
+  const int64_t wanted = (n + kZPerBlock - 1) / kZPerBlock;
+  return static_cast<int>(wanted < 1 ? 1 : wanted > kZBlocks ? kZBlocks : wanted);
+}
+template <bool SQUARE>
+static int sum_launch(const ZLossParams& p, int blocks, bool mean, ZPartial* partial, float* out, float* count, hipStream_t stream) {
+  hipLaunchKernelGGL(z_loss_sum_kernel<SQUARE>, dim3(blocks), dim3(kZThreads), 0, stream, p, mean, partial, out, count);
+  if (blocks > 1)
+    hipLaunchKernelGGL(z_loss_total_kernel, dim3(1), dim3(kZThreads), 0, stream, partial, blocks, mean, out, count);
+  return status_from_hip(hipGetLastError());
+}
+
+int64_t row_total_workspace_bytes(int64_t n) { return sum_blocks(n) > 1 ? kZBlocks * static_cast<int64_t>(sizeof(ZPartial)) : 0; }
+int row_total_launch(const float* values, int64_t n, bool mean, float* out, void* workspace, hipStream_t stream) {
+  const ZLossParams p = {values, nullptr, n, 0, 0, static_cast<int>(n), static_cast<int>(n > 0 ? n : 1)};
+  return sum_launch<false>(p, sum_blocks(n), mean, static_cast<ZPartial*>(workspace), out, nullptr, stream);
+}
+
 }  // namespace cce
 
 using namespace cce;
@@ -392,16 +413,12 @@ extern "C" int cce_z_loss_forward(const float* lse, int64_t lse_stride, const in
     return status_from_hip(hipGetLastError());
   }
   const bool mean = reduction == CCE_REDUCTION_MEAN;
-  const int64_t wanted = (n + kZPerBlock - 1) / kZPerBlock;
-  const int blocks = static_cast<int>(wanted < 1 ? 1 : wanted > kZBlocks ? kZBlocks : wanted);
+  const int blocks = sum_blocks(n);
   if (blocks > 1 && (workspace == nullptr || workspace_bytes < cce_z_loss_workspace_bytes(rows, cols)))
     return CCE_ERR_WORKSPACE_TOO_SMALL;
   if ((reinterpret_cast<uintptr_t>(workspace) & 7u) != 0) return CCE_ERR_MISALIGNED;
   ZPartial* const partial = static_cast<ZPartial*>(workspace);
-  hipLaunchKernelGGL(z_loss_sum_kernel, dim3(blocks), dim3(kZThreads), 0, stream, p, mean, partial, out, count);
-  if (blocks > 1)
-    hipLaunchKernelGGL(z_loss_total_kernel, dim3(1), dim3(kZThreads), 0, stream, partial, blocks, mean, out, count);
-  return status_from_hip(hipGetLastError());
+  return sum_launch<true>(p, blocks, mean, partial, out, count, stream);
 }
 
 extern "C" int cce_z_loss_backward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows,

@@ -21,6 +21,7 @@ DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1}
 STAT_ROWS = 32
 STAT_COLS = 32
 NUM_COUNTERS = 4
+ERR_WORKSPACE_TOO_SMALL = 10003
 STATIC_SCRATCH_BYTES = 8 * 1024 * 1024
 
 _i64, _i32, _f32, _ptr = ctypes.c_int64, ctypes.c_int, ctypes.c_float, ctypes.c_void_p
@@ -74,6 +75,8 @@ _SIGNATURES = {
     "cce_z_loss_backward": (_i32, [_ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _ptr, _i32, _ptr, _ptr, _ptr]),
     "cce_valid_rows": (_i32, [_ptr, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr]),
     "cce_loss_forward": (_i32, [_ptr] * 9 + [_i64] + [_i64] * 4 + [_i64] * 3 + [_i64, _i64, _f32, _i32, _ptr]),
+    "cce_loss_call_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32, _i32]),
+    "cce_loss_call": (_i32, [_ptr] * 11 + [_i64] * 8 + [_i64] * 3 + [_f32, _i32, _i32, _i32, _ptr]),
     "cce_fp32_forward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),
     "cce_fp32_forward": (_i32, [_ptr] * 8 + [_i64] + [_i64] * 4 + [_i64] * 3 + [_i64, _i64, _f32, _i32, _ptr]),
     "cce_fp32_backward_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32]),

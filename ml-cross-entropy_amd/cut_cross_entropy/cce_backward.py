@@ -80,7 +80,7 @@ class _FlaggedMonitor:
     forgotten = False  # what was measured so far does not count any more
 
     def __init__(self, device: torch.device):
-        self.scratch: dict = {}  # stream -> the word its measurements count in
+        self.scratch: dict = {}  # handle of a stream -> the word its measurements count in, and the stream
         self.host = torch.zeros((1,), dtype=torch.int64, pin_memory=True)
         self.event = torch.cuda.Event()
         self.pending_cells = 0   # cells of the measurement in flight (0: none)
@@ -105,15 +105,15 @@ class _FlaggedMonitor:
             self.fraction, self.forgotten = None, False
 
     def measure(self, lib, tile_max, lse, B: int, V: int, filter_eps: float, dev: torch.device) -> None:
-        stream = torch.cuda.current_stream(dev)
-        scratch = self.scratch.get(stream.cuda_stream)
-        if scratch is None:
+        handle = _hip.current_stream_ptr(dev)
+        if handle not in self.scratch:
             if len(self.scratch) >= 16:  # streams come and go; whatever of theirs is still running holds its own memory
                 self.scratch.clear()
-            scratch = self.scratch[stream.cuda_stream] = torch.zeros((1,), dtype=torch.int64, device=dev)
+            self.scratch[handle] = torch.zeros((1,), dtype=torch.int64, device=dev), torch.cuda.current_stream(dev)
+        scratch, stream = self.scratch[handle]
         with _hip.on_device(dev):
             status = lib.cce_measure_flagged_cells(tile_max.data_ptr(), lse.data_ptr(), B, V, float(filter_eps),
-                                                   scratch.data_ptr(), self.host.data_ptr(), stream.cuda_stream)
+                                                   scratch.data_ptr(), self.host.data_ptr(), handle)
         _hip.check(status, "cce_measure_flagged_cells")
         self.event.record(stream)
         self.pending_cells = lib.cce_tile_stat_elems(B, V)

@@ -1,11 +1,15 @@
 """Launcher of the fused matmul + log-sum-exp kernel
 (reference: cut_cross_entropy/cce_lse_forward.py:170-237)."""
 
+import threading
 from typing import Optional, Tuple, Union
 
 import torch
 
 from cut_cross_entropy import _hip
+
+REDUCTION_CODES = {"none": 0, "sum": 1, "mean": 2}
+_pinned = threading.local()  # the word of pinned host memory that a thread receives its counts in
 
 
 def lse_forward(
@@ -113,6 +117,67 @@ def loss_forward(
         )
     _hip.check(status, "cce_loss_forward")
     return lse, nll, tile_max
+
+
+def loss_call(
+    e: torch.Tensor,
+    c: torch.Tensor,
+    bias: Optional[torch.Tensor],
+    targets: torch.Tensor,
+    shift: int,
+    ignore_index: int,
+    softcap: Optional[float],
+    target_offset: int,
+    reduction: str,
+    return_lse: bool,
+    want_tile_max: bool,
+    terms: int,
+):
+    """The whole forward in one library call: ``(rows, count, outputs)``.  ``rows[:count]`` are the valid rows of the flattened
+    ``e`` for labels ``targets`` [batch.., steps]; ``outputs`` is ``(loss, lse_out | None, lse[count], tile_max | None)``, or
+    None where so few rows count that their plan wants more scratch than was set aside (the single calls take any).
+    ``terms``: cross terms per product of fp32 inputs, 0 for 16-bit ones."""
+    dev = e.device
+    _hip.require_one_gpu(e, c, bias, targets)
+    assert c.dtype == e.dtype and e.ndim == 2 and c.ndim == 2 and e.shape[1] == c.shape[1]
+    n, (v, d), steps = e.shape[0], c.shape, targets.size(-1)
+    assert targets.numel() == n
+    code = 2 if terms else _hip.dtype_code(e.dtype)
+    lib = _hip.load()
+    if bias is not None:
+        assert bias.ndim == 1 and bias.shape[0] == v
+        bias = bias.to(e.dtype).contiguous()
+    batch = targets.shape
+    kept = batch[:-1] + (steps - shift,) if shift else batch
+    targets = targets.to(torch.int64).contiguous()
+    rows = torch.empty((n,), dtype=torch.int32, device=dev)
+    lse = torch.empty((n,), dtype=torch.float32, device=dev)
+    tile_max = torch.empty((lib.cce_tile_stat_elems(n, v),), dtype=torch.float32, device=dev) if want_tile_max else None
+    loss = torch.empty(kept if reduction == "none" else (), dtype=torch.float32, device=dev)
+    lse_out = torch.empty(kept, dtype=torch.float32, device=dev) if return_lse else None
+    ws_bytes = lib.cce_loss_call_workspace_bytes(n, v, d, code, terms)
+    ws = torch.empty((ws_bytes + 256,), dtype=torch.uint8, device=dev)
+    count = getattr(_pinned, "count", None)
+    if count is None:
+        count = _pinned.count = torch.zeros((1,), dtype=torch.int64, pin_memory=True)
+    with _hip.on_device(dev), _hip.timed("forward_fp32" if terms else "lse_forward", dev):
+        status = lib.cce_loss_call(
+            e.data_ptr(), c.data_ptr(), _hip.ptr(bias), targets.data_ptr(), rows.data_ptr(), count.data_ptr(), lse.data_ptr(),
+            _hip.ptr(tile_max), loss.data_ptr(), _hip.ptr(lse_out), (ws.data_ptr() + 255) // 256 * 256, ws_bytes,
+            n, steps, v, d, e.stride(0), c.stride(0), c.stride(1), shift, ignore_index, target_offset,
+            float(softcap) if softcap is not None else 0.0, REDUCTION_CODES[reduction], code, terms,
+            _hip.current_stream_ptr(dev))
+    b = count.item()
+    if status == _hip.ERR_WORKSPACE_TOO_SMALL and b >= 0:
+        return rows, b, None
+    _hip.check(status, "cce_loss_call")
+    if return_lse and b == n and not shift:
+        lse_out = lse.view(batch)
+    if b < n:
+        lse = lse[:b]
+        if tile_max is not None:
+            tile_max = tile_max[: lib.cce_tile_stat_elems(b, v)]
+    return rows, b, (loss, lse_out, lse, tile_max)
 
 
 def cce_lse_forward_kernel(

@@ -834,3 +834,52 @@ def test_the_dense_implementation_needs_no_library(monkeypatch, shift, ignored):
     (g_e, g_c), value = torch.func.grad_and_value(loss_of, argnums=(0, 1))(e.detach(), c.detach(), t)
     assert torch.allclose(value, loss.detach())
     assert torch.allclose(g_e, e.grad, atol=1e-7) and torch.allclose(g_c, c.grad, atol=1e-7)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+@pytest.mark.parametrize("shape,shift,keep", [((1, 1), 0, 1.0), ((2, 200), 0, 1.0), ((2, 200), 0, 0.6), ((3, 130), 2, 0.7), ((4, 300), 1, 0.02),
+                                              ((2, 50), 1, 0.0), ((1, 17000), 0, 0.9)])
+def test_the_forward_call_equals_its_single_calls(monkeypatch, dtype, reduction, shape, shift, keep):
+    """The forward in one library call, against the list of rows, the loss and the reduction called one by one, which is also what runs where
+    few rows need more scratch than was set aside: the same losses, log-sum-exps and gradients."""
+    from cut_cross_entropy import cce, linear_cross_entropy
+
+    g = torch.Generator().manual_seed(sum(shape))
+    e = torch.randn((*shape, 128), generator=g).to(dtype).cuda().requires_grad_(True)
+    c = (torch.randn((1000, 128), generator=g) * 0.2).to(dtype).cuda().requires_grad_(True)
+    t = torch.randint(0, 1000, shape, generator=g)
+    t[torch.rand(shape, generator=g) >= keep] = -100
+    t = t.cuda()
+
+    def results():
+        loss, lse = linear_cross_entropy(e, c, t, reduction=reduction, shift=shift, return_lse=True, impl="cce_exact")
+        assert loss.shape == (lse.shape if reduction == "none" else ()) and lse.shape == (*shape[:-1], shape[-1] - shift)
+        e.grad = c.grad = None
+        (loss.sum() + 0.1 * lse.sum()).backward()
+        return loss.detach(), lse.detach(), e.grad, c.grad
+
+    one = results()
+    whole = cce.loss_call
+    monkeypatch.setattr(cce, "loss_call", lambda *a: whole(*a)[:2] + (None,))
+    single = results()
+    for x, y in zip(one, single):
+        if x.ndim == 0:  # sums of up to 17000 values in fp64 and in fp32
+            assert torch.allclose(x, y, rtol=1e-5, atol=0, equal_nan=True)
+        else:
+            assert torch.equal(x, y)
+
+
+def test_the_forward_call_refuses_a_capture():
+    """A captured stream runs nothing, and the number of valid rows would never arrive: an error, not a wait."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    e, c, t, _ = (x.cuda() if x is not None else None for x in make_inputs(64, 300, 128, torch.bfloat16, seed=1))
+    want = linear_cross_entropy(e, c, t)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError):
+        with torch.cuda.graph(graph):
+            linear_cross_entropy(e, c, t)
+    torch.cuda.synchronize()
+    assert torch.equal(linear_cross_entropy(e, c, t), want)
