@@ -678,3 +678,24 @@ def test_z_loss_kernels_against_tensor_operations(shape, shift, reduction, label
         assert torch.allclose(tangent.sum(), all_ones.sum(), rtol=1e-5, atol=1e-5, equal_nan=True)
         pair = torch.vmap(lambda x: utils.compute_z_loss(x, t, shift, reduction=reduction))(torch.stack([plain, plain]))
         assert torch.allclose(pair[1], out.detach(), rtol=1e-6, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("shape,budget", [((4744, 6303, 320), 7 << 20), ((5308, 4438, 128), 5 << 20), ((9380, 4245, 320), 16 << 20),
+                                          ((10691, 3041, 192), 11 << 20)])
+def test_cut_reductions_in_more_launches(monkeypatch, shape, budget):
+    """Buffers in which the slots of a cut reduction fit only beside smaller chunks than whole reductions would take: dC cut chunk by
+    chunk, dE cut block by block, several launches of either.  Against the formulas in fp64."""
+    from cut_cross_entropy import cce_backward as bw
+    from cut_cross_entropy import linear_cross_entropy
+
+    monkeypatch.setattr(bw, "DENSE_DZ_BYTES", budget)
+    monkeypatch.setattr(bw, "DENSE_DZ_MIN_CLASSES", 256)
+    N, V, D = shape
+    e, c, t, _ = make_inputs(N, V, D, torch.bfloat16, seed=9, planted=False, c_std=0.3)
+    e, c, t = e.cuda().requires_grad_(True), c.cuda().requires_grad_(True), t.cuda()
+    linear_cross_entropy(e, c, t, reduction="sum", impl="cce_exact").backward()
+    p = torch.softmax(e.detach().double() @ c.detach().double().T, 1)
+    p[torch.arange(N, device="cuda"), t] -= 1.0
+    for got, want in ((e.grad, p @ c.detach().double()), (c.grad, p.T @ e.detach().double())):
+        # dz and the result are rounded to bf16, 2^-9 of every product and of the sum: the bound of the cuts above
+        assert torch.isfinite(got).all() and (got.double() - want).norm() <= 6e-3 * want.norm()
