@@ -944,39 +944,60 @@ inline int compute_units() {
   return n;
 }
 
-// Vocabulary spans per row block for the kernels that cut the (row block, vocabulary) plane into
-// items of one row block x one span of tiles.  Two things are weighed: the rounds of 256 workgroups
-// the items make, and the L2 traffic of the 32 workgroups that run on one XCD at a time, which cover
-// 32 / s row blocks (one E block each) times s spans (one stream of C tiles each): s + 32 / s streams,
-// least for s = 4 .. 8, and 32 + 1 for any s beyond 32.  The weight 0.165 is fitted to measurements at
-// E [65536, 3584] x C [152064, 3584] (1, 2, 4, 8, 16 spans: 70.8, 62.5, 53.9, 56.8, 59.4 ms).
-// Up to 64 spans are weighed, and as many as fill the chip where the row blocks are fewer than that takes: one row
-// block against 256000 classes of 2304 columns is 847 us in 64 spans (a quarter of the compute units) and 262 us in 250 (4.5 TB/s).
+// How the (row block, vocabulary) plane is cut into items of one row block x one span of tiles, and in which order the items
+// are numbered.  The 32 workgroups that run on one XCD at a time take consecutive numbers and share its L2: what they stream is
+// one block of E per row block and one stream of C tiles per span among them.  Numbered block_rows row blocks x block_spans
+// spans at a time (span by span inside a row block, then the next row block), 32 items are about A + 32 / A streams, least for A
+// = 4 .. 8; numbered row block by row block (block_rows == 1, block_spans == spans) s + 32 / s for s spans.
 struct SpanChoice {
-  int count;
-  double cost;  // of the launch, in times of one tile
+  int count;                   // spans per row block
+  int block_rows, block_spans;
+  double cost;                 // of the launch, in times of one tile
 };
+__device__ __forceinline__ void item_place(int item, int nrb, int nsplit, int block_rows, int block_spans, int& rb, int& split) {
+  const int rows_first = item / (block_rows * nsplit) * block_rows;
+  const int rows = min(block_rows, nrb - rows_first);
+  item -= rows_first * nsplit;
+  const int spans_first = item / (rows * block_spans) * block_spans;
+  const int spans = min(block_spans, nsplit - spans_first);
+  item -= rows * spans_first;
+  rb = rows_first + item / spans;
+  split = spans_first + item % spans;
+}
+
+// Two things are weighed: the rounds of 256 workgroups the items make, and those streams.  The weight 0.165 is fitted to
+// measurements at E [65536, 3584] x C [152064, 3584] (1, 2, 4, 8, 16 spans, row block by row block: 70.8, 62.5, 53.9, 56.8, 59.4
+// ms).  Up to 64 spans are weighed, and as many as fill the chip where the row blocks are fewer than that takes: one row
+// block against 256000 classes of 2304 columns is 847 us in 64 spans (a quarter of the compute units) and 262 us in 250 (4.5 TB/s).
+// Blocks are for few row blocks, which have to be cut into more than 20 spans to fill the chip: 32 streams become 11 - 18.  Forward, row
+// block by row block / in blocks, us: 900 x 1024 x 50257 (four row blocks) 97 / 91, 900 x 1000 x 50257 142 / 126, 1024 x 4096 x 128256
+// 860 / 818, 307 x 5120 x 131072 521 / 496.  With many row blocks the longer spans of fewer items are the faster ones whatever the
+// estimate says (60 row blocks x 501 tiles: 4 spans of 126 tiles take less than 17 of 30, forward and backward 51.3 / 51.9 ms; 32 x
+// 1000 in 8 spans, 4 x 8 or 5 x 7 at a time: 8.70 / 8.79; 15 row blocks x 142 tiles 0.393 / 0.403).
+constexpr int kFewRowBlocks = 12;
 inline SpanChoice choose_spans(int nrb, int nvt) {
   const int num_cu = compute_units();  // (the size query and the launch must see the same device)
-  int best = 1;
-  double best_cost = 1e300;
+  SpanChoice best = {1, 1, 1, 1e300};
   const int most = num_cu / nrb > 64 ? num_cu / nrb : 64;
   const int max_split = nvt < most ? nvt : most;
   for (int s = 1; s <= max_split; ++s) {
     const int64_t items = static_cast<int64_t>(nrb) * s;
     const int64_t rounds = (items + num_cu - 1) / num_cu;
     const int tiles_per_item = (nvt + s - 1) / s;
-    const double streams = (s <= 32) ? s + 32.0 / s : 33.0;
+    double streams = (s <= 32) ? s + 32.0 / s : 33.0;
+    int rows = 1;
+    for (int a = 2; a <= 8 && a <= nrb && nrb < kFewRowBlocks; ++a) {
+      if ((32 + a - 1) / a <= s && a + 32.0 / a < streams - 0.5) {
+        streams = a + 32.0 / a;
+        rows = a;
+      }
+    }
     const double traffic = 1.0 + 0.165 * (streams / 11.3137 - 1.0);
     const double cost = static_cast<double>(rounds) * tiles_per_item * traffic + 0.002 * s;
-    if (cost < best_cost - 1e-9) {
-      best_cost = cost;
-      best = s;
-    }
+    if (cost < best.cost - 1e-9) best = {s, rows, rows == 1 ? s : (32 + rows - 1) / rows, cost};
   }
-  return {best, best_cost};
+  return best;
 }
-inline int choose_span_count(int nrb, int nvt) { return choose_spans(nrb, nvt).count; }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -31,6 +31,7 @@ struct DzParams {
   int pad_store;  // also store the (zero) gradients of the classes between v and the end of their 16-byte piece,
                   // up to column ldz: the product kernels read dz in whole 64-class stages
   int nrb, nvt, nsplit, nitems, items_per_xcd;
+  int block_rows, block_spans;  // the order of the items (item_place)
   Softcap sc;
   // operands and dz in 16-bit parts (kDzParts): d is the width of a part, rows of e are compact (valids only says which
   // targets and upstream gradients they belong to), dz is [b_store][parts][ldz], rows past b zeros
@@ -62,8 +63,8 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz_kernel(DzParams p) {
   if (slot >= p.items_per_xcd) return;
   const int item = xcd * p.items_per_xcd + slot;
   if (item >= p.nitems) return;
-  const int rb = item / p.nsplit;
-  const int split = item % p.nsplit;
+  int rb, split;
+  item_place(item, p.nrb, p.nsplit, p.block_rows, p.block_spans, rb, split);
   const int vt_begin = static_cast<int>((static_cast<int64_t>(p.nvt) * split) / p.nsplit);
   const int vt_end = static_cast<int>((static_cast<int64_t>(p.nvt) * (split + 1)) / p.nsplit);
 
@@ -278,8 +279,8 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   if (slot >= p.items_per_xcd) return;
   const int item = xcd * p.items_per_xcd + slot;
   if (item >= p.nitems) return;
-  const int rb = item / p.nsplit;
-  const int split = item % p.nsplit;
+  int rb, split;
+  item_place(item, p.nrb, p.nsplit, p.block_rows, p.block_spans, rb, split);
   const int vt_begin = static_cast<int>((static_cast<int64_t>(p.nvt) * split) / p.nsplit);
   const int vt_end = static_cast<int>((static_cast<int64_t>(p.nvt) * (split + 1)) / p.nsplit);
   if (vt_begin >= vt_end) return;
@@ -531,7 +532,10 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
   p.pad_store = pad_store;
   p.nrb = static_cast<int>((b + kDzTile - 1) / kDzTile);
   p.nvt = static_cast<int>((v + kDzTile - 1) / kDzTile);
-  p.nsplit = choose_span_count(p.nrb, p.nvt);
+  const SpanChoice spans = choose_spans(p.nrb, p.nvt);
+  p.nsplit = spans.count;
+  p.block_rows = spans.block_rows;
+  p.block_spans = spans.block_spans;
   p.nitems = p.nrb * p.nsplit;
   p.items_per_xcd = (p.nitems + 7) / 8;
   p.sc = make_softcap(softcap);
@@ -612,7 +616,10 @@ int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_par
   p.d_out_is_scalar = d_out_is_scalar;
   p.nrb = static_cast<int>((b + kDzTile - 1) / kDzTile);
   p.nvt = static_cast<int>((v + kDzTile - 1) / kDzTile);
-  p.nsplit = choose_span_count(p.nrb, p.nvt);
+  const SpanChoice spans = choose_spans(p.nrb, p.nvt);
+  p.nsplit = spans.count;
+  p.block_rows = spans.block_rows;
+  p.block_spans = spans.block_spans;
   p.nitems = p.nrb * p.nsplit;
   p.items_per_xcd = (p.nitems + 7) / 8;
   p.sc = make_softcap(softcap);

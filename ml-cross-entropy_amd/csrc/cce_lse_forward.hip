@@ -30,6 +30,7 @@ struct LseFwdParams {
   int64_t b, v, d, n_rows;
   int64_t stride_e, stride_cv, stride_cd;
   int nrb, nvt, nsplit, nitems, items_per_xcd;
+  int block_rows, block_spans;  // the order of the items (item_place)
   int stat_cols;
   Softcap sc;
   float avg_scale;  // ln 2 / b: turns a column sum in log2 units into its share of logit_avg
@@ -116,8 +117,8 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward_kernel(LseFwdParam
   if (slot >= p.items_per_xcd) return;
   const int item = xcd * p.items_per_xcd + slot;
   if (item >= p.nitems) return;
-  const int rb = item / p.nsplit;
-  const int split = item % p.nsplit;
+  int rb, split;
+  item_place(item, p.nrb, p.nsplit, p.block_rows, p.block_spans, rb, split);
   const int vt_begin = static_cast<int>((static_cast<int64_t>(p.nvt) * split) / p.nsplit);
   const int vt_end = static_cast<int>((static_cast<int64_t>(p.nvt) * (split + 1)) / p.nsplit);
 
@@ -420,8 +421,8 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward16_kernel(LseFwdPar
   if (slot >= p.items_per_xcd) return;
   const int item = xcd * p.items_per_xcd + slot;
   if (item >= p.nitems) return;
-  const int rb = item / p.nsplit;
-  const int split = item % p.nsplit;
+  int rb, split;
+  item_place(item, p.nrb, p.nsplit, p.block_rows, p.block_spans, rb, split);
   const int vt_begin = static_cast<int>((static_cast<int64_t>(p.nvt) * split) / p.nsplit);
   const int vt_end = static_cast<int>((static_cast<int64_t>(p.nvt) * (split + 1)) / p.nsplit);
 
@@ -673,18 +674,27 @@ __global__ void fill_zero_kernel(float* p, int64_t n) {
   if (i < n) p[i] = 0.0f;
 }
 
-static int choose_nsplit(int nrb, int nvt) { return choose_span_count(nrb, nvt); }
-
 struct RowBlocks {
-  int rows, nrb, nvt, nsplit;
+  int rows, nrb, nvt, nsplit, block_rows, block_spans;
   int64_t partial_bytes(int64_t b) const { return static_cast<int64_t>(nsplit) * b * static_cast<int64_t>(sizeof(float2)); }
 };
 static RowBlocks blocks_of(int rows, int64_t b, int64_t v, double* cost = nullptr) {
-  RowBlocks r = {rows, static_cast<int>((b + rows - 1) / rows), static_cast<int>((v + kFwdTile - 1) / kFwdTile), 0};
+  RowBlocks r = {rows, static_cast<int>((b + rows - 1) / rows), static_cast<int>((v + kFwdTile - 1) / kFwdTile), 0, 0, 0};
   const SpanChoice s = choose_spans(r.nrb, r.nvt);
   r.nsplit = s.count;
+  r.block_rows = s.block_rows;
+  r.block_spans = s.block_spans;
   if (cost != nullptr) *cost = s.cost;
   return r;
+}
+static void take_blocks(LseFwdParams& p, const RowBlocks& r) {
+  p.nrb = r.nrb;
+  p.nvt = r.nvt;
+  p.nsplit = r.nsplit;
+  p.block_rows = r.block_rows;
+  p.block_spans = r.block_spans;
+  p.nitems = p.nrb * p.nsplit;
+  p.items_per_xcd = (p.nitems + 7) / 8;
 }
 // Rows per block of the 16 x 16 x 32 kernel: 256, or 192 where that leaves fewer rows of padding or an emptier last round
 // less work.  A tile of 192 rows has three quarters of the products but 56 of the 64 KB of loads per stage, and more
@@ -731,11 +741,7 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64
     if (best.partial_bytes(p.b) <= workspace_bytes) blocks = best;
   }
   const bool mid = blocks.rows == kFwdMidRows;
-  p.nrb = blocks.nrb;
-  p.nvt = blocks.nvt;
-  p.nsplit = blocks.nsplit;
-  p.nitems = p.nrb * p.nsplit;
-  p.items_per_xcd = (p.nitems + 7) / 8;
+  take_blocks(p, blocks);
   const bool general = want_la || (p.bias != nullptr) || (p.v % Tile::TILE_V != 0);
   const int grid = p.items_per_xcd * 8;
   hipError_t err;
@@ -792,7 +798,7 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64
 
 // ---- the forward over one chunk of classes with operands in 16-bit parts (cce_fp32.hip) ------------------------
 int lse_terms_splits(int64_t b, int64_t v) {
-  return choose_nsplit(static_cast<int>((b + 255) / 256), static_cast<int>((v + 255) / 256));
+  return blocks_of(kFwdTile, b, v).nsplit;
 }
 
 int lse_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
@@ -810,11 +816,7 @@ int lse_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_pa
   p.stride_e = ld_e;
   p.stride_cv = ld_c;
   p.stride_cd = 1;
-  p.nrb = static_cast<int>((b + 255) / 256);
-  p.nvt = static_cast<int>((v + 255) / 256);
-  p.nsplit = choose_nsplit(p.nrb, p.nvt);
-  p.nitems = p.nrb * p.nsplit;
-  p.items_per_xcd = (p.nitems + 7) / 8;
+  take_blocks(p, blocks_of(kFwdTile, b, v));
   p.sc = make_softcap(softcap);
   p.cap_inv = p.sc.on ? 1.0f / (-2.0f * p.sc.out_scale) : 0.0f;
   using Fast = DmaLogitTile16<BF16, kF16WV, kF16WT, kFwdNWV, kFwdNWT, true>;
