@@ -59,9 +59,18 @@ struct BwdParams {
   int parts;
   float* slots;
   uint32_t* part_bits;  // [parts][ntg][bit_words]
+  // Gradients of surviving sub-tiles kept by the dE pass for what comes after it (fast kernels): candidate k of a row group, in
+  // the order of its list, has slot k of the group's dz_quota (later ones are formed again where they are needed).
+  int dz_mode;          // kDzNone, kDzStore (slice 0 of this dE pass), kDzRead
+  int dz_quota;
+  uint16_t* dz_slots;   // [ntg][dz_quota][32 rows][32 classes]
+  uint32_t* cand_bits;  // [ntg][bit_words]: the candidates, as kept_bits has the survivors; a slot is found by counting bits
+  int slice_first;      // slice of D of the first workgroups
   Softcap sc;
 };
 
+constexpr int kDzNone = 0, kDzStore = 1, kDzRead = 2;
+constexpr int kDzSlotElems = 32 * 32;
 constexpr int kStageCols = 256;               // columns of D per LDS stage
 constexpr int kStageRowBytes = kStageCols * 2;
 constexpr int kMaxChunks = 9;                 // 9 * 256 = 2304 columns of D per workgroup
@@ -704,7 +713,9 @@ __device__ __forceinline__ void wait_vmcnt_upto_wide(int n) {
   }
 }
 
-template <typename T, bool IS_DE, bool LIGHT = false, bool TAIL = false>
+// KEEP: gradients of surviving sub-tiles are kept or read (p.dz_mode); a variant of its own, since what every trip asks for it
+// costs the others 1 - 3 %.
+template <typename T, bool IS_DE, bool LIGHT = false, bool TAIL = false, bool KEEP = false>
 __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_kernel(BwdParams p) {
   static_assert(!(LIGHT && IS_DE), "the light variant is a dC pass");
   using Lds = FastLds<LIGHT>;
@@ -733,7 +744,7 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   const int parts = IS_DE ? p.parts : 1;
   const int part = IS_DE ? static_cast<int>(blockIdx.x) % parts : 0;
   int own = blockIdx.x / (p.nslices * parts);
-  const int slice = (blockIdx.x / parts) % p.nslices;
+  const int slice = (KEEP ? p.slice_first : 0) + (blockIdx.x / parts) % p.nslices;
   if (IS_DE && blockIdx.x == 0 && threadIdx.x == 0 && p.heavy_list != nullptr) p.heavy_list[0] = 0;  // for the dC passes
   if (!IS_DE && !LIGHT && p.light_on) {
     // the full dC pass after the light one: only the class groups that one listed
@@ -767,7 +778,8 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
       const float mn = wave_min(my_lse);
       if (lane == 0) reinterpret_cast<float*>(sMisc)[2] = mn;
     }
-    for (int w = tid; w < p.bit_words; w += kBwdThreads) sBits[w] = 0u;
+    for (int w = tid; w < p.bit_words; w += kBwdThreads)
+      sBits[w] = KEEP && p.dz_mode == kDzRead ? p.kept_bits[static_cast<int64_t>(own) * p.bit_words + w] : 0u;
   } else if (tid < 32) {
     const int64_t pos = static_cast<int64_t>(own) * 32 + tid;
     int cid = -1;
@@ -861,6 +873,15 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
           if (IS_DE) {
             const int m = (base + lane < seg_n) ? sFlag[base + lane] : 0;
             const int cnt = __popc(m);
+            if (KEEP && p.dz_mode == kDzStore && slice == 0 && part == 0) {  // eight cells make a word of candidate bits
+              uint32_t w = static_cast<uint32_t>(m) << (4 * (lane & 7));
+              w |= __shfl_xor(w, 1, 64);
+              w |= __shfl_xor(w, 2, 64);
+              w |= __shfl_xor(w, 4, 64);
+              const int at = (seg + base + lane) >> 3;
+              if ((lane & 7) == 0 && base + lane < seg_n && at < p.bit_words)
+                p.cand_bits[static_cast<int64_t>(own) * p.bit_words + at] = w;
+            }
             int incl = cnt;
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) {
@@ -927,6 +948,7 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
         }
       }
       if (tid == 0) sMisc[1] = 0;
+      if (KEEP && tid == 0) sMisc[3] = 0;
       __syncthreads();
       const int* other_ids = IS_DE ? sCellCid : meta.row;
       // Waves and entries: with 3 or 4 entries in the trip wave w recomputes entry w over all of D; with
@@ -971,6 +993,55 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
         for (int q = 0; q < 8; ++q) issue_load(q, col0, slot, entries);
       };
 
+      // ---- gradients that the dE pass has kept: no logits, if every entry of the trip that survived has a slot ----------
+      bool kept_dz = false;
+      if (KEEP && p.dz_mode == kDzRead) {
+        bool mine = false;  // an entry of this wave's that enters the product
+        int64_t group = own;
+        int rank = 0;
+        if (wave < nent) {
+          const int id = sList[li + wave];
+          if (IS_DE) {
+            mine = ((sBits[id >> 5] >> (id & 31)) & 1u) != 0u;
+            rank = (trip - 1) * 4 + wave;
+          } else {
+            mine = true;
+            group = id;
+            const uint32_t* words = p.cand_bits + group * p.bit_words;
+            for (int w = lane; w <= (own >> 5); w += 64)
+              rank += __popc(w < (own >> 5) ? words[w] : words[w] & ((1u << (own & 31)) - 1u));
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) rank += __shfl_xor(rank, off, 64);
+          }
+        }
+        if (mine && rank >= p.dz_quota && lane == 0) atomicOr(&sMisc[3], 1);
+        __syncthreads();
+        kept_dz = sMisc[3] == 0;
+        if (kept_dz && mine) {
+          const uint16_t* slot = p.dz_slots + (group * p.dz_quota + rank) * kDzSlotElems + l32 * 32 + 4 * half;
+          uint2 pk[4];
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4) pk[r4] = *reinterpret_cast<const uint2*>(slot + 8 * r4);
+#pragma unroll
+          for (int r4 = 0; r4 < 4; ++r4) {
+            if (IS_DE) {
+              const int k = wave * 32 + 8 * r4 + 4 * half;
+              *reinterpret_cast<uint2*>(sDz + l32 * 256 + ((((k >> 3) ^ (l32 & 7)) << 4) | ((k & 7) << 1))) = pk[r4];
+            } else {
+              const int k = wave * 32 + l32;
+              const uint32_t w[2] = {pk[r4].x, pk[r4].y};
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int cls = 8 * r4 + 4 * half + j;
+                *reinterpret_cast<uint16_t*>(sDz + cls * 256 + ((((k >> 3) ^ (cls & 7)) << 4) | ((k & 7) << 1))) =
+                    static_cast<uint16_t>(w[j >> 1] >> (16 * (j & 1)));
+              }
+            }
+          }
+          if (lane == 0) atomicOr(&sMisc[1], 1 << wave);
+        }
+      }
+      if (!kept_dz) {
       // ---- logits^T of (entry of this wave) x (own rows): 2 nent + 2 loads per wave and stage -----------
       // One wave per SIMD issues every instruction of this loop by itself, so the loop is written once per
       // number of entries: ring geometry, wait counts and which loads exist are then compile-time facts and
@@ -1108,6 +1179,10 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
               pk.x = Elem<T>::pack2(s[r4 * 4 + 0], s[r4 * 4 + 1]);
               pk.y = Elem<T>::pack2(s[r4 * 4 + 2], s[r4 * 4 + 3]);
               *reinterpret_cast<uint2*>(sDz + l32 * 256 + ((((k >> 3) ^ (l32 & 7)) << 4) | ((k & 7) << 1))) = pk;
+              const int rank = (trip - 1) * 4 + ew;
+              if (KEEP && p.dz_mode == kDzStore && slice == 0 && rank < p.dz_quota)
+                *reinterpret_cast<uint2*>(p.dz_slots + (static_cast<int64_t>(own) * p.dz_quota + rank) * kDzSlotElems + l32 * 32 +
+                                          8 * r4 + 4 * half) = pk;
             }
           } else {
             const int k = ew * 32 + l32;
@@ -1127,6 +1202,7 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
           if (lane == 0) atomicOr(&sMisc[1], 1 << ew);
         }
       }
+      }  // !kept_dz
       __syncthreads();
       const uint32_t mask = static_cast<uint32_t>(sMisc[1]);
       const bool product = write_out && (mask != 0u);
@@ -1447,12 +1523,26 @@ static int64_t round16(int64_t x) { return (x + 15) / 16 * 16; }
 // what the parts keep behind the lists: bits, then slots
 static int64_t part_bits_bytes(int64_t b, int64_t v, int parts) { return parts > 1 ? round16(parts * kept_bits_bytes(b, v)) : 0; }
 static int64_t lists_bytes(int64_t b, int64_t v) { return kept_bits_bytes(b, v) + (1 + (v + 31) / 32) * 4; }
+// Slots per row group for the gradients of its candidates, 2 KB each: 40 (32 rows have a label each) where D is in slices and
+// every row group has a workgroup per slice.  Logits would be formed once per slice in either pass there: what is fetched for a
+// surviving sub-tile is 32 rows x D of C and of E twice or three times in the dE pass and as often in the dC pass, and once
+// less in the first and once in all in the second with its gradient kept.  Not with one slice: where D is narrow, the memory
+// of the loss path is the point (E [8192, 2304] x C [256000, 2304]: 9 MB, and 20 MB of slots).
+// E [65536, 3584] x C [152064, 3584], peaked: dE 6.9 -> 4.9 ms in two launches, dC 7.4 -> 2.9, forward and backward 62.8 -> 56.3, for 168 MB.
+static int dz_quota(int64_t b, int64_t v, int64_t d) {
+  return b > 0 && d > 0 && owner_slices(d) > 1 && owner_parts(b, v, d) == 1 ? 40 : 0;
+}
+// candidate bits, then slots
+static int64_t dz_bytes(int64_t b, int64_t v, int64_t d) {
+  const int64_t quota = dz_quota(b, v, d);
+  return quota == 0 ? 0 : round16(kept_bits_bytes(b, v)) + (b + 31) / 32 * quota * kDzSlotElems * 2;
+}
 
 extern "C" int64_t cce_backward_workspace_bytes(int64_t b, int64_t v, int64_t d) {
   if (b <= 0 || v <= 0) return 0;
   const int parts = owner_parts(b, v, d);
-  if (parts == 1) return lists_bytes(b, v);
-  return round16(lists_bytes(b, v)) + part_bits_bytes(b, v, parts) + parts * ((b + 31) / 32 * 32) * d * 4;
+  if (parts > 1) return round16(lists_bytes(b, v)) + part_bits_bytes(b, v, parts) + parts * ((b + 31) / 32 * 32) * d * 4;
+  return dz_quota(b, v, d) == 0 ? lists_bytes(b, v) : round16(lists_bytes(b, v)) + dz_bytes(b, v, d);
 }
 
 extern "C" int cce_backward(const void* e, const void* c, const void* bias,
@@ -1562,7 +1652,12 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
   } while (0)
 #define CCE_LAUNCH_OWNER(IS_DE_, GRID)                                                              \
   do {                                                                                              \
-    if (dtype == CCE_DTYPE_BF16) {                                                                  \
+    if (p.dz_mode != kDzNone) {                                                                     \
+      if (dtype == CCE_DTYPE_BF16 && tail) CCE_LAUNCH((bwd_owner_fast_kernel<BF16, IS_DE_, false, true, true>), kFLdsBytes, GRID); \
+      else if (dtype == CCE_DTYPE_BF16) CCE_LAUNCH((bwd_owner_fast_kernel<BF16, IS_DE_, false, false, true>), kFLdsBytes, GRID);  \
+      else if (tail) CCE_LAUNCH((bwd_owner_fast_kernel<F16, IS_DE_, false, true, true>), kFLdsBytes, GRID); \
+      else CCE_LAUNCH((bwd_owner_fast_kernel<F16, IS_DE_, false, false, true>), kFLdsBytes, GRID);   \
+    } else if (dtype == CCE_DTYPE_BF16) {                                                           \
       if (fast && tail) CCE_LAUNCH((bwd_owner_fast_kernel<BF16, IS_DE_, false, true>), kFLdsBytes, GRID); \
       else if (fast) CCE_LAUNCH((bwd_owner_fast_kernel<BF16, IS_DE_>), kFLdsBytes, GRID);           \
       else if (aligned) CCE_LAUNCH((bwd_owner_kernel<BF16, true, IS_DE_>), kBwdLdsBytes, GRID);     \
@@ -1575,21 +1670,47 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
     }                                                                                               \
   } while (0)
   const int full_slices = p.nslices;
+  p.dz_mode = kDzNone;
+  p.dz_quota = 0;
+  p.dz_slots = nullptr;
+  p.cand_bits = nullptr;
+  p.slice_first = 0;
   if (need_de_pass) {
     p.nslices = (d_e != nullptr) ? full_slices : 1;
-    // (a caller who brings less workspace than the size query names gets one workgroup per row group)
+    // (a caller who brings less workspace than the size query names gets one workgroup per row group and no kept gradients)
     const int parts = owner_parts(b, v, d);
-    if (fast && parts > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
+    if (fast && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
         workspace_bytes >= cce_backward_workspace_bytes(b, v, d)) {
-      unsigned char* const ws = static_cast<unsigned char*>(workspace) + round16(lists_bytes(b, v));
-      p.parts = parts;
-      p.part_bits = reinterpret_cast<uint32_t*>(ws);
-      p.slots = reinterpret_cast<float*>(ws + part_bits_bytes(b, v, parts));
+      unsigned char* ws = static_cast<unsigned char*>(workspace) + round16(lists_bytes(b, v));
+      if (parts > 1) {
+        p.parts = parts;
+        p.part_bits = reinterpret_cast<uint32_t*>(ws);
+        p.slots = reinterpret_cast<float*>(ws + part_bits_bytes(b, v, parts));
+      }
+      // dBias sums the gradients in fp32: with it they are formed again.  Without a candidate list there is no order to find them by.
+      if (dz_quota(b, v, d) > 0 && p.shortcut && need_bits && d_bias == nullptr) {
+        p.dz_mode = kDzStore;
+        p.dz_quota = dz_quota(b, v, d);
+        p.cand_bits = reinterpret_cast<uint32_t*>(ws);
+        p.dz_slots = reinterpret_cast<uint16_t*>(ws + round16(kept_bits_bytes(b, v)));
+      }
     }
-    const unsigned grid = static_cast<unsigned>(p.ntg) * static_cast<unsigned>(p.nslices) * static_cast<unsigned>(p.parts);
-    CCE_LAUNCH_OWNER(true, grid);
+    // Where the row groups fill the chip by themselves, the slices after the first are a launch of their own that reads what the
+    // first one kept; fewer row groups take all slices at once.
+    const bool later = p.dz_mode == kDzStore && p.nslices > 1 && p.ntg >= compute_units();
+    if (later) p.nslices = 1;
+    CCE_LAUNCH_OWNER(true, static_cast<unsigned>(p.ntg) * static_cast<unsigned>(p.nslices) * static_cast<unsigned>(p.parts));
     err = hipGetLastError();
     if (err != hipSuccess) return status_from_hip(err);
+    if (p.dz_mode == kDzStore) p.dz_mode = kDzRead;
+    if (later) {
+      p.nslices = full_slices - 1;
+      p.slice_first = 1;
+      CCE_LAUNCH_OWNER(true, static_cast<unsigned>(p.ntg) * static_cast<unsigned>(p.nslices));
+      err = hipGetLastError();
+      if (err != hipSuccess) return status_from_hip(err);
+      p.slice_first = 0;
+    }
     if (p.parts > 1) {
       const int64_t items = (d_e != nullptr ? b * (d / 8) : 0) + (p.kept_bits != nullptr ? static_cast<int64_t>(p.ntg) * p.bit_words : 0);
       const dim3 blocks(static_cast<unsigned>((items + 255) / 256));
@@ -1616,8 +1737,15 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
         hipLaunchKernelGGL(kern, dim3(grid), dim3(kBwdThreads), kFLightLdsBytes, stream, q);
         return hipGetLastError();
       };
-      static LdsLimitOnce limits[4];
-      if (dtype == CCE_DTYPE_BF16) {
+      static LdsLimitOnce limits[8];
+      if (q.dz_mode != kDzNone) {
+        if (dtype == CCE_DTYPE_BF16)
+          err = tail ? launch(bwd_owner_fast_kernel<BF16, false, true, true, true>, limits[4])
+                     : launch(bwd_owner_fast_kernel<BF16, false, true, false, true>, limits[5]);
+        else
+          err = tail ? launch(bwd_owner_fast_kernel<F16, false, true, true, true>, limits[6])
+                     : launch(bwd_owner_fast_kernel<F16, false, true, false, true>, limits[7]);
+      } else if (dtype == CCE_DTYPE_BF16) {
         err = tail ? launch(bwd_owner_fast_kernel<BF16, false, true, true>, limits[0])
                    : launch(bwd_owner_fast_kernel<BF16, false, true>, limits[1]);
       } else {

@@ -699,3 +699,34 @@ def test_cut_reductions_in_more_launches(monkeypatch, shape, budget):
     for got, want in ((e.grad, p @ c.detach().double()), (c.grad, p.T @ e.detach().double())):
         # dz and the result are rounded to bf16, 2^-9 of every product and of the sum: the bound of the cuts above
         assert torch.isfinite(got).all() and (got.double() - want).norm() <= 6e-3 * want.norm()
+
+
+@pytest.mark.parametrize("shape", [(8200, 2500, 2432), (4500, 1000, 2312), (8192, 3000, 4736)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("few_labels", [False, True])
+def test_gradients_kept_between_the_filtered_passes(monkeypatch, shape, dtype, few_labels):
+    """Widths in slices: the dE pass keeps the gradients of surviving sub-tiles, slices after the first (a launch of their own from 256 row
+    groups on) and the dC pass read them.  Row groups with fewer candidates than slots and with more (every class a label), a partial
+    last stage, against the same call with a bias of zeros, for whose gradient everything is formed again."""
+    from cut_cross_entropy import cce_backward as bw
+    from cut_cross_entropy import linear_cross_entropy
+
+    monkeypatch.setattr(bw, "FILTERED_BACKWARD_PATH", "sparse")
+    N, V, D = shape
+    g = torch.Generator(device="cuda").manual_seed(N + V)
+    c = (torch.randn((V, D), generator=g, device="cuda") * 0.02).to(dtype)
+    t = torch.randint(0, 40 if few_labels else V, (N,), generator=g, device="cuda")
+    other = torch.randint(0, V, (N,), generator=g, device="cuda")
+    gain = (30.0 / D) ** 0.5 / 0.02
+    e = gain * (c[t].float() + 0.9 * c[other].float()) * 0.2 + torch.randn((N, D), generator=g, device="cuda") * 0.1
+    e = e.to(dtype)
+    got = []
+    for bias in (None, torch.zeros((V,), dtype=dtype, device="cuda", requires_grad=True)):
+        e1, c1 = e.clone().requires_grad_(True), c.clone().requires_grad_(True)
+        linear_cross_entropy(e1, c1, t, bias=bias, softcap=50.0, reduction="sum", filter_eps=2.0**-9).backward()
+        got.append((e1.grad.double(), c1.grad.double()))
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and a.abs().max() > 0
+        # dz is rounded to the type from logits summed in another order: 2^-9 (bf16) of single products, and of the results
+        assert (a - b).norm() <= 2e-3 * b.norm()
+        assert ((a - b).abs() <= 2e-2 * b.abs() + 2e-2 * b.abs().amax(dim=1, keepdim=True)).all()
