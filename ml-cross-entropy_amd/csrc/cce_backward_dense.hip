@@ -22,13 +22,13 @@
 // of 800 stages on 256 compute units, and its mirror image, dC of a small vocabulary under many rows), the reduction
 // itself is cut: a tile becomes several items, each with a range of the reduction and an fp32 slot [rows, d] of its
 // own in the workspace, and split_sum_kernel adds the slots in a fixed order at the end (deterministic, no atomics).
-// Both products run on the tile loop of cce_tile4.h (direct-to-LDS loads, LDS transpose reads for the
+// Both products run on the tile loop of cce_tile8.h (direct-to-LDS loads, LDS transpose reads for the
 // operand whose reduction index is the row index).  Everything is enqueued on the caller's stream; nothing
 // is allocated, no host synchronisation.
 #include <algorithm>
 
 #include "cce_dense.h"
-#include "cce_tile4.h"
+#include "cce_tile8.h"
 
 namespace cce {
 
@@ -74,7 +74,7 @@ struct ProductParams {
   int cls_out;
 };
 
-constexpr int kProdThreads = 256;  // four waves, one per SIMD
+constexpr int kProdThreads = 512;  // eight waves, two per SIMD
 
 // Item `block` of a group of `items` = tiles x splits items (tiles_n column tiles wide).  Block ids that land on one XCD get
 // consecutive places in an order that keeps the 32 tiles an XCD works on at a time on few operand panels: a tile
@@ -138,38 +138,56 @@ __device__ __forceinline__ void store_piece(float* row, int col, int d, bool vec
   }
 }
 
+// Where the operands of a tile lie: dE = dz . C (rows m0 on, columns n0 on, classes k0 on) and dC = dz^T . E (classes m0 on, rows
+// k0 on).  Rows past the end repeat the last one, chunks past the `cols` columns of a matrix the last one inside it: their
+// results are dropped.
+template <typename Tile>
+__device__ __forceinline__ void de_source(typename Tile::Source& s, const ProductParams& p, const typename Tile::Geometry& g,
+                                          int64_t m0, int n0, int k0, int cols) {
+  s.a_base = reinterpret_cast<const unsigned char*>(p.dz + m0 * p.ldz + k0);
+  const int last = static_cast<int>(min(p.b - m0, static_cast<int64_t>(Tile::TILE))) - 1;
+#pragma unroll
+  for (int q = 0; q < Tile::NQ; ++q)
+    s.a_off[q] = 2u * (static_cast<unsigned>(min(Tile::row_direct(q, g.wave, g.lane), last)) * static_cast<unsigned>(p.ldz) +
+                       static_cast<unsigned>(Tile::chunk_direct(g.wave, g.lane)));
+  s.a_stride = 0;
+  s.b_base = reinterpret_cast<const unsigned char*>(p.c + k0 * p.stride_cv);
+  s.b_stride = static_cast<uint32_t>(2 * p.stride_cv);
+  s.b_off = (g.lane >> 5) * s.b_stride + 2u * static_cast<unsigned>(min(n0 + Tile::chunk_kmajor(g.wave, g.lane), cols - 8));
+  s.b_rows = nullptr;
+  s.k_total = min(p.de_len, p.n_cls - k0);
+}
+template <typename Tile, bool GATHER>
+__device__ __forceinline__ void dc_source(typename Tile::Source& s, const ProductParams& p, const typename Tile::Geometry& g, int m0,
+                                          int n0, int64_t k0, int64_t dz_cols, int cols) {
+  const int chunk = Tile::chunk_kmajor(g.wave, g.lane);
+  s.a_base = reinterpret_cast<const unsigned char*>(p.dz + k0 * p.ldz);
+  s.a_stride = static_cast<uint32_t>(2 * p.ldz);
+  s.a_off[0] = (g.lane >> 5) * s.a_stride + 2u * static_cast<unsigned>(min(static_cast<int64_t>(m0 + chunk), dz_cols - 8));
+  s.b_base = reinterpret_cast<const unsigned char*>(p.e + (GATHER ? 0 : k0 * p.stride_e));
+  s.b_stride = static_cast<uint32_t>(2 * p.stride_e);
+  s.b_off = (GATHER ? 0u : (g.lane >> 5) * s.b_stride) + 2u * static_cast<unsigned>(min(n0 + chunk, cols - 8));
+  s.b_rows = GATHER ? p.valids + k0 : nullptr;
+  s.k_total = static_cast<int>(min(static_cast<int64_t>(p.dc_len), p.b - k0));
+}
+
 // The two products of operands in parts, fp32 results: the tiles below without what 16-bit gradients need.
 __device__ __forceinline__ void terms_de_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
-  using Tile = Tile4<BF16, false, true, false, true>;
+  using Tile = Tile8<BF16, false, false, true>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int64_t m0 = static_cast<int64_t>(tm) * Tile::TILE;
   const int n0 = tn * Tile::TILE;
   const int k0 = split * p.de_len;
   typename Tile::Source s;
-#pragma unroll
-  for (int q = 0; q < Tile::NQ1; ++q) {
-    int64_t i = m0 + Tile::row_direct(q, g.wave, g.lane);
-    i = (i < p.b) ? i : p.b - 1;  // rows past the end repeat the last one; their results are dropped
-    s.a_row[q] = p.dz + i * p.ldz + k0 + Tile::chunk_direct(g.wave, g.lane);
-  }
-  s.b_row[0] = nullptr;
-  s.a_km = nullptr;
-  s.a_stride = 0;
-  s.b_km = p.c + k0 * p.stride_cv + min(n0 + Tile::chunk_kmajor(g.wave, g.lane), p.part_d - 8);
-  s.b_stride = p.stride_cv;
-  s.b_rows = nullptr;
-  s.k_total = min(p.de_len, p.n_cls - k0);
-  s.a_part = p.dz_part;
-  s.b_part = p.part_d;
+  de_source<Tile>(s, p, g, m0, n0, k0, p.part_d);
+  s.a_part = 2 * static_cast<int64_t>(p.dz_part);
+  s.b_part = 2 * static_cast<int64_t>(p.part_d);
   s.terms = p.terms;
+  Tile::plan(s);
   float* const de = p.de_f32 + split * p.de_slot;
 
-  f32x16 acc[Tile::WM][Tile::WN];
-  typename Tile::Loop loop = Tile::plan(s, g);
-  typename Tile::Ids ids;
-  typename Tile::Ptrs ptrs;
-  Tile::prefetch(s, loop, ptrs, ids, g);
-  Tile::run(acc, s, loop, ptrs, ids, smem, g);
+  f32x4 acc[Tile::WM][Tile::WN];
+  Tile::run(acc, s, smem, g);
   Tile::for_each_row_piece(acc, smem, g, [&](int row, int col, const float (&v)[8]) {
     const int64_t ri = m0 + row;
     const int cg = n0 + col;
@@ -189,32 +207,21 @@ __device__ __forceinline__ void terms_de_tile(const ProductParams& p, int split,
 }
 
 __device__ __forceinline__ void terms_dc_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
-  using Tile = Tile4<BF16, true, true, false, true>;
+  using Tile = Tile8<BF16, true, false, true>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int m0 = tm * Tile::TILE;
   const int n0 = tn * Tile::TILE;
   const int64_t k0 = static_cast<int64_t>(split) * p.dc_len;
-  const int chunk = Tile::chunk_kmajor(g.wave, g.lane);
   typename Tile::Source s;
-  s.a_row[0] = nullptr;
-  s.b_row[0] = nullptr;
-  s.a_km = p.dz + k0 * p.ldz + min(m0 + chunk, p.dz_part - 8);
-  s.a_stride = p.ldz;
-  s.b_km = p.e + k0 * p.stride_e + min(n0 + chunk, p.part_d - 8);
-  s.b_stride = p.stride_e;
-  s.b_rows = nullptr;
-  s.k_total = static_cast<int>(min(static_cast<int64_t>(p.dc_len), p.b - k0));
-  s.a_part = p.dz_part;
-  s.b_part = p.part_d;
+  dc_source<Tile, false>(s, p, g, m0, n0, k0, p.dz_part, p.part_d);
+  s.a_part = 2 * static_cast<int64_t>(p.dz_part);
+  s.b_part = 2 * static_cast<int64_t>(p.part_d);
   s.terms = p.terms;
+  Tile::plan(s);
   float* const dc = static_cast<float*>(p.d_c) + split * p.dc_slot;
 
-  f32x16 acc[Tile::WM][Tile::WN];
-  typename Tile::Loop loop = Tile::plan(s, g);
-  typename Tile::Ids ids;
-  typename Tile::Ptrs ptrs;
-  Tile::prefetch(s, loop, ptrs, ids, g);
-  Tile::run(acc, s, loop, ptrs, ids, smem, g);
+  f32x4 acc[Tile::WM][Tile::WN];
+  Tile::run(acc, s, smem, g);
   Tile::for_each_row_piece(acc, smem, g, [&](int row, int col, const float (&v)[8]) {
     const int cls = m0 + row;
     const int cg = n0 + col;
@@ -236,27 +243,15 @@ __device__ __forceinline__ void terms_dc_tile(const ProductParams& p, int split,
 // dE[row][col] += sum_class dz[row][class] * C[class][col]
 template <typename T, bool SPLIT_DE>
 __device__ __forceinline__ void dense_de_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
-  using Tile = Tile4<T, false, true>;
+  using Tile = Tile8<T, false>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int64_t m0 = static_cast<int64_t>(tm) * Tile::TILE;
   const int n0 = tn * Tile::TILE;
   const int k0 = split * p.de_len;
 
   typename Tile::Source s;
-#pragma unroll
-  for (int q = 0; q < Tile::NQ1; ++q) {
-    int64_t i = m0 + Tile::row_direct(q, g.wave, g.lane);
-    i = (i < p.b) ? i : p.b - 1;  // rows past the end repeat the last one; their results are dropped
-    s.a_row[q] = p.dz + i * p.ldz + k0 + Tile::chunk_direct(g.wave, g.lane);
-  }
-  s.b_row[0] = nullptr;
-  s.a_km = nullptr;
-  s.a_stride = 0;
-  // (columns past d: the last chunk inside the matrix once more; what they feed is dropped below)
-  s.b_km = p.c + k0 * p.stride_cv + min(n0 + Tile::chunk_kmajor(g.wave, g.lane), p.d - 8);
-  s.b_stride = p.stride_cv;
-  s.b_rows = nullptr;
-  s.k_total = min(p.de_len, p.n_cls - k0);
+  de_source<Tile>(s, p, g, m0, n0, k0, p.d);
+  Tile::plan(s);
   float* const de_f32 = SPLIT_DE ? nullptr : p.de_f32 + split * p.de_slot;
 
   // What memory holds of a piece so far, fetched ahead of its use.
@@ -284,17 +279,10 @@ __device__ __forceinline__ void dense_de_tile(const ProductParams& p, int split,
     }
     return o;
   };
-  f32x16 acc[Tile::WM][Tile::WN];
-  typename Tile::Loop loop = Tile::plan(s, g);
-  typename Tile::Ids ids;
-  typename Tile::Ptrs ptrs;
-  Tile::prefetch(s, loop, ptrs, ids, g);
-  Tile::run(acc, s, loop, ptrs, ids, smem, g);
+  f32x4 acc[Tile::WM][Tile::WN];
+  Tile::run(acc, s, smem, g);
 
-  // (fetching the first slabs before the main loop instead would hold 80 registers across it: they spill)
-  typename Tile::template Rmw<Old> rmw;
-  Tile::rmw_begin(rmw, g, fetch);
-  Tile::for_each_row_piece_rmw(acc, smem, g, rmw, fetch, [&](int row, int col, const float (&v)[8], const Old& o) {
+  Tile::template for_each_row_piece_rmw<Old>(acc, smem, g, fetch, [&](int row, int col, const float (&v)[8], const Old& o) {
     if (o.re < 0) return;
     const int64_t ri = m0 + row;
     const int cg = n0 + col;
@@ -333,30 +321,18 @@ __device__ __forceinline__ void dense_de_tile(const ProductParams& p, int split,
 // dC[class][col] = sum_row dz[row][class] * E[row][col]; GATHER: the rows of E come through valids
 template <typename T, bool GATHER>
 __device__ __forceinline__ void dense_dc_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
-  using Tile = Tile4<T, true, true, GATHER>;
+  using Tile = Tile8<T, true, GATHER>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int m0 = tm * Tile::TILE;
   const int n0 = tn * Tile::TILE;
   const int64_t k0 = static_cast<int64_t>(split) * p.dc_len;
 
   typename Tile::Source s;
-  s.a_row[0] = nullptr;
-  s.b_row[0] = nullptr;
-  const int chunk = Tile::chunk_kmajor(g.wave, g.lane);
-  // (columns past the matrix: the last chunk inside it once more; what they feed is dropped below)
-  s.a_km = p.dz + k0 * p.ldz + min(static_cast<int64_t>(m0 + chunk), p.ldz - 8);
-  s.a_stride = p.ldz;
-  s.b_km = p.e + (GATHER ? 0 : k0 * p.stride_e) + min(n0 + chunk, p.d - 8);
-  s.b_stride = p.stride_e;
-  s.b_rows = GATHER ? p.valids + k0 : nullptr;
-  s.k_total = static_cast<int>(min(static_cast<int64_t>(p.dc_len), p.b - k0));
+  dc_source<Tile, GATHER>(s, p, g, m0, n0, k0, p.ldz, p.d);
+  Tile::plan(s);
 
-  f32x16 acc[Tile::WM][Tile::WN];
-  typename Tile::Loop loop = Tile::plan(s, g);
-  typename Tile::Ids ids;
-  typename Tile::Ptrs ptrs;
-  Tile::prefetch(s, loop, ptrs, ids, g);
-  Tile::run(acc, s, loop, ptrs, ids, smem, g);
+  f32x4 acc[Tile::WM][Tile::WN];
+  Tile::run(acc, s, smem, g);
 
   if (p.dc_lo != nullptr) {
     // a 16-bit dC carried over blocks of rows: value so far = hi + lo, as dE is carried over chunks of classes
@@ -379,9 +355,7 @@ __device__ __forceinline__ void dense_dc_tile(const ProductParams& p, int split,
       }
       return o;
     };
-    typename Tile::template Rmw<Old> rmw;
-    Tile::rmw_begin(rmw, g, fetch);
-    Tile::for_each_row_piece_rmw(acc, smem, g, rmw, fetch, [&](int row, int col, const float (&v)[8], const Old& o) {
+    Tile::template for_each_row_piece_rmw<Old>(acc, smem, g, fetch, [&](int row, int col, const float (&v)[8], const Old& o) {
       if (!o.ok) return;
       const int cls = m0 + row;
       const int cg = n0 + col;
@@ -911,7 +885,7 @@ int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t*
   p.de_first = std::min<int64_t>(de_len, cls_pad) > std::min<int64_t>(dc_len, b_pad) ? 1 : 0;
   const int blocks = (p.dc_per_xcd + p.de_per_xcd) * 8;
   if (blocks == 0) return CCE_OK;
-  const int lds = Tile4<BF16, true, true>::LDS_BYTES;
+  const int lds = Tile8<BF16, true>::LDS_BYTES;
   auto kern = terms_products_kernel;
   static LdsLimitOnce lds_limit;
   const hipError_t err = lds_limit.set(kern, lds);
@@ -1047,7 +1021,7 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
     p.de_first = (std::min<int64_t>(p.de_len, cls) > std::min<int64_t>(p.dc_len, rows)) ? 1 : 0;
   };
 
-  using TileB = Tile4<BF16, true, true>;
+  using TileB = Tile8<BF16, true>;
   const int lds = TileB::LDS_BYTES;
   hipError_t err;
 #define CCE_LAUNCH_PRODUCT(KERN, BLOCKS)                                                            \
@@ -1201,7 +1175,7 @@ extern "C" int cce_backward_products(const void* dz, int64_t ldz, const void* c,
   p.de_per_xcd = (p.de_tiles + 7) / 8;
   p.de_first = (n_cls > b) ? 1 : 0;
   const int blocks = (p.dc_per_xcd + p.de_per_xcd) * 8;
-  const int lds = Tile4<BF16, true, true>::LDS_BYTES;
+  const int lds = Tile8<BF16, true>::LDS_BYTES;
   hipError_t err;
   if (dtype == CCE_DTYPE_BF16) {
     auto kern = dense_products_kernel<BF16, false>;
