@@ -1001,4 +1001,19 @@ inline SpanChoice choose_spans(int nrb, int nvt) {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Rows per block of the 16 x 16 x 32 kernels of the 16-bit types that form logits (forward, dz): 256, or 192 where that leaves
+// fewer rows of padding or an emptier last round less work.  A tile of 192 rows has three quarters of the products but 56 of the
+// 64 KB of loads per stage, and more fragment reads per product (10 for 24 instead of 12 for 32), so that it costs 0.82 - 0.94 of
+// a whole one; at equal rounds it wins, for one round more in ten it does not.  Forward of R rows, blocks of 256 / 192, us:
+// 307 x 5120 x 131072 633 / 521, 192 x 2048 x 32000 52 / 46, 900 x 1024 x 50257 104 / 97.5, 900 x 1000 x 50257 (soft-cap, bias)
+// 147 / 142, 600 x 640 x 8000 24.8 / 23.5; and 960 x 4096 x 128256 854 / 948, 3891 x 1024 x 32000 215 / 229, 8192 x 2304 x 256000
+// 6979 / 8811.  dz: 900 x 1000 x 50257 (soft-cap, bias) 155 / 132; whole steps 5476 x 4096 x 1024 300 / 288, 8888 x 3712 x 3677
+// 886 / 858, 12737 x 4864 x 640 458 / 442, 633 x 4352 x 9760 348 / 339.
+constexpr int kRowBlock = 256, kMidRowBlock = 192;
+constexpr double kMidTileCost = 0.92;
+inline bool mid_row_blocks(int64_t b, int64_t v) {
+  auto cost = [&](int rows) { return choose_spans(static_cast<int>((b + rows - 1) / rows), static_cast<int>((v + 255) / 256)).cost; };
+  return cost(kMidRowBlock) * kMidTileCost < cost(kRowBlock);
+}
+
 }  // namespace cce

@@ -250,11 +250,11 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz_kernel(DzParams p) {
 
 // ---------------------------------------------------------------------------------------------
 // The same kernel on the 16 x 16 x 32 main loop (DmaLogitTile16).  A lane holds, per 16-row block ti of its wave,
-// ONE token row (lane % 16) and the classes 16 vi + 4 (lane / 16) + r of the wave's 128; what a row needs (its
+// ONE token row (lane % 16) and the classes 16 vi + 4 (lane / 16) + r of the wave's 128 (64); what a row needs (its
 // log-sum-exp, upstream gradients, target) sits in LDS, one entry per row of the workgroup, instead of in
 // registers.  The whole ring is busy during the epilogue (the main loop fetches both first stages of the next
 // tile under its last two stages), so the staging blocks have LDS of their own: 16 rows x 128 bytes per wave,
-// half the classes of a row block at a time.
+// 64 classes of a row block at a time.
 // ---------------------------------------------------------------------------------------------
 constexpr int kDz16WV = 8, kDz16WT = 4;
 constexpr int kDz16StageBytes = 16 * kDzStageRow;  // 16 rows of 128 bytes per wave
@@ -264,15 +264,30 @@ struct DzRow {
   int tgt;
 };
 
-template <typename T, bool GENERAL, DzOut OUT, bool TAIL = false>
+// Who holds what of a tile of ROWS x 256: 2 x 4 waves of 128 classes x 64 rows, or 4 x 2 of 64 x 96.
+template <int ROWS>
+struct Dz16Shape {
+  static_assert(ROWS == kDzTile || ROWS == kMidRowBlock, "rows of a tile");
+  static constexpr bool MID = ROWS == kMidRowBlock;
+  static constexpr int WV = MID ? 4 : kDz16WV, WT = MID ? 6 : kDz16WT;
+  static constexpr int NWV = MID ? 4 : kDzNWV, NWT = MID ? 2 : kDzNWT;
+  template <typename T, bool PARTS, bool TAIL>
+  using Tile = DmaLogitTile16<T, WV, WT, NWV, NWT, PARTS, TAIL>;
+  static constexpr int LDS_BYTES =
+      Tile<BF16, false, false>::LDS_BYTES + 2 * kDzTile * 4 + ROWS * static_cast<int>(sizeof(DzRow)) + NWV * NWT * kDz16StageBytes;
+};
+
+template <typename T, bool GENERAL, DzOut OUT, bool TAIL = false, int ROWS = kDzTile>
 __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   constexpr bool OUT32 = OUT == kDzFp32;
   constexpr bool PARTS = OUT == kDzParts;
-  using Fast = DmaLogitTile16<T, kDz16WV, kDz16WT, kDzNWV, kDzNWT, PARTS, TAIL>;
+  using Shape = Dz16Shape<ROWS>;
+  constexpr int WV = Shape::WV, WT = Shape::WT;
+  using Fast = typename Shape::template Tile<T, PARTS, TAIL>;
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_addend = reinterpret_cast<float*>(smem + Fast::LDS_BYTES);                                   // [2][256]
-  DzRow* s_rows = reinterpret_cast<DzRow*>(smem + Fast::LDS_BYTES + 2 * kDzTile * 4);                    // [256]
-  unsigned char* s_stage = smem + Fast::LDS_BYTES + 2 * kDzTile * 4 + kDzTile * sizeof(DzRow);           // [8 waves]
+  DzRow* s_rows = reinterpret_cast<DzRow*>(smem + Fast::LDS_BYTES + 2 * kDzTile * 4);                    // [ROWS]
+  unsigned char* s_stage = smem + Fast::LDS_BYTES + 2 * kDzTile * 4 + ROWS * sizeof(DzRow);              // [8 waves]
 
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
@@ -288,11 +303,11 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wv = wave / kDzNWT;
-  const int wt = wave % kDzNWT;
+  const int wv = wave / Shape::NWT;
+  const int wt = wave % Shape::NWT;
   const int r16 = lane & 15;
   const int kq = lane >> 4;
-  const int64_t t0 = static_cast<int64_t>(rb) * kDzTile;
+  const int64_t t0 = static_cast<int64_t>(rb) * ROWS;
 
   typename Fast::Source src;
   src.e_base = reinterpret_cast<const unsigned char*>(p.e);
@@ -320,7 +335,7 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   Fast::prefetch(src, smem, static_cast<int>(p.d));
   // What the rows of this workgroup need, fixed for the whole item (published by the first barrier of the main loop;
   // fetched behind the first stages of the ring, so that the two latencies overlap).
-  if (tid < kDzTile) {
+  if (tid < ROWS) {
     const int64_t i = t0 + tid;
     DzRow r = {INFINITY, 0.0f, 0.0f, -1};
     if (i < p.b) {
@@ -351,26 +366,26 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
         addend[tid] = a;
       }
     }
-    f32x4 acc[kDz16WV][kDz16WT];
+    f32x4 acc[WV][WT];
     Fast::run(acc, src, smem, static_cast<int>(p.d), buf, vt == vt_begin, [&] {
       if (vt + 1 < vt_end) set_class_tile(vt + 1);
     });
 
-    const int cls0 = static_cast<int>(v0) + wv * (16 * kDz16WV);  // first class of this wave
-    const float* wave_addend = addend + wv * (16 * kDz16WV);
+    const int cls0 = static_cast<int>(v0) + wv * (16 * WV);  // first class of this wave
+    const float* wave_addend = addend + wv * (16 * WV);
     const int sw = (r16 >> 1) & 7;  // 16-byte chunks of a staged row are XOR-swizzled with (row >> 1) & 7
     // (left to itself the compiler forms the row part of every store address before the tile loop, holds the pairs
     // of registers through the main loop by spilling them, and the reload at the top of the epilogue waits for
     // the loads just issued for the next tile)
-    int64_t wrow0 = t0 + wt * (16 * kDz16WT);  // first row of this wave
+    int64_t wrow0 = t0 + wt * (16 * WT);  // first row of this wave
     asm volatile("" : "+s"(wrow0));
     constexpr int kEs = OUT32 ? 4 : 2;                  // bytes per stored element
     constexpr int kViPer = kDzStageRow / (16 * kEs);    // 16-class blocks per staged row (4, or 2 for fp32)
-    constexpr int kParts = kDz16WV / kViPer;            // staged blocks per row block
+    constexpr int kParts = WV / kViPer;                 // staged blocks per row block
     constexpr int kPieceElems = 16 / kEs;               // elements per 16-byte piece
 #pragma unroll
-    for (int ti = 0; ti < kDz16WT; ++ti) {
-      const DzRow rr = s_rows[wt * (16 * kDz16WT) + ti * 16 + r16];
+    for (int ti = 0; ti < WT; ++ti) {
+      const DzRow rr = s_rows[wt * (16 * WT) + ti * 16 + r16];
 #pragma unroll
       for (int vh = 0; vh < kParts; ++vh) {
         float rest[PARTS ? kViPer : 1][4];  // PARTS: what the parts stored so far leave of the gradients
@@ -530,7 +545,11 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
   p.grad_scale = grad_scale;
   p.d_out_is_scalar = d_out_is_scalar;
   p.pad_store = pad_store;
-  p.nrb = static_cast<int>((b + kDzTile - 1) / kDzTile);
+  // the 16 x 16 x 32 kernel addresses rows by 32-bit byte offsets and streams at least two stages per tile
+  const bool k16 = dense_k16(n_rows, d, stride_e, stride_cv);
+  const bool mid = k16 && !dz_is_fp32 && mid_row_blocks(b, v);
+  const int block = mid ? kMidRowBlock : kDzTile;
+  p.nrb = static_cast<int>((b + block - 1) / block);
   p.nvt = static_cast<int>((v + kDzTile - 1) / kDzTile);
   const SpanChoice spans = choose_spans(p.nrb, p.nvt);
   p.nsplit = spans.count;
@@ -542,15 +561,25 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
 
   using FastB = DmaLogitTile<BF16, kDzWV, kDzWT, kDzNWV, kDzNWT>;
   const int lds = FastB::LDS_BYTES + 2 * kDzTile * 4;
-  const int lds16 = lds + kDzTile * static_cast<int>(sizeof(DzRow)) + kDzNWV * kDzNWT * kDz16StageBytes;
+  const int lds16 = mid ? Dz16Shape<kMidRowBlock>::LDS_BYTES : Dz16Shape<kDzTile>::LDS_BYTES;
   const bool general = (bias != nullptr) || (v % kDzTile != 0);
-  // the 16 x 16 x 32 kernel addresses rows by 32-bit byte offsets and streams at least two stages per tile
-  const bool k16 = dense_k16(n_rows, d, stride_e, stride_cv);
   const int grid = p.items_per_xcd * 8;
   hipError_t err;
 #define CCE_LAUNCH_DZ2(TT, GE, O32)                                                               \
   do {                                                                                            \
-    if (k16 && tail) {                                                                            \
+    if (mid && tail) {                                                                            \
+      auto kern = dense_dz16_kernel<TT, GE, kDz16Bit, true, kMidRowBlock>;                        \
+      static LdsLimitOnce lds_limit;                                                              \
+      err = lds_limit.set(kern, lds16);                                                           \
+      if (err != hipSuccess) return status_from_hip(err);                                         \
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(kDzThreads), lds16, stream, p);                   \
+    } else if (mid) {                                                                             \
+      auto kern = dense_dz16_kernel<TT, GE, kDz16Bit, false, kMidRowBlock>;                       \
+      static LdsLimitOnce lds_limit;                                                              \
+      err = lds_limit.set(kern, lds16);                                                           \
+      if (err != hipSuccess) return status_from_hip(err);                                         \
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(kDzThreads), lds16, stream, p);                   \
+    } else if (k16 && tail) {                                                                     \
       auto kern = dense_dz16_kernel<TT, GE, kDz16Bit, true>;                                      \
       static LdsLimitOnce lds_limit;                                                              \
       err = lds_limit.set(kern, lds16);                                                           \

@@ -302,12 +302,11 @@ __global__ __launch_bounds__(kFwdThreads, 1) void lse_forward_kernel(LseFwdParam
 // ---------------------------------------------------------------------------------------------
 constexpr int kF16WV = 8, kF16WT = 4;  // 16-row blocks per wave: 128 classes x 64 rows
 constexpr int kF16RunBytes = kF16WT * kFwdThreads * static_cast<int>(sizeof(float2));  // running (max, sum) pairs
-constexpr int kFwdMidRows = 192;
 // Who holds what of a tile of ROWS x 256: 2 x 4 waves of 128 classes x 64 rows, or 4 x 2 of 64 x 96.
 template <int ROWS>
 struct Fwd16Shape {
-  static_assert(ROWS == kFwdTile || ROWS == kFwdMidRows, "rows of a tile");
-  static constexpr bool MID = ROWS == kFwdMidRows;
+  static_assert(ROWS == kFwdTile || ROWS == kMidRowBlock, "rows of a tile");
+  static constexpr bool MID = ROWS == kMidRowBlock;
   static constexpr int WV = MID ? 4 : kF16WV, WT = MID ? 6 : kF16WT;
   static constexpr int NWV = MID ? 4 : kFwdNWV, NWT = MID ? 2 : kFwdNWT;
   static constexpr int RUN_BYTES = WT * kFwdThreads * static_cast<int>(sizeof(float2));
@@ -678,13 +677,12 @@ struct RowBlocks {
   int rows, nrb, nvt, nsplit, block_rows, block_spans;
   int64_t partial_bytes(int64_t b) const { return static_cast<int64_t>(nsplit) * b * static_cast<int64_t>(sizeof(float2)); }
 };
-static RowBlocks blocks_of(int rows, int64_t b, int64_t v, double* cost = nullptr) {
+static RowBlocks blocks_of(int rows, int64_t b, int64_t v) {
   RowBlocks r = {rows, static_cast<int>((b + rows - 1) / rows), static_cast<int>((v + kFwdTile - 1) / kFwdTile), 0, 0, 0};
   const SpanChoice s = choose_spans(r.nrb, r.nvt);
   r.nsplit = s.count;
   r.block_rows = s.block_rows;
   r.block_spans = s.block_spans;
-  if (cost != nullptr) *cost = s.cost;
   return r;
 }
 static void take_blocks(LseFwdParams& p, const RowBlocks& r) {
@@ -696,19 +694,7 @@ static void take_blocks(LseFwdParams& p, const RowBlocks& r) {
   p.nitems = p.nrb * p.nsplit;
   p.items_per_xcd = (p.nitems + 7) / 8;
 }
-// Rows per block of the 16 x 16 x 32 kernel: 256, or 192 where that leaves fewer rows of padding or an emptier last round
-// less work.  A tile of 192 rows has three quarters of the products but 56 of the 64 KB of loads per stage, and more
-// fragment reads per product (10 for 24 instead of 12 for 32), so that it costs 0.82 - 0.94 of a whole one; at equal
-// rounds it wins, for one round more in ten it does not.  Forward of R rows, blocks of 256 / 192, us: 307 x 5120 x 131072 633 / 521,
-// 192 x 2048 x 32000 52 / 46, 900 x 1024 x 50257 104 / 97.5, 900 x 1000 x 50257 (soft-cap, bias) 147 / 142, 600 x 640 x 8000
-// 24.8 / 23.5; and 960 x 4096 x 128256 854 / 948, 3891 x 1024 x 32000 215 / 229, 8192 x 2304 x 256000 6979 / 8811.
-constexpr double kMidTileCost = 0.92;
-static RowBlocks best_blocks(int64_t b, int64_t v) {
-  double whole, mid;
-  const RowBlocks w = blocks_of(kFwdTile, b, v, &whole);
-  const RowBlocks m = blocks_of(kFwdMidRows, b, v, &mid);
-  return mid * kMidTileCost < whole ? m : w;
-}
+static RowBlocks best_blocks(int64_t b, int64_t v) { return blocks_of(mid_row_blocks(b, v) ? kMidRowBlock : kFwdTile, b, v); }
 
 template <typename T>
 static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64_t workspace_bytes, hipStream_t stream) {
@@ -720,7 +706,7 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64
   using Few = DmaLogitTile16<T, kF16WV, kF16WT, kFwdNWV, kFwdNWT, false, false, true>;
   constexpr int lds_few = Few::LDS_BYTES + kFwdBiasBytes + kF16RunBytes / 2;
   static_assert(lds_few <= 160 * 1024, "three stages fit");
-  using MidShape = Fwd16Shape<kFwdMidRows>;
+  using MidShape = Fwd16Shape<kMidRowBlock>;
   constexpr int lds_mid = DmaLogitTile16<T, MidShape::WV, MidShape::WT, MidShape::NWV, MidShape::NWT>::LDS_BYTES + kFwdBiasBytes +
                           MidShape::RUN_BYTES;
   // the 16 x 16 x 32 kernel addresses token rows by 32-bit byte offsets from e and class rows by offsets from the
@@ -740,7 +726,7 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64
     const RowBlocks best = best_blocks(p.b, p.v);
     if (best.partial_bytes(p.b) <= workspace_bytes) blocks = best;
   }
-  const bool mid = blocks.rows == kFwdMidRows;
+  const bool mid = blocks.rows == kMidRowBlock;
   take_blocks(p, blocks);
   const bool general = want_la || (p.bias != nullptr) || (p.v % Tile::TILE_V != 0);
   const int grid = p.items_per_xcd * 8;
@@ -769,11 +755,11 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64
     if (general) CCE_LAUNCH_FWD16(true, false, false, true, kFwdTile);
     else CCE_LAUNCH_FWD16(false, false, false, true, kFwdTile);
   } else if (mid && tail) {
-    if (general) CCE_LAUNCH_FWD16(true, false, true, false, kFwdMidRows);
-    else CCE_LAUNCH_FWD16(false, false, true, false, kFwdMidRows);
+    if (general) CCE_LAUNCH_FWD16(true, false, true, false, kMidRowBlock);
+    else CCE_LAUNCH_FWD16(false, false, true, false, kMidRowBlock);
   } else if (mid) {
-    if (general) CCE_LAUNCH_FWD16(true, false, false, false, kFwdMidRows);
-    else CCE_LAUNCH_FWD16(false, false, false, false, kFwdMidRows);
+    if (general) CCE_LAUNCH_FWD16(true, false, false, false, kMidRowBlock);
+    else CCE_LAUNCH_FWD16(false, false, false, false, kMidRowBlock);
   } else if (fast16 && tail) {
     if (want_la) CCE_LAUNCH_FWD16(true, true, true, false, kFwdTile);
     else if (general) CCE_LAUNCH_FWD16(true, false, true, false, kFwdTile);

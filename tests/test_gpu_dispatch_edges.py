@@ -730,3 +730,42 @@ def test_gradients_kept_between_the_filtered_passes(monkeypatch, shape, dtype, f
         # dz is rounded to the type from logits summed in another order: 2^-9 (bf16) of single products, and of the results
         assert (a - b).norm() <= 2e-3 * b.norm()
         assert ((a - b).abs() <= 2e-2 * b.abs() + 2e-2 * b.abs().amax(dim=1, keepdim=True)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [129, 191, 192, 193, 300, 384, 385, 576])
+@pytest.mark.parametrize("width,classes", [(128, 256), (136, 1000), (192, 256 * 40 + 1), (704, 256 * 130)])
+def test_logit_gradients_in_blocks_of_192_rows(dtype, rows, width, classes):
+    """The blocks of test_forward_in_blocks_of_192_rows in the kernel that forms dz: gathered rows, partial stages, cut tiles, several
+    tiles per item, soft-cap and bias.  Seen through dBias (the sums of dz over the rows) and the two products."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    g = torch.Generator().manual_seed(rows + width)
+    e0 = torch.randn((rows + 5, width), generator=g).to(dtype).cuda()
+    c0 = (torch.randn((classes, width), generator=g) * 0.1).to(dtype).cuda()
+    b0 = torch.randn((classes,), generator=g).to(dtype).cuda()
+    t = torch.randint(0, classes, (rows + 5,), generator=g).cuda()
+    t[:5] = -100
+    for softcap, biased in ((None, False), (20.0, True)):
+        e, c, bias = (x.clone().requires_grad_(True) for x in (e0, c0, b0))
+        nll = linear_cross_entropy(e, c, t, bias=bias if biased else None, softcap=softcap, reduction="none", impl="cce_exact")
+        up = torch.rand(nll.shape, generator=torch.Generator().manual_seed(1)).cuda() + 0.5
+        nll.backward(up.to(nll.dtype))
+        z = e0.double() @ c0.double().T + (b0.double() if biased else 0.0)
+        x = softcap * torch.tanh(z / softcap) if softcap else z
+        dz = torch.softmax(x, 1)
+        dz[5:].scatter_add_(1, t[5:, None], -torch.ones((rows, 1), dtype=torch.float64, device="cuda"))
+        if softcap:
+            dz *= 1 - (x / softcap) ** 2
+        dz *= up.to(nll.dtype).double()[:, None]
+        dz[:5] = 0.0
+        # the bounds of test_backward_dense_cuts_long_reductions: dz and the results are rounded to 8 (11) bits once each
+        for got, want in ((e.grad, dz @ c0.double()), (c.grad, dz.T @ e0.double())):
+            scale = want.abs().amax(dim=1, keepdim=True)
+            assert ((got.double() - want).abs() <= 1e-2 * scale + 1e-2 * want.abs() + 1e-6).all()
+            assert (got.double() - want).norm() <= 6e-3 * want.norm()
+        if biased:  # terms of 8 significant bits: half a unit in the last place is up to 2^-8 of each, and of their sum once more;
+            # below 2^-14 a fp16 term is off by up to 2^-25 whatever its size
+            want = dz.sum(0)
+            tiny = (rows + 1) * 2.0**-25 if dtype == torch.float16 else 0.0
+            assert ((bias.grad.double() - want).abs() <= 2.0**-8 * (dz.abs().sum(0) * 1.01 + want.abs()) + tiny + 1e-6).all()
