@@ -1293,12 +1293,13 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
       // Nothing survived for this class group: its rows are zeros, written as whole 16-byte pieces, a wave
       // instruction inside one row (the launcher guarantees 16-byte aligned rows and D a multiple of 8).
       const int ppr = (d_end - d_begin) / 8;  // 16-byte pieces per row
-      const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+      typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+      const u32x4 zero = {0u, 0u, 0u, 0u};
       for (int row = wave; row < 32; row += kBwdThreads / 64) {  // (a division per piece costs more than its store)
         const int id = own_ids[row];
         if (id < 0) continue;
-        uint4* const dst = reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.d_c) + static_cast<int64_t>(id) * own_sr + d_begin);
-        for (int j = lane; j < ppr; j += 64) dst[j] = zero;
+        u32x4* const dst = reinterpret_cast<u32x4*>(static_cast<uint16_t*>(p.d_c) + static_cast<int64_t>(id) * own_sr + d_begin);
+        for (int j = lane; j < ppr; j += 64) __builtin_nontemporal_store(zero, dst + j);
       }
     }
   } else if (write_out && (touched || !IS_DE || to_slot)) {  // dC rows and slots are always written; the launcher guarantees 16-byte aligned rows
