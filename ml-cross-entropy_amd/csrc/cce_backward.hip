@@ -651,8 +651,8 @@ struct FastLds {
 };
 constexpr int kFLdsBytes = FastLds<false>::kBytes;
 constexpr int kFLightLdsBytes = FastLds<true>::kBytes;
-constexpr int kFLightMaxEntries = 2;
-constexpr int kLightStores = 4;                     // store instructions per wave and 128-column chunk of the light dC pass                // entries of a class group the light dC pass takes on
+constexpr int kFLightMaxEntries = 2;  // entries of a class group the light dC pass takes on
+constexpr int kLightStores = 2;  // store instructions per wave and 128-column chunk of the light dC pass
 constexpr int kFSegCells = 512;                     // dE: cells scanned per pass (<= 2048 entries)
 constexpr int kFListCap = 2048;
 static_assert(kFLdsBytes <= 160 * 1024 && 2 * kFLightLdsBytes <= 160 * 1024, "LDS budget of gfx950");
@@ -816,20 +816,29 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   // light variant: the 32 own rows x 128 columns of one chunk, 16-bit, straight from the accumulator block of
   // this wave (lane = own row, registers = 4 x 4 consecutive columns)
   auto store_chunk_direct = [&](int ci, const f32x16& a) {
+    // The halves of the wave hold columns 0 .. 3 and 4 .. 7 of every eight.  They change places two by two, so that a lane has
+    // eight in a row and a store instruction 32 bytes of each of 32 rows, not 16: light dC pass of 8192 rows x 2304 x 256000 679 -> 603 us,
+    // of 307 x 5120 x 131072 341 -> 315.  (64 bytes of 16 rows, by another exchange, are no faster; stored past the caches, parts of
+    // lines cost three times as much.)
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 val[kLightStores];
+#pragma unroll
+    for (int k = 0; k < kLightStores; ++k) {
+      const auto lo = __builtin_amdgcn_permlane32_swap(Elem<T>::pack2(a[8 * k + 0], a[8 * k + 1]), Elem<T>::pack2(a[8 * k + 4], a[8 * k + 5]), false, false);
+      const auto hi = __builtin_amdgcn_permlane32_swap(Elem<T>::pack2(a[8 * k + 2], a[8 * k + 3]), Elem<T>::pack2(a[8 * k + 6], a[8 * k + 7]), false, false);
+      val[k] = u32x4{lo[0], hi[0], lo[1], hi[1]};
+    }
     const int id = own_ids[l32];
     if (id < 0) return;
-    const int col = d_begin + ci * kFCols + wave * 32 + 4 * half;
+    const int col = d_begin + ci * kFCols + wave * 32 + 8 * half;
     uint16_t* dst = static_cast<uint16_t*>(p.d_c) + static_cast<int64_t>(id) * own_sr + col;
     // exactly kLightStores store instructions per wave and chunk (the product loop below counts them: stores share
-    // the counter its loads are awaited on), whatever the compiler would make of four plain assignments; fewer in a
+    // the counter its loads are awaited on), whatever the compiler would make of plain assignments; fewer in a
     // partial chunk, which is the last one: nothing is counted after it
 #pragma unroll
-    for (int r4 = 0; r4 < kLightStores; ++r4) {
-      if (TAIL && col + 8 * r4 >= D) break;
-      uint2 pk;
-      pk.x = Elem<T>::pack2(a[r4 * 4 + 0], a[r4 * 4 + 1]);
-      pk.y = Elem<T>::pack2(a[r4 * 4 + 2], a[r4 * 4 + 3]);
-      asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(dst + 8 * r4), "v"(pk) : "memory");
+    for (int k = 0; k < kLightStores; ++k) {
+      if (TAIL && col + 16 * k >= D) break;
+      asm volatile("global_store_dwordx4 %0, %1, off" ::"v"(dst + 16 * k), "v"(val[k]) : "memory");
     }
   };
 
@@ -1291,7 +1300,9 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
   if constexpr (LIGHT) {
     if (write_out && !touched) {
       // Nothing survived for this class group: its rows are zeros, written as whole 16-byte pieces, a wave
-      // instruction inside one row (the launcher guarantees 16-byte aligned rows and D a multiple of 8).
+      // instruction inside one row (the launcher guarantees 16-byte aligned rows and D a multiple of 8), past the caches: they
+      // are written once, and pushed out what the next kernels read again (307 rows x 5120 x 131072: this pass 376 -> 342 us, the
+      // forward of the step after it 520 -> 494; a kernel of its own for the zeros takes 229 us beside 183 of the rest).
       const int ppr = (d_end - d_begin) / 8;  // 16-byte pieces per row
       typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
       const u32x4 zero = {0u, 0u, 0u, 0u};
