@@ -669,6 +669,11 @@ def test_z_loss_kernels_against_tensor_operations(shape, shift, reduction, label
         (g2,) = torch.autograd.grad(g1.sum(), lse)
         assert torch.allclose(g2 * lse.detach(), want_grad, rtol=1e-6, atol=0)
         plain = lse.detach()
+        # several upstream gradients at once, which autograd batches without storage
+        pair = torch.stack([up, 2 * up])
+        (both,) = torch.autograd.grad(out, lse, pair, retain_graph=True, is_grads_batched=True)
+        for one, k in zip(both, (1, 2)):
+            assert torch.allclose(one, k * want_grad, rtol=4e-7, atol=0, equal_nan=True)
         import torch.autograd.forward_ad as fwAD
 
         with fwAD.dual_level():
