@@ -361,8 +361,10 @@ extern "C" int cce_rows_to_batch(const float* values, const int32_t* rows, int64
 
 extern "C" int cce_rows_to_steps(const float* first, const float* second, const int32_t* rows, int64_t count, int64_t n, int64_t steps,
                                  int64_t shift, float* out_first, float* out_second, void* stream) {
-  if (n < 0 || n >= (int64_t(1) << 31) - 8192 || count < 0 || count > n || steps <= 0 || shift < 0) return CCE_ERR_INVALID_ARGUMENT;
-  if (n == 0 || shift >= steps) return CCE_OK;
+  if (n < 0 || n >= (int64_t(1) << 31) - 8192 || count < 0 || count > n || shift < 0) return CCE_ERR_INVALID_ARGUMENT;
+  if (n == 0) return CCE_OK;  // (sequences of no steps among them)
+  if (steps <= 0) return CCE_ERR_INVALID_ARGUMENT;
+  if (shift >= steps) return CCE_OK;
   if (n % steps != 0 || (count > 0 && rows == nullptr)) return CCE_ERR_INVALID_ARGUMENT;
   if (count > 0 && ((out_first != nullptr && first == nullptr) || (out_second != nullptr && second == nullptr)))
     return CCE_ERR_INVALID_ARGUMENT;
@@ -375,8 +377,9 @@ extern "C" int cce_rows_to_steps(const float* first, const float* second, const 
 
 extern "C" int cce_steps_to_batch(const float* first, const float* second, int64_t n, int64_t steps, int64_t shift, float* out_first,
                                   float* out_second, void* stream) {
-  if (n < 0 || n >= (int64_t(1) << 31) - 8192 || steps <= 0 || shift < 0 || shift > steps) return CCE_ERR_INVALID_ARGUMENT;
+  if (n < 0 || n >= (int64_t(1) << 31) - 8192 || shift < 0) return CCE_ERR_INVALID_ARGUMENT;
   if (n == 0) return CCE_OK;
+  if (steps <= 0 || shift > steps) return CCE_ERR_INVALID_ARGUMENT;
   if (n % steps != 0 || (out_first != nullptr && first == nullptr) || (out_second != nullptr && second == nullptr))
     return CCE_ERR_INVALID_ARGUMENT;
   const TwoSets sets = {{first, second}, {out_first, out_second}};

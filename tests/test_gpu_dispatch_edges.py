@@ -614,6 +614,23 @@ def test_rows_to_steps_and_back(shape, shift, keep):
                 assert torch.equal(flat.cpu(), want.view(-1))
 
 
+@pytest.mark.parametrize("shape", [(0,), (3, 0), (0, 5)])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+def test_no_labels_at_all(shape, reduction):
+    """Batches without a position: nothing to sum, values in the (empty) batch shape, gradients of zeros."""
+    from cut_cross_entropy.cce import cce_linear_cross_entropy
+
+    e = torch.randn(shape + (64,), device="cuda", dtype=torch.bfloat16).requires_grad_(True)
+    c = torch.randn((100, 64), device="cuda", dtype=torch.bfloat16).requires_grad_(True)
+    t = torch.zeros(shape, dtype=torch.int64, device="cuda")
+    loss, lse = cce_linear_cross_entropy(e, c, t, reduction=reduction, return_lse=True)
+    assert lse.shape == shape and loss.shape == (shape if reduction == "none" else ())
+    if reduction != "none":
+        assert loss.isnan() if reduction == "mean" else loss.item() == 0.0
+    (loss.sum() + lse.sum()).backward()
+    assert e.grad.shape == e.shape and not c.grad.any()
+
+
 @pytest.mark.parametrize("shape,shift", [((1,), 0), ((2, 1), 0), ((70,), 3), ((3, 85), 2), ((2, 3, 50), 1), ((1, 16384), 0), ((1, 16385), 0),
                                          ((5, 3277), 1), ((3, 1400001), 1)])
 @pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
