@@ -1134,6 +1134,18 @@ extern "C" int cce_backward_products(const void* dz, int64_t ldz, const void* c,
   if (ldz >= (int64_t(1) << 30) || stride_cv >= (int64_t(1) << 30) || stride_e >= (int64_t(1) << 30))
     return CCE_ERR_INVALID_ARGUMENT;
   if (d_e == nullptr && d_c == nullptr) return CCE_OK;
+  // The tiles of dE reach their 256 rows of dz by 32-bit offsets.  Wider rows than that allows go block by block.
+  if (d_e != nullptr && ldz > 0 && std::min<int64_t>(b, 256) * ldz * 2 >= (int64_t(1) << 32)) {
+    const int64_t most = ((int64_t(1) << 32) - 1) / (2 * ldz);
+    for (int64_t i = 0; i < b; i += most) {
+      const int st = cce_backward_products(static_cast<const uint16_t*>(dz) + i * ldz, ldz, c, stride_cv,
+                                           (e == nullptr || valids != nullptr) ? e : static_cast<const uint16_t*>(e) + i * stride_e,
+                                           stride_e, valids == nullptr ? nullptr : valids + i, d_e + i * ld_de, ld_de, d_c, ld_dc,
+                                           (d_c_accumulate || i > 0) ? 1 : 0, std::min(most, b - i), n_cls, d, dtype, stream_);
+      if (st != CCE_OK) return st;
+    }
+    return CCE_OK;
+  }
   if (!aligned16(dz) || ldz % 8 != 0 || ldz < (n_cls + 63) / 64 * 64 || d % 8 != 0) return CCE_ERR_MISALIGNED;
   if (d_e != nullptr && (!aligned16(c) || stride_cv % 8 != 0 || !aligned16(d_e) || ld_de % 4 != 0 || ld_de < d))
     return CCE_ERR_MISALIGNED;

@@ -493,6 +493,35 @@ def test_entry_points_reject_bad_arguments_before_launching():
     assert lib.cce_error_string(INVALID) and lib.cce_error_string(MISALIGNED) and lib.cce_error_string(DTYPE)
 
 
+@pytest.mark.parametrize("gather", [False, True])
+def test_backward_products_of_rows_far_apart(gather):
+    """256 rows of dz that span more than 4 GB, past what a 32-bit offset reaches; bounds as below."""
+    lib = _lib()
+    dev = torch.device("cuda:0")
+    B, M, D, ldz = 300, 130, 72, 9_000_000
+    g = torch.Generator().manual_seed(4)
+    dz = (torch.randn((B, M), generator=g) * 0.1).to(torch.bfloat16)
+    c = torch.randn((M, D), generator=g).to(torch.bfloat16)
+    e = torch.randn((B + 9, D), generator=g).to(torch.bfloat16)
+    valids = torch.arange(B, dtype=torch.int32) + (9 if gather else 0)
+    wide = torch.empty((B, ldz), dtype=torch.bfloat16, device=dev)
+    wide[:, :192] = 0.0
+    wide[:, :M] = dz.to(dev)
+    de0, dc0 = torch.randn((B, D), generator=g), torch.randn((M, D), generator=g)
+    want_de = de0.double() + dz.double() @ c.double()
+    cd, ed, vd = c.to(dev), e.to(dev), valids.to(dev)
+    for accumulate in (0, 1):
+        ded, dcd = de0.to(dev), dc0.to(dev)
+        st = lib.cce_backward_products(wide.data_ptr(), ldz, cd.data_ptr(), D, ed.data_ptr(), D, vd.data_ptr() if gather else None,
+                                       ded.data_ptr(), D, dcd.data_ptr(), D, accumulate, B, M, D, 0,
+                                       torch.cuda.current_stream().cuda_stream)
+        assert st == 0, lib.cce_error_string(st)
+        torch.cuda.synchronize()
+        want_dc = dz.double().T @ e[valids.long()].double() + (dc0.double() if accumulate else 0.0)
+        for got, want in ((ded, want_de), (dcd, want_dc)):
+            assert (got.cpu().double() - want).abs().max().item() <= 1e-5 * want.abs().max().item()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(256, 512, 128), (300, 500, 72), (1000, 130, 264), (33, 64, 8),
                                    (63, 40, 64), (65, 257, 520), (1, 7, 8), (130, 64, 1032)])
