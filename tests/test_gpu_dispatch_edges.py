@@ -702,6 +702,37 @@ def test_z_loss_kernels_against_tensor_operations(shape, shift, reduction, label
         assert torch.allclose(pair[1], out.detach(), rtol=1e-6, atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("layout", ["sliced", "permuted", "expanded", "several"])
+@pytest.mark.parametrize("reduction", ["mean", "none"])
+def test_z_loss_of_layouts_with_dimensions_of_one_entry(layout, reduction):
+    """Dimensions of one entry between larger ones: layouts that one stride leads through and layouts that it does not, for the
+    log-sum-exps and for the labels."""
+    from cut_cross_entropy import utils
+
+    def laid_out(x):
+        x = x.cuda()
+        return {"sliced": lambda: x.view(4, 1, 12, 8)[:, :, :5], "permuted": lambda: x[:160].view(5, 4, 1, 8).permute(1, 2, 0, 3),
+                "expanded": lambda: x[:32].view(4, 1, 1, 8).expand(4, 1, 3, 8),
+                "several": lambda: x.view(4, 1, 3, 1, 32)[:, :, 1:2, :, 1:9]}[layout]()
+
+    g = torch.Generator().manual_seed(5)
+    values = torch.randn((384,), generator=g) * 3 + 9
+    labels = torch.randint(0, 50, (384,), generator=g)
+    labels[torch.rand((384,), generator=g) < 0.3] = -100
+    for lse, t in ((laid_out(values), laid_out(labels)), (laid_out(values).contiguous(), laid_out(labels)),
+                   (laid_out(values), laid_out(labels).contiguous())):
+        lse = lse.detach().requires_grad_(True)
+        out = utils.compute_z_loss(lse, t, reduction=reduction)
+        up = torch.rand(out.shape, generator=g).cuda() + 0.5
+        (grad,) = torch.autograd.grad(out, lse, up)
+        ref = lse.detach().contiguous().requires_grad_(True)
+        sq = ref.square().masked_fill(t == -100, 0.0)
+        want = sq if reduction == "none" else sq.sum() / (t != -100).sum()
+        (want_grad,) = torch.autograd.grad(want, ref, up)
+        # at most 384 fp32 additions of values of one sign in the reference
+        assert torch.allclose(out, want, rtol=384 * 2.0**-24, atol=0) and torch.allclose(grad, want_grad, rtol=2e-7, atol=0)
+
+
 @pytest.mark.parametrize("shape,budget", [((4744, 6303, 320), 7 << 20), ((5308, 4438, 128), 5 << 20), ((9380, 4245, 320), 16 << 20),
                                           ((10691, 3041, 192), 11 << 20)])
 def test_cut_reductions_in_more_launches(monkeypatch, shape, budget):

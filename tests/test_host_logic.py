@@ -203,3 +203,41 @@ def test_forgotten_measurements_keep_their_word_until_it_has_been_written(monkey
     assert word() is not None
     assert bw._filtered_backward_runs_dense(None, None, None, 32, 512, 64, 1e-4, torch.bfloat16, dev) is False
     assert len(seen) == 2 and Event.waited == 2  # its own cells, and those for the backward after it
+
+
+def test_rows_of_steps_lead_to_the_elements_they_name():
+    """Slices, permutations, expansions and dimensions of one entry, up to five dimensions: either the strides answered lead to the
+    elements in order, or no one stride does (``view`` to a matrix of dense rows knows)."""
+    import itertools
+
+    from cut_cross_entropy.utils import _rows_of_steps
+
+    def check(t):
+        rows = _rows_of_steps(t)
+        try:
+            matrix = t.view(-1, t.size(-1))
+        except RuntimeError:
+            matrix = None
+        if matrix is not None and matrix.stride(1) != 1 and matrix.size(1) > 1:
+            matrix = None
+        assert (rows is None) == (matrix is None), (t.shape, t.stride())
+        if rows is not None:
+            n, cols, step = rows
+            assert n * cols == t.numel()
+            assert torch.equal(t.as_strided((n, cols), (step, 1)), t.reshape(n, cols)), (t.shape, t.stride())
+
+    for ndim in range(1, 6):
+        for shape in itertools.product((1, 2, 3), repeat=ndim):
+            base = torch.arange(int(torch.tensor(shape).prod())).view(shape)
+            for order in itertools.permutations(range(ndim)) if ndim < 5 else [(0, 1, 2, 3, 4), (1, 2, 0, 3, 4), (3, 0, 1, 2, 4), (0, 3, 2, 1, 4)]:
+                t = base.permute(order)
+                check(t)
+                for d in range(ndim):
+                    if t.size(d) == 3:
+                        check(t.narrow(d, 1, 2))
+                        check(t.narrow(d, 2, 1))
+                    if t.size(d) == 1:
+                        check(t.expand(*t.shape[:d], 2, *t.shape[d + 1 :]))
+    # what was read at the wrong places
+    check(torch.arange(384).view(4, 1, 12, 8)[:, :, :5])
+    check(torch.arange(160).view(5, 4, 1, 8).permute(1, 2, 0, 3))
