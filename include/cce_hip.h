@@ -319,18 +319,19 @@ int cce_steps_to_batch(const float* first, const float* second, int64_t n, int64
 /*
  * The z-loss (cut_cross_entropy/utils.py:64-102): squares of lse[rows][cols], zero where labels[rows][cols] (NULL: nowhere) is
  * `ignored`; CCE_REDUCTION_NONE writes out[rows * cols], the others one value, and how many positions count to *count where
- * that is not NULL.  The strides lead from row to row.  Backward: d_lse[rows * cols] from the upstream gradient (one value, or one
- * per position), divided by *count where that is not NULL (the mean).
+ * that is not NULL.  kept[rows * cols] (NULL: not wanted) is 1 where a position counts, else 0.  The strides lead from row to row.
+ * Backward: d_lse[rows * cols] from the upstream gradient (one value, or one per position), divided by *count where that is not
+ * NULL (the mean), for the positions that `kept` of the forward names (NULL: all), so that the labels may have changed since.
  */
 #define CCE_REDUCTION_NONE 0
 #define CCE_REDUCTION_SUM 1
 #define CCE_REDUCTION_MEAN 2
 int64_t cce_z_loss_workspace_bytes(int64_t rows, int64_t cols);
 int cce_z_loss_forward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows, int64_t cols,
-                       int64_t ignored, int reduction, float* out, float* count, void* workspace, int64_t workspace_bytes,
-                       void* stream);
-int cce_z_loss_backward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows, int64_t cols,
-                        int64_t ignored, const float* grad, int grad_is_scalar, const float* count, float* d_lse, void* stream);
+                       int64_t ignored, int reduction, float* out, float* count, uint8_t* kept, void* workspace,
+                       int64_t workspace_bytes, void* stream);
+int cce_z_loss_backward(const float* lse, int64_t lse_stride, const uint8_t* kept, int64_t rows, int64_t cols, const float* grad,
+                        int grad_is_scalar, const float* count, float* d_lse, void* stream);
 
 /*
  * cce_lse_forward (without logit_avg) and cce_indexed_neg_dot in one call: lse[b], and nll[b] = lse + neg_dot, the loss of

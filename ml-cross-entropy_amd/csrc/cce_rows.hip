@@ -112,6 +112,7 @@ struct ZLossParams {
   const int64_t* labels;  // nullptr: everything counts
   int64_t lse_stride, label_stride, ignored;
   int n, cols;
+  uint8_t* kept;  // one byte per position, dense: the forward says which positions counted (nullptr: not wanted), the backward reads it
 };
 __device__ __forceinline__ bool z_loss_counts(const ZLossParams& p, int r, int c) {
   return p.labels == nullptr || p.labels[r * p.label_stride + c] != p.ignored;
@@ -152,7 +153,9 @@ __global__ __launch_bounds__(kZThreads) void z_loss_sum_kernel(ZLossParams p, bo
   ZPartial mine = {0.0, 0};
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kZThreads + threadIdx.x; i < p.n; i += static_cast<int64_t>(gridDim.x) * kZThreads) {
     const int r = static_cast<int>(i) / p.cols, c = static_cast<int>(i) - r * p.cols;
-    if (z_loss_counts(p, r, c)) {
+    const bool counts = z_loss_counts(p, r, c);
+    if (SQUARE && p.kept != nullptr) p.kept[i] = counts ? 1 : 0;
+    if (counts) {
       const float x = p.lse[r * p.lse_stride + c];
       mine.sum += static_cast<double>(SQUARE ? x * x : x);
       ++mine.count;
@@ -177,12 +180,14 @@ __global__ __launch_bounds__(256) void z_loss_map_kernel(ZLossParams p, const fl
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= p.n) return;
   const int r = static_cast<int>(i) / p.cols, c = static_cast<int>(i) - r * p.cols;
-  const bool counts = z_loss_counts(p, r, c);
   const float x = p.lse[r * p.lse_stride + c];
   if (!GRAD) {
+    const bool counts = z_loss_counts(p, r, c);
+    if (p.kept != nullptr) p.kept[i] = counts ? 1 : 0;
     out[i] = counts ? x * x : 0.0f;
     return;
   }
+  const bool counts = p.kept == nullptr || p.kept[i] != 0;
   float g = one_grad ? grad[0] : grad[i];
   if (count != nullptr) g /= count[0];
   out[i] = (counts ? g : 0.0f) * (2.0f * x);
@@ -329,7 +334,7 @@ static int sum_launch(const ZLossParams& p, int blocks, bool mean, ZPartial* par
 
 int64_t row_total_workspace_bytes(int64_t n) { return sum_blocks(n) > 1 ? kZBlocks * static_cast<int64_t>(sizeof(ZPartial)) : 0; }
 int row_total_launch(const float* values, int64_t n, bool mean, float* out, void* workspace, hipStream_t stream) {
-  const ZLossParams p = {values, nullptr, n, 0, 0, static_cast<int>(n), static_cast<int>(n > 0 ? n : 1)};
+  const ZLossParams p = {values, nullptr, n, 0, 0, static_cast<int>(n), static_cast<int>(n > 0 ? n : 1), nullptr};
   return sum_launch<false>(p, sum_blocks(n), mean, static_cast<ZPartial*>(workspace), out, nullptr, stream);
 }
 
@@ -400,15 +405,15 @@ extern "C" int64_t cce_z_loss_workspace_bytes(int64_t rows, int64_t cols) {
 }
 
 extern "C" int cce_z_loss_forward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows,
-                                  int64_t cols, int64_t ignored, int reduction, float* out, float* count, void* workspace,
-                                  int64_t workspace_bytes, void* stream_) {
+                                  int64_t cols, int64_t ignored, int reduction, float* out, float* count, uint8_t* kept,
+                                  void* workspace, int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   int64_t n = 0;
   const int st = z_loss_check(lse, rows, cols, &n);
   if (st != CCE_OK) return st;
   if (reduction < CCE_REDUCTION_NONE || reduction > CCE_REDUCTION_MEAN) return CCE_ERR_INVALID_ARGUMENT;
   if (out == nullptr && (n > 0 || reduction != CCE_REDUCTION_NONE)) return CCE_ERR_INVALID_ARGUMENT;
-  const ZLossParams p = {lse, labels, lse_stride, label_stride, ignored, static_cast<int>(n), static_cast<int>(cols > 0 ? cols : 1)};
+  const ZLossParams p = {lse, labels, lse_stride, label_stride, ignored, static_cast<int>(n), static_cast<int>(cols > 0 ? cols : 1), kept};
   if (reduction == CCE_REDUCTION_NONE) {
     if (n == 0) return CCE_OK;
     hipLaunchKernelGGL(z_loss_map_kernel<false>, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, stream, p, nullptr, false,
@@ -424,14 +429,13 @@ extern "C" int cce_z_loss_forward(const float* lse, int64_t lse_stride, const in
   return sum_launch<true>(p, blocks, mean, partial, out, count, stream);
 }
 
-extern "C" int cce_z_loss_backward(const float* lse, int64_t lse_stride, const int64_t* labels, int64_t label_stride, int64_t rows,
-                                   int64_t cols, int64_t ignored, const float* grad, int grad_is_scalar, const float* count,
-                                   float* d_lse, void* stream) {
+extern "C" int cce_z_loss_backward(const float* lse, int64_t lse_stride, const uint8_t* kept, int64_t rows, int64_t cols,
+                                   const float* grad, int grad_is_scalar, const float* count, float* d_lse, void* stream) {
   int64_t n = 0;
   const int st = z_loss_check(lse, rows, cols, &n);
   if (st != CCE_OK || n == 0) return st;
   if (grad == nullptr || d_lse == nullptr) return CCE_ERR_INVALID_ARGUMENT;
-  const ZLossParams p = {lse, labels, lse_stride, label_stride, ignored, static_cast<int>(n), static_cast<int>(cols)};
+  const ZLossParams p = {lse, nullptr, lse_stride, 0, 0, static_cast<int>(n), static_cast<int>(cols), const_cast<uint8_t*>(kept)};
   hipLaunchKernelGGL(z_loss_map_kernel<true>, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), p, grad, grad_is_scalar != 0, count, d_lse);
   return status_from_hip(hipGetLastError());

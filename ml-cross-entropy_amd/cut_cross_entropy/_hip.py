@@ -16,7 +16,7 @@ _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "li
 _lib: Optional[ctypes.CDLL] = None
 _lock = threading.Lock()
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1}
 STAT_ROWS = 32
 STAT_COLS = 32
@@ -71,8 +71,8 @@ _SIGNATURES = {
     "cce_rows_to_steps": (_i32, [_ptr] * 3 + [_i64] * 4 + [_ptr] * 3),
     "cce_steps_to_batch": (_i32, [_ptr] * 2 + [_i64] * 3 + [_ptr] * 3),
     "cce_z_loss_workspace_bytes": (_i64, [_i64, _i64]),
-    "cce_z_loss_forward": (_i32, [_ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _i32, _ptr, _ptr, _ptr, _i64, _ptr]),
-    "cce_z_loss_backward": (_i32, [_ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _ptr, _i32, _ptr, _ptr, _ptr]),
+    "cce_z_loss_forward": (_i32, [_ptr, _i64, _ptr, _i64, _i64, _i64, _i64, _i32, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
+    "cce_z_loss_backward": (_i32, [_ptr, _i64, _ptr, _i64, _i64, _ptr, _i32, _ptr, _ptr, _ptr]),
     "cce_valid_rows": (_i32, [_ptr, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr]),
     "cce_loss_forward": (_i32, [_ptr] * 9 + [_i64] + [_i64] * 4 + [_i64] * 3 + [_i64, _i64, _f32, _i32, _ptr]),
     "cce_loss_call_workspace_bytes": (_i64, [_i64, _i64, _i64, _i32, _i32]),

@@ -702,6 +702,32 @@ def test_z_loss_kernels_against_tensor_operations(shape, shift, reduction, label
         assert torch.allclose(pair[1], out.detach(), rtol=1e-6, atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("shape,shift", [((3, 85), 2), ((5, 3277), 1)])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+def test_labels_overwritten_after_the_z_loss(shape, shift, reduction):
+    """A label buffer that the next batch is written to before the gradients are taken: those of the labels that the loss saw, also
+    for a graph of the gradient and for several upstream gradients at once."""
+    from cut_cross_entropy import utils
+
+    g = torch.Generator().manual_seed(3)
+    lse = (torch.randn(shape, generator=g) * 3 + 9).cuda()[:, shift:].detach().requires_grad_(True)
+    t = torch.randint(0, 50, shape, generator=g)
+    t[torch.rand(shape, generator=g) < 0.3] = -100
+    t = t.cuda()
+    masked = t[:, shift:] == -100
+    sq = lse.square().masked_fill(masked, 0.0)
+    want = sq if reduction == "none" else sq.sum() / (1 if reduction == "sum" else (~masked).sum())
+    out = utils.compute_z_loss(lse, t, shift, reduction=reduction)
+    t.copy_(torch.where(t == -100, 7, -100))
+    up = torch.rand(out.shape, generator=g).cuda() + 0.5
+    (want_grad,) = torch.autograd.grad(want, lse, up)
+    (graphed,) = torch.autograd.grad(out, lse, up, create_graph=True)
+    (both,) = torch.autograd.grad(out, lse, torch.stack([up, up]), retain_graph=True, is_grads_batched=True)
+    (grad,) = torch.autograd.grad(out, lse, up)
+    for got in (grad, graphed, both[0], both[1]):
+        assert torch.allclose(got, want_grad, rtol=4e-7, atol=0)
+
+
 @pytest.mark.parametrize("layout", ["sliced", "permuted", "expanded", "several"])
 @pytest.mark.parametrize("reduction", ["mean", "none"])
 def test_z_loss_of_layouts_with_dimensions_of_one_entry(layout, reduction):
