@@ -218,6 +218,20 @@ def test_a_shift_past_the_sequences_is_refused(shape, shift):
             _build_flat_valids(torch.zeros(shape, dtype=torch.int64, device=device), -100, shift)
 
 
+@pytest.mark.parametrize("shape,shift", [((2, 4), 4), ((2, 4), 5), ((0, 4), 4), ((2, 0), 1)])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_the_operator_refuses_a_shift_past_the_sequences(shape, shift, reduction, dtype):
+    """The same through the operator itself, empty batches among them."""
+    from cut_cross_entropy.cce import cce_linear_cross_entropy
+
+    e = torch.randn(shape + (64,), device="cuda", dtype=dtype).requires_grad_(True)
+    c = torch.randn((100, 64), device="cuda", dtype=dtype).requires_grad_(True)
+    t = torch.zeros(shape, dtype=torch.int64, device="cuda")
+    with pytest.raises(RuntimeError, match="No label lies shift="):
+        cce_linear_cross_entropy(e, c, t, shift=shift, reduction=reduction, return_lse=True)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(2, 3, 8), (5, 256 * 70, 128), (130, 700, 123), (1000, 2000, 192)])
 @pytest.mark.parametrize("softcap,bias,shift", [(None, False, 0), (15.0, True, 1)])
