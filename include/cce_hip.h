@@ -350,7 +350,8 @@ int cce_loss_forward(const void* e, const void* c, const void* bias, const int32
  * per position without the first `shift` steps, and lse_out (may be NULL) like that, which is left alone where it would be lse:
  * no shift and *count == n.  rows[n], lse[n] (the first *count
  * are written) and tile_max (may be NULL; cce_tile_stat_elems(n, v) floats) are kept for a backward.  `workspace` 256-byte
- * aligned.  CCE_ERR_WORKSPACE_TOO_SMALL after a wait (*count >= 0): rows and *count are written, the rest is for the single calls.
+ * aligned.  CCE_ERR_WORKSPACE_TOO_SMALL after a wait (*count >= 0): rows and *count are written, the rest is for the single calls;
+ * *count is -1 after any refusal before the wait.
  * Refuses a stream that is being captured.
  */
 int64_t cce_loss_call_workspace_bytes(int64_t n, int64_t v, int64_t d, int dtype, int terms);

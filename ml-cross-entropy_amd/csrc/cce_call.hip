@@ -57,6 +57,8 @@ extern "C" int cce_loss_call(const void* e, const void* c, const void* bias, con
                              int64_t shift, int64_t ignored, int64_t target_offset, float softcap, int reduction, int dtype, int terms,
                              void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
+  // before anything is refused: a caller that keeps the word from call to call can tell a refusal from rows that are written
+  if (count != nullptr) __atomic_store_n(count, int64_t(-1), __ATOMIC_RELEASE);
   if (n <= 0 || steps <= 0 || n % steps != 0 || shift < 0 || shift >= steps || v <= 0 || d <= 0) return CCE_ERR_INVALID_ARGUMENT;
   if (reduction < CCE_REDUCTION_NONE || reduction > CCE_REDUCTION_MEAN) return CCE_ERR_INVALID_ARGUMENT;
   if (dtype != CCE_DTYPE_BF16 && dtype != CCE_DTYPE_F16 && dtype != CCE_DTYPE_F32) return CCE_ERR_UNSUPPORTED_DTYPE;
@@ -69,7 +71,6 @@ extern "C" int cce_loss_call(const void* e, const void* c, const void* bias, con
   if (err != hipSuccess) return status_from_hip(err);
   if (capturing != hipStreamCaptureStatusNone) return status_from_hip(hipErrorStreamCaptureUnsupported);  // nothing would run
 
-  __atomic_store_n(count, int64_t(-1), __ATOMIC_RELEASE);
   int st = cce_valid_rows(labels, n, steps, shift, ignored, rows, count, stream_);
   if (st != CCE_OK) return st;
   int64_t b = 0;

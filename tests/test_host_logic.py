@@ -241,3 +241,27 @@ def test_rows_of_steps_lead_to_the_elements_they_name():
     # what was read at the wrong places
     check(torch.arange(384).view(4, 1, 12, 8)[:, :, :5])
     check(torch.arange(160).view(5, 4, 1, 8).permute(1, 2, 0, 3))
+
+
+def test_a_refused_loss_call_leaves_no_count_of_an_earlier_one():
+    """The word that receives the count is kept from call to call: -1 after a refusal, so that a workspace too small from the start is
+    told from one too small for the rows found.  Nothing is launched: the addresses are never followed."""
+    import ctypes
+
+    from cut_cross_entropy import _hip
+
+    lib = _hip.load()
+    count, somewhere = ctypes.c_int64(77), ctypes.addressof(ctypes.create_string_buffer(512))
+    somewhere = (somewhere + 255) // 256 * 256
+
+    def call(workspace, workspace_bytes, n=64, dtype=0):
+        count.value = 77
+        return lib.cce_loss_call(somewhere, somewhere, None, somewhere, somewhere, ctypes.addressof(count), somewhere, None, somewhere,
+                                 None, workspace, workspace_bytes, n, 64, 512, 128, 128, 128, 1, 0, -100, 0, 0.0, 2, dtype, 0, None)
+
+    assert call(None, 0) == _hip.ERR_WORKSPACE_TOO_SMALL and count.value == -1
+    needed = lib.cce_loss_call_workspace_bytes(64, 512, 128, 0, 0)
+    assert call(somewhere, needed - 1) == _hip.ERR_WORKSPACE_TOO_SMALL and count.value == -1
+    assert call(somewhere + 8, needed) != 0 and count.value == -1
+    assert call(somewhere, needed, n=65) != 0 and count.value == -1
+    assert call(somewhere, needed, dtype=7) != 0 and count.value == -1
