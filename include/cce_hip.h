@@ -224,7 +224,7 @@ int cce_backward_dz(const void* e, const void* c, const void* bias,
  * whole 256-class tiles of b rows, at most 16384 classes -- or, where it walks by rows, to whole 256-row blocks of all
  * classes -- and never goes below one tile), plus the 16-bit compensation term of the gradient it carries from
  * launch to launch when `d_e_in_workspace` (d_e wanted in the 16-bit input type): [b, d] for dE, or [v, d] for dC
- * where b >= 2 v and the walk goes by blocks of rows (see cce_backward_dense).
+ * where b >= 2 v, v <= 2^23 and the walk goes by blocks of rows (see cce_backward_dense).
  * cce_backward_dense_fixed_bytes is the second part alone; cce_backward_dense_dz_bytes the size of a dz buffer of
  * `units` classes per chunk (rows per block where the walk goes by rows), for a caller that sizes the workspace
  * against a limit of its own. */

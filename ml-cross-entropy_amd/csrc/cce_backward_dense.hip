@@ -605,8 +605,11 @@ struct DensePlan {
   int64_t dz_bytes;
   int64_t slot_bytes;   // of all slots
 };
+// (A block's rows of dz are whole vocabularies apart, and a tile of dE reaches 256 of them by 32-bit byte offsets: wider ones
+// go by classes.)
 static bool dense_walks_by_rows(int64_t b, int64_t v, bool gradients_16bit) {
-  return gradients_16bit && b >= 2 * ((v + 255) / 256 * 256);
+  const int64_t v_pad = (v + 255) / 256 * 256;
+  return gradients_16bit && b >= 2 * v_pad && v_pad <= (int64_t(1) << 23);
 }
 
 // A split of n steps of 64: multiples of whole stages, so that only the last one has a partial stage.

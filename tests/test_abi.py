@@ -104,6 +104,25 @@ def test_dense_backward_plans_by_classes_or_by_rows():
         assert dz <= a256(B) * v_pad * 2
 
 
+def test_dense_backward_goes_by_rows_only_where_offsets_reach_a_block():
+    """Rows of dz of a walk by rows are a vocabulary apart, and 256 of them are reached by 32-bit byte offsets: up to 2^23 classes.
+    More go by classes, in chunks whose 256 rows are reached."""
+    lib = _lib()
+    a256 = lambda x: (x + 255) // 256 * 256
+    D = 64
+    for V in (1 << 23, (1 << 23) + 1):
+        B = 2 * a256(V)
+        by_rows = V == 1 << 23
+        assert lib.cce_backward_dense_fixed_bytes(B, V, D, 1) == a256((V if by_rows else B) * D * 2)
+        units = 4096
+        dz = lib.cce_backward_dense_dz_bytes(B, V, D, 1, units)
+        assert dz == units * (a256(V) if by_rows else B) * 2
+        row = a256(V) if by_rows else units  # classes from one row of dz to the next
+        assert (255 * row + 56) * 2 < 1 << 32
+        total = lib.cce_backward_dense_workspace_bytes(B, V, D, 1, dz)
+        assert total >= a256((V if by_rows else B) * D * 2) + 256 * (a256(V) if by_rows else B) * 2
+
+
 @pytest.mark.parametrize("sizes", [(0, 10, 64), (10, 0, 64), (10, 10, 0), (0, 0, 0)])
 def test_size_queries_answer_for_empty_matrices(sizes):
     """A query is asked before the call that refuses such sizes, so it has to answer."""
