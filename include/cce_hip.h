@@ -133,10 +133,14 @@ int cce_indexed_neg_dot(const void* e, const void* c, const int64_t* targets, co
                         int64_t shift, int64_t target_offset,
                         float softcap, int dtype, void* stream);
 
-/* Scratch bytes cce_backward needs: one survivor bit per 32 x 32 sub-tile, each 32-row group's bits
+/* Scratch bytes for cce_backward: one survivor bit per 32 x 32 sub-tile, each 32-row group's bits
  * padded to whole 32-bit words, then a count and one int32 per 32-class group (the class groups its second,
- * full dC pass takes over from the light one). */
+ * full dC pass takes over from the light one); where few row groups are dealt to several workgroups, bits and an fp32 slot for each;
+ * and for wide rows the gradients that its first pass keeps for its later ones.  These are kept only by a call with tile_max that
+ * wants d_c filtered, d_e filtered or not at all, and no d_bias or vocab_order: any other does with what
+ * cce_backward_unkept_workspace_bytes answers, and so does this one, which then forms them again. */
 int64_t cce_backward_workspace_bytes(int64_t b, int64_t v, int64_t d);
+int64_t cce_backward_unkept_workspace_bytes(int64_t b, int64_t v, int64_t d);
 
 /*
  * Gradients of  sum_i d_out_i * nll_i + d_lse_i * lse_i  w.r.t. e, c and bias.

@@ -1549,11 +1549,17 @@ static int64_t dz_bytes(int64_t b, int64_t v, int64_t d) {
   return quota == 0 ? 0 : round16(kept_bits_bytes(b, v)) + (b + 31) / 32 * quota * kDzSlotElems * 2;
 }
 
-extern "C" int64_t cce_backward_workspace_bytes(int64_t b, int64_t v, int64_t d) {
+extern "C" int64_t cce_backward_unkept_workspace_bytes(int64_t b, int64_t v, int64_t d) {
   if (b <= 0 || v <= 0) return 0;
   const int parts = owner_parts(b, v, d);
   if (parts > 1) return round16(lists_bytes(b, v)) + part_bits_bytes(b, v, parts) + parts * ((b + 31) / 32 * 32) * d * 4;
-  return dz_quota(b, v, d) == 0 ? lists_bytes(b, v) : round16(lists_bytes(b, v)) + dz_bytes(b, v, d);
+  return lists_bytes(b, v);
+}
+
+extern "C" int64_t cce_backward_workspace_bytes(int64_t b, int64_t v, int64_t d) {
+  if (b <= 0 || v <= 0) return 0;
+  // (with several workgroups per row group nothing is kept)
+  return dz_quota(b, v, d) == 0 ? cce_backward_unkept_workspace_bytes(b, v, d) : round16(lists_bytes(b, v)) + dz_bytes(b, v, d);
 }
 
 extern "C" int cce_backward(const void* e, const void* c, const void* bias,
@@ -1688,10 +1694,10 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
   p.slice_first = 0;
   if (need_de_pass) {
     p.nslices = (d_e != nullptr) ? full_slices : 1;
-    // (a caller who brings less workspace than the size query names gets one workgroup per row group and no kept gradients)
+    // (a caller who brings less workspace than the size queries name gets one workgroup per row group, or no kept gradients)
     const int parts = owner_parts(b, v, d);
     if (fast && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
-        workspace_bytes >= cce_backward_workspace_bytes(b, v, d)) {
+        workspace_bytes >= cce_backward_unkept_workspace_bytes(b, v, d)) {
       unsigned char* ws = static_cast<unsigned char*>(workspace) + round16(lists_bytes(b, v));
       if (parts > 1) {
         p.parts = parts;
@@ -1699,7 +1705,9 @@ extern "C" int cce_backward(const void* e, const void* c, const void* bias,
         p.slots = reinterpret_cast<float*>(ws + part_bits_bytes(b, v, parts));
       }
       // dBias sums the gradients in fp32: with it they are formed again.  Without a candidate list there is no order to find them by.
-      if (dz_quota(b, v, d) > 0 && p.shortcut && need_bits && d_bias == nullptr) {
+      // (cce_backward.py asks for the larger workspace by the same rule)
+      if (dz_quota(b, v, d) > 0 && p.shortcut && need_bits && d_bias == nullptr &&
+          workspace_bytes >= cce_backward_workspace_bytes(b, v, d)) {
         p.dz_mode = kDzStore;
         p.dz_quota = dz_quota(b, v, d);
         p.cand_bits = reinterpret_cast<uint32_t*>(ws);

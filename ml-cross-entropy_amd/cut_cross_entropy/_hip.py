@@ -33,6 +33,7 @@ _SIGNATURES = {
     "cce_tile_stat_elems": (_i64, [_i64, _i64]),
     "cce_lse_forward_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "cce_backward_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "cce_backward_unkept_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "cce_lse_forward": (
         _i32,
         [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64]

@@ -56,7 +56,8 @@ FILTERED_BACKWARD_PATH = "auto"
 # of workspace (the dz buffer, plus the 16-bit compensation buffer of the gradient that is carried between launches:
 # [B, D] for dE, or [V, D] for dC where rows outnumber classes two to one): the ownership kernels need well
 # under 16 MB (with few rows up to half the bytes of C on top, fp32 slots for workgroups that share a row group: 53 MB at
-# 307 rows of 5120 columns against 131072 classes), and a caller who picked a filtered preset did not ask for more.  The defaults, 256 MB and 1.0, say:
+# 307 rows of 5120 columns against 131072 classes; with more rows of more than 2304 columns 2.5 KB per row, gradients kept from
+# pass to pass: 169 MB at 65536 rows, beside 470 MB of E), and a caller who picked a filtered preset did not ask for more.  The defaults, 256 MB and 1.0, say:
 # never more than the operands the caller already holds take themselves, and 256 MB where they are smaller (the
 # second term matters when rows are many: at E [65536, 3584] x C [19008, 3584] the compensation buffer alone is
 # 448 MB and the operands are 578 MB; the ownership kernels take 167 ms there, the unfiltered path 22 - 30).  The dz chunk
@@ -378,7 +379,12 @@ def cce_backward_kernel(
         assert counters.is_contiguous() and counters.device == dev
 
     if B > 0 and (de_sparse or dc_sparse):
-        ws_bytes = lib.cce_backward_workspace_bytes(B, c.size(0), e.size(1))
+        # Gradients are kept from pass to pass (wide rows: 80 KB per 32 of them) by calls whose passes all go by one list of
+        # candidates, and not beside a dBias, which sums them in fp32: any other call does without the room for them.
+        keeps = (tile_max is not None and vocab_ordering is None and filter_eps_or_none(filter_eps) > 0.0 and dc_sparse and want_dc
+                 and not want_dbias and filter_c_grad and (filter_e_grad or not de_sparse))
+        room = lib.cce_backward_workspace_bytes if keeps else lib.cce_backward_unkept_workspace_bytes
+        ws_bytes = room(B, c.size(0), e.size(1))
         workspace = torch.empty((max(ws_bytes, 8) // 8 + 1,), dtype=torch.int64, device=dev)
         with _hip.on_device(dev), _hip.timed("backward_sparse", dev):
             status = lib.cce_backward(

@@ -64,6 +64,11 @@ def test_host_only_queries():
     # survivor bits (256 row groups x 250 words) + a count and one id per class group for the second dC pass
     assert lib.cce_backward_workspace_bytes(8192, 256000, 2304) == 256 * 250 * 4 + (1 + 8000) * 4
     assert lib.cce_backward_workspace_bytes(0, 5, 5) == 0
+    # rows of more than one slice: room for kept gradients on top, which not every call uses (candidate bits, 40 slots of 2 KB)
+    lists = 2048 * 149 * 4 + (1 + 4752) * 4
+    assert lib.cce_backward_unkept_workspace_bytes(65536, 152064, 3584) == lists
+    kept = 2048 * 149 * 4 + 2048 * 40 * 2048
+    assert lib.cce_backward_workspace_bytes(65536, 152064, 3584) == (lists + 15) // 16 * 16 + kept
 
 
 def test_header_constants_match_binding():

@@ -825,6 +825,41 @@ def test_gradients_kept_between_the_filtered_passes(monkeypatch, shape, dtype, f
         assert ((a - b).abs() <= 2e-2 * b.abs() + 2e-2 * b.abs().amax(dim=1, keepdim=True)).all()
 
 
+@pytest.mark.parametrize("call,keeps", [("plain", True), ("frozen e", True), ("frozen c", False), ("bias", False), ("frozen bias", True),
+                                        ("unfiltered c", False), ("unfiltered e", True), ("no filter", None)])
+def test_room_for_kept_gradients_only_where_they_are_kept(monkeypatch, call, keeps):
+    """Which calls bring the larger workspace.  With dE unfiltered the ownership kernels are left with dC, whose passes keep."""
+    from cut_cross_entropy import _hip
+    from cut_cross_entropy import cce_backward as bw
+    from cut_cross_entropy import linear_cross_entropy
+
+    monkeypatch.setattr(bw, "FILTERED_BACKWARD_PATH", "sparse")
+    N, V, D = 1200, 1000, 2432
+    lib, brought = _hip.load(), []
+    least, most = lib.cce_backward_unkept_workspace_bytes(N, V, D), lib.cce_backward_workspace_bytes(N, V, D)
+    assert most - least >= (N // 32) * 40 * 2048
+
+    class Recorded:
+        def __getattr__(self, name):
+            if name == "cce_backward":
+                return lambda *a: brought.append(a[15]) or lib.cce_backward(*a)
+            return getattr(lib, name)
+
+    monkeypatch.setattr(_hip, "load", lambda: Recorded())
+    g = torch.Generator().manual_seed(4)
+    e = torch.randn((N, D), generator=g).to(torch.bfloat16).cuda().requires_grad_(call != "frozen e")
+    c = (torch.randn((V, D), generator=g) * 0.05).to(torch.bfloat16).cuda().requires_grad_(call != "frozen c")
+    t = torch.randint(0, V, (N,), generator=g).cuda()
+    bias = torch.zeros((V,), dtype=torch.bfloat16, device="cuda", requires_grad=call == "bias") if "bias" in call else None
+    impl = {"unfiltered c": "cce_kahan_full_c", "unfiltered e": "cce_kahan_full_e", "no filter": "cce_exact"}.get(call, "cce")
+    linear_cross_entropy(e, c, t, bias=bias, impl=impl).backward()
+    if keeps is None:
+        assert not brought
+    else:
+        (got,) = brought
+        assert got >= most if keeps else least <= got < least + 16
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows", [129, 191, 192, 193, 300, 384, 385, 576])
 @pytest.mark.parametrize("width,classes", [(128, 256), (136, 1000), (192, 256 * 40 + 1), (704, 256 * 130)])
