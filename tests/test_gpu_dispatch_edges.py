@@ -742,6 +742,37 @@ def test_labels_overwritten_after_the_z_loss(shape, shift, reduction):
         assert torch.allclose(got, want_grad, rtol=4e-7, atol=0)
 
 
+@pytest.mark.parametrize("reduction", ["mean", "none"])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_upstream_gradients_that_are_lazily_negated(reduction, shift, dtype):
+    """What sends the gradients of imaginary parts back through a conjugate sends views with the negative bit set: the same gradients
+    as from plain tensors, of the loss, of the log-sum-exps and of the z-loss."""
+    from cut_cross_entropy import linear_cross_entropy, utils
+
+    class Negated(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return torch._neg_view((-g).contiguous())
+
+    g = torch.Generator().manual_seed(2)
+    e0 = torch.randn((3, 40, 128), generator=g).to(dtype).cuda()
+    c0 = (torch.randn((500, 128), generator=g) * 0.1).to(dtype).cuda()
+    t = torch.randint(0, 500, (3, 40), generator=g).cuda()
+    got = []
+    for through in (lambda x: x.clone(), Negated.apply):
+        e, c = e0.clone().requires_grad_(True), c0.clone().requires_grad_(True)
+        loss, lse = linear_cross_entropy(e, c, t, shift=shift, reduction=reduction, return_lse=True)
+        z = utils.compute_z_loss(lse, t, shift, reduction=reduction)
+        (through(loss).sum() + 1e-2 * through(lse).sum() + 1e-2 * through(z).sum()).backward()
+        got.append((e.grad, c.grad))
+    assert got[0][0].any() and torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("layout", ["sliced", "permuted", "expanded", "several"])
 @pytest.mark.parametrize("reduction", ["mean", "none"])
 def test_z_loss_of_layouts_with_dimensions_of_one_entry(layout, reduction):
