@@ -773,6 +773,26 @@ def test_upstream_gradients_that_are_lazily_negated(reduction, shift, dtype):
     assert got[0][0].any() and torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+def test_a_trace_of_the_z_loss_can_be_saved(reduction):
+    """torch.jit.trace records tensor operations: the trace is saved, loaded and run on other labels and values."""
+    import io
+
+    from cut_cross_entropy import utils
+
+    g = torch.Generator().manual_seed(1)
+    lse, other = (torch.randn((3, 6), generator=g).cuda() + 5 for _ in range(2))
+    t = torch.tensor([[0, -100, 1, 2, 3, 4, 5]] * 3).cuda()
+    traced = torch.jit.trace(lambda x, labels: utils.compute_z_loss(x, labels, 1, reduction=reduction), (lse, t))
+    file = io.BytesIO()
+    torch.jit.save(traced, file)
+    file.seek(0)
+    loaded = torch.jit.load(file)
+    for x, labels in ((lse, t), (other, t.roll(2, 1))):
+        # at most 18 additions of one sign, in either order
+        assert torch.allclose(loaded(x, labels), utils.compute_z_loss(x, labels, 1, reduction=reduction), rtol=18 * 2.0**-23, atol=0)
+
+
 @pytest.mark.parametrize("layout", ["sliced", "permuted", "expanded", "several"])
 @pytest.mark.parametrize("reduction", ["mean", "none"])
 def test_z_loss_of_layouts_with_dimensions_of_one_entry(layout, reduction):
