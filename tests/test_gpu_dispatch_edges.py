@@ -850,8 +850,8 @@ def test_cut_reductions_in_more_launches(monkeypatch, shape, budget):
 @pytest.mark.parametrize("few_labels", [False, True])
 def test_gradients_kept_between_the_filtered_passes(monkeypatch, shape, dtype, few_labels):
     """Widths in slices: the dE pass keeps the gradients of surviving sub-tiles, slices after the first (a launch of their own from 256 row
-    groups on) and the dC pass read them.  Row groups with fewer candidates than slots and with more (every class a label), a partial
-    last stage, against the same call with a bias of zeros, for whose gradient everything is formed again."""
+    groups on) and the dC pass read them.  Candidates that all have a slot (the labels of 32 rows), a partial last stage, against the
+    same call with a bias of zeros, for whose gradient everything is formed again.  (More candidates than slots: below.)"""
     from cut_cross_entropy import cce_backward as bw
     from cut_cross_entropy import linear_cross_entropy
 
@@ -872,6 +872,62 @@ def test_gradients_kept_between_the_filtered_passes(monkeypatch, shape, dtype, f
     for a, b in zip(*got):
         assert torch.isfinite(a).all() and a.abs().max() > 0
         # dz is rounded to the type from logits summed in another order: 2^-9 (bf16) of single products, and of the results
+        assert (a - b).norm() <= 2e-3 * b.norm()
+        assert ((a - b).abs() <= 2e-2 * b.abs() + 2e-2 * b.abs().amax(dim=1, keepdim=True)).all()
+
+
+@pytest.mark.parametrize("shape,likely", [((8200, 2500, 2432), 6), ((4500, 1900, 2312), 3), ((8192, 3000, 4736), 2), ((4500, 60000, 2432), 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_more_candidates_than_slots_for_kept_gradients(monkeypatch, shape, likely, dtype):
+    """Rows with several likely classes: row groups with more candidates than the 40 slots beside groups with fewer, so that trips read
+    kept gradients, form them again, and do either for some of their entries; and, with classes many against the rows, class groups of one
+    or two survivors, which the light dC pass takes.  What each is here for is counted in plain torch.  Reference and bounds as above."""
+    from cut_cross_entropy import cce_backward as bw
+    from cut_cross_entropy import linear_cross_entropy
+    from cut_cross_entropy.cce_lse_forward import loss_forward
+
+    monkeypatch.setattr(bw, "FILTERED_BACKWARD_PATH", "sparse")
+    N, V, D = shape
+    eps, softcap, quota = 2.0**-9, 50.0, 40
+    g = torch.Generator(device="cuda").manual_seed(N + V)
+    c = (torch.randn((V, D), generator=g, device="cuda") * 0.02).to(dtype)
+    # a logit of 12 for each of `likely` classes; every fourth row group has its labels alone, all in one sub-tile
+    pick = torch.randint(0, V, (likely, N), generator=g, device="cuda")
+    few = (torch.arange(N, device="cuda") // 32) % 4 == 0
+    pick[:, few] = torch.randint(0, 32, (1, int(few.sum())), generator=g, device="cuda")
+    t = pick[0].clone()
+    e = torch.randn((N, D), generator=g, device="cuda") * 0.1
+    for classes in pick:
+        add = 12.0 / (D * 0.02**2) * c[classes].float()
+        e += torch.where(few[:, None], add / likely, add)
+    e = e.to(dtype)
+
+    # candidates of a row group: sub-tiles whose largest logit can make a probability of eps in one of its rows, and those of its labels
+    lse, _, tile_max = loss_forward(e, c, None, t, None, 0, softcap, 0, True)
+    groups, blocks = -(-N // 32), -(-V // 32)
+    low = torch.nn.functional.pad(lse, (0, groups * 32 - N), value=float("inf")).view(groups, 32).amin(1)
+    candidate = tile_max.view(groups, blocks) - low[:, None] >= torch.log(torch.tensor(eps)).item()
+    candidate[torch.arange(N, device="cuda") // 32, t // 32] = True
+    per_group = candidate.sum(1)
+    p = torch.exp(softcap * torch.tanh((e.float() @ c.float().T) / softcap) - lse[:, None])
+    p[torch.arange(N, device="cuda"), t] -= 1.0
+    p = torch.nn.functional.pad(p.abs(), (0, blocks * 32 - V, 0, groups * 32 - N)).view(groups, 32, blocks, 32).amax((1, 3)) >= eps
+    if V < 10000:
+        assert (per_group > quota).sum() > groups // 2 and (per_group <= quota).any()
+        # survivors behind the last slot, and class groups whose list holds survivors of either kind
+        late = p & candidate & (candidate.cumsum(1) > quota)
+        assert (late.any(0) & (p & candidate & ~late).any(0)).sum() > 4
+    else:
+        light = ((p & candidate).sum(0) >= 1) & ((p & candidate).sum(0) <= 2)
+        assert light.sum() > 500 and (p.sum(0) > 2).any()
+
+    got = []
+    for bias in (None, torch.zeros((V,), dtype=dtype, device="cuda", requires_grad=True)):
+        e1, c1 = e.clone().requires_grad_(True), c.clone().requires_grad_(True)
+        linear_cross_entropy(e1, c1, t, bias=bias, softcap=softcap, reduction="sum", filter_eps=eps).backward()
+        got.append((e1.grad.double(), c1.grad.double()))
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and a.abs().max() > 0
         assert (a - b).norm() <= 2e-3 * b.norm()
         assert ((a - b).abs() <= 2e-2 * b.abs() + 2e-2 * b.abs().amax(dim=1, keepdim=True)).all()
 
