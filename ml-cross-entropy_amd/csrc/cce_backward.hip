@@ -1301,8 +1301,8 @@ __global__ __launch_bounds__(kBwdThreads, LIGHT ? 2 : 1) void bwd_owner_fast_ker
     if (write_out && !touched) {
       // Nothing survived for this class group: its rows are zeros, written as whole 16-byte pieces, a wave
       // instruction inside one row (the launcher guarantees 16-byte aligned rows and D a multiple of 8), past the caches: they
-      // are written once, and pushed out what the next kernels read again (307 rows x 5120 x 131072: this pass 376 -> 342 us, the
-      // forward of the step after it 520 -> 494; a kernel of its own for the zeros takes 229 us beside 183 of the rest).
+      // are written once, and pushed out what the next kernels read again (307 rows x 5120 x 131072: this pass 376 -> 342 us; and where
+      // the step after it runs on the same C, part of which is then still in the caches, its forward 520 -> 494; a kernel of its own for the zeros takes 229 us beside 183 of the rest).
       const int ppr = (d_end - d_begin) / 8;  // 16-byte pieces per row
       typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
       const u32x4 zero = {0u, 0u, 0u, 0u};
