@@ -965,6 +965,11 @@ def test_room_for_kept_gradients_only_where_they_are_kept(monkeypatch, call, kee
     else:
         (got,) = brought
         assert got >= most if keeps else least <= got < least + 16
+    if keeps:  # the same gradient where everything is formed again (a bias of zeros that wants one); bound as above
+        e1, c1 = e.detach().clone().requires_grad_(e.requires_grad), c.detach().clone().requires_grad_(True)
+        linear_cross_entropy(e1, c1, t, bias=torch.zeros((V,), dtype=c.dtype, device="cuda", requires_grad=True), impl=impl).backward()
+        for x, y in ((c, c1),) if call == "frozen e" else ((e, e1), (c, c1)):
+            assert y.grad.any() and (x.grad.double() - y.grad.double()).norm() <= 2e-3 * y.grad.double().norm()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
