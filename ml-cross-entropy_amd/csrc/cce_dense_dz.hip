@@ -539,10 +539,11 @@ __global__ __launch_bounds__(kDzThreads, 1) void dz_terms_kernel(DzParams p) {
 __global__ __launch_bounds__(1024) void dz_scale_kernel(const float* d_out, int d_out_is_scalar, const float* d_lse, const int32_t* valids,
                                                         int64_t n_rows, int64_t b, float grad_scale, int64_t shift, DzScale* out) {
   float most = 0.0f, least = INFINITY;
-  const int64_t n = (d_out_is_scalar && d_lse == nullptr) ? 1 : b;  // one row stands for all of them
+  const bool uniform = d_out_is_scalar && d_lse == nullptr;  // one row stands for all of them, and no position is read
+  const int64_t n = uniform ? 1 : b;
   for (int64_t i = threadIdx.x; i < n; i += 1024) {
     const int64_t at = (valids != nullptr ? static_cast<int64_t>(valids[i]) : i) + shift;
-    if (n > 1 && at >= n_rows) continue;
+    if (!uniform && at >= n_rows) continue;
     float w = fabsf(grad_scale * d_out[d_out_is_scalar ? 0 : at]);
     if (d_lse != nullptr) w += fabsf(d_lse[at]);
     if (!(w > 0.0f && w < INFINITY)) continue;

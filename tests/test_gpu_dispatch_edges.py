@@ -190,6 +190,28 @@ def test_fp32_passes_abi(shape, keep, extra, terms):
     assert (de[ignored] == 0).all()
 
 
+@pytest.mark.parametrize("scalar,with_dlse", [(0, False), (0, True), (1, True), (1, False)])
+def test_fp32_backward_of_one_row_whose_label_is_past_the_end(scalar, with_dlse):
+    """One row, no list of rows and a shift: the row has no label, so its gradients are zeros whatever stands behind the one upstream
+    gradient that there is."""
+    lib = _lib()
+    V, D = 300, 72
+    e, c, t, _, _, _, _, _ = _fp32_case(1, V, D, 1.0, 3)
+    lse = torch.logsumexp(e @ c.T, 1)
+    w = torch.full((64,), float("nan"), device="cuda")
+    h = torch.full((64,), 1e30, device="cuda")
+    w[0] = h[0] = 1.0
+    de, dc, db = torch.zeros((1, D), device="cuda"), torch.full((V, D), float("nan"), device="cuda"), torch.zeros((V,), device="cuda")
+    n_ws = lib.cce_fp32_backward_workspace_bytes(1, V, D, 6)
+    buf = torch.full((n_ws // 4 + 64,), float("nan"), device="cuda")
+    ws = (buf.data_ptr() + 255) // 256 * 256
+    p = lambda x: x.data_ptr()
+    st = lib.cce_fp32_backward(p(e), p(c), None, p(lse), p(w), scalar, p(h) if with_dlse else None, None, p(t), p(de), p(dc), p(db), ws,
+                               n_ws, 1, 1, V, D, D, D, 1, D, D, 1.0, 1, 0, 0.0, 6, torch.cuda.current_stream().cuda_stream)
+    assert st == 0, lib.cce_error_string(st)
+    assert (de == 0).all() and (dc == 0).all() and (db == 0).all()
+
+
 @pytest.mark.parametrize("where", ["inside", "e", "c", "late c", "upstream", "nan"])
 @pytest.mark.parametrize("bias", [False, True])
 def test_fp32_values_without_room_in_halves_go_by_parts(where, bias):
