@@ -72,10 +72,6 @@ struct ProductParams {
   int terms, part_d, dz_part, out_vec;
   int64_t rows_out;
   int cls_out;
-  // *wide == 0: the parts are halves, packed two to a row, of c and e at *_unit of their size and of dz at that of dz_scale
-  const int* wide;
-  const DzScale* dz_scale;
-  float c_unit, e_unit;
 };
 
 constexpr int kProdThreads = 512;  // eight waves, two per SIMD
@@ -176,9 +172,8 @@ __device__ __forceinline__ void dc_source(typename Tile::Source& s, const Produc
 }
 
 // The two products of operands in parts, fp32 results: the tiles below without what 16-bit gradients need.
-template <typename T>
 __device__ __forceinline__ void terms_de_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
-  using Tile = Tile8<T, false, false, true>;
+  using Tile = Tile8<BF16, false, false, true>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int64_t m0 = static_cast<int64_t>(tm) * Tile::TILE;
   const int n0 = tn * Tile::TILE;
@@ -190,7 +185,6 @@ __device__ __forceinline__ void terms_de_tile(const ProductParams& p, int split,
   s.terms = p.terms;
   Tile::plan(s);
   float* const de = p.de_f32 + split * p.de_slot;
-  const float unit = Tile::HALVES ? p.dz_scale->unit * p.c_unit : 1.0f;
 
   f32x4 acc[Tile::WM][Tile::WN];
   Tile::run(acc, s, smem, g);
@@ -202,19 +196,18 @@ __device__ __forceinline__ void terms_de_tile(const ProductParams& p, int split,
     float out[8];
     if (p.de_init) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) out[k] = v[k] * unit;
+      for (int k = 0; k < 8; ++k) out[k] = v[k];
     } else {
       load_piece(de + re * p.ld_de, cg, p.d, p.out_vec != 0, out);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) out[k] = fmaf(v[k], unit, out[k]);
+      for (int k = 0; k < 8; ++k) out[k] += v[k];
     }
     store_piece(de + re * p.ld_de, cg, p.d, p.out_vec != 0, out);
   });
 }
 
-template <typename T>
 __device__ __forceinline__ void terms_dc_tile(const ProductParams& p, int split, int tm, int tn, unsigned char* smem) {
-  using Tile = Tile8<T, true, false, true>;
+  using Tile = Tile8<BF16, true, false, true>;
   typename Tile::Geometry g = Tile::geometry(smem);
   const int m0 = tm * Tile::TILE;
   const int n0 = tn * Tile::TILE;
@@ -226,7 +219,6 @@ __device__ __forceinline__ void terms_dc_tile(const ProductParams& p, int split,
   s.terms = p.terms;
   Tile::plan(s);
   float* const dc = static_cast<float*>(p.d_c) + split * p.dc_slot;
-  const float unit = Tile::HALVES ? p.dz_scale->unit * p.e_unit : 1.0f;
 
   f32x4 acc[Tile::WM][Tile::WN];
   Tile::run(acc, s, smem, g);
@@ -237,7 +229,7 @@ __device__ __forceinline__ void terms_dc_tile(const ProductParams& p, int split,
     float* dst = dc + static_cast<int64_t>(cls) * p.ld_dc;
     float out[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) out[k] = v[k] * unit;
+    for (int k = 0; k < 8; ++k) out[k] = v[k];
     if (p.dc_accumulate) {
       float old[8];
       load_piece(dst, cg, p.d, p.out_vec != 0, old);
@@ -433,31 +425,19 @@ __global__ __launch_bounds__(kProdThreads, 1) void dense_products_kernel(Product
   }
 }
 
-// The same for operands in parts, of the kind that the device found them to need.
-template <typename T>
-__device__ __forceinline__ void terms_products_item(const ProductParams& p, unsigned char* smem) {
+// The same for operands in parts.
+__global__ __launch_bounds__(kProdThreads, 1) void terms_products_kernel(ProductParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
   const int first_blocks = (p.de_first ? p.de_per_xcd : p.dc_per_xcd) * 8;
   const bool first = static_cast<int>(blockIdx.x) < first_blocks;
   const int block = first ? blockIdx.x : blockIdx.x - first_blocks;
   int split, tm, tn;
   if (first != (p.de_first != 0)) {
     if (!product_tile_of(block, p.dc_tiles, p.dc_splits, p.dc_per_xcd, p.tiles_n, split, tm, tn)) return;
-    terms_dc_tile<T>(p, split, tm, tn, smem);
+    terms_dc_tile(p, split, tm, tn, smem);
   } else {
     if (!product_tile_of(block, p.de_tiles, p.de_splits, p.de_per_xcd, p.tiles_n, split, tm, tn)) return;
-    terms_de_tile<T>(p, split, tm, tn, smem);
-  }
-}
-__global__ __launch_bounds__(kProdThreads, 1) void terms_products_kernel(ProductParams given) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  if (__builtin_amdgcn_readfirstlane(*given.wide) == 0) {
-    ProductParams p = given;
-    p.terms = kHalvesTerms;
-    p.ldz = kHalvesParts * static_cast<int64_t>(p.dz_part);
-    p.stride_cv = p.stride_e = kHalvesParts * static_cast<int64_t>(p.part_d);
-    terms_products_item<F16>(p, smem);
-  } else {
-    terms_products_item<BF16>(given, smem);
+    terms_de_tile(p, split, tm, tn, smem);
   }
 }
 
@@ -506,26 +486,20 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* slots, int 
 constexpr int kColsumClasses = 64, kColsumLanes = 128;
 template <typename T>
 __global__ __launch_bounds__(1024) void dz_colsum_kernel(uint16_t* dz, int64_t ldz, int parts, int64_t b, int n_cls, int blocks, int ranges,
-                                                         float* d_bias, const int* wide, const DzScale* dz_scale) {
+                                                         float* d_bias) {
   __shared__ float s_sum[1024 / 64][kColsumClasses];
   const int cl = threadIdx.x % 8, rl = threadIdx.x / 8;
   const int block = blockIdx.x % blocks, range = blockIdx.x / blocks;
   const int64_t begin = b * range / ranges, end = b * (range + 1) / ranges;
   const int cls = block * kColsumClasses + cl * 8;
   float sum[8] = {};
-  const bool halves = wide != nullptr && *wide == 0;
-  if (halves) parts = kHalvesParts;
   if (cls < n_cls) {  // (a row of dz goes on in whole 16-byte pieces)
     auto value = [&](int64_t i, float (&x)[8]) {
       for (int part = parts - 1; part >= 0; --part) {
         const uint4 v = *reinterpret_cast<const uint4*>(dz + (i * parts + part) * ldz + cls);
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const uint16_t bits = static_cast<uint16_t>(w[k >> 1] >> (16 * (k & 1)));
-          if (halves) x[k] = fmaf(x[k], part == 0 ? 1.0f / kLowerHalf : 1.0f, Elem<F16>::to_float(bits));
-          else x[k] += Elem<T>::to_float(bits);
-        }
+        for (int k = 0; k < 8; ++k) x[k] += Elem<T>::to_float(static_cast<uint16_t>(w[k >> 1] >> (16 * (k & 1))));
       }
     };
     // (the last time a row that does not exist is the last one again, and not added)
@@ -561,28 +535,26 @@ __global__ __launch_bounds__(1024) void dz_colsum_kernel(uint16_t* dz, int64_t l
     for (int w = 0; w < 1024 / 64; ++w) all += s_sum[w][threadIdx.x];
     const int c = block * kColsumClasses + threadIdx.x;
     if (ranges == 1) {
-      if (c < n_cls) d_bias[c] += all * (halves ? dz_scale->unit : 1.0f);
+      if (c < n_cls) d_bias[c] += all;
     } else if ((c & ~7) < n_cls) {
       reinterpret_cast<float*>(dz + (begin * parts + ((c >> 2) & 1)) * ldz + (c & ~7))[c & 3] = all;
     }
   }
 }
 __global__ __launch_bounds__(256) void colsum_merge_kernel(const uint16_t* dz, int64_t ldz, int parts, int64_t b, int n_cls, int ranges,
-                                                           float* d_bias, const int* wide, const DzScale* dz_scale) {
+                                                           float* d_bias) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= n_cls) return;
-  const bool halves = wide != nullptr && *wide == 0;
-  if (halves) parts = kHalvesParts;
   float all = 0.0f;
 #pragma unroll 8
   for (int s = 0; s < ranges; ++s)
     all += reinterpret_cast<const float*>(dz + (b * s / ranges * parts + ((c >> 2) & 1)) * ldz + (c & ~7))[c & 3];
-  d_bias[c] += all * (halves ? dz_scale->unit : 1.0f);
+  d_bias[c] += all;
 }
 
 // The last reader of dz: its contents are gone afterwards.
-int dz_colsum_launch(uint16_t* dz, int64_t ldz, int parts, int64_t b, int64_t n_cls, float* d_bias, int dtype, const int* wide,
-                     const DzScale* dz_scale, hipStream_t stream) {
+int dz_colsum_launch(uint16_t* dz, int64_t ldz, int parts, int64_t b, int64_t n_cls, float* d_bias, int dtype,
+                     hipStream_t stream) {
   const int blocks = static_cast<int>((n_cls + kColsumClasses - 1) / kColsumClasses);
   // two workgroups to a compute unit, and at least one row per row lane: never fewer than the two rows that the sums take
   int64_t ranges = 2 * compute_units() / blocks;
@@ -592,13 +564,13 @@ int dz_colsum_launch(uint16_t* dz, int64_t ldz, int parts, int64_t b, int64_t n_
   const dim3 grid(static_cast<unsigned>(blocks * ranges));
   if (dtype == CCE_DTYPE_BF16)
     hipLaunchKernelGGL(dz_colsum_kernel<BF16>, grid, dim3(1024), 0, stream, dz, ldz, parts, b, static_cast<int>(n_cls), blocks,
-                       static_cast<int>(ranges), d_bias, wide, dz_scale);
+                       static_cast<int>(ranges), d_bias);
   else
     hipLaunchKernelGGL(dz_colsum_kernel<F16>, grid, dim3(1024), 0, stream, dz, ldz, parts, b, static_cast<int>(n_cls), blocks,
-                       static_cast<int>(ranges), d_bias, wide, dz_scale);
+                       static_cast<int>(ranges), d_bias);
   if (ranges > 1)
     hipLaunchKernelGGL(colsum_merge_kernel, dim3(static_cast<unsigned>((n_cls + 255) / 256)), dim3(256), 0, stream, dz, ldz, parts, b,
-                       static_cast<int>(n_cls), static_cast<int>(ranges), d_bias, wide, dz_scale);
+                       static_cast<int>(n_cls), static_cast<int>(ranges), d_bias);
   return status_from_hip(hipGetLastError());
 }
 
@@ -902,12 +874,8 @@ int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t*
                           int64_t ld_e, const int32_t* valids, float* d_e, int64_t ld_de, bool de_by_number, bool de_init,
                           int64_t de_slot, int de_len, float* d_c, int64_t ld_dc, bool dc_add, int64_t dc_slot, int dc_len,
                           bool out_vec, int64_t b, int64_t b_pad, int64_t cls, int64_t cls_pad, int64_t d, int64_t part_d, int terms,
-                          int parts, const int* wide, const DzScale* dz_scale, float c_unit, float e_unit, hipStream_t stream) {
+                          int parts, hipStream_t stream) {
   ProductParams p = {};
-  p.wide = wide;
-  p.dz_scale = dz_scale;
-  p.c_unit = c_unit;
-  p.e_unit = e_unit;
   p.dz = dz_parts;
   p.ldz = parts * ldz;
   p.dz_part = static_cast<int>(ldz);
@@ -1104,7 +1072,7 @@ extern "C" int cce_backward_dense(const void* e, const void* c, const void* bias
         else CCE_LAUNCH_PRODUCT((dense_products_kernel<F16, false>), blocks);
       }
     }
-    if (bias_out != nullptr) return dz_colsum_launch(dz, ldz, 1, rows, cls, bias_out, dtype, nullptr, nullptr, stream);
+    if (bias_out != nullptr) return dz_colsum_launch(dz, ldz, 1, rows, cls, bias_out, dtype, stream);
     return status_from_hip(hipGetLastError());
   };
 #undef CCE_LAUNCH_PRODUCT

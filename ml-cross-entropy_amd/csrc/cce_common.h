@@ -609,18 +609,9 @@ struct DmaLogitTile {
 //   hi lo, lo hi, mid mid, hi mid, mid hi, hi hi          (two bits per term; the last three are the product of two parts)
 constexpr int kTermsAll = 6;
 constexpr unsigned kTermsFirst = 0x118u, kTermsSecond = 0x052u;
-// The parts are three (terms == 6) or two (3) of bf16, or two of fp16.  Two halves of 11 bits hold 22 - 23 of the 24 bits of a
-// value as long as its magnitude fits them, in half the products; cce_fp32.hip says when they are taken.
+// The parts are three (terms == 6) or two (3) of bf16.  Logits go by two halves of fp16 and the last three terms where those have
+// room for the values (cce_fp32.hip).
 constexpr int kHalvesTerms = 3, kHalvesParts = 2;
-// Gradients of logits span more powers of two than the operands: the lower half of one is stored kLowerHalf times larger, and
-// the term of their lower halves, lo hi, comes first: the sums so far are divided by it before hi lo and hi hi are added.
-constexpr float kLowerHalf = 2048.0f;
-constexpr unsigned kHalvesFirst = 0x01u, kHalvesSecond = 0x04u;
-// What the upstream gradients of a call say about the gradients of its logits.
-struct DzScale {
-  float scale, unit;  // |dz| scale < 2^15, a power of two; unit = 1 / scale
-  int out_of_range;   // no one scale serves all rows
-};
 __host__ __device__ __forceinline__ int term_part(unsigned table, int term) {
   return static_cast<int>((table >> (2 * term)) & 3u);
 }

@@ -29,8 +29,8 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
 // ---- fp32 operands as 16-bit parts (cce_fp32.hip) ---------------------------------------------------------------
 // A row of e_parts / c_parts holds its parts [hi | mid | lo] side by side, part_d (a multiple of 64) columns each;
 // ld_e / ld_c elements from row to row, a multiple of 8.  terms: 6 cross terms of three parts, or 3 of two.
-// Where the device finds *wide == 0 the rows are [hi | lo] of fp16 instead, packed, whose products are 1 / halves_scale times what
-// they stand for (a power of two).
+// Logits are formed from rows [hi | lo] of fp16 instead, packed, where the device finds *wide == 0: their products are 1 /
+// halves_scale times what they stand for (a power of two).  lse_terms_launch finds these halves in the place of the parts.
 
 // Spans per row block that lse_terms_launch makes of v classes: the float2 partials [spans][b] it writes.
 int lse_terms_splits(int64_t b, int64_t v);
@@ -38,17 +38,14 @@ int lse_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_pa
                      float2* partial, int64_t b, int64_t v, int64_t part_d, int terms, const int* wide, float halves_scale,
                      float softcap, hipStream_t stream);
 
-// *out: the scale of the gradients of logits that the upstream gradients of the b rows allow.
-int dz_scale_launch(const float* d_out, int d_out_is_scalar, const float* d_lse, const int32_t* valids, int64_t n_rows, int64_t b,
-                    float grad_scale, int64_t shift, DzScale* out, hipStream_t stream);
-
-// dz of v classes as parts [b_store][parts][ldz], bf16 or halves of dz_scale->scale dz like the operands; ldz = v rounded up to 64; columns past v and rows b .. b_store
+// dz of v classes as bf16 parts [b_store][parts][ldz], ldz = v rounded up to 64; columns past v and rows b .. b_store
 // (b rounded up to 64) are zeros.  valids: the rows of the batch that the (compact) rows of e_parts are.
-int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
+int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const uint16_t* e_halves,
+                    const uint16_t* c_halves, const int* wide, float halves_scale, const float* bias,
                     const float* lse, const float* d_out, int d_out_is_scalar, const float* d_lse,
                     const int32_t* valids, const int64_t* targets, uint16_t* dz_parts, int64_t ldz,
-                    int64_t n_rows, int64_t b, int64_t b_store, int64_t v, int64_t part_d, int terms, int parts, const int* wide,
-                    float halves_scale, const DzScale* dz_scale, float grad_scale, int64_t shift, int64_t target_offset, float softcap, hipStream_t stream);
+                    int64_t n_rows, int64_t b, int64_t b_store, int64_t v, int64_t part_d, int terms, int parts,
+                    float grad_scale, int64_t shift, int64_t target_offset, float softcap, hipStream_t stream);
 
 // Chunks of classes and cuts of the reductions of dE and dC for terms_products_launch.
 struct TermsPlan {
@@ -65,10 +62,9 @@ int terms_products_launch(const uint16_t* dz_parts, int64_t ldz, const uint16_t*
                           int64_t ld_e, const int32_t* valids, float* d_e, int64_t ld_de, bool de_by_number, bool de_init,
                           int64_t de_slot, int de_len, float* d_c, int64_t ld_dc, bool dc_add, int64_t dc_slot, int dc_len,
                           bool out_vec, int64_t b, int64_t b_pad, int64_t cls, int64_t cls_pad, int64_t d, int64_t part_d, int terms,
-                          int parts, const int* wide, const DzScale* dz_scale, float c_unit, float e_unit, hipStream_t stream);
-// d_bias[class] += column sums of dz [b][parts][ldz] in dtype, or of its halves; dz is used up
-int dz_colsum_launch(uint16_t* dz, int64_t ldz, int parts, int64_t b, int64_t n_cls, float* d_bias, int dtype, const int* wide,
-                     const DzScale* dz_scale, hipStream_t stream);
+                          int parts, hipStream_t stream);
+// d_bias[class] += column sums of dz [b][parts][ldz] in dtype; dz is used up
+int dz_colsum_launch(uint16_t* dz, int64_t ldz, int parts, int64_t b, int64_t n_cls, float* d_bias, int dtype, hipStream_t stream);
 // out[row(i)][0 .. d) (+)= sum over the slots [count][rows][ld_slot]
 int split_sum_launch(const float* slots, int count, int64_t rows, int64_t d, int64_t ld_slot, const int32_t* ids, float* out,
                      int64_t ld, bool add, bool out_vec, hipStream_t stream);

@@ -38,10 +38,11 @@ struct DzParams {
   const float* bias32;
   int terms, parts;
   int64_t b_store;
-  // *wide == 0: halves, two to a row and packed; the logit is halves_scale times their product, and dz leaves times dz_scale->scale
+  // *wide == 0: the logits from halves, two to a row and packed, whose product is 1 / halves_scale times the logit
   const int* wide;
+  const uint16_t* e_halves;
+  const uint16_t* c_halves;
   float halves_scale;
-  const DzScale* dz_scale;
   float softcap;
 };
 
@@ -318,18 +319,15 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
   const int64_t t0 = static_cast<int64_t>(rb) * ROWS;
 
   typename Fast::Source src;
-  src.e_base = reinterpret_cast<const unsigned char*>(p.e);
+  src.e_base = reinterpret_cast<const unsigned char*>(HALVES ? p.e_halves : p.e);
   src.chunk_bytes = 2u * static_cast<unsigned>(Fast::chunk_elems(wave, lane));
   src.row_in_block = static_cast<unsigned>(lane >> 3);
   const int64_t stride_e = HALVES ? kHalvesParts * p.d : p.stride_e, stride_cv = HALVES ? kHalvesParts * p.d : p.stride_cv;
   src.c_stride_bytes = static_cast<unsigned>(stride_cv * 2);
   src.terms = !PARTS ? 1 : HALVES ? kHalvesTerms : p.terms;
-  int parts = HALVES ? kHalvesParts : p.parts;
-  if (HALVES) asm volatile("" : "+s"(parts));  // (as a constant it has the compiler unroll itself out of scalar registers)
   // a sum in an accumulator times `unit` is a logit (a power of two); without an addend it rides in the first factor
   const float unit = HALVES ? p.halves_scale : 1.0f;
   const float in_scale = GENERAL ? p.sc.in_scale : p.sc.in_scale * unit;
-  const float dz_scale = HALVES ? p.dz_scale->scale : 1.0f;
   if constexpr (TAIL) Fast::set_tail(src, static_cast<int>(p.d));
 #pragma unroll
   for (int q = Fast::NQC; q < Fast::NQ; ++q) {
@@ -341,7 +339,7 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
   auto set_class_tile = [&](int vt) {
     const int64_t v0 = static_cast<int64_t>(vt) * kDzTile;
     const int left = static_cast<int>(min(p.v - v0, static_cast<int64_t>(kDzTile)));
-    Fast::set_class_tile(src, reinterpret_cast<const unsigned char*>(p.c) + v0 * stride_cv * 2, left, wave);
+    Fast::set_class_tile(src, reinterpret_cast<const unsigned char*>(HALVES ? p.c_halves : p.c) + v0 * stride_cv * 2, left, wave);
   };
 
   unsigned char* stage = s_stage + wave * kDz16StageBytes;
@@ -439,7 +437,7 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
             unsigned char* dst = stage + r16 * kDzStageRow + ((((col >> 4) ^ sw) << 4) | (col & 15));
             if (PARTS) {
 #pragma unroll
-              for (int r = 0; r < 4; ++r) rest[vj][r] = dzv[r] * dz_scale;
+              for (int r = 0; r < 4; ++r) rest[vj][r] = dzv[r];
             } else if (OUT32) {
               *reinterpret_cast<float4*>(dst) = make_float4(dzv[0], dzv[1], dzv[2], dzv[3]);
             } else {
@@ -468,7 +466,7 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
             const int64_t gcol = static_cast<int64_t>(cls0) + vh * (16 * kViPer) + pc * kPieceElems;
             if constexpr (PARTS) {
               if (gi < p.b_store && gcol < p.ldz)
-                *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.dz) + (gi * parts + part) * p.ldz + gcol) = val;
+                *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.dz) + (gi * p.parts + part) * p.ldz + gcol) = val;
             } else if (gi < p.b) {
               unsigned char* dst = static_cast<unsigned char*>(p.dz) + (gi * p.ldz + gcol) * kEs;
               if (!GENERAL || gcol + kPieceElems <= p.v || (p.pad_store && gcol + kPieceElems <= p.ldz)) {
@@ -489,24 +487,19 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // reads done before the next block is staged
         };
         if constexpr (PARTS) {
-          // x = hi + mid + lo, each the bf16 nearest to what the ones before it leave, or hi + lo / kLowerHalf in fp16; one
-          // staged block per part
+          // x = hi + mid + lo, each the bf16 nearest to what the ones before it leave; one staged block per part
 #pragma unroll
           for (int part = 0; part < 3; ++part) {
-            if (part >= parts) break;
+            if (part >= p.parts) break;
 #pragma unroll
             for (int vj = 0; vj < kViPer; ++vj) {
               uint2 pk;
-              pk.x = Elem<T>::pack2(rest[vj][0], rest[vj][1]);
-              pk.y = Elem<T>::pack2(rest[vj][2], rest[vj][3]);
-              rest[vj][0] -= Elem<T>::to_float(static_cast<uint16_t>(pk.x));
-              rest[vj][1] -= Elem<T>::to_float(static_cast<uint16_t>(pk.x >> 16));
-              rest[vj][2] -= Elem<T>::to_float(static_cast<uint16_t>(pk.y));
-              rest[vj][3] -= Elem<T>::to_float(static_cast<uint16_t>(pk.y >> 16));
-              if (HALVES) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) rest[vj][r] *= kLowerHalf;
-              }
+              pk.x = Elem<BF16>::pack2(rest[vj][0], rest[vj][1]);
+              pk.y = Elem<BF16>::pack2(rest[vj][2], rest[vj][3]);
+              rest[vj][0] -= Elem<BF16>::to_float(static_cast<uint16_t>(pk.x));
+              rest[vj][1] -= Elem<BF16>::to_float(static_cast<uint16_t>(pk.x >> 16));
+              rest[vj][2] -= Elem<BF16>::to_float(static_cast<uint16_t>(pk.y));
+              rest[vj][3] -= Elem<BF16>::to_float(static_cast<uint16_t>(pk.y >> 16));
               const int col = (vj * 16 + 4 * kq) * 2;
               *reinterpret_cast<uint2*>(stage + r16 * kDzStageRow + ((((col >> 4) ^ sw) << 4) | (col & 15))) = pk;
             }
@@ -527,61 +520,11 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz16_kernel(DzParams p) {
   dense_dz16_item<T, GENERAL, OUT, TAIL, ROWS>(p);
 }
 
-// Operands in parts, of the kind that the device found them to need.
+// Operands in parts: logits from halves of fp16 where the device found room for the values in them.
 template <bool GENERAL>
 __global__ __launch_bounds__(kDzThreads, 1) void dz_terms_kernel(DzParams p) {
   if (*p.wide == 0) dense_dz16_item<F16, GENERAL, kDzParts>(p);
   else dense_dz16_item<BF16, GENERAL, kDzParts>(p);
-}
-
-// |dz| <= |g| + |h| of its row.  Halves of fp16 under one scale hold 20 bits and more of a gradient down to 2^-31 of the largest
-// that there can be; rows whose bounds lie more than 2^16 apart ask for the bf16 parts.  (Bounds that are no numbers ask for nothing.)
-__global__ __launch_bounds__(1024) void dz_scale_kernel(const float* d_out, int d_out_is_scalar, const float* d_lse, const int32_t* valids,
-                                                        int64_t n_rows, int64_t b, float grad_scale, int64_t shift, DzScale* out) {
-  float most = 0.0f, least = INFINITY;
-  const bool uniform = d_out_is_scalar && d_lse == nullptr;  // one row stands for all of them, and no position is read
-  const int64_t n = uniform ? 1 : b;
-  for (int64_t i = threadIdx.x; i < n; i += 1024) {
-    const int64_t at = (valids != nullptr ? static_cast<int64_t>(valids[i]) : i) + shift;
-    if (!uniform && at >= n_rows) continue;
-    float w = fabsf(grad_scale * d_out[d_out_is_scalar ? 0 : at]);
-    if (d_lse != nullptr) w += fabsf(d_lse[at]);
-    if (!(w > 0.0f && w < INFINITY)) continue;
-    most = fmaxf(most, w);
-    least = fminf(least, w);
-  }
-  __shared__ float s_most[16], s_least[16];
-  most = wave_max(most);
-  least = wave_min(least);
-  if ((threadIdx.x & 63) == 0) {
-    s_most[threadIdx.x >> 6] = most;
-    s_least[threadIdx.x >> 6] = least;
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int w = 1; w < 16; ++w) {
-    most = fmaxf(most, s_most[w]);
-    least = fminf(least, s_least[w]);
-  }
-  DzScale r = {1.0f, 1.0f, 0};
-  if (most > 0.0f) {
-    int exponent;
-    frexpf(most, &exponent);  // most < 2^exponent
-    if (exponent < -90 || exponent > 90 || least < most * 0x1p-16f) {
-      r.out_of_range = 1;
-    } else {
-      r.scale = ldexpf(1.0f, 15 - exponent);
-      r.unit = ldexpf(1.0f, exponent - 15);
-    }
-  }
-  *out = r;
-}
-
-int dz_scale_launch(const float* d_out, int d_out_is_scalar, const float* d_lse, const int32_t* valids, int64_t n_rows, int64_t b,
-                    float grad_scale, int64_t shift, DzScale* out, hipStream_t stream) {
-  hipLaunchKernelGGL(dz_scale_kernel, dim3(1), dim3(1024), 0, stream, d_out, d_out_is_scalar, d_lse, valids, n_rows, b, grad_scale, shift,
-                     out);
-  return status_from_hip(hipGetLastError());
 }
 
 int dense_dz_launch(const void* e, const void* c, const void* bias,
@@ -696,17 +639,18 @@ int dense_dz_launch(const void* e, const void* c, const void* bias,
 }
 
 // ---- dz of one chunk of classes with operands and result in bf16 parts (cce_fp32.hip) --------------------------
-int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const float* bias,
+int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_parts, int64_t ld_c, const uint16_t* e_halves,
+                    const uint16_t* c_halves, const int* wide, float halves_scale, const float* bias,
                     const float* lse, const float* d_out, int d_out_is_scalar, const float* d_lse,
                     const int32_t* valids, const int64_t* targets, uint16_t* dz_parts, int64_t ldz,
-                    int64_t n_rows, int64_t b, int64_t b_store, int64_t v, int64_t part_d, int terms, int parts, const int* wide,
-                    float halves_scale, const DzScale* dz_scale, float grad_scale, int64_t shift, int64_t target_offset, float softcap,
-                    hipStream_t stream) {
+                    int64_t n_rows, int64_t b, int64_t b_store, int64_t v, int64_t part_d, int terms, int parts,
+                    float grad_scale, int64_t shift, int64_t target_offset, float softcap, hipStream_t stream) {
   DzParams p = {};
   p.wide = wide;
+  p.e_halves = e_halves;
+  p.c_halves = c_halves;
   p.halves_scale = halves_scale;
   p.softcap = softcap;
-  p.dz_scale = dz_scale;
   p.e = e_parts;
   p.c = c_parts;
   p.bias32 = bias;

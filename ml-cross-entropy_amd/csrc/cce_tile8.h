@@ -35,10 +35,9 @@
 //
 // TERMS: the operands are fp32 values in 16-bit parts, a_part / b_part bytes from part to part, and the reduction runs over the
 // cross terms of the parts one after the other (kTermsFirst / kTermsSecond of cce_common.h: A is the first operand), whole
-// stages only.  With T = F16 they are halves (kHalvesFirst / kHalvesSecond), the lower one of A kLowerHalf times larger.
+// stages only.
 #pragma once
 
-#include <type_traits>
 #include <utility>
 
 #include "cce_common.h"
@@ -59,8 +58,6 @@ struct Tile8 {
   static constexpr int B_BASE = 2 * OP_BYTES;     // A stage 0, A stage 1, B stage 0, B stage 1
   static constexpr int LDS_BYTES = 4 * OP_BYTES;
   static constexpr int NQ = 4;                    // loads per wave, stage and operand
-  static constexpr bool HALVES = TERMS && std::is_same<T, F16>::value;
-  static constexpr unsigned kFirst = HALVES ? kHalvesFirst : kTermsFirst, kSecond = HALVES ? kHalvesSecond : kTermsSecond;
   using vec8 = typename Elem<T>::vec8;
 
   // ---- what a lane fetches ---------------------------------------------------------------------------
@@ -131,9 +128,9 @@ struct Tile8 {
   static __device__ __forceinline__ Pos first_pos(const Source& s) {
     Pos p = {s.partial ? s.k_total / BK * BK : 0, 0, 0, 0};
     if constexpr (TERMS) {
-      p.term = HALVES ? 0 : kTermsAll - s.terms;
-      p.a = term_part(kFirst, p.term) * s.a_part;
-      p.b = term_part(kSecond, p.term) * s.b_part;
+      p.term = kTermsAll - s.terms;
+      p.a = term_part(kTermsFirst, p.term) * s.a_part;
+      p.b = term_part(kTermsSecond, p.term) * s.b_part;
     }
     return p;
   }
@@ -144,8 +141,8 @@ struct Tile8 {
       if (p.k == s.k_total) {
         p.k = 0;
         ++p.term;
-        p.a = term_part(kFirst, p.term) * s.a_part;
-        p.b = term_part(kSecond, p.term) * s.b_part;
+        p.a = term_part(kTermsFirst, p.term) * s.a_part;
+        p.b = term_part(kTermsSecond, p.term) * s.b_part;
       }
     } else {
       p.k = (t - s.partial) * BK;
@@ -340,27 +337,15 @@ struct Tile8 {
       if (kReadsA == 2) read_a(i, 1, a, lds, 0, 0, g);
     }
 
-    auto end_of_lower = [&](int st) {  // the stages before `st` were those of the first term
-      if constexpr (HALVES) {
-        if (st * BK == s.k_total) {
-#pragma unroll
-          for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; ++j) acc[i][j] *= 1.0f / kLowerHalf;
-        }
-      }
-    };
     int cur = 0;
 #pragma unroll 1
     for (int st = 0; st + 2 < nk; ++st) {
-      end_of_lower(st);
       advance(at, s, st + 2);
       step<true, false, false, true>(acc, a, b0, b1, lds, cur, 1, s, at, 0, ids, at.k, g);
       step<true, true, true, false>(acc, a, b1, b0, lds, OP_BYTES - cur, 0, s, at, cur, ids, 0, g);
       cur = OP_BYTES - cur;
     }
     if (nk > 1) {
-      end_of_lower(nk - 2);
       step<true, false, false, false>(acc, a, b0, b1, lds, cur, 1, s, at, 0, ids, 0, g);
       step<true, false, true, false>(acc, a, b1, b0, lds, OP_BYTES - cur, 0, s, at, 0, ids, 0, g);
       cur = OP_BYTES - cur;

@@ -1,20 +1,20 @@
 """fp32 inputs on matrix cores that multiply 16-bit numbers.
 
 gfx950 has no fast fp32 matrix path (the reference leans on Triton's tf32x3 / ieee dot for fp32 inputs,
-cce_lse_forward.py:81, constants via tl_utils).  The library splits every fp32 value into two halves of fp16
-(22 - 23 bits) and takes a product as hi*hi + hi*lo + lo*hi, in one reduction of its 16-bit kernels with fp32
-accumulators.  Where a value of E is past 255.5, one of C past 15.9, or the upstream gradients of rows lie more than
-2^16 apart, the device goes by three bfloat16 parts instead, x = hi + mid + lo (8 + 8 + 8 bits), and six cross terms
+cce_lse_forward.py:81, constants via tl_utils).  For the products of the gradients the library splits every fp32 value
+into three bfloat16 parts, x = hi + mid + lo (8 + 8 + 8 significant bits), and takes a product as its six leading cross terms
 
     hi*hi + hi*mid + mid*hi + mid*mid + hi*lo + lo*hi          (what is left is below 2^-24 relative)
 
-``cce_fp32_forward`` and ``cce_fp32_backward`` run the whole of either pass in one call.  The gradient filter threshold
-of fp32 is far below anything a soft-max produces, so the backward is the unfiltered one.
+in one reduction of its 16-bit kernels with fp32 accumulators.  The logits, in either pass, go by two halves of fp16 (22 - 23
+bits) and hi*hi + hi*lo + lo*hi, unless a value of E is past 255.5 or one of C past 15.9: then by the same parts and terms as the
+gradients, which the device decides.  ``cce_fp32_forward`` and ``cce_fp32_backward`` run the whole of either pass in one call.  The
+gradient filter threshold of fp32 is far below anything a soft-max produces, so the backward is the unfiltered one.
 
-``torch.set_float32_matmul_precision``: with "high" or "medium" the caller has asked for fast fp32 products (the
-reference then lets Triton use tf32, 10 mantissa bits, cce_lse_forward.py:129-131), and where bf16 parts are taken
-they are two, and three terms hi*hi + hi*mid + mid*hi (16 bits).  dBias is no product: it is a sum of fp32 values
-either way.
+``torch.set_float32_matmul_precision``: "highest" (the default) takes the terms above; with "high" or "medium" the caller has asked
+for fast fp32 products (the reference then lets Triton use tf32, 10 mantissa bits, cce_lse_forward.py:129-131), and products of
+bf16 parts are formed from two of them and three terms, hi*hi + hi*mid + mid*hi (16 bits), half the work.  dBias is no product: it is a
+sum of fp32 values either way.
 """
 
 from typing import Optional, Tuple

@@ -212,6 +212,74 @@ def test_fp32_backward_of_one_row_whose_label_is_past_the_end(scalar, with_dlse)
     assert (de == 0).all() and (dc == 0).all() and (db == 0).all()
 
 
+def _fp32_gradients(e, c, t, b):
+    """Gradients of linear_cross_entropy under uneven weights, and the same in fp64: (dE, dC, dBias), (dE, dC, dBias)."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    N = e.size(0)
+    w = torch.rand((N,), generator=torch.Generator(device="cuda").manual_seed(9), device="cuda") + 0.5
+    for x in (e, c, b):
+        x.requires_grad_(True)
+    linear_cross_entropy(e, c, t, bias=b, reduction="none").backward(w)
+    with torch.no_grad():
+        x = e.double() @ c.double().T + b.double()
+        dz = torch.softmax(x, dim=1)
+        dz[torch.arange(N, device="cuda"), t] -= 1.0
+        dz *= w.double()[:, None]
+        return (e.grad, c.grad, b.grad), (dz @ c.double(), dz.T @ e.double(), dz.sum(0))
+
+
+@pytest.mark.parametrize("size", [1e-4, 1e-6, 1e-8, 1e-12])
+@pytest.mark.parametrize("which", ["e", "c", "columns of e", "columns of c"])
+@pytest.mark.parametrize("shape", [(300, 3000, 200), (20, 700, 64)])
+def test_fp32_gradients_of_small_operands(which, size, shape):
+    """dC is proportional to E and dE to C: an operand, or a feature, that is small everywhere has gradients as exact, for their own
+    size, as any other."""
+    N, V, D = shape
+    e, c, t, b, _, _, _, _ = _fp32_case(N, V, D, 1.0, 11, bias=True)
+    small = e if which.endswith("e") else c
+    if which.startswith("columns"):
+        small[:, 3:9] *= size
+    else:
+        small *= size
+    got, want = _fp32_gradients(e, c, t, b)
+    for x, exact in zip(got[:2], want[:2]):
+        assert torch.isfinite(x).all()
+        # per column: fp32 sums of at most 3000 products (sqrt(3000) 2^-24 if all roundings met the largest sum), and what dz inherits
+        # from logits and log-sum-exps of up to 16 rounded to fp32, 2^-20
+        err, norm = (x.double() - exact).norm(dim=0), exact.norm(dim=0)
+        assert (err <= 4e-6 * norm).all(), (err / norm).max().item()
+
+
+def test_fp32_gradients_keep_all_bits_of_their_operands():
+    """Few rows and a head that has not learnt: a row of dC is one row of E times a dz of about -1, a value next to one product."""
+    for seed in range(4):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        e, c = torch.randn((16, 64), generator=g, device="cuda"), torch.randn((2000, 64), generator=g, device="cuda") * 0.02
+        t = torch.randint(0, 2000, (16,), generator=g, device="cuda")
+        got, want = _fp32_gradients(e, c, t, torch.zeros((2000,), device="cuda"))
+        # two roundings to 24 bits, of dz and of the result, each 2^-24 / sqrt(3) at most as a root mean square, and what dz inherits
+        assert (got[1].double() - want[1]).norm() <= 2.0**-23.5 * want[1].norm()
+
+
+@pytest.mark.parametrize("gap", [10.0, 25.0, 40.0, 70.0])
+@pytest.mark.parametrize("rows", [5, 300])
+def test_fp32_gradients_of_improbable_classes(gap, rows):
+    """Classes that no row expects: their rows of dC and their dBias are small, and as exact for their own size as their probabilities."""
+    V, D = 3000, 200
+    e, c, t, b, _, _, _, _ = _fp32_case(rows, V, D, 1.0, 12, bias=True)
+    b[1000:2000] -= gap
+    t %= 1000
+    got, want = _fp32_gradients(e, c, t, b)
+    # a probability e^-x inherits the roundings of its logit, of x and of x log2(e), half a unit of 2^-23 of gap + 16 each; sums of rows
+    rel = 4 * 2.0**-24 * (gap + 16.0)
+    dc, want_dc = got[1].double()[1000:2000], want[1][1000:2000]
+    err, norm = (dc - want_dc).norm(dim=1), want_dc.norm(dim=1)
+    assert (norm > 0).all() and (err <= rel * norm).all(), (err / norm).max().item()
+    db, want_db = got[2].double()[1000:2000], want[2][1000:2000]
+    assert ((db - want_db).abs() <= rel * want_db.abs()).all()
+
+
 @pytest.mark.parametrize("where", ["inside", "e", "c", "late c", "upstream", "nan"])
 @pytest.mark.parametrize("bias", [False, True])
 def test_fp32_values_without_room_in_halves_go_by_parts(where, bias):
