@@ -9,6 +9,7 @@
 // statistics a register-local reduction.
 #pragma once
 
+#include <type_traits>
 #include <atomic>
 #include <utility>
 
@@ -612,6 +613,9 @@ constexpr unsigned kTermsFirst = 0x118u, kTermsSecond = 0x052u;
 // The parts are three (terms == 6) or two (3) of bf16.  Logits go by two halves of fp16 and the last three terms where those have
 // room for the values (cce_fp32.hip).
 constexpr int kHalvesTerms = 3, kHalvesParts = 2;
+// The lower half is stored kLowerHalf times larger, in the range of the upper one; the two terms with a lower half in them come first, and
+// their sum is divided by it before hi hi is added.
+constexpr float kLowerHalf = 2048.0f;
 __host__ __device__ __forceinline__ int term_part(unsigned table, int term) {
   return static_cast<int>((table >> (2 * term)) & 3u);
 }
@@ -631,6 +635,7 @@ struct DmaLogitTile16 {
   static constexpr int STAGE_BYTES = FEW ? (TILE_V + TILE_T / 2) * kDmaRowBytes : Base::STAGE_BYTES;
   static constexpr int LDS_BYTES = RING * STAGE_BYTES;
   static constexpr bool SPREAD = WV == 4;  // (blocks of 192 rows)
+  static constexpr bool HALVES = TERMS && std::is_same<T, F16>::value;
   using vec8 = typename Elem<T>::vec8;
 
   static __device__ __forceinline__ int wv_of(int wave) { return FEW ? wave % NWV : wave / NWT; }
@@ -913,10 +918,21 @@ struct DmaLogitTile16 {
                                   wave);
       cur = nxt;
     }
+    auto end_of_lower = [&](int s) {  // the stages before `s` were those of the terms with a lower half
+      if constexpr (HALVES) {
+        if (s == (kHalvesTerms - 1) * (D / kDmaBK)) {
+#pragma unroll
+          for (int vi = 0; vi < WV; ++vi)
+#pragma unroll
+            for (int ti = 0; ti < WT; ++ti) acc[vi][ti] *= 1.0f / kLowerHalf;
+        }
+      }
+    };
     constexpr Loads kFirst = SPREAD ? kTokenLoads : kNoLoads, kSecond = SPREAD ? kClassLoads : kAllLoads;
 #pragma unroll 1
     for (int s = 1; s < nk - 1; ++s) {
       const int nxt = next_stage(cur);
+      end_of_lower(s);
       ahead(s);
       step<true, kFirst, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, w.off_c, w.off_e, lds_base, cur, wave);
       if (s == nk - RING) next_tile();
@@ -926,6 +942,7 @@ struct DmaLogitTile16 {
     }
     // the last stage: its second step reads nothing (the next tile's first fragments would sit in registers
     // through the epilogue) and fetches the second stage of the next tile
+    end_of_lower(nk - 1);
     ahead(nk - 1);
     step<true, kFirst, false>(acc, a, b0, b1, c_row + cur + chunk1, e_row + cur + chunk1, src, w.off_c, w.off_e, lds_base, cur, wave);
     step<false, kSecond, true>(acc, a, b1, b0, c_row, e_row, src, w.off_c, w.off_e, lds_base, cur, wave);

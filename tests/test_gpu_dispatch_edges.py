@@ -251,6 +251,23 @@ def test_fp32_gradients_of_small_operands(which, size, shape):
         assert (err <= 4e-6 * norm).all(), (err / norm).max().item()
 
 
+@pytest.mark.parametrize("width", [64, 128, 65536])
+def test_fp32_losses_of_small_logits_from_large_factors(width):
+    """E ~ 1e-6 and C ~ 5: what is lost of a small operand meets a large one, and the losses, log 2 and a little, show it."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    N, V = 500, 2
+    g = torch.Generator(device="cuda").manual_seed(1)
+    e = torch.randn((N, width), generator=g, device="cuda") * 1e-6
+    c = torch.randn((V, width), generator=g, device="cuda").clamp_(-3, 3) * 5.0
+    t = torch.randint(0, V, (N,), generator=g, device="cuda")
+    loss = linear_cross_entropy(e, c, t, reduction="none")
+    x = e.double() @ c.double().T
+    want = torch.logsumexp(x, 1) - x[torch.arange(N, device="cuda"), t]
+    # three roundings of half a unit of 2^-24 at most: of the loss (0.69), of the logarithm in base 2 and of the sum of two exponentials
+    assert (loss.double() - want).square().mean().sqrt() <= 3**0.5 * 2.0**-25
+
+
 def test_fp32_gradients_keep_all_bits_of_their_operands():
     """Few rows and a head that has not learnt: a row of dC is one row of E times a dz of about -1, a value next to one product."""
     for seed in range(4):
