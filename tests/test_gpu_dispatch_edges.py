@@ -297,19 +297,19 @@ def test_fp32_gradients_of_improbable_classes(gap, rows):
     assert ((db - want_db).abs() <= rel * want_db.abs()).all()
 
 
-@pytest.mark.parametrize("where", ["inside", "e", "c", "late c", "upstream", "nan"])
+@pytest.mark.parametrize("where", ["inside", "e", "e, two chunks", "c", "early c", "late c", "upstream", "nan"])
 @pytest.mark.parametrize("bias", [False, True])
 def test_fp32_values_without_room_in_halves_go_by_parts(where, bias):
-    """The largest values that halves of fp16 are used for and the smallest past them, in E, in C, in the second chunk of C alone;
+    """The largest values that halves of fp16 are used for and the smallest past them, in E, in C, in the first or the second of two chunks of C;
     upstream gradients further apart than one scale serves; one row of NaN.  Against fp64, rows of gradients of their own size."""
     from cut_cross_entropy import linear_cross_entropy
 
     dev = torch.device("cuda:0")
-    N, V, D = (70, 45000, 2048) if where == "late c" else (300, 700, 200)
+    N, V, D = (70, 45000, 2048) if where in ("e, two chunks", "early c", "late c") else (300, 700, 200)
     e, c, t, b, w, _, _, _ = _fp32_case(N, V, D, 1.0, 4, bias=bias)
     inside = where in ("inside", "upstream", "nan")
-    e[5, 3], c[:, 3] = (255.5 if where != "e" else 255.6), c[:, 3] * 1e-2
-    c[V - 1, 2], e[:, 2] = (15.96875 if inside or where == "e" else 16.0), e[:, 2] * 1e-2
+    e[5, 3], c[:, 3] = (255.6 if where.startswith("e,") or where == "e" else 255.5), c[:, 3] * 1e-2
+    c[0 if where == "early c" else V - 1, 2], e[:, 2] = (16.0 if where.endswith("c") else 15.96875), e[:, 2] * 1e-2
     if where == "upstream":
         w[7] = 1e-6
     if where == "nan":
