@@ -29,6 +29,8 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+// What there and back again, kLn2 times kLog2e, falls short of 1.
+constexpr float kLog2Slack = static_cast<float>(1.0 - static_cast<double>(kLn2) * static_cast<double>(kLog2e));
 constexpr int kBK = 64;          // reduction elements per LDS stage
 constexpr int kRowBytes = 128;   // kBK * sizeof(16-bit element)
 

@@ -43,7 +43,6 @@ struct DzParams {
   const uint16_t* e_halves;
   const uint16_t* c_halves;
   float halves_scale;
-  float softcap;
 };
 
 // How dz leaves: in the input type, as fp32, or as an fp32 value in two or three bf16 parts
@@ -265,12 +264,25 @@ __global__ __launch_bounds__(kDzThreads, 1) void dense_dz_kernel(DzParams p) {
 constexpr int kDz16WV = 8, kDz16WT = 4;
 constexpr int kDz16StageBytes = 16 * kDzStageRow;  // 16 rows of 128 bytes per wave
 
-// lse: in log2 units; with operands in parts as it is, since the difference of natural logarithms is exact where p is near 1 (the
-// gradients of large logits, [300, 5120] x [30000, 5120], come 3 % nearer to 64 bits)
 struct DzRow {
-  float lse, g, gh;
+  float lse2, g, gh;
   int tgt;
 };
+
+// 2^(x2 - lse2) for gradients in fp32.  The difference as a whole number and a fraction of up to a half: rounded as one number, of 16 or so, it
+// is off by 2^-21, and the result by as much.  x2, and lse2 = log-sum-exp times kLog2e, are rounded as they were in the forward, also by its
+// soft-capping factor: of a row that one logit makes up it is that logit again, and the difference 0 (as a difference of natural
+// logarithms it was 5e-7 there, and one with a factor of its own 9e-8 of a soft-capped logit).  Where they are far apart, lse2 falls short
+// of the forward's by kLog2Slack of itself, which is of the difference.
+// Distance from 64 bits, 2-norm, as a difference rounded as one number / of natural logarithms / so: dE of [64, 1000] x [50003, 1000] with soft-cap
+// 30 2.57e-7 / 2.26e-7 / 2.09e-7, of [500, 2048] x [20000, 2048] 3.29e-7 / 3.1e-7 / 2.42e-7, of [400, 3072] x [3000, 3072] with targets of logits up
+// to 15 8.09e-7 / 7.75e-7 / 8.00e-7, and with soft-cap 30 1.49e-6 / 1.73e-6 / 1.48e-6.  Six instructions per logit: nothing to be seen in
+// the time of [2046, 3072] x [32064, 3072].
+__device__ __forceinline__ float exp2_difference(float x2, float lse2) {
+  const float n = fmaxf(rintf(x2 - lse2), -256.0f);
+  const float f = fmaf(n, kLog2Slack, x2 - (n + lse2));  // n + lse2: exact unless x2 is past lse2
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
+}
 
 // Who holds what of a tile of ROWS x 256: 2 x 4 waves of 128 classes x 64 rows, or 4 x 2 of 64 x 96.
 template <int ROWS>
@@ -328,6 +340,7 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
   // a sum in an accumulator times `unit` is a logit (a power of two); without an addend it rides in the first factor
   const float unit = HALVES ? p.halves_scale : 1.0f;
   const float in_scale = GENERAL ? p.sc.in_scale : p.sc.in_scale * unit;
+  const float log2e = GENERAL ? kLog2e : kLog2e * unit;
   if constexpr (TAIL) Fast::set_tail(src, static_cast<int>(p.d));
 #pragma unroll
   for (int q = Fast::NQC; q < Fast::NQ; ++q) {
@@ -353,7 +366,7 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
     DzRow r = {INFINITY, 0.0f, 0.0f, -1};
     if (i < p.b) {
       const int64_t row = p.valids ? static_cast<int64_t>(p.valids[i]) : i;
-      r.lse = PARTS ? p.lse[i] : p.lse[i] * kLog2e;
+      r.lse2 = p.lse[i] * kLog2e;
       const int64_t tpos = row + p.shift;
       if (tpos < p.n_rows) {
         const int64_t t = p.targets[tpos] - p.target_offset;
@@ -418,17 +431,16 @@ __device__ __forceinline__ void dense_dz16_item(const DzParams& p) {
                 dead = (add == -INFINITY);
                 x = dead ? 0.0f : fmaf(x, unit, add);
               }
-              float arg, damp = 1.0f;  // of p = 2^arg
+              float pr, damp = 1.0f;
               if (decltype(capped)::value) {
                 const float t = __builtin_amdgcn_exp2f(x * in_scale);
                 const float w = __builtin_amdgcn_rcpf(1.0f + t);
                 const float th = 1.0f - 2.0f * w;
-                arg = PARTS ? fmaf(p.softcap, th, -rr.lse) * kLog2e : p.sc.out_scale * th - rr.lse;
+                pr = PARTS ? exp2_difference(p.sc.out_scale * th, rr.lse2) : __builtin_amdgcn_exp2f(p.sc.out_scale * th - rr.lse2);
                 damp = 1.0f - th * th;
               } else {
-                arg = PARTS ? (GENERAL ? x - rr.lse : fmaf(x, unit, -rr.lse)) * kLog2e : x * kLog2e - rr.lse;
+                pr = PARTS ? exp2_difference(x * log2e, rr.lse2) : __builtin_amdgcn_exp2f(x * kLog2e - rr.lse2);
               }
-              const float pr = __builtin_amdgcn_exp2f(arg);
               float dz = pr * rr.gh - ((cls0 + cl == rr.tgt) ? rr.g : 0.0f);
               if (decltype(capped)::value) dz *= damp;
               dzv[r] = dead ? 0.0f : dz;
@@ -650,7 +662,6 @@ int dz_terms_launch(const uint16_t* e_parts, int64_t ld_e, const uint16_t* c_par
   p.e_halves = e_halves;
   p.c_halves = c_halves;
   p.halves_scale = halves_scale;
-  p.softcap = softcap;
   p.e = e_parts;
   p.c = c_parts;
   p.bias32 = bias;

@@ -251,6 +251,27 @@ def test_fp32_gradients_of_small_operands(which, size, shape):
         assert (err <= 4e-6 * norm).all(), (err / norm).max().item()
 
 
+@pytest.mark.parametrize("softcap", [7.0, 15.0, 30.0, None])
+def test_fp32_probability_of_the_only_class_is_one(softcap):
+    """One class: the log-sum-exp is its logit, and the backward finds it to be: a row that is sure of its label has no gradient."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    N, D = 8192, 64
+    top = softcap or 20.0
+    e = (torch.linspace(0.1, 1.5, N, device="cuda") * top / D).repeat(D, 1).T.contiguous().requires_grad_(True)
+    c = torch.ones((1, D), device="cuda")
+    linear_cross_entropy(e, c, torch.zeros((N,), dtype=torch.int64, device="cuda"), softcap=softcap, reduction="sum").backward()
+    x = e.detach().double().sum(1)
+    if softcap:
+        # either pass forms the soft-capped logit by a hardware exponential and a reciprocal, of one unit in the last place each, and by
+        # the same rounded factor; what is left has no sign in common but for those
+        th = torch.tanh(x / softcap)
+        off = e.grad.double()[:, 0] / (1.0 - th * th)  # p - 1
+        assert abs(off.mean()) <= 2.0**-24 * (softcap * th).mean()
+    else:
+        assert e.grad.double().square().mean().sqrt() <= 2.0**-23
+
+
 @pytest.mark.parametrize("width", [64, 128, 65536])
 def test_fp32_losses_of_small_logits_from_large_factors(width):
     """E ~ 1e-6 and C ~ 5: what is lost of a small operand meets a large one, and the losses, log 2 and a little, show it."""
