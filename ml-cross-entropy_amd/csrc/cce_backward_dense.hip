@@ -480,10 +480,20 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* slots, int 
 // added up in a fixed order, those of a wave by exchanges between its lanes, then the 16 waves in LDS.  Bound by reading dz.  Few
 // classes make few workgroups: the rows are then cut into ranges, each with a workgroup, which leaves its sums, as floats, in
 // the first two rows of its own range (no one reads dz any more, the workgroup itself has), and colsum_merge_kernel adds them up in
-// their order.  (Narrower columns of whole reductions, down to a 16-byte one, read as many times the lines: [54888] x 1088 in halves
-// 443 us / 75 + 20 so, [14264] x 4448 52 / 24 + 5, [4096] x 32000 47 / 44 + 5; and with a row at a time where fewer than four are left, and a tree of
-// barriers in LDS, [900] x 50257 30 / 25.)
+// their order.  (Narrower columns of whole reductions, down to a 16-byte one, with a tree of barriers in LDS, read as many times the lines.
+// They took / it takes, us, dz in bf16: [54888] x 1088 80 / 20 + 6, [14264] x 4448 52 / 23 + 4, [4096] x 32000 50 / 47, [900] x 50257 26 / 19; in three
+// parts: 253 / 34 + 10, 196 / 91 + 5, 123 / 96 + 5, 88 / 65, the first in two chunks of classes.)
 constexpr int kColsumClasses = 64, kColsumLanes = 128;
+// As a tree: a large entry among many small ones is rounded with every number that is added to it.  (The waves and the ranges one after the
+// other: classes that are the label of one of 8192 rows had their dBias off by 4.0e-7, root mean square, now 2.9e-8.)
+template <int N>
+__device__ __forceinline__ float pairwise_sum(float (&v)[N]) {
+#pragma unroll
+  for (int half = N / 2; half >= 1; half /= 2)
+#pragma unroll
+    for (int k = 0; k < half; ++k) v[k] += v[k + half];
+  return v[0];
+}
 template <typename T>
 __global__ __launch_bounds__(1024) void dz_colsum_kernel(uint16_t* dz, int64_t ldz, int parts, int64_t b, int n_cls, int blocks, int ranges,
                                                          float* d_bias) {
@@ -530,9 +540,10 @@ __global__ __launch_bounds__(1024) void dz_colsum_kernel(uint16_t* dz, int64_t l
   }
   __syncthreads();
   if (threadIdx.x < kColsumClasses) {
-    float all = 0.0f;
+    float wave_sum[1024 / 64];
 #pragma unroll
-    for (int w = 0; w < 1024 / 64; ++w) all += s_sum[w][threadIdx.x];
+    for (int w = 0; w < 1024 / 64; ++w) wave_sum[w] = s_sum[w][threadIdx.x];
+    const float all = pairwise_sum(wave_sum);
     const int c = block * kColsumClasses + threadIdx.x;
     if (ranges == 1) {
       if (c < n_cls) d_bias[c] += all;
@@ -545,11 +556,16 @@ __global__ __launch_bounds__(256) void colsum_merge_kernel(const uint16_t* dz, i
                                                            float* d_bias) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= n_cls) return;
-  float all = 0.0f;
-#pragma unroll 8
-  for (int s = 0; s < ranges; ++s)
-    all += reinterpret_cast<const float*>(dz + (b * s / ranges * parts + ((c >> 2) & 1)) * ldz + (c & ~7))[c & 3];
-  d_bias[c] += all;
+  float sums[8] = {};
+  for (int first = 0; first < ranges; first += 8) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t s = min(first + k, ranges - 1);
+      const float x = reinterpret_cast<const float*>(dz + (b * s / ranges * parts + ((c >> 2) & 1)) * ldz + (c & ~7))[c & 3];
+      sums[k] += first + k < ranges ? x : 0.0f;
+    }
+  }
+  d_bias[c] += pairwise_sum(sums);
 }
 
 // The last reader of dz: its contents are gone afterwards.

@@ -406,6 +406,26 @@ def test_bias_gradient_in_ranges_of_rows(shape, dtype):
     assert ((bias.grad.double() - dz.sum(0)).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("rows", [2048, 8192, 65536])
+def test_bias_gradient_of_one_large_entry_among_small_ones(rows):
+    """Classes that are the label of one row and improbable in all others: their dBias is rounded with every partial sum that meets the
+    large entry, so these are added as trees."""
+    from cut_cross_entropy import linear_cross_entropy
+
+    V, D = 64, 64
+    bias = torch.zeros((V,), device="cuda")
+    bias[0] = 17.0
+    bias.requires_grad_(True)
+    t = torch.zeros((rows,), dtype=torch.int64)
+    t[torch.randperm(rows, generator=torch.Generator().manual_seed(1))[: V - 1]] = torch.arange(1, V)
+    linear_cross_entropy(torch.zeros((rows, D), device="cuda"), torch.zeros((V, D), device="cuda"), t.cuda(), bias=bias,
+                         reduction="sum").backward()
+    want = rows * torch.softmax(bias.detach().double(), 0) - torch.bincount(t, minlength=V).cuda()
+    # at most 2^-25 each: the entry; rows of a lane, 3 exchanges, 4 levels of waves, and of up to 64 ranges 8 in a row and 3 levels; the result
+    per_lane = -(-rows // (64 * 512))
+    assert (bias.grad.double() - want)[1:].square().mean().sqrt() <= (17 + per_lane) ** 0.5 * 2.0**-25 / 3**0.5
+
+
 @pytest.mark.parametrize("shape", [(1, 16384), (1, 16385), (9, 7001), (40000, 2), (1, 32 * 8192), (1, 32 * 8192 + 1), (3, 200003)])
 @pytest.mark.parametrize("keep", [0.0, 0.4, 1.0])
 def test_valid_rows_of_several_workgroups_match_the_host(shape, keep):
