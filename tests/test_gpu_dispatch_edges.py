@@ -128,11 +128,36 @@ def test_fp32_passes_abi(shape, keep, extra, terms):
     """cce_fp32_forward / cce_fp32_backward against fp64: widths that are no multiple of anything, one and several chunks
     of classes (33000 x 2048), cut reductions of dE and of dC, rows gathered or taken as they lie, more rows than 32-bit
     offsets reach in one copy (two blocks of rows), a classifier with gaps between its rows."""
+    _check_fp32_passes(shape, terms, extra.get("softcap"), *_fp32_case(*shape, keep, 21, **extra))
+
+
+@pytest.mark.parametrize("shape,keep,extra,past", [
+    ((65, 257, 65), 1.0, {"softcap": 5.0}, "e"), ((300, 9001, 123), 0.7, {"bias": True, "d_lse": True}, "e"),
+    ((300, 9001, 123), 0.7, {"bias": True, "d_lse": True}, "c"), ((130, 600, 1000), 0.5, {"strided": True}, "c"),
+    ((40, 33000, 2048), 1.0, {"bias": True}, "last class"), ((40, 33000, 2048), 1.0, {"bias": True}, "e"),
+    ((6000, 300, 200), 0.9, {"d_lse": True, "softcap": 20.0}, "e"), ((1500, 1400, 96), 1.0, {"strided": True, "bias": True}, "c"),
+    ((176000, 70, 4096), 1.0, {}, "first row"), ((176000, 70, 4096), 1.0, {}, "last row"), ((180000, 70, 4096), 0.98, {}, "last row"),
+    ((30000, 5000, 64), 1.0, {"bias": True}, "e"),
+])
+@pytest.mark.parametrize("terms", [6, 3])
+def test_fp32_passes_abi_by_parts(shape, keep, extra, past, terms):
+    """The same with a value past what halves of fp16 hold, so that the logits go by bf16 parts as well: in E or in C, in the last of
+    several chunks of classes alone, in the first or the second block of rows alone."""
+    e, c, t, bias, w, h, rows, valids = _fp32_case(*shape, keep, 21, **extra)
+    if past in ("c", "last class"):
+        e[:, 0] *= 1e-2
+        c[-1, 0] = 16.5
+    else:
+        c[:, 0] *= 1e-2
+        e[rows[0] if past in ("e", "first row") else rows[-1], 0] = 300.0
+    _check_fp32_passes(shape, terms, extra.get("softcap"), e, c, t, bias, w, h, rows, valids)
+
+
+def _check_fp32_passes(shape, terms, cap, e, c, t, bias, w, h, rows, valids):
     lib = _lib()
     dev = torch.device("cuda:0")
     N, V, D = shape
-    e, c, t, bias, w, h, rows, valids = _fp32_case(N, V, D, keep, 21, **extra)
-    B, cap = rows.numel(), extra.get("softcap")
+    B = rows.numel()
     p = lambda x: x.data_ptr() if x is not None else None
     lse = torch.full((B,), float("nan"), device=dev)
     nll = torch.full((B,), float("nan"), device=dev)
@@ -328,7 +353,6 @@ def test_fp32_values_without_room_in_halves_go_by_parts(where, bias):
     dev = torch.device("cuda:0")
     N, V, D = (70, 45000, 2048) if where in ("e, two chunks", "early c", "late c") else (300, 700, 200)
     e, c, t, b, w, _, _, _ = _fp32_case(N, V, D, 1.0, 4, bias=bias)
-    inside = where in ("inside", "upstream", "nan")
     e[5, 3], c[:, 3] = (255.6 if where.startswith("e,") or where == "e" else 255.5), c[:, 3] * 1e-2
     c[0 if where == "early c" else V - 1, 2], e[:, 2] = (16.0 if where.endswith("c") else 15.96875), e[:, 2] * 1e-2
     if where == "upstream":
@@ -745,9 +769,10 @@ def test_a_row_that_is_not_a_number_says_so(dtype, softcap, rows, width):
 
 
 @pytest.mark.parametrize("shape", [(1, 700, 64), (300, 2000, 200), (3000, 100, 72)])
-def test_fp32_column_sums_keep_their_bits_with_three_terms(shape):
+@pytest.mark.parametrize("past", [False, True])
+def test_fp32_column_sums_keep_their_bits_with_three_terms(shape, past):
     """dBias is a sum of fp32 values and no product: with operands of 8 significant bits, whose logits three terms give
-    exactly, it is bit for bit what six terms give."""
+    exactly, it is bit for bit what six terms give; the logits from halves of fp16, or with a value past those from bf16 parts."""
     lib = _lib()
     N, V, D = shape
     g = torch.Generator(device="cuda").manual_seed(N)
@@ -755,6 +780,8 @@ def test_fp32_column_sums_keep_their_bits_with_three_terms(shape):
     c = (torch.randn((V, D), generator=g, device="cuda") / D**0.5).bfloat16().float()
     t = torch.randint(0, V, (N,), generator=g, device="cuda")
     w = torch.rand((N,), generator=g, device="cuda") + 0.5
+    if past:
+        e[0, 0], c[:, 0] = 320.0, c[:, 0] / 64
     lse = torch.logsumexp((e.double() @ c.double().T), 1).float()
     p = lambda x: x.data_ptr()
     sums = []
@@ -1158,11 +1185,12 @@ def test_more_candidates_than_slots_for_kept_gradients(monkeypatch, shape, likel
 
 
 @pytest.mark.parametrize("shape,likely", [((1, 4000, 128), 1), ((33, 20000, 72), 1), ((300, 30000, 2432), 2), ((130, 9000, 2056), 1),
-                                          ((90, 30000, 4736), 1), ((3200, 26000, 256), 4)])
+                                          ((90, 30000, 4736), 1), ((3200, 26000, 256), 4), ((64, 30000, 2056), 48)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gradients_kept_where_few_row_groups_are_dealt_out(monkeypatch, shape, likely, dtype):
     """Row groups dealt to 2 - 16 workgroups keep the gradients of what survives too, 40 slots for each workgroup, in one slice of D or
-    several; from 2048 columns on the light dC pass is in two slices, the last one partial (2056 = 1152 + 904); the last shape has row groups with more candidates than that.  Against the same call with a bias of zeros, as above."""
+    several; from 2048 columns on the light dC pass is in two slices, the last one partial (2056 = 1152 + 904); the last two shapes have row
+    groups with more candidates than that, one of them for the light pass in two slices.  Against the same call with a bias of zeros, as above."""
     from cut_cross_entropy import _hip
     from cut_cross_entropy import cce_backward as bw
     from cut_cross_entropy import linear_cross_entropy
@@ -1187,7 +1215,7 @@ def test_gradients_kept_where_few_row_groups_are_dealt_out(monkeypatch, shape, l
     lse, _, tile_max = loss_forward(e, c, None, t, None, 0, softcap, 0, True)
     low = torch.nn.functional.pad(lse, (0, groups * 32 - N), value=float("inf")).view(groups, 32).amin(1)
     candidates = (tile_max.view(groups, blocks) - low[:, None] >= torch.log(torch.tensor(eps)).item()).sum(1)
-    assert (candidates > quota).any() == (N == 3200)
+    assert (candidates > quota).any() == (N in (64, 3200))
 
     got = []
     for bias in (None, torch.zeros((V,), dtype=dtype, device="cuda", requires_grad=True)):

@@ -646,15 +646,19 @@ def test_fp32_mean_and_lse_and_shard(highest_matmul_precision):
     assert torch.allclose(one.cpu().double(), torch.logsumexp(logits, 1) - corr, atol=2e-5, rtol=0)
 
 
+@pytest.mark.parametrize("past", [False, True])
 @pytest.mark.parametrize("softcap", [None, 20.0])
-def test_fp32_inputs_under_fast_matmul_precision(softcap):
+def test_fp32_inputs_under_fast_matmul_precision(softcap, past):
     """``torch.set_float32_matmul_precision("high")`` asks for fast fp32 products (the reference then uses tf32, 10
-    mantissa bits): the logits are formed from three 16-bit terms instead of six and must still be far better than
-    tf32 would be -- 1e-4 on the per-token loss, 2e-3 on the gradients against the fp64 oracle."""
+    mantissa bits): products of bf16 parts -- of the gradients, and of the logits where a value has no room in halves of
+    fp16 -- are formed from three 16-bit terms instead of six and must still be far better than tf32 would be: 1e-4 on the per-token
+    loss, 2e-3 on the gradients against the fp64 oracle."""
     from cut_cross_entropy import fp32_path, linear_cross_entropy
     from oracle import dense_lce
 
     e, c, t, _ = make_inputs(512, 2000, 256, torch.float32, seed=14, invalid_frac=0.1)
+    if past:
+        e[0, 0], c[:, 0] = 300.0, c[:, 0] * 1e-3
     el = e.double().requires_grad_(True)
     cl = c.double().requires_grad_(True)
     want, _ = dense_lce.dense_linear_cross_entropy(el, cl, t, softcap=softcap, reduction="none")
