@@ -826,7 +826,7 @@ static DensePlan dense_plan(int64_t b, int64_t v, int64_t d, bool g16, int64_t m
 // The walk over the classes for a dz of `dz_bytes_per_class` and a copy of C of `c_bytes_per_class`, either at most
 // `most_bytes`, in chunks that are multiples of 256 classes; the reductions are cut as in cce_backward_dense.
 static TermsPlan terms_plan_uncached(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class,
-                                     int64_t c_bytes_per_class, int64_t most_bytes, bool cut_dc) {
+                                     int64_t c_bytes_per_class, int64_t most_bytes) {
   TermsPlan pl = {256, 1, 1};
   static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   const int64_t v_pad = (v + 255) / 256 * 256;
@@ -841,7 +841,7 @@ static TermsPlan terms_plan_uncached(int64_t b, int64_t v, int64_t d, int terms,
     for (int se : kSplits) {
       if (se > 1 && ((unit + 63) / 64 * terms < se * kMinSplitStages || se * b * d * 4 > most_bytes || unit / 64 < se)) break;
       for (int sc : kSplits) {
-        if (sc > 1 && (!cut_dc || (b + 63) / 64 * terms < sc * kMinSplitStages || sc * std::min(unit, v) * d * 4 > most_bytes ||
+        if (sc > 1 && ((b + 63) / 64 * terms < sc * kMinSplitStages || sc * std::min(unit, v) * d * 4 > most_bytes ||
                        b / 64 < sc))
           break;
         auto launch = [&](int64_t cls) {
@@ -863,11 +863,10 @@ static TermsPlan terms_plan_uncached(int64_t b, int64_t v, int64_t d, int terms,
 
 // (asked by the size query and again by the call, with every step of a training loop, like dense_plan: 7 - 50 us each)
 TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class, int64_t c_bytes_per_class,
-                     int64_t most_bytes, bool cut_dc) {
+                     int64_t most_bytes) {
   struct Memo {
     int64_t b, v, d, dz, c, most;
     int terms, cus;
-    bool cut_dc;
     TermsPlan answer;
   };
   constexpr int kMemos = 8;
@@ -877,11 +876,11 @@ TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_byte
   for (int i = 0; i < kMemos; ++i) {
     const Memo& m = memo[i];
     if (m.b == b && m.v == v && m.d == d && m.dz == dz_bytes_per_class && m.c == c_bytes_per_class && m.most == most_bytes &&
-        m.terms == terms && m.cus == cus && m.cut_dc == cut_dc)
+        m.terms == terms && m.cus == cus)
       return m.answer;
   }
-  const TermsPlan answer = terms_plan_uncached(b, v, d, terms, dz_bytes_per_class, c_bytes_per_class, most_bytes, cut_dc);
-  memo[next_slot] = {b, v, d, dz_bytes_per_class, c_bytes_per_class, most_bytes, terms, cus, cut_dc, answer};
+  const TermsPlan answer = terms_plan_uncached(b, v, d, terms, dz_bytes_per_class, c_bytes_per_class, most_bytes);
+  memo[next_slot] = {b, v, d, dz_bytes_per_class, c_bytes_per_class, most_bytes, terms, cus, answer};
   next_slot = (next_slot + 1) % kMemos;
   return answer;
 }

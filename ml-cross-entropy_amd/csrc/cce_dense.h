@@ -53,7 +53,7 @@ struct TermsPlan {
   int de_splits, dc_splits;
 };
 TermsPlan terms_plan(int64_t b, int64_t v, int64_t d, int terms, int64_t dz_bytes_per_class, int64_t c_bytes_per_class,
-                     int64_t most_bytes, bool cut_dc);
+                     int64_t most_bytes);
 
 // dE (+)= dz . C and dC (+)= dz^T . E of one chunk, fp32 results.  dz_parts as written by dz_terms_launch, c_parts and
 // e_parts with zero rows up to cls_pad and b_pad (multiples of 64).  Range s of a reduction (de_len classes, dc_len rows,

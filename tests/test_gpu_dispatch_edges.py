@@ -121,13 +121,13 @@ def _fp32_case(N, V, D, keep, seed, softcap=None, bias=False, d_lse=False, strid
     ((64, 256, 64), 1.0, {}), ((130, 600, 1000), 0.5, {"strided": True}), ((40, 33000, 2048), 1.0, {"bias": True}),
     ((6000, 300, 200), 0.9, {"d_lse": True, "softcap": 20.0}), ((1500, 1400, 96), 1.0, {"strided": True, "bias": True}),
     ((176000, 70, 4096), 1.0, {}), ((180000, 70, 4096), 0.98, {}),
-    ((30000, 5000, 64), 1.0, {"bias": True}),
+    ((30000, 5000, 64), 1.0, {"bias": True}), ((30000, 1500, 4096), 0.95, {"softcap": 10.0, "d_lse": True, "bias": True}),
 ])
 @pytest.mark.parametrize("terms", [6, 3])
 def test_fp32_passes_abi(shape, keep, extra, terms):
     """cce_fp32_forward / cce_fp32_backward against fp64: widths that are no multiple of anything, one and several chunks
     of classes (33000 x 2048), cut reductions of dE and of dC, rows gathered or taken as they lie, more rows than 32-bit
-    offsets reach in one copy (two blocks of rows), a classifier with gaps between its rows."""
+    offsets reach in one copy (blocks of rows: two forward, seven backward), a classifier with gaps between its rows."""
     _check_fp32_passes(shape, terms, extra.get("softcap"), *_fp32_case(*shape, keep, 21, **extra))
 
 
@@ -142,7 +142,7 @@ def test_fp32_passes_abi(shape, keep, extra, terms):
 @pytest.mark.parametrize("terms", [6, 3])
 def test_fp32_passes_abi_by_parts(shape, keep, extra, past, terms):
     """The same with a value past what halves of fp16 hold, so that the logits go by bf16 parts as well: in E or in C, in the last of
-    several chunks of classes alone, in the first or the second block of rows alone."""
+    several chunks of classes alone, in the first or the last block of rows alone."""
     e, c, t, bias, w, h, rows, valids = _fp32_case(*shape, keep, 21, **extra)
     if past in ("c", "last class"):
         e[:, 0] *= 1e-2
