@@ -368,16 +368,20 @@ int cce_loss_call(const void* e, const void* c, const void* bias, const int64_t*
                   int64_t shift, int64_t ignored, int64_t target_offset, float softcap, int reduction, int dtype, int terms, void* stream);
 
 /*
- * fp32 inputs.  The matrix cores multiply 16-bit numbers: every value is split into bf16 parts, x = hi + mid + lo, and a
- * product is taken as its leading cross terms (`terms`: 6, what is left is below 2^-24 relative; or 3 of two parts,
- * 16 bits), all in fp32 accumulators.  The reference gives this dtype to tl.dot (cut_cross_entropy/cce_lse_forward.py:81,
+ * fp32 inputs.  The matrix cores multiply 16-bit numbers.  For the products of the gradients every value is split into bf16 parts,
+ * x = hi + mid + lo, and a product is taken as its leading cross terms (`terms`: 6, what is left is below 2^-24 relative; or 3 of
+ * two parts, 16 bits), all in fp32 accumulators.  The logits, in either pass, are formed from two halves of fp16 (22 - 23 bits of a
+ * value, and no less than 2^-44 of e and 2^-48 of c) in three terms, whatever `terms` says; where a number in e is past 255.5 or one in c
+ * past 15.96875 in magnitude the device forms them from the parts and terms of the gradients instead: in the forward from the first chunk of
+ * classes on that has such a number, in the backward in the chunks that have one, and everywhere for one in e.  So how a row's logits are
+ * rounded may depend on other rows.  The reference gives this dtype to tl.dot (cut_cross_entropy/cce_lse_forward.py:81,
  * cce_backward.py:170-302).
  *
  * cce_fp32_forward: lse[b] and nll[b] as cce_loss_forward defines them; bias [v] float or NULL.
  * cce_fp32_backward: the unfiltered gradients, arguments as for cce_backward_dense: d_e [n_rows, d] is added to (row
  * stride ld_de), d_c [v, d] written (row stride ld_dc), d_bias [v] added to (sums of fp32 values whatever `terms` says).
  * Any alignment and width; stride_cd must be 1, else CCE_ERR_MISALIGNED.  `workspace` 256-byte aligned, of at least the
- * bytes that the size query names (copies of e and of a chunk of c in parts; dz of a chunk).
+ * bytes that the size query names (copies of e and of a chunk of c in halves or parts, in the backward both; dz of a chunk).
  */
 int64_t cce_fp32_forward_workspace_bytes(int64_t b, int64_t v, int64_t d, int terms);
 int cce_fp32_forward(const float* e, const float* c, const float* bias, const int32_t* valids, const int64_t* targets,

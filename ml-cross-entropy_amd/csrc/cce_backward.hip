@@ -1538,9 +1538,10 @@ static int64_t parts_bytes(int64_t b, int64_t v, int64_t d) {
   return parts > 1 ? part_bits_bytes(b, v, parts) + parts * ((b + 31) / 32 * 32) * d * 4 : 0;
 }
 static int64_t lists_bytes(int64_t b, int64_t v) { return kept_bits_bytes(b, v) + (1 + (v + 31) / 32) * 4; }
-// Slots per row group for the gradients of its candidates, 2 KB each: 40 (32 rows have a label each) where D is in slices.  Logits would be formed once per slice in either pass there: what is fetched for a
-// surviving sub-tile is 32 rows x D of C and of E twice or three times in the dE pass and as often in the dC pass, and once
-// less in the first and once in all in the second with its gradient kept.  Not with one slice and a workgroup for every row group: where D is narrow, the memory
+// Slots per row group for the gradients of its candidates, 2 KB each: 40 (32 rows have a label each) where D is in slices.  Logits
+// would be formed once per slice in either pass there: what is fetched for a surviving sub-tile is 32 rows x D of C and of E twice
+// or three times in the dE pass and as often in the dC pass, and once less in the first and once in all in the second with its
+// gradient kept.  Not with one slice and a workgroup for every row group: where D is narrow, the memory
 // of the loss path is the point (E [8192, 2304] x C [256000, 2304]: 9 MB, and 20 MB of slots).
 // E [65536, 3584] x C [152064, 3584], peaked: dE 6.9 -> 4.9 ms in two launches, dC 7.4 -> 2.9, forward and backward 62.8 -> 56.3, for 168 MB.
 // Few row groups, dealt to several workgroups: 40 for each of these, whatever the width (20 MB at most: 256 workgroups in all), so

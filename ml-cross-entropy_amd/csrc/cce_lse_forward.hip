@@ -765,7 +765,7 @@ static int launch_lse_forward(LseFwdParams& p, bool aligned, bool want_la, int64
   } while (0)
 #define CCE_LAUNCH_FWD16(GE, LA, TAIL, FEW, ROWS)                                                 \
   do {                                                                                            \
-    auto kern = lse_forward16_kernel<T, GE, LA, TAIL, FEW, ROWS>;                          \
+    auto kern = lse_forward16_kernel<T, GE, LA, TAIL, FEW, ROWS>;                                 \
     static LdsLimitOnce lds_limit;                                                                \
     const int bytes = (ROWS) != kFwdTile ? lds_mid : (FEW) ? lds_few : lds16 + ((LA) ? kF16ColsumBytes : 0); \
     err = lds_limit.set(kern, bytes);                                                             \

@@ -379,8 +379,9 @@ def cce_backward_kernel(
         assert counters.is_contiguous() and counters.device == dev
 
     if B > 0 and (de_sparse or dc_sparse):
-        # Gradients are kept from pass to pass (wide rows: 80 KB per 32 of them; few rows: 20 MB at most) by calls whose passes all go by one list of
-        # candidates, and not beside a dBias, which sums them in fp32: any other call does without the room for them.
+        # Gradients are kept from pass to pass (wide rows: 80 KB per 32 of them; few rows: 20 MB at most) by calls whose passes
+        # all go by one list of candidates, and not beside a dBias, which sums them in fp32: any other call does without the
+        # room for them.
         keeps = (tile_max is not None and vocab_ordering is None and filter_eps_or_none(filter_eps) > 0.0 and dc_sparse and want_dc
                  and not want_dbias and filter_c_grad and (filter_e_grad or not de_sparse))
         room = lib.cce_backward_keeping_workspace_bytes if keeps else lib.cce_backward_unkept_workspace_bytes
