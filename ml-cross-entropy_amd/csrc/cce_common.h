@@ -597,8 +597,9 @@ struct DmaLogitTile {
 //
 // SPREAD (blocks of 192 rows): the token fragments of the next step are held apart, so they can all be read at the start of the
 // first step, and after one more barrier the token half of the ring stage is free there: its loads then go out under the first
-// step and those of the class rows under the second, where all of them together came faster than a compute unit takes
-// them in.  Forward, us: 900 x 1000 x 50257 115 / 104, forward and unfiltered backward 400 / 380.  Blocks of 256 rows reach 1.95 PFLOP/s
+// step and those of the class rows under the second, and not all of them under the second.  Forward, us: 900 x 1000 x 50257 115 / 104,
+// forward and unfiltered backward 400 / 380; counters of that forward with soft-cap and bias: compute units busy 6.47e7 / 5.64e7 cycles,
+// their matrix pipes 37 / 43 % of these.  Blocks of 256 rows reach 1.95 PFLOP/s
 // instead of 1.60 so with operands of zeros ([8192, 2304] x [256000, 2304]), but under real ones, where power is the limit, 6.66 / 6.75
 // ms, and keep the older order.  So does the first stage of a tile, at whose start the waves may still be an epilogue apart.
 //
