@@ -279,7 +279,7 @@ struct DzRow {
 // to 15 8.09e-7 / 7.75e-7 / 8.00e-7, and with soft-cap 30 1.49e-6 / 1.73e-6 / 1.48e-6.  Six instructions per logit: nothing to be seen in
 // the time of [2046, 3072] x [32064, 3072].
 __device__ __forceinline__ float exp2_difference(float x2, float lse2) {
-  const float n = fmaxf(rintf(x2 - lse2), -256.0f);
+  const float n = __builtin_amdgcn_fmed3f(rintf(x2 - lse2), -256.0f, 256.0f);  // (rows past the end: lse2 = infinity, and 0)
   const float f = fmaf(n, kLog2Slack, x2 - (n + lse2));  // n + lse2: exact unless x2 is past lse2
   return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
 }
