@@ -414,7 +414,7 @@ def main():
         "fwd_bwd_frac_alg": f_alg / (ms_per_step * 1e-3) / 1e12 / peak,
         "fwd_bwd_frac_dense_equiv": f_dense / (ms_per_step * 1e-3) / 1e12 / peak,
         "roofline": {
-            "kernel": ("the fp32 forward (three-way bf16 split of e and c, lse_forward16_kernel per vocabulary chunk, merge)"
+            "kernel": ("the fp32 forward (split of e and c into halves of fp16, lse_terms_kernel per vocabulary chunk, merge)"
                        if args.dtype == "fp32" else
                        "lse_forward16_kernel (fused E.C^T + softcap + online log-sum-exp)")
                       + ", device events around its launches inside the timed steps",
